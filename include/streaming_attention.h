@@ -33,6 +33,8 @@
  *     src/streaming_attention/kernel.py:1065-1066), whatever `prescale_qk` the caller of the Python
  *     operator passed: their probabilities differ from the forward's by about |score| * 2^-9 (bf16) /
  *     2^-12 (fp16) relative, inside the 16-bit accuracy bar.  Forward and dQ scale in float32.
+ *   - float32 at D <= 128: every product is formed from three bfloat16 parts per operand, which hold all 24
+ *     significand bits, and summed in float32; a non-finite input element gives NaN wherever it is used.
  */
 #ifndef STREAMING_ATTENTION_H
 #define STREAMING_ATTENTION_H
@@ -101,8 +103,8 @@ int sa_bwd_dkdv(const void* q, const void* k, const void* v,
                 int dtype, void* stream);
 
 /* Whole backward on one stream; `delta` is a caller-provided [B,H,T] float32 workspace that holds
- * rowsum(O * dO) afterwards.  For float32 and for head dimensions 16 and 32 this is sa_bwd_delta +
- * sa_bwd_dkdv + sa_bwd_dq.  For float16 / bfloat16 at head dimensions 32, 64, 128 and 256 the dQ kernel
+ * rowsum(O * dO) afterwards.  For float32 at head dimension 256 and for 16-bit types at 16 this is
+ * sa_bwd_delta + sa_bwd_dkdv + sa_bwd_dq.  Everywhere else the dQ kernel
  * forms the row sums itself from the dO rows it holds anyway (it reads O once more and writes
  * `delta` for the dK/dV kernel, which runs after it), so the separate pass over O and dO -- the
  * reference's `_streaming_attn_bwd_precompute` launch, kernel.py:433-514 -- is not launched; the

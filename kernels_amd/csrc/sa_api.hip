@@ -180,9 +180,11 @@ int sa_bwd_dkdv(const void* q, const void* k, const void* v, const int32_t* lens
     return D == 256 ? launch_dkdv<E, 1>(p, D, (hipStream_t)stream) : launch_dkdv<E, 0>(p, D, (hipStream_t)stream); });
 }
 
-// The dQ kernels for the 16-bit types at head dimensions 64, 128 and 256 hold each query's dO row and form
-// delta = rowsum(O * dO) in their prologue; the separate pass over O and dO is then not launched.
-static bool delta_inside_dq(int D, int dtype) { return dtype != SA_DTYPE_F32 && Cfg<__bf16>::fwd2(D); }
+// Most dQ kernels hold each query's dO row and form delta = rowsum(O * dO) in their prologue; the separate pass
+// over O and dO is then launched only for 16-bit elements at head dimension 16 and float32 at 256.
+static bool delta_inside_dq(int D, int dtype) {
+  return dtype == SA_DTYPE_F32 ? Cfg<float>::split(D) : Cfg<__bf16>::fwd2(D);
+}
 
 // The launches behind sa_backward and sa_backward_static: delta, dK/dV, dQ -- or dQ (forming delta), dK/dV.
 static int backward_launches(const void* q, const void* k, const void* v, const int32_t* lens, int64_t lens_stride,

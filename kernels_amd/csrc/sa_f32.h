@@ -1,0 +1,608 @@
+// float32 kernels on the 16-bit matrix pipe, head dimensions 16 to 128.
+//
+// v_mfma_f32_32x32x2_f32 does 64 flop per cycle and SIMD, v_mfma_f32_32x32x16_bf16 1024.  A float32
+// number is exactly the sum of three bfloat16 numbers (24 = 8 + 8 + 8 significand bits, same exponent
+// range; each part is the rounded remainder of the ones before), so a float32 product is
+//   x*y = x1*y1 + (x1*y2 + x2*y1) + (x1*y3 + x2*y2 + x3*y1) + [x2*y3 + x3*y2 + x3*y3],
+// every term of which the bfloat16 instruction forms exactly and adds up in float32.  The bracket is
+// left out: it is below 2^-26 of |x*y|, a quarter of the 2^-24 to which float32 rounds a product (or a
+// running sum).  Six products at 16 times the rate take 6/16 of the matrix time, and the sums have fewer
+// roundings (16 contraction slots per instruction instead of 2).  Measured on problems of 200 to 4096
+// positions against float64: errors of O, dQ, dK, dV at or below those of the float32 instruction
+// kernels (see the comment at each kernel for times).  A non-finite input element makes the results that
+// depend on it NaN: its remainder is not a number.
+//
+// The parts of the resident operand are formed once per wave and stay in registers; those of the streamed
+// tiles are formed once per workgroup on the way into LDS, where each part is a bfloat16 tile of its own
+// (the swizzled layout and transposing reads of the 16-bit kernels apply unchanged).  Probabilities and dS
+// are split in registers.
+#pragma once
+#include "sa_common.h"
+
+namespace sa {
+
+// Three bfloat16 fragments that add up to eight float32 values.
+struct Split8 {
+  bf16x8 p[3];
+};
+// The parts of two values, packed: one conversion for both, widened again with one shift and one mask.
+SA_DEV void split2(float x0, float x1, uint32_t (&u)[3]) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  f32x2 r = {x0, x1};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    u[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+    r[0] -= __uint_as_float(u[k] << 16);
+    r[1] -= __uint_as_float(u[k] & 0xFFFF0000u);
+  }
+}
+// Elements 2*e and 2*e+1 of a fragment.
+SA_DEV void split_pair(Split8& s, int e, float x0, float x1) {
+  uint32_t u[3];
+  split2(x0, x1, u);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    u32x4 w = __builtin_bit_cast(u32x4, s.p[k]);
+    w[e] = u[k];
+    s.p[k] = __builtin_bit_cast(bf16x8, w);
+  }
+}
+SA_DEV Split8 split8(const float (&x)[8]) {
+  Split8 s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) split_pair(s, e, x[2 * e], x[2 * e + 1]);
+  return s;
+}
+// The six products, smallest first.
+SA_DEV void mma6(f32x16& acc, const Split8& a, const Split8& b) {
+  mma(acc, a.p[2], b.p[0]);
+  mma(acc, a.p[0], b.p[2]);
+  mma(acc, a.p[1], b.p[1]);
+  mma(acc, a.p[1], b.p[0]);
+  mma(acc, a.p[0], b.p[1]);
+  mma(acc, a.p[0], b.p[0]);
+}
+
+// One LDS tile of ROWS rows: three bfloat16 tiles, one per part.
+template <int D, int ROWS> struct SplitTile {
+  using G = TileGeom<__bf16, D>;
+  static constexpr int PLANE = ROWS * G::PITCH;   // elements
+  static constexpr int ELEMS = 3 * PLANE;
+};
+
+// Copy of a [ROWS][D] float32 tile through registers into a SplitTile, eight elements per thread and step.
+// Rows are clamped to last_row (the values are masked by the caller).
+template <int D, int ROWS, int NT> struct SplitStager {
+  using G = TileGeom<__bf16, D>;
+  static constexpr int CPR = D / 8, TOTAL = ROWS * CPR, N = (TOTAL + NT - 1) / NT;
+  f32x4 regs[N][2];
+
+  SA_DEV void load(const float* base, int64_t row_stride, int row0, int last_row, int tid) {
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int ch = tid + it * NT;
+      if (TOTAL % NT == 0 || ch < TOTAL) {
+        int gr = row0 + ch / CPR;
+        gr = gr < last_row ? gr : last_row;
+        const float* src = base + (int64_t)gr * row_stride + (ch % CPR) * 8;
+        regs[it][0] = *reinterpret_cast<const f32x4*>(src);
+        regs[it][1] = *reinterpret_cast<const f32x4*>(src + 4);
+      }
+    }
+  }
+  SA_DEV void store_step(__bf16* tile, int tid, int it) const {
+    const int ch = tid + it * NT;
+    if (TOTAL % NT == 0 || ch < TOTAL) {
+      const float x[8] = {regs[it][0][0], regs[it][0][1], regs[it][0][2], regs[it][0][3],
+                          regs[it][1][0], regs[it][1][1], regs[it][1][2], regs[it][1][3]};
+      const Split8 s = split8(x);
+      __bf16* dst = tile + G::off(ch / CPR, (ch % CPR) * 8);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * SplitTile<D, ROWS>::PLANE) = s.p[k];
+    }
+  }
+  SA_DEV void store(__bf16* tile, int tid) const {
+#pragma unroll
+    for (int it = 0; it < N; ++it) store_step(tile, tid, it);
+  }
+};
+
+// The split fragments of one float32 row (as a B operand), multiplied by sign.
+template <int D> SA_DEV void load_row_split(Split8 (&f)[D / 16], const float* row, int h, bool negative) {
+#pragma unroll
+  for (int g = 0; g < D / 16; ++g) {
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(row + g * 16 + h * 8);
+    const f32x4 hi = *reinterpret_cast<const f32x4*>(row + g * 16 + h * 8 + 4);
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = negative ? -lo[e] : lo[e], x[4 + e] = negative ? -hi[e] : hi[e];
+    f[g] = split8(x);
+  }
+}
+
+// acc[row r][col c] += sum_k tile[r][k] * B[k][c] for the 32 rows of a split tile.  side(g) is vector work placed
+// behind the matrix instructions of step g: a wave that has a SIMD to itself has nothing else to fill them with.
+struct NoSide {
+  SA_DEV void operator()(int) const {}
+};
+template <int D, int ROWS, typename Side = NoSide>
+SA_DEV void mma_rows_split(f32x16& acc, const __bf16* tile, const Split8 (&b)[D / 16], int lane, Side&& side = Side()) {
+  using G = TileGeom<__bf16, D>;
+  const int c = lane & 31, h = lane >> 5;
+  const __bf16* base = tile + c * G::PITCH;
+  const int sw = G::swz(c);
+  pipeline<D / 16, 1>(
+      [&](int g) {
+        Split8 a;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          a.p[k] = *reinterpret_cast<const bf16x8*>(base + k * SplitTile<D, ROWS>::PLANE + (((g * 2 + h) ^ sw) * 8));
+        return a;
+      },
+      [&](int g, const Split8& a) { mma6(acc, a, b[g]); side(g); });
+}
+
+// acc[m] += X^T * P for 16*NH rows of a split tile X, from row 16*half0; P is a C fragment, split by the caller (rows
+// 16*(half0 + j) and up in b[j]).  Step it = j * NM + m.
+template <int D, int ROWS, int NM, int NH, typename Side = NoSide>
+SA_DEV void mma_tr_split(f32x16 (&acc)[NM], const __bf16* X, const Split8 (&b)[NH], int lane, Side&& side = Side(),
+                         int half0 = 0) {
+  using G = TileGeom<__bf16, D>;
+  static_assert(NM == G::DB, "one accumulator per 32-wide block of the head dimension");
+  const int g16 = lane >> 4, j = lane & 15;
+  const int r_lo = 4 * (g16 >> 1) + (j >> 2);
+  const int col = (g16 & 1) * 16 + 4 * (j & 3);
+  pipeline<NH * NM, 1>(
+      [&](int it) {
+        const int half = half0 + it / NM, m = it % NM;
+        Split8 a;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const __bf16* p0 = X + k * SplitTile<D, ROWS>::PLANE + G::off(half * 16 + r_lo, m * 32 + col);
+          const __bf16* p1 = X + k * SplitTile<D, ROWS>::PLANE + G::off(half * 16 + 8 + r_lo, m * 32 + col);
+          s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS s16x4*)(p0));
+          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS s16x4*)(p1));
+          a.p[k] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+        return a;
+      },
+      [&](int it, const Split8& a) { mma6(acc[it % NM], a, b[it / NM]); side(it); });
+}
+// The split B operand of mma_tr_split from a whole C fragment.
+SA_DEV void split_c(Split8 (&b)[2], const f32x16& P) {
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) split_pair(b[i / 8], (i % 8) / 2, P[i], P[i + 1]);
+}
+
+// The windows of a wave's 32 queries, of one lane's query, and of the workgroup.
+struct QueryWindow {
+  int lo, hi;            // this lane's keys
+  int lo_max, hi_min;    // keys every query of the wave sees
+  int lo_min, hi_max;    // keys any query of the wave sees (empty for a wave of padding)
+  int lo_wg, hi_wg;      // keys any query of the workgroup sees
+  SA_DEV QueryWindow(int q0, int wave, int TQ, int qrow, int L, int C, int R, ChunkDiv cd) {
+    auto low = [&](int q) { const int x = div_by(q, cd); return (x > R ? x - R : 0) * C; };
+    auto high = [&](int q) { const int e = (div_by(q, cd) + 1) * C; return e < L ? e : L; };
+    auto valid = [&](int q) { return q < L ? q : L - 1; };   // rows past L mimic the last valid row
+    lo = low(valid(qrow)), hi = high(valid(qrow));
+    const int first = valid(q0 + wave * 32), last = valid(q0 + wave * 32 + 31);
+    lo_max = low(last), hi_min = high(first);
+    lo_min = low(first), hi_max = q0 + wave * 32 < L ? high(last) : 0;
+    lo_wg = low(q0), hi_wg = high(valid(q0 + TQ - 1));
+  }
+};
+
+// Forward.  One wave per 32 queries, tiles of 32 keys in NST stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
+// bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back: D=128 685 us with the float32 instruction, 425 here;
+// D=64 (ragged) 266 -> 153; D=32 147 -> 92; D=16 116 -> 73.
+template <int D, int NW, int NST>
+__global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p) {
+  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TILE = SplitTile<D, TK>::ELEMS;
+  constexpr float kRescaleGap = 8.0f;
+  constexpr float kSumLimit = 256.0f;
+
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  __bf16* smem = reinterpret_cast<__bf16*>(smem_raw);   // [stage][K|V][part][TK][PITCH]
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  int bh, qt;
+  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, growing_tiles(p.C, p.R, p.T, TQ));
+  const int hd = bh % p.H, b = bh / p.H;
+  const int T_ = p.T;
+  int L = T_;
+  if (p.lens) {
+    L = p.lens[(int64_t)b * p.lens_stride];
+    L = L < 0 ? 0 : (L > T_ ? T_ : L);
+  }
+  const int q0 = qt * TQ;
+  float* o_base = reinterpret_cast<float*>(p.o) + (int64_t)bh * T_ * D;
+  float* lse_base = p.lse ? p.lse + (int64_t)bh * T_ : nullptr;
+  const int q_end = q0 + TQ < T_ ? q0 + TQ : T_;
+  if (q0 >= L) {
+    zero_rows<float, D, NT>(o_base, q0, q_end, tid);
+    if (lse_base)
+      for (int r = q0 + tid; r < q_end; r += NT) lse_base[r] = 0.0f;
+    return;
+  }
+
+  const int qrow = q0 + wave * 32 + c;
+  const QueryWindow w(q0, wave, TQ, qrow, L, p.C, p.R, p.cdiv);
+  const int kt0 = w.lo_wg / TK, kt1 = (w.hi_wg + TK - 1) / TK;
+  // never exactly 0, so that a masked score of -inf stays -inf after scaling
+  const float sl2e = fmaxf(fabsf(p.scale_log2e), 1e-30f);
+
+  const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
+  const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
+  SplitStager<D, TK, NT> sk, sv;
+  sk.load(kbase, p.k_st, kt0 * TK, L - 1, tid);
+  sv.load(vbase, p.v_st, kt0 * TK, L - 1, tid);
+
+  Split8 qf[D / 16];
+  load_row_split<D>(qf, reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
+                            (int64_t)(qrow < L ? qrow : L - 1) * p.q_st, h, p.scale_log2e < 0.0f);
+
+  f32x16 oacc[DB];
+#pragma unroll
+  for (int m = 0; m < DB; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+
+  sk.store(smem, tid);
+  sv.store(smem + TILE, tid);
+  __syncthreads();
+
+  for (int t = kt0; t < kt1; ++t) {
+    const __bf16* Kt = smem + ((t - kt0) % NST) * 2 * TILE;
+    const __bf16* Vt = Kt + TILE;
+    const bool more = t + 1 < kt1;
+    if (more) {
+      sk.load(kbase, p.k_st, (t + 1) * TK, L - 1, tid);
+      sv.load(vbase, p.v_st, (t + 1) * TK, L - 1, tid);
+    }
+    const int k0 = t * TK;
+    if (k0 + TK > w.lo_min && k0 < w.hi_max) {   // some query of this wave sees the tile
+      f32x16 s;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+      mma_rows_split<D, TK>(s, Kt, qf, lane);
+      if (!(k0 >= w.lo_max && k0 + TK <= w.hi_min)) {
+        const uint32_t rm = row_mask(w.lo - k0, w.hi - k0, h);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = keep_or_neg_inf(s[i], keep_bits(rm, i));
+      }
+      // probabilities against the running maximum as it stands; it is searched for when their sum shows that
+      // it has been left behind, or when a lane has none yet (see fwd2_kernel)
+      f32x16 pr;
+      float rs0, rs1;
+      auto probabilities = [&](float m_use) {
+        rs0 = rs1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pr[i] = fast_exp2(__builtin_fmaf(s[i], sl2e, -m_use));
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) rs0 += pr[i], rs1 += pr[i + 1];
+      };
+      probabilities(m_run == -INFINITY ? 0.0f : m_run);
+      const bool behind = !(rs0 + rs1 <= kSumLimit) || m_run == -INFINITY;   // true for NaN too
+      if (__builtin_amdgcn_ballot_w64(behind) != 0) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) mx = fast_max3(mx, s[i], s[i + 1]);
+        mx = half_max(mx) * sl2e;
+        const bool move = mx > m_run + kRescaleGap;   // false for mx = -inf or NaN
+        if (__builtin_amdgcn_ballot_w64(move) != 0) {
+          const float alpha = move ? fast_exp2(m_run - mx) : 1.0f;
+          m_run = move ? mx : m_run;
+          l_run *= alpha;
+#pragma unroll
+          for (int m = 0; m < DB; ++m)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) oacc[m][i] *= alpha;
+          probabilities(m_run == -INFINITY ? 0.0f : m_run);
+        }
+      }
+      l_run += rs0 + rs1;
+      Split8 pb[2];
+      split_c(pb, pr);
+      mma_tr_split<D, TK>(oacc, Vt, pb, lane);   // O^T[d][q] += V^T P^T
+    }
+    if (more) {
+      if (NST == 1) __syncthreads();   // the only stage has no reader left
+      __bf16* nxt = smem + ((t + 1 - kt0) % NST) * 2 * TILE;
+      sk.store(nxt, tid);
+      sv.store(nxt + TILE, tid);
+    }
+    __syncthreads();
+  }
+
+  const float l_tot = half_sum(l_run);
+  const bool valid = qrow < L;
+  if (qrow < T_) {
+    const float inv = valid ? 1.0f / l_tot : 0.0f;
+    if (!valid) {
+#pragma unroll
+      for (int m = 0; m < DB; ++m)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
+    }
+    store_acc_T<float, D, DB>(o_base + (int64_t)qrow * D, oacc, inv, h);
+    if (lse_base && h == 0) lse_base[qrow] = valid ? m_run + __builtin_amdgcn_logf(l_tot) : 0.0f;
+  }
+}
+
+// dQ, one wave per 32 queries, tiles of 32 keys, two stages.  delta = rowsum(O * dO) is formed in the prologue (the
+// O row is read beside the dO row) and written for the dK/dV kernel that runs after this one, or read when the caller
+// has computed it (p.delta_out == null).  Same problem as above: D=128 1015 -> 650 us (one wave per SIMD: the parts of Q
+// and dO are 192 registers), D=64 380 -> 215; forming delta here saves a pass of 49 us over O and dO at D=128.
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(const BwdParams p) {
+  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TILE = SplitTile<D, TK>::ELEMS;
+
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  __bf16* smem = reinterpret_cast<__bf16*>(smem_raw);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  int bh, qt;
+  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, growing_tiles(p.C, p.R, p.T, TQ));
+  const int hd = bh % p.H, b = bh / p.H;
+  const int T_ = p.T;
+  int L = T_;
+  if (p.lens) {
+    L = p.lens[(int64_t)b * p.lens_stride];
+    L = L < 0 ? 0 : (L > T_ ? T_ : L);
+  }
+  const int q0 = qt * TQ;
+  float* dq_base = reinterpret_cast<float*>(p.dq) + (int64_t)bh * T_ * D;
+  const int q_end = q0 + TQ < T_ ? q0 + TQ : T_;
+  if (q0 >= L) {
+    zero_rows<float, D, NT>(dq_base, q0, q_end, tid);
+    if (p.delta_out)
+      for (int r = q0 + tid; r < q_end; r += NT) p.delta_out[(int64_t)bh * T_ + r] = 0.0f;
+    return;
+  }
+
+  const int qrow = q0 + wave * 32 + c;
+  const QueryWindow w(q0, wave, TQ, qrow, L, p.C, p.R, p.cdiv);
+  const int kt0 = w.lo_wg / TK, kt1 = (w.hi_wg + TK - 1) / TK;
+  const float sl2e = fabsf(p.scale_log2e);
+
+  const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
+  const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
+  SplitStager<D, TK, NT> sk, sv;
+  sk.load(kbase, p.k_st, kt0 * TK, L - 1, tid);
+  sv.load(vbase, p.v_st, kt0 * TK, L - 1, tid);
+
+  Split8 qf[NF], gf[NF];
+  const int qr = qrow < L ? qrow : L - 1;
+  const float lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qr] : INFINITY;   // rows past L: P = exp2(-inf) = 0
+  float delta_q;
+  {
+    const float* gp = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh +
+                      (int64_t)qr * p.do_st;
+    load_row_split<D>(qf, reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
+                              (int64_t)qr * p.q_st, h, p.scale_log2e < 0.0f);
+    load_row_split<D>(gf, gp, h, false);
+    if (p.delta_out) {
+      const float* op = reinterpret_cast<const float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh +
+                        (int64_t)qr * p.o_st;
+      float sum = 0.0f;
+#pragma unroll
+      for (int g = 0; g < 2 * NF; ++g) {   // this lane's half of the row, as in load_row_split
+        const int d = (g >> 1) * 16 + h * 8 + (g & 1) * 4;
+        const f32x4 o4 = *reinterpret_cast<const f32x4*>(op + d), g4 = *reinterpret_cast<const f32x4*>(gp + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(o4[e], g4[e], sum);
+      }
+      delta_q = half_sum(sum);
+      if (h == 0 && qrow < T_) p.delta_out[(int64_t)bh * T_ + qrow] = qrow < L ? delta_q : 0.0f;
+    } else {
+      delta_q = p.delta[(int64_t)bh * T_ + qr];
+    }
+  }
+
+  f32x16 acc[DB];
+#pragma unroll
+  for (int m = 0; m < DB; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+  sk.store(smem, tid);
+  sv.store(smem + TILE, tid);
+  __syncthreads();
+
+  for (int t = kt0; t < kt1; ++t) {
+    const __bf16* Kt = smem + ((t - kt0) & 1) * 2 * TILE;
+    const __bf16* Vt = Kt + TILE;
+    const bool more = t + 1 < kt1;
+    if (more) {
+      sk.load(kbase, p.k_st, (t + 1) * TK, L - 1, tid);
+      sv.load(vbase, p.v_st, (t + 1) * TK, L - 1, tid);
+    }
+    const int k0 = t * TK;
+    if (k0 + TK > w.lo_min && k0 < w.hi_max) {
+      f32x16 s, dp;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f, dp[i] = -delta_q;
+      mma_rows_split<D, TK>(s, Kt, qf, lane);
+      mma_rows_split<D, TK>(dp, Vt, gf, lane, [&](int g) {
+#pragma unroll
+        for (int i = g * 16 / NF; i < (g + 1) * 16 / NF; ++i) s[i] = fast_exp2(__builtin_fmaf(s[i], sl2e, -lse_q));
+      });
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] *= dp[i];   // dS
+      if (!(k0 >= w.lo_max && k0 + TK <= w.hi_min)) {
+        const uint32_t rm = row_mask(w.lo - k0, w.hi - k0, h);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = keep_or_zero(s[i], keep_bits(rm, i));
+      }
+      Split8 sb[2];
+      split_c(sb, s);
+      mma_tr_split<D, TK>(acc, Kt, sb, lane);   // dQ^T[d][q] += K^T dS^T
+    }
+    if (more) {
+      __bf16* nxt = smem + ((t + 1 - kt0) & 1) * 2 * TILE;
+      sk.store(nxt, tid);
+      sv.store(nxt + TILE, tid);
+    }
+    __syncthreads();
+  }
+
+  if (qrow < T_) {
+    if (qrow >= L) {
+#pragma unroll
+      for (int m = 0; m < DB; ++m)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+    }
+    store_acc_T<float, D, DB>(dq_base + (int64_t)qrow * D, acc, p.scale, h);
+  }
+}
+
+// dK and dV, one wave per 32 keys, tiles of 32 queries, two stages.  Four products per tile; the vector work sits behind
+// their matrix instructions (the exponentials and the parts of P behind dP, dS and its parts behind dV): from head
+// dimension 64 on a wave has its SIMD to itself.  Held to 256 registers for a second wave, D=64 spilled and measured
+// the same (335 us) or slower.  Same problem as above: D=128 1470 -> 835 us, D=64 495 -> 330.
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_kernel(const BwdParams p) {
+  constexpr int TKB = NW * 32, NT = NW * 64, TQ = 32, NF = D / 16, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TILE = SplitTile<D, TQ>::ELEMS;
+  constexpr int STAGE_BYTES = 2 * TILE * 2 + 2 * TQ * 4;   // [Q][dO][lse, delta]
+
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  int bh, kt, L;
+  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
+                  p.lens_stride, bh, kt, L);
+  const int hd = bh % p.H, b = bh / p.H;
+  const int T_ = p.T, C = p.C, R = p.R;
+  const int k0 = kt * TKB;
+  float* dk_base = reinterpret_cast<float*>(p.dk) + (int64_t)bh * T_ * D;
+  float* dv_base = reinterpret_cast<float*>(p.dv) + (int64_t)bh * T_ * D;
+  const int k_end = k0 + TKB < T_ ? k0 + TKB : T_;
+  if (k0 >= L) {
+    zero_rows<float, D, NT>(dk_base, k0, k_end, tid);
+    zero_rows<float, D, NT>(dv_base, k0, k_end, tid);
+    return;
+  }
+
+  // query window [qlo, qhi) of a key: its own chunk and the R chunks after it, below L
+  auto win_lo = [&](int key) { return div_by(key, p.cdiv) * C; };
+  auto win_hi = [&](int key) {
+    const int64_t e = ((int64_t)div_by(key, p.cdiv) + R + 1) * (int64_t)C;
+    return e < (int64_t)L ? (int)e : L;
+  };
+  auto valid = [&](int key) { return key < L ? key : L - 1; };   // keys past L mimic the last valid key
+  const int krow = k0 + wave * 32 + c;
+  const int qlo = win_lo(valid(krow)), qhi = win_hi(valid(krow));
+  const int wk_first = valid(k0 + wave * 32), wk_last = valid(k0 + wave * 32 + 31);
+  const int qhi_min = win_hi(wk_first), qlo_max = win_lo(wk_last);
+  const int qlo_min = win_lo(wk_first), qhi_max = k0 + wave * 32 < L ? win_hi(wk_last) : 0;
+  const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(valid(k0 + TKB - 1)) + TQ - 1) / TQ;
+  const float sl2e = fabsf(p.scale_log2e);
+
+  const float* qbase = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
+  const float* gbase = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
+  const float* row_base = (tid < TQ ? p.lse : p.delta) + (int64_t)bh * T_;
+  SplitStager<D, TQ, NT> sq, sg;
+  float r_row = 0.0f;   // threads [0, TQ) stage lse, [TQ, 2*TQ) delta
+  auto load_tile = [&](int t) {
+    sq.load(qbase, p.q_st, t * TQ, L - 1, tid);
+    sg.load(gbase, p.do_st, t * TQ, L - 1, tid);
+    if (tid < 2 * TQ) r_row = row_base[valid(t * TQ + tid % TQ)];
+  };
+  auto stage_ptr = [&](int t) { return smem_raw + ((t - qt0) & 1) * STAGE_BYTES; };
+  auto store_tile = [&](int t) {
+    __bf16* st = reinterpret_cast<__bf16*>(stage_ptr(t));
+    sq.store(st, tid);
+    sg.store(st + TILE, tid);
+    if (tid < 2 * TQ) reinterpret_cast<float*>(st + 2 * TILE)[tid] = r_row;
+  };
+  static_assert(2 * TQ <= NT, "one thread per staged row value");
+  load_tile(qt0);
+
+  Split8 kf[NF], vf[NF];
+  {
+    const int kr = valid(krow);
+    load_row_split<D>(kf, reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
+                              (int64_t)kr * p.k_st, h, p.scale_log2e < 0.0f);
+    load_row_split<D>(vf, reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
+                              (int64_t)kr * p.v_st, h, false);
+  }
+
+  f32x16 dk[DB], dv[DB];
+#pragma unroll
+  for (int m = 0; m < DB; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
+  store_tile(qt0);
+  __syncthreads();
+
+  for (int t = qt0; t < qt1; ++t) {
+    const __bf16* Qt = reinterpret_cast<const __bf16*>(stage_ptr(t));
+    const __bf16* Gt = Qt + TILE;
+    const float* rows = reinterpret_cast<const float*>(Qt + 2 * TILE);
+    const bool more = t + 1 < qt1;
+    if (more) load_tile(t + 1);
+    const int qs = t * TQ;
+    if (qs + TQ > qlo_min && qs < qhi_max) {
+      const bool interior = qs >= qlo_max && qs + TQ <= qhi_min;
+      const uint32_t rm = interior ? ~0u : row_mask(qlo - qs, qhi - qs, h);
+      f32x16 s, dp, lse_r;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(rows + 8 * g4 + 4 * h);
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(rows + TQ + 8 * g4 + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[4 * g4 + e] = 0.0f, dp[4 * g4 + e] = -d4[e], lse_r[4 * g4 + e] = l4[e];
+      }
+      Split8 pb[2], sb[2];
+      mma_rows_split<D, TQ>(s, Qt, kf, lane);                // S[q][key]
+      mma_rows_split<D, TQ>(dp, Gt, vf, lane, [&](int g) {   // dP[q][key] - delta[q]
+#pragma unroll
+        for (int i = g * 16 / NF; i < (g + 1) * 16 / NF; i += 2) {
+          s[i] = fast_exp2(__builtin_fmaf(s[i], sl2e, -lse_r[i]));
+          s[i + 1] = fast_exp2(__builtin_fmaf(s[i + 1], sl2e, -lse_r[i + 1]));
+          if (!interior) s[i] = keep_or_zero(s[i], keep_bits(rm, i)), s[i + 1] = keep_or_zero(s[i + 1], keep_bits(rm, i + 1));
+          split_pair(pb[i / 8], (i % 8) / 2, s[i], s[i + 1]);
+        }
+      });
+      mma_tr_split<D, TQ>(dv, Gt, pb, lane, [&](int it) {    // dV^T[d][key] += dO^T P
+#pragma unroll
+        for (int i = it * 8 / DB; i < (it + 1) * 8 / DB; i += 2) {
+          float a = s[i] * dp[i], e = s[i + 1] * dp[i + 1];
+          // a masked dP may hold anything (NaN included): P = 0 does not clear it
+          if (!interior) a = keep_or_zero(a, keep_bits(rm, i)), e = keep_or_zero(e, keep_bits(rm, i + 1));
+          split_pair(sb[i / 8], (i % 8) / 2, a, e);
+        }
+      });
+      mma_tr_split<D, TQ>(dk, Qt, sb, lane);                 // dK^T[d][key] += Q^T dS
+    }
+    if (more) store_tile(t + 1);
+    __syncthreads();
+  }
+
+  if (krow < T_) {
+    if (krow >= L) {
+#pragma unroll
+      for (int m = 0; m < DB; ++m)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
+    }
+    store_acc_T<float, D, DB>(dk_base + (int64_t)krow * D, dk, p.scale, h);
+    store_acc_T<float, D, DB>(dv_base + (int64_t)krow * D, dv, 1.0f, h);
+  }
+}
+
+}  // namespace sa

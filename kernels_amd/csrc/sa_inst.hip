@@ -4,6 +4,7 @@
 //   SA_DGROUP: 0 head dims 16..128, 1 head dim 256
 #include <mutex>
 #include "sa_launch.h"
+#include "sa_f32.h"
 #if SA_KIND == 0
 #include "sa_fwd.h"
 #ifndef SA_NO_ASM_KERNELS
@@ -118,6 +119,19 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
   }
 #endif
 }
+#if SA_DTYPE_ID == 0
+template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipStream_t st) {
+  constexpr size_t lds = (size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
+  auto kern = fwd_split_kernel<D, NW, NST>;
+  static PrepareState once;
+  if (int rc = prepare(kern, lds, once)) return rc;
+  p.n_tiles = (int)ceil_div(p.T, NW * 32);
+  const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
+#endif
 template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D)) {
@@ -132,6 +146,16 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
     } else {
       if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
       return fwd2_launch<D, C::NARROW_NW, false>(p, st);
+    }
+  } else if constexpr (C::split(D)) {
+    // Head dimension 128: eight waves share one workgroup's two 48 KiB stages, two waves per SIMD, once that makes a
+    // workgroup per CU; smaller grids run twice as many four-wave workgroups with one stage (B*H=24, T=1024: 34
+    // against 44 us; B*H=64, T=2048, 512 of the large ones: 91 against 82 us).
+    if constexpr (D == 128) {
+      if ((int64_t)p.B * p.H * ceil_div(p.T, 256) < 256) return fwd_split_launch<D, 4, 1>(p, st);
+      return fwd_split_launch<D, 8, 2>(p, st);
+    } else {
+      return fwd_split_launch<D, 4, 2>(p, st);
     }
   } else {
     constexpr int TQ = C::NW * 32;
@@ -212,6 +236,17 @@ template <int D> static int dq_d(BwdParams p, hipStream_t st) {
       if (launch_choice(D, p.C, p.R).dq == DQ_PIPELINED) return dq3_launch<D>(p, st);
     }
     return dq2_launch<D, C::NARROW_NW>(p, st);
+  } else if constexpr (C::split(D)) {
+    constexpr int NW = 4, TQ = NW * 32;
+    constexpr size_t lds = (size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
+    auto kern = dq_split_kernel<D, NW>;
+    static PrepareState once;
+    if (int rc = prepare(kern, lds, once)) return rc;
+    p.n_tiles = (int)ceil_div(p.T, TQ);
+    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
+    return (int)hipGetLastError();
   } else {
     if (p.delta_out) return SA_ERR_ARG;
     constexpr int TQ = C::NW * 32;
@@ -303,6 +338,17 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::DKDV2_NW * 64), lds, st, p);
+    return (int)hipGetLastError();
+  } else if constexpr (C::split(D)) {
+    constexpr int NW = 4, TKB = NW * 32;
+    constexpr size_t lds = (size_t)2 * (2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + 2 * 32 * sizeof(float));
+    auto kern = dkdv_split_f32_kernel<D, NW>;
+    static PrepareState once;
+    if (int rc = prepare(kern, lds, once)) return rc;
+    p.n_tiles = (int)ceil_div(p.T, TKB);
+    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
   } else {
     constexpr int TKB = C::NW * 32;

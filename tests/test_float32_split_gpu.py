@@ -1,0 +1,38 @@
+"""float32 kernels that form their products from bfloat16 parts (head dimensions 16 to 128): float32 accuracy at the edges of
+the 32-row tiles and of the 128- and 256-row workgroups, on ordinary, very large and very small magnitudes."""
+import pytest
+import torch
+
+from oracle import sa_oracle
+from tests.helpers import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+# (B*H, T): two rows; tile and workgroup edges; B*H*ceil(T/256) below and from 256 on (the two forward shapes at D=128)
+@pytest.mark.parametrize("B,H,T,C,R", [(1, 1, 2, 4, 1), (2, 3, 129, 32, 2), (2, 2, 257, 1000, 0), (1, 2, 415, 100, 1),
+                                      (8, 16, 260, 48, 2), (8, 32, 96, 10, 3)])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("gain", [1.0, 1e15, 1e-15])
+def test_float32_accuracy(B, H, T, C, R, D, gain):
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    q, k, v, d_o = (t.to(dev) for t in make_inputs(B, H, T, D, seed=71))
+    # scores and dP keep their size; the tensors cover thirty decades (bfloat16 has float32's exponents)
+    q, k, v, d_o = q * gain, k / gain, v * gain, d_o / gain
+    lens = torch.tensor([T - (b * 37) % max(T // 2, 1) for b in range(B)], dtype=torch.int32, device=dev)
+    qd, kd, vd = (t.clone().requires_grad_() for t in (q, k, v))
+    out, lse = streaming_attention(qd, kd, vd, lens, C, R, return_lse=True)
+    out.backward(d_o)
+    want = sa_oracle.windowed(q, k, v, lens, C, R, d_out=d_o, dtype=torch.float64)
+    # float32 rounds to 2^-24; a sum of n terms in any order is off by about sqrt(n) roundings, and the longest chain here
+    # (scores over D, sums over a window of up to 415 keys, delta over D) has fewer than 1024 terms in all: 32 roundings
+    bound = 32 * 2.0 ** -24
+    for name, got, ref in zip(("O", "LSE", "dQ", "dK", "dV"), (out, lse, qd.grad, kd.grad, vd.grad), want):
+        got = got.detach().double()
+        assert torch.isfinite(got).all(), name
+        rel = ((got - ref).norm() / ref.norm()).item()
+        assert rel <= bound, f"{name}: relative error {rel:.2e}"
+    for b in range(B):
+        assert not out[b, :, int(lens[b]):].any() and not qd.grad[b, :, int(lens[b]):].any()
