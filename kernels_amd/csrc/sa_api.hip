@@ -186,7 +186,7 @@ static bool delta_inside_dq(int D, int dtype) {
   return dtype == SA_DTYPE_F32 ? Cfg<float>::split(D) : Cfg<__bf16>::fwd2(D);
 }
 
-// The launches behind sa_backward and sa_backward_static: delta, dK/dV, dQ -- or dQ (forming delta), dK/dV.
+// The launches behind sa_backward and sa_backward_static: delta, dK/dV, dQ -- or dQ (forming delta), dK/dV -- or one for all.
 static int backward_launches(const void* q, const void* k, const void* v, const int32_t* lens, int64_t lens_stride,
                              const void* o, const void* d_o, const float* lse, float* delta, void* dq, void* dk,
                              void* dv, const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
@@ -198,10 +198,17 @@ static int backward_launches(const void* q, const void* k, const void* v, const 
     if (!dq || !dk || !dv || !delta) return SA_ERR_ARG;
     if (!aligned16(dq) || !aligned16(dk) || !aligned16(dv)) return SA_ERR_LAYOUT;
     if (int rc = check_layout(o, os, dtype, T, D)) return rc;
-    BwdParams probe{};
-    if (int rc = fill_bwd(probe, q, k, v, lens, lens_stride, d_o, lse, delta, qs, ks, vs, gs, B, H, T, D,
-                          context_size, back_contexts, sm_scale, dtype))
+    BwdParams p{};
+    if (int rc = fill_bwd(p, q, k, v, lens, lens_stride, d_o, lse, delta, qs, ks, vs, gs, B, H, T, D, context_size,
+                          back_contexts, sm_scale, dtype))
       return rc;
+    if (dtype != SA_DTYPE_F32 && fused_backward(D, p.C, p.R)) {
+      p.dq = dq; p.dk = dk; p.dv = dv;
+      p.o = o; p.o_sb = os[0]; p.o_sh = os[1]; p.o_st = os[2];
+      p.delta_out = delta;
+      return dtype == SA_DTYPE_F16 ? launch_bwd_fused<_Float16>(p, D, (hipStream_t)stream)
+                                   : launch_bwd_fused<__bf16>(p, D, (hipStream_t)stream);
+    }
   }
   if (delta_inside_dq(D, dtype) && B > 0 && H > 0 && T > 0) {
     if (int rc = run_dq(q, k, v, lens, lens_stride, d_o, lse, delta, dq, qs, ks, vs, gs, B, H, T, D, context_size,

@@ -404,13 +404,99 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 // asynchronous global->LDS copies into a ring of NST stages, one barrier per tile.
 // ---------------------------------------------------------------------------------------
 
+// The window of one lane's row (a query's keys, or a key's queries), of all rows of its wave and of any of them.
+struct WaveWindow {
+  int lo, hi;
+  int lo_max, hi_min;   // seen by every row of the wave
+  int lo_min, hi_max;   // seen by some row of the wave (empty for a wave of padding)
+};
+
+// -dQ^T += K^T (-dS^T) for the TK keys from k0 on: S, dP and dS of one 32-key block at a time, blocks outside the wave's
+// windows left out.  gf holds -dO and dinit delta, so that the dP accumulator ends at delta - dP.
+template <typename T, int D, int TK, int NF, int DB>
+SA_DEV void dq2_tile(f32x16 (&acc)[DB], const T* Kt, const T* Vt, int k0, const WaveWindow& win,
+                     const typename Elem<T>::Frag (&qf)[NF], const typename Elem<T>::Frag (&gf)[NF], float sl2e,
+                     float lse_q, const f32x16& dinit, int lane) {
+  const int h = lane >> 5;
+#pragma unroll
+  for (int kb = 0; kb < TK / 32; ++kb) {
+    const int kb0 = k0 + kb * 32;
+    if (kb0 + 32 <= win.lo_min || kb0 >= win.hi_max) continue;
+    const bool interior = (kb0 >= win.lo_max) && (kb0 + 32 <= win.hi_min);
+    f32x16 s[1], dp[1];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[0][i] = 0.0f;
+    dp[0] = dinit;
+    mma_rows_pair<T, D>(s[0], dp[0], Kt, Vt, kb * 32, qf, gf, lane);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float pr = fast_exp2(__builtin_fmaf(s[0][i], sl2e, -lse_q));
+      s[0][i] = pr * dp[0][i];   // = -dS
+    }
+    if (!interior) {
+      const uint32_t rm = row_mask(win.lo - kb0, win.hi - kb0, h);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[0][i] = keep_or_zero(s[0][i], keep_bits(rm, i));
+    }
+    mma_tr<T, D>(acc, Kt, kb, s[0], lane);   // -dQ^T[d][q] += K^T (-dS^T)
+  }
+}
+
+// dV^T += dO^T P and -dK^T += Q^T (-dS) for the TQ queries from qs on.  rows(r) gives the four lse and the four delta
+// values of the tile's rows r to r+3.  kf holds K * (-scale * log2 e), vf holds -V.
+template <typename T, int D, int TQ, int PG, int NF, int DB, typename Rows>
+SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T* Gt, int qs, const WaveWindow& win,
+                       const typename Elem<T>::Frag (&kf)[NF], const typename Elem<T>::Frag (&vf)[NF], Rows&& rows,
+                       int lane) {
+  const int h = lane >> 5;
+#pragma unroll
+  for (int qb = 0; qb < TQ / 32; ++qb) {
+    const int qb0 = qs + qb * 32;
+    if (qb0 + 32 <= win.lo_min || qb0 >= win.hi_max) continue;
+    const bool interior = (qb0 >= win.lo_max) && (qb0 + 32 <= win.hi_min);
+    f32x16 s[1], dp[1];
+    // lse / delta of the 16 rows this lane holds, fetched ahead of the products and read
+    // straight into the score and dP accumulators
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      f32x4 l4, d4;
+      rows(qb * 32 + 8 * g4 + 4 * h, l4, d4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[0][4 * g4 + e] = l4[e], dp[0][4 * g4 + e] = d4[e];
+    }
+    // S[q][key] = Q K^T and dP[q][key] = dO V^T
+    mma_rows_pair<T, D, NF, PG>(s[0], dp[0], Qt, Gt, qb * 32, kf, vf, lane);
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * g4 + e;
+        const float pr = fast_exp2(-s[0][i]);
+        s[0][i] = pr;
+        dp[0][i] = pr * dp[0][i];   // = -dS
+      }
+    }
+    if (!interior) {
+      const uint32_t rm = row_mask(win.lo - qb0, win.hi - qb0, h);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t keep = keep_bits(rm, i);
+        s[0][i] = keep_or_zero(s[0][i], keep);
+        dp[0][i] = keep_or_zero(dp[0][i], keep);
+      }
+    }
+    // dV^T[d][key] += dO^T P and -dK^T[d][key] += Q^T (-dS)
+    mma_tr_pair<T, D, DB, PG>(dv, dk, Gt, Qt, qb, s[0], dp[0], lane);
+  }
+}
+
 template <typename T, int D, int NW, int TK, int NST>
 __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ && (NST == 2 || NST == 3), "swizzled 16-bit tiles, 2 or 3 stages");
-  constexpr int TQ = NW * 32, NT = NW * 64, KBN = TK / 32;
+  constexpr int TQ = NW * 32, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TK * D, STAGE = 2 * TILE;
   using Loader = AsyncTile<T, D, TK, NW>;
@@ -457,6 +543,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   const bool wave_live = q0 + wave * 32 < L;
   const int lo_min = (cdiv(wq_first) > R ? cdiv(wq_first) - R : 0) * C;
   const int hi_max = !wave_live ? 0 : ((cdiv(wq_last) + 1) * C < L ? (cdiv(wq_last) + 1) * C : L);
+  const WaveWindow win{lo, hi, lo_max, hi_min, lo_min, hi_max};
   const int gq_last = q0 + TQ - 1 < L ? q0 + TQ - 1 : L - 1;
   const int lo_wg = (cdiv(q0) > R ? cdiv(q0) - R : 0) * C;
   const int hi_wg = (cdiv(gq_last) + 1) * C < L ? (cdiv(gq_last) + 1) * C : L;
@@ -539,31 +626,9 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
     const T* Kt = smem + ((t - kt0) % NST) * STAGE;
     const T* Vt = Kt + TILE;
     const int k0 = t * TK;
-    if (k0 + TK <= lo_min || k0 >= hi_max) continue;   // outside this wave's windows
+    if (k0 + TK <= win.lo_min || k0 >= win.hi_max) continue;   // outside this wave's windows
 
-#pragma unroll
-    for (int kb = 0; kb < KBN; ++kb) {
-      // the same two tests per 32-key block: short windows end inside a tile
-      const int kb0 = k0 + kb * 32;
-      if (kb0 + 32 <= lo_min || kb0 >= hi_max) continue;
-      const bool interior = (kb0 >= lo_max) && (kb0 + 32 <= hi_min);
-      f32x16 s[1], dp[1];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[0][i] = 0.0f;
-      dp[0] = dinit;
-      mma_rows_pair<T, D>(s[0], dp[0], Kt, Vt, kb * 32, qf, gf, lane);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pr = fast_exp2(__builtin_fmaf(s[0][i], sl2e, -lse_q));
-        s[0][i] = pr * dp[0][i];   // = -dS
-      }
-      if (!interior) {
-        const uint32_t rm = row_mask(lo - (k0 + kb * 32), hi - (k0 + kb * 32), h);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[0][i] = keep_or_zero(s[0][i], keep_bits(rm, i));
-      }
-      mma_tr<T, D>(acc, Kt, kb, s[0], lane);   // -dQ^T[d][q] += K^T (-dS^T)
-    }
+    dq2_tile<T, D, TK>(acc, Kt, Vt, k0, win, qf, gf, sl2e, lse_q, dinit, lane);
   }
 
   if (qrow >= L) {
@@ -592,7 +657,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ && (NST == 2 || NST == 3), "swizzled 16-bit tiles, 2 or 3 stages");
-  constexpr int TKB = NW * 32, NT = NW * 64, QBN = TQ / 32;
+  constexpr int TKB = NW * 32, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TQ * D;
   constexpr int RPW = TQ / NW;   // rows of lse / delta each wave stages
@@ -638,6 +703,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   // queries that can see any key of this wave; a wave whose keys are all padding has none
   const bool wave_live = k0 + wave * 32 < L;
   const int qlo_min = win_lo(wk_first), qhi_max = wave_live ? win_hi(wk_last) : 0;
+  const WaveWindow win{qlo, qhi, qlo_max, qhi_min, qlo_min, qhi_max};
   const int gk_last = k0 + TKB - 1 < L ? k0 + TKB - 1 : L - 1;
   const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(gk_last) + TQ - 1) / TQ;
 
@@ -706,50 +772,13 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
     const T* Gt = Qt + TILE;
     const float* ld_t = reinterpret_cast<const float*>(stage_ptr(t) + 2 * TILE * sizeof(T));
     const int qs = t * TQ;
-    if (qs + TQ <= qlo_min || qs >= qhi_max) continue;   // outside this wave's windows
+    if (qs + TQ <= win.lo_min || qs >= win.hi_max) continue;   // outside this wave's windows
 
-#pragma unroll
-    for (int qb = 0; qb < QBN; ++qb) {
-      // the same two tests per 32-query block: short windows end inside a tile
-      const int qb0 = qs + qb * 32;
-      if (qb0 + 32 <= qlo_min || qb0 >= qhi_max) continue;
-      const bool interior = (qb0 >= qlo_max) && (qb0 + 32 <= qhi_min);
-      f32x16 s[1], dp[1];
-      // lse / delta of the 16 rows this lane holds, fetched ahead of the products and read
-      // straight into the score and dP accumulators
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int r = qb * 32 + 8 * g4 + 4 * h;     // tile row of 4 consecutive C-fragment rows
-        const float* chunk = ld_t + (r / RPW) * 2 * RPW + (r % RPW);
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(chunk);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(chunk + RPW);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[0][4 * g4 + e] = l4[e], dp[0][4 * g4 + e] = d4[e];
-      }
-      // S[q][key] = Q K^T and dP[q][key] = dO V^T
-      mma_rows_pair<T, D, NF, PG>(s[0], dp[0], Qt, Gt, qb * 32, kf, vf, lane);
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 4 * g4 + e;
-          const float pr = fast_exp2(-s[0][i]);
-          s[0][i] = pr;
-          dp[0][i] = pr * dp[0][i];   // = -dS
-        }
-      }
-      if (!interior) {
-        const uint32_t rm = row_mask(qlo - (qs + qb * 32), qhi - (qs + qb * 32), h);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint32_t keep = keep_bits(rm, i);
-          s[0][i] = keep_or_zero(s[0][i], keep);
-          dp[0][i] = keep_or_zero(dp[0][i], keep);
-        }
-      }
-      // dV^T[d][key] += dO^T P and -dK^T[d][key] += Q^T (-dS)
-      mma_tr_pair<T, D, DB, PG>(dv, dk, Gt, Qt, qb, s[0], dp[0], lane);
-    }
+    dkdv2_tile<T, D, TQ, PG>(dk, dv, Qt, Gt, qs, win, kf, vf, [&](int r, f32x4& l4, f32x4& d4) {
+      const float* chunk = ld_t + (r / RPW) * 2 * RPW + (r % RPW);
+      l4 = *reinterpret_cast<const f32x4*>(chunk);
+      d4 = *reinterpret_cast<const f32x4*>(chunk + RPW);
+    }, lane);
   }
 
   if (krow >= L) {

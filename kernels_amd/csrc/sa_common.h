@@ -768,6 +768,7 @@ struct BwdParams {
   int64_t o_sb, o_sh, o_st;
   float* delta_out;
   ChunkDiv cdiv;      // division by C
+  int fused_rows;     // one-launch backward only: query rows whose lse and delta a workgroup keeps
 };
 
 struct DeltaParams {

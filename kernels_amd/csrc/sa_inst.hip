@@ -1,6 +1,6 @@
 // Kernel instantiations for one element type and one kernel family.
 // Compiled once per (SA_DTYPE_ID, SA_KIND) pair so that the families build in parallel.
-//   SA_DTYPE_ID: 0 fp32, 1 fp16, 2 bf16        SA_KIND: 0 forward, 1 delta + dQ, 2 dK/dV
+//   SA_DTYPE_ID: 0 fp32, 1 fp16, 2 bf16        SA_KIND: 0 forward, 1 delta + dQ, 2 dK/dV, 3 one-launch backward
 //   SA_DGROUP: 0 head dims 16..128, 1 head dim 256
 #include <mutex>
 #include "sa_launch.h"
@@ -17,6 +17,7 @@
 #include "sa_bwd4.h"
 #endif
 #include "sa_bwd_split.h"
+#include "sa_bwd_fused.h"
 #endif
 
 namespace sa {
@@ -266,7 +267,7 @@ template <> int launch_dq<ElemT, SA_DGROUP>(const BwdParams& p, int D, hipStream
   SA_FOR_EACH_D(X)
 #undef X
 }
-#else
+#elif SA_KIND == 2
 template <int D> static int dkdv3_launch(BwdParams p, hipStream_t st) {
 #ifdef SA_NO_ASM_KERNELS
   (void)p; (void)st;
@@ -379,6 +380,28 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
 }
 template <> int launch_dkdv<ElemT, SA_DGROUP>(const BwdParams& p, int D, hipStream_t st) {
 #define X(d) return dkdv_d<d>(p, st)
+  SA_FOR_EACH_D(X)
+#undef X
+}
+#else
+template <int D> static int bwd_fused_d(BwdParams p, hipStream_t st) {
+  if constexpr (fused_backward_exists<ElemT>(D)) {
+    p.fused_rows = fused_rows(p.C, p.R);
+    const size_t lds = BwdFused::lds_bytes<ElemT, D>(p.fused_rows);
+    auto kern = bwd_fused_kernel<ElemT, D>;
+    static PrepareState once;
+    if (int rc = prepare(kern, BwdFused::lds_bytes<ElemT, D>(BWD_FUSED_MAX_ROWS), once)) return rc;
+    p.n_tiles = (int)ceil_div(p.T, BwdFused::ROWS);
+    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(BwdFused::NW * 64), lds, st, p);
+    return (int)hipGetLastError();
+  } else {
+    return SA_ERR_HEAD_DIM;
+  }
+}
+template <> int launch_bwd_fused<ElemT>(const BwdParams& p, int D, hipStream_t st) {
+#define X(d) return bwd_fused_d<d>(p, st)
   SA_FOR_EACH_D(X)
 #undef X
 }

@@ -14,6 +14,7 @@ template <typename T, int DGROUP> int launch_fwd(const FwdParams& p, int D, hipS
 template <typename T, int DGROUP> int launch_delta(const DeltaParams& p, int D, hipStream_t st);
 template <typename T, int DGROUP> int launch_dq(const BwdParams& p, int D, hipStream_t st);
 template <typename T, int DGROUP> int launch_dkdv(const BwdParams& p, int D, hipStream_t st);
+template <typename T> int launch_bwd_fused(const BwdParams& p, int D, hipStream_t st);
 
 // tile sizes, shared between the launchers and sa_query()
 #ifndef SA_FWD2_QB
@@ -92,6 +93,32 @@ inline LaunchChoice launch_choice(int D, int chunk, int back) {
   if (!pipelined && c.dq == DQ_PIPELINED) c.dq = DQ_NARROW;
   if (!pipelined && c.fwd == FWD_PIPELINED) c.fwd = FWD_NARROW;
   return c;
+}
+
+// The one-launch backward (sa_bwd_fused.h), 16-bit elements.
+template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 32 || D == 64); }
+// Query rows that a workgroup of 128 rows goes through for dK and dV, in whole 64-row tiles: the most over all positions.
+constexpr int BWD_FUSED_MAX_ROWS = 320;
+inline int fused_rows(int chunk, int back) {
+  int period = chunk;   // the pattern repeats after chunk / gcd(chunk, 128) workgroups
+  while (period % 2 == 0 && period > chunk / 128) period /= 2;
+  int most = 0;
+  for (int i = 0; i < period; ++i) {
+    const int first = 128 * i / chunk * chunk / 64, last = ((128 * i + 127) / chunk + back + 1) * chunk;
+    most = (last + 63) / 64 - first > most ? (last + 63) / 64 - first : most;
+  }
+  return most * 64;
+}
+// Used while those rows are few: beyond its own 128 a workgroup reads and multiplies rows that belong to its neighbours.
+// Measured against the two launches (B=8, H=16, T=4096, D=64 and batches of the sizes in sa_bwd_fused.h), rows: gain --
+// 128: 1.27; 192: 1.27, 1.17; 256: 1.13; 320: 1.07, 1.01; 384: 0.94; 448: 0.91.  D=32 -- 192: 1.02, 1.05; 320: 0.98; 384: 0.91.
+inline bool fused_backward(int D, int chunk, int back) {
+  if (!fused_backward_exists<__bf16>(D)) return false;
+  // a pinned dQ or dK/dV variant asks for the launches of their own
+  if (g_tune_override[1].load(std::memory_order_relaxed) >= 0 || g_tune_override[2].load(std::memory_order_relaxed) >= 0)
+    return false;
+  if ((long long)chunk * ((long long)back + 1) > BWD_FUSED_MAX_ROWS) return false;
+  return fused_rows(chunk, back) <= (D == 64 ? BWD_FUSED_MAX_ROWS : 256);
 }
 
 template <typename T> struct Cfg {
