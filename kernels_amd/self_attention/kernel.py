@@ -7,51 +7,27 @@ positions ``t >= lens[b]`` are zero, as the reference's ``zeros_like`` leaves th
 """
 from __future__ import annotations
 
-from typing import Optional
-
 import torch
 import torch.nn.functional as F
 
-from streaming_attention import _lib
-from streaming_attention.ops import _dtype_id, _kernel_layout, _lens_args, _on_device, _stream, _validate_placement
+from streaming_attention._native import self_attention as _eager_call  # (the module registers the op)
+from streaming_attention.api import _takes_native_call
+from streaming_attention.ops import _validate_placement
 
 _HEAD_DIMS = (16, 32, 64, 128, 256)
 
 
-@torch.library.custom_op("alexdremov_flash_attention::forward", mutates_args=(), device_types=("cuda",))
-def attention_forward_adapter(
-    q: torch.Tensor,
-    k: torch.Tensor,
-    v: torch.Tensor,
-    lens: Optional[torch.Tensor],
-    sm_scale: float,
-    autotune: bool,
-    prescale: bool,
-) -> torch.Tensor:
+def _validate(q, k, v, lens):
+    """Called by the native implementation with arguments it cannot serve, to name the condition
+    (the same ones as src/self_attention/kernel.py:372-379)."""
     _validate_placement(q, k, v, lens)
     batch, heads, T, head_dim = q.shape
-    # same conditions as src/self_attention/kernel.py:372-379
     assert head_dim in _HEAD_DIMS
     assert head_dim == k.shape[-1] and head_dim == v.shape[-1]
     assert T == k.shape[-2] and T == v.shape[-2]
-    assert sm_scale is not None
     assert lens is None or (lens.dtype == torch.int32 and batch == len(lens) and lens.ndim == 1)
     assert q.dtype == k.dtype == v.dtype
-
-    lib = _lib.load()
-    O = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    if q.numel() == 0:
-        return O
-    qk, kk, vk = _kernel_layout(q), _kernel_layout(k), _kernel_layout(v)
-    lens_ptr, lens_stride = _lens_args(lens)
-    with _on_device(q.device):
-        rc = lib.sa_forward(
-            qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), lens_ptr, lens_stride, O.data_ptr(), None,
-            _lib.strides4(qk), _lib.strides4(kk), _lib.strides4(vk),
-            batch, heads, T, head_dim, max(T, 1), 0, float(sm_scale), _dtype_id(q.dtype), _stream(q.device),
-        )
-    _lib.check(rc, "sa_forward (self attention)")
-    return O
+    assert q.dtype in (torch.float32, torch.float16, torch.bfloat16), f"unsupported dtype {q.dtype}"
 
 
 @torch.library.register_fake("alexdremov_flash_attention::forward")
@@ -86,6 +62,8 @@ def self_attention_reference_naive(q, k, v, lens):
 def self_attention(q, k, v, lens, sm_scale=None, autotune=True, prescale=False):
     """Dense attention over the first ``lens[b]`` positions of every sequence (all of them when
     ``lens`` is None).  ``autotune`` and ``prescale`` are accepted for signature compatibility."""
+    if not torch.compiler.is_compiling() and _takes_native_call(q, k, v, lens):
+        return _eager_call(q, k, v, lens, sm_scale, autotune, prescale)
     if sm_scale is None:
         sm_scale = q.size(-1) ** -0.5
     return torch.ops.alexdremov_flash_attention.forward(q, k, v, lens, sm_scale, autotune, prescale)

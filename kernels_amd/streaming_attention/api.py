@@ -2,13 +2,14 @@
 from __future__ import annotations
 
 import contextlib
-import os
 import threading
 
 import torch
 import torch.nn.functional as F
 
 from . import ops  # noqa: F401  (registers the dispatcher ops)
+from ._native import env_asks_for_wrapper as _env_asks_for_wrapper
+from ._native import streaming_attention as _eager_call
 
 
 def streaming_attention_reference(q, k, v, context_size, back_contexts, lens, scale=None):
@@ -73,9 +74,18 @@ def _use_compiled_wrapper() -> bool:
     scoped = getattr(_call_path, "compiled", None)
     if scoped is not None:
         return scoped
-    if os.environ.get("STREAMING_ATTENTION_COMPILED") == "1":
-        return True
-    return os.environ.get("STREAMING_ATTENTION_EAGER") == "0"
+    return _env_asks_for_wrapper()
+
+
+_plain_types = (torch.Tensor, type(None))
+_torch_function_modes = torch._C._len_torch_function_stack
+
+
+def _takes_native_call(q, k, v, lens) -> bool:
+    """Plain tensors with no torch-function mode around go from Python to the dispatcher in one native call; subclasses,
+    proxies and modes need the Python op call, which they can intercept."""
+    return (type(q) is torch.Tensor and type(k) is torch.Tensor and type(v) is torch.Tensor
+            and type(lens) in _plain_types and not _torch_function_modes())
 
 
 def _compiled_forward():
@@ -125,6 +135,9 @@ def streaming_attention(
     AOTAutograd wrappers cost about 0.1 ms of host time per forward+backward, as much as all four
     kernels of a small problem take on the GPU.
     """
+    direct = torch.compiler.is_compiling() or not _use_compiled_wrapper()
+    if direct and not torch.compiler.is_compiling() and _takes_native_call(q, k, v, lens):
+        return _eager_call(q, k, v, lens, context_size, back_contexts, sm_scale, autotune, return_lse, prescale_qk, precision)
     if sm_scale is None:
         sm_scale = q.size(-1) ** -0.5
     args = dict(
@@ -132,7 +145,7 @@ def streaming_attention(
         sm_scale=sm_scale, autotune=autotune, return_lse=return_lse, prescale_qk=prescale_qk,
         precision=precision,
     )
-    if torch.compiler.is_compiling() or not _use_compiled_wrapper():
+    if direct:
         return _forward_op(**args)
     for t in (q, k, v):
         torch._dynamo.mark_static(t, 1)
