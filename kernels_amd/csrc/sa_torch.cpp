@@ -21,7 +21,6 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
-#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/library.h>
@@ -247,18 +246,18 @@ struct StreamingAttention : torch::autograd::Function<StreamingAttention> {
     ctx->saved_data["flags"] = (int64_t)(autotune ? 1 : 0) | (prescale_qk ? 2 : 0);
     ctx->saved_data["precision"] = std::move(precision);
     ctx->mark_non_differentiable({lse});
-    ctx->set_materialize_grads(false);   // the log-sum-exp never has a gradient: no zeros for it
+    ctx->set_materialize_grads(false);   // the log-sum-exp never has a gradient: no zeros for it; O's are made in backward
     return {o, lse};
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
     torch::autograd::variable_list out(11);
-    if (!grads[0].defined()) return out;
     const auto saved = ctx->get_saved_variables();
+    const Tensor d_o = grads[0].defined() ? grads[0] : at::zeros_like(saved[3]);
     const int64_t flags = ctx->saved_data["flags"].toInt();
     const std::string precision = ctx->saved_data["precision"].toStringRef();
     auto [dq, dk, dv] = backward_op().call(saved[0], saved[1], saved[2], saved[5].defined() ? OptTensor(saved[5]) : OptTensor(),
-                                           saved[3], saved[4], grads[0], ctx->saved_data["context_size"].toSymInt(),
+                                           saved[3], saved[4], d_o, ctx->saved_data["context_size"].toSymInt(),
                                            ctx->saved_data["back_contexts"].toSymInt(), ctx->saved_data["sm_scale"].toDouble(),
                                            (flags & 1) != 0, (flags & 2) != 0, precision);
     out[0] = std::move(dq), out[1] = std::move(dk), out[2] = std::move(dv);
@@ -273,9 +272,18 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
   return false;
 }
 
+bool has_tangent(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->_fw_grad(0).defined()) return true;
+  return false;
+}
+
 std::tuple<Tensor, Tensor> forward_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& lens,
                                             SymInt context_size, SymInt back_contexts, double sm_scale, bool autotune,
                                             bool return_lse, bool prescale_qk, c10::string_view precision) {
+  // a tangent must not be dropped in silence
+  TORCH_CHECK_NOT_IMPLEMENTED(!has_tangent({&q, &k, &v}),
+                              "alexdremov_streaming_attention::forward has no forward-mode derivative");
   if (!wants_grad({&q, &k, &v})) {
     at::AutoDispatchBelowADInplaceOrView below;
     return forward_op().call(q, k, v, lens, std::move(context_size), std::move(back_contexts), sm_scale, autotune, return_lse,
@@ -336,45 +344,81 @@ Tensor dense_gpu(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   return o;
 }
 using DenseOp = Tensor(const Tensor&, const Tensor&, const Tensor&, const OptTensor&, double, bool, bool);
+const c10::TypedOperatorHandle<DenseOp>& dense_op() {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("alexdremov_flash_attention::forward", "").typed<DenseOp>();
+  return op;
+}
+
+// Forward only: the result of inputs that require a gradient requires one too, and asking for it raises.
+struct DenseAttention : torch::autograd::Function<DenseAttention> {
+  static Tensor forward(torch::autograd::AutogradContext*, const Tensor& q, const Tensor& k, const Tensor& v,
+                        const OptTensor& lens, double sm_scale, bool autotune, bool prescale) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return dense_op().call(q, k, v, lens, sm_scale, autotune, prescale);
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext*, torch::autograd::variable_list) {
+    TORCH_CHECK(false, "Trying to backward through alexdremov_flash_attention.forward.default but no autograd formula was "
+                       "registered: dense attention is forward only");
+  }
+};
+Tensor dense_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& lens, double sm_scale,
+                      bool autotune, bool prescale) {
+  if (wants_grad({&q, &k, &v})) return DenseAttention::apply(q, k, v, lens, sm_scale, autotune, prescale);
+  at::AutoDispatchBelowADInplaceOrView below;
+  return dense_op().call(q, k, v, lens, sm_scale, autotune, prescale);
+}
 
 // ---- eager call path of the public functions ------------------------------------------------------------------------
 // Arguments come positionally and already complete from the Python functions, which keep their signatures and defaults.
-bool tensor_arg(PyObject* x, Tensor& t) {
-  if (!THPVariable_Check(x)) return false;
-  t = THPVariable_Unpack(x);
+// An argument that is not of the plain type (a flag given as an int, a scale as a tensor, a mistake) returns NotImplemented:
+// the Python functions then call the op itself, which converts or refuses it.
+bool tensor_args(PyObject* const* args, Tensor (&t)[4], bool& has_lens) {
+  has_lens = args[3] != Py_None;
+  for (int i = 0; i < (has_lens ? 4 : 3); ++i) {
+    if (!THPVariable_Check(args[i])) return false;
+    t[i] = THPVariable_Unpack(args[i]);
+  }
+  return t[0].dim() > 0;
+}
+bool int_arg(PyObject* x, int64_t& value) {
+  int overflow = 0;
+  if (!PyLong_CheckExact(x)) return false;
+  value = PyLong_AsLongLongAndOverflow(x, &overflow);
+  return overflow == 0;
+}
+bool scale_arg(PyObject* x, const Tensor& q, double& value) {
+  if (x != Py_None && !PyFloat_CheckExact(x)) return false;
+  value = x == Py_None ? 1.0 / std::sqrt((double)q.size(-1)) : PyFloat_AS_DOUBLE(x);
+  return true;
+}
+bool flag_args(PyObject* const* args, int n) {
+  for (int i = 0; i < n; ++i)
+    if (!PyBool_Check(args[i])) return false;
   return true;
 }
 
 // streaming_attention(q, k, v, lens, context_size, back_contexts, sm_scale or None, autotune, return_lse, prescale_qk, precision)
 PyObject* py_streaming_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Tensor q, k, v, lens;
-  const bool has_lens = n == 11 && args[3] != Py_None;
-  Py_ssize_t len = 0;
-  const char* precision = n == 11 ? PyUnicode_AsUTF8AndSize(args[10], &len) : nullptr;
-  if (n == 11 && !precision) return nullptr;
-  if (n != 11 || !tensor_arg(args[0], q) || !tensor_arg(args[1], k) || !tensor_arg(args[2], v) ||
-      (has_lens && !tensor_arg(args[3], lens))) {
-    PyErr_SetString(PyExc_TypeError, "streaming_attention: q, k, v and lens must be tensors");
-    return nullptr;
-  }
-  const long long context_size = PyLong_AsLongLong(args[4]), back_contexts = PyLong_AsLongLong(args[5]);
-  if (PyErr_Occurred()) return nullptr;
+  Tensor t[4];
+  bool has_lens;
+  int64_t context_size, back_contexts;
   double sm_scale;
-  if (args[6] == Py_None) {
-    sm_scale = 1.0 / std::sqrt((double)q.size(-1));
-  } else {
-    sm_scale = PyFloat_AsDouble(args[6]);
-    if (PyErr_Occurred()) return nullptr;
-  }
-  const bool autotune = PyObject_IsTrue(args[7]), return_lse = PyObject_IsTrue(args[8]), prescale = PyObject_IsTrue(args[9]);
+  if (n != 11 || !tensor_args(args, t, has_lens) || !int_arg(args[4], context_size) || !int_arg(args[5], back_contexts) ||
+      !scale_arg(args[6], t[0], sm_scale) || !flag_args(args + 7, 3) || !PyUnicode_CheckExact(args[10]))
+    Py_RETURN_NOTIMPLEMENTED;
+  Py_ssize_t len = 0;
+  const char* precision = PyUnicode_AsUTF8AndSize(args[10], &len);
+  if (!precision) return nullptr;
+  const bool autotune = args[7] == Py_True, return_lse = args[8] == Py_True, prescale = args[9] == Py_True;
   // the log-sum-exp is needed by the backward pass whenever a gradient is wanted
-  const bool need_lse = return_lse || q.requires_grad() || k.requires_grad() || v.requires_grad();
+  const bool need_lse = return_lse || t[0].requires_grad() || t[1].requires_grad() || t[2].requires_grad();
   std::tuple<Tensor, Tensor> r;
   {
     pybind11::gil_scoped_release no_gil;
-    r = forward_op().call(q, k, v, has_lens ? OptTensor(lens) : OptTensor(), context_size, back_contexts, sm_scale, autotune,
-                          need_lse, prescale, c10::string_view(precision, (size_t)len));
+    r = forward_op().call(t[0], t[1], t[2], has_lens ? OptTensor(t[3]) : OptTensor(), context_size, back_contexts, sm_scale,
+                          autotune, need_lse, prescale, c10::string_view(precision, (size_t)len));
   }
   PyObject* o = THPVariable_Wrap(std::get<0>(r));
   if (!return_lse || !o) return o;
@@ -385,27 +429,16 @@ PyObject* py_streaming_attention(PyObject*, PyObject* const* args, Py_ssize_t n)
 // self_attention(q, k, v, lens, sm_scale or None, autotune, prescale)
 PyObject* py_self_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  static const auto op =
-      c10::Dispatcher::singleton().findSchemaOrThrow("alexdremov_flash_attention::forward", "").typed<DenseOp>();
-  Tensor q, k, v, lens;
-  const bool has_lens = n == 7 && args[3] != Py_None;
-  if (n != 7 || !tensor_arg(args[0], q) || !tensor_arg(args[1], k) || !tensor_arg(args[2], v) ||
-      (has_lens && !tensor_arg(args[3], lens))) {
-    PyErr_SetString(PyExc_TypeError, "self_attention: q, k, v and lens must be tensors");
-    return nullptr;
-  }
+  Tensor t[4];
+  bool has_lens;
   double sm_scale;
-  if (args[4] == Py_None) {
-    sm_scale = 1.0 / std::sqrt((double)q.size(-1));
-  } else {
-    sm_scale = PyFloat_AsDouble(args[4]);
-    if (PyErr_Occurred()) return nullptr;
-  }
-  const bool autotune = PyObject_IsTrue(args[5]), prescale = PyObject_IsTrue(args[6]);
+  if (n != 7 || !tensor_args(args, t, has_lens) || !scale_arg(args[4], t[0], sm_scale) || !flag_args(args + 5, 2))
+    Py_RETURN_NOTIMPLEMENTED;
+  const bool autotune = args[5] == Py_True, prescale = args[6] == Py_True;
   Tensor o;
   {
     pybind11::gil_scoped_release no_gil;
-    o = op.call(q, k, v, has_lens ? OptTensor(lens) : OptTensor(), sm_scale, autotune, prescale);
+    o = dense_op().call(t[0], t[1], t[2], has_lens ? OptTensor(t[3]) : OptTensor(), sm_scale, autotune, prescale);
   }
   return THPVariable_Wrap(o);
   END_HANDLE_TH_ERRORS
@@ -452,7 +485,7 @@ TORCH_LIBRARY(alexdremov_flash_attention, m) {
 }
 TORCH_LIBRARY_IMPL(alexdremov_flash_attention, CUDA, m) { m.impl("forward", TORCH_FN(dense_gpu)); }
 TORCH_LIBRARY_IMPL(alexdremov_flash_attention, Autograd, m) {
-  m.impl("forward", torch::autograd::autogradNotImplementedFallback());   // forward only: differentiating raises
+  m.impl("forward", TORCH_FN(dense_autograd));
 }
 
 PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }

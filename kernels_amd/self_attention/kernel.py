@@ -63,7 +63,9 @@ def self_attention(q, k, v, lens, sm_scale=None, autotune=True, prescale=False):
     """Dense attention over the first ``lens[b]`` positions of every sequence (all of them when
     ``lens`` is None).  ``autotune`` and ``prescale`` are accepted for signature compatibility."""
     if not torch.compiler.is_compiling() and _takes_native_call(q, k, v, lens):
-        return _eager_call(q, k, v, lens, sm_scale, autotune, prescale)
+        result = _eager_call(q, k, v, lens, sm_scale, autotune, prescale)
+        if result is not NotImplemented:
+            return result
     if sm_scale is None:
         sm_scale = q.size(-1) ** -0.5
     return torch.ops.alexdremov_flash_attention.forward(q, k, v, lens, sm_scale, autotune, prescale)

@@ -137,7 +137,9 @@ def streaming_attention(
     """
     direct = torch.compiler.is_compiling() or not _use_compiled_wrapper()
     if direct and not torch.compiler.is_compiling() and _takes_native_call(q, k, v, lens):
-        return _eager_call(q, k, v, lens, context_size, back_contexts, sm_scale, autotune, return_lse, prescale_qk, precision)
+        result = _eager_call(q, k, v, lens, context_size, back_contexts, sm_scale, autotune, return_lse, prescale_qk, precision)
+        if result is not NotImplemented:
+            return result
     if sm_scale is None:
         sm_scale = q.size(-1) ** -0.5
     args = dict(
