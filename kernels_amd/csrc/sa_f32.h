@@ -9,8 +9,8 @@
 // running sum).  Six products at 16 times the rate take 6/16 of the matrix time, and the sums have fewer
 // roundings (16 contraction slots per instruction instead of 2).  Measured on problems of 200 to 4096
 // positions against float64: errors of O, dQ, dK, dV at or below those of the float32 instruction
-// kernels (see the comment at each kernel for times).  A non-finite input element makes the results that
-// depend on it NaN: its remainder is not a number.
+// kernels (see the comment at each kernel for times).  Elements beyond bfloat16's range, infinities among them,
+// take a path of their own (split2_wide).
 //
 // The parts of the resident operand are formed once per wave and stay in registers; those of the streamed
 // tiles are formed once per workgroup on the way into LDS, where each part is a bfloat16 tile of its own
@@ -48,10 +48,60 @@ SA_DEV void split_pair(Split8& s, int e, float x0, float x1) {
     s.p[k] = __builtin_bit_cast(bf16x8, w);
   }
 }
+// The same for input elements that may round to an infinite first part: the first part of a finite one is cut off
+// instead of rounded, and an infinity is (1, 0, infinity) with its sign, which the six products with another split
+// number take to what the number itself gives (x3 meets y1 only, so no remainder of y spoils the sign).
+SA_DEV void split2_wide(float x0, float x1, uint32_t (&u)[3]) {
+  uint32_t inf[2], cut[2];
+  float y[2] = {x0, x1};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const uint32_t bits = __float_as_uint(y[j]), mag = bits & 0x7FFFFFFFu;
+    inf[j] = mag == 0x7F800000u ? bits >> 16 : 0u;
+    cut[j] = mag >= 0x7F7F8000u && mag < 0x7F800000u ? bits >> 16 : 0u;
+    if (inf[j]) y[j] = __uint_as_float((bits & 0x80000000u) | 0x3F800000u);
+    if (cut[j]) y[j] = __uint_as_float(bits) - __uint_as_float(cut[j] << 16);
+  }
+  split2(y[0], y[1], u);
+  // a cut-off element is (cut, y1, y2): its y has 16 significand bits, so y3 is zero
+  const uint32_t m = (cut[0] ? 0x0000FFFFu : 0u) | (cut[1] ? 0xFFFF0000u : 0u);
+  u[2] = (u[1] & m) | (u[2] & ~m) | inf[0] | (inf[1] << 16);
+  u[1] = (u[0] & m) | (u[1] & ~m);
+  u[0] = (cut[0] | (cut[1] << 16)) | (u[0] & ~m);
+}
+// The largest magnitude among eight values and m; a NaN counts for nothing (and needs nothing).
+SA_DEV float magnitude8(const f32x4& lo, const f32x4& hi, float m) {
+  auto max3 = [](float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  };
+  return max3(max3(lo[0], lo[1], lo[2]), max3(lo[3], hi[0], hi[1]), max3(hi[2], hi[3], m));
+}
+// Whether some lane of the wave holds elements that need split2_wide, from their largest magnitude (it gives all others
+// the same parts, so the whole wave takes one way).
+SA_DEV bool any_wide(float m) {
+  return __builtin_expect(__builtin_amdgcn_ballot_w64(m >= __uint_as_float(0x7F7F8000u)) != 0, 0);
+}
 SA_DEV Split8 split8(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int e = 0; e < 4; ++e) split_pair(s, e, x[2 * e], x[2 * e + 1]);
+  return s;
+}
+SA_DEV Split8 split8_wide(const float (&x)[8]) {
+  Split8 s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    uint32_t u[3];
+    split2_wide(x[2 * e], x[2 * e + 1], u);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      u32x4 w = __builtin_bit_cast(u32x4, s.p[k]);
+      w[e] = u[k];
+      s.p[k] = __builtin_bit_cast(bf16x8, w);
+    }
+  }
   return s;
 }
 // The six products, smallest first.
@@ -91,35 +141,74 @@ template <int D, int ROWS, int NT> struct SplitStager {
       }
     }
   }
-  SA_DEV void store_step(__bf16* tile, int tid, int it) const {
-    const int ch = tid + it * NT;
-    if (TOTAL % NT == 0 || ch < TOTAL) {
-      const float x[8] = {regs[it][0][0], regs[it][0][1], regs[it][0][2], regs[it][0][3],
-                          regs[it][1][0], regs[it][1][1], regs[it][1][2], regs[it][1][3]};
-      const Split8 s = split8(x);
-      __bf16* dst = tile + G::off(ch / CPR, (ch % CPR) * 8);
+  SA_DEV float magnitude(float m) const {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * SplitTile<D, ROWS>::PLANE) = s.p[k];
+    for (int it = 0; it < N; ++it)
+      if (TOTAL % NT == 0 || (int)threadIdx.x + it * NT < TOTAL) m = magnitude8(regs[it][0], regs[it][1], m);
+    return m;
+  }
+  template <bool WIDE> SA_DEV void store(__bf16* tile, int tid) const {
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int ch = tid + it * NT;
+      if (TOTAL % NT == 0 || ch < TOTAL) {
+        const float x[8] = {regs[it][0][0], regs[it][0][1], regs[it][0][2], regs[it][0][3],
+                            regs[it][1][0], regs[it][1][1], regs[it][1][2], regs[it][1][3]};
+        __bf16* dst = tile + G::off(ch / CPR, (ch % CPR) * 8);
+        if constexpr (WIDE) {   // pair by pair, in few registers
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            uint32_t u[3];
+            split2_wide(x[2 * e], x[2 * e + 1], u);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) reinterpret_cast<uint32_t*>(dst + k * SplitTile<D, ROWS>::PLANE)[e] = u[k];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          const Split8 s = split8(x);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * SplitTile<D, ROWS>::PLANE) = s.p[k];
+        }
+      }
     }
   }
-  SA_DEV void store(__bf16* tile, int tid) const {
-#pragma unroll
-    for (int it = 0; it < N; ++it) store_step(tile, tid, it);
-  }
 };
-
-// The split fragments of one float32 row (as a B operand), multiplied by sign.
-template <int D> SA_DEV void load_row_split(Split8 (&f)[D / 16], const float* row, int h, bool negative) {
-#pragma unroll
-  for (int g = 0; g < D / 16; ++g) {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(row + g * 16 + h * 8);
-    const f32x4 hi = *reinterpret_cast<const f32x4*>(row + g * 16 + h * 8 + 4);
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = negative ? -lo[e] : lo[e], x[4 + e] = negative ? -hi[e] : hi[e];
-    f[g] = split8(x);
+// Two tiles, one check for both.
+template <typename S> SA_DEV void store_tiles(const S& a, __bf16* ta, const S& b, __bf16* tb, int tid) {
+  if (any_wide(b.magnitude(a.magnitude(0.0f)))) {
+    a.template store<true>(ta, tid);
+    b.template store<true>(tb, tid);
+  } else {
+    a.template store<false>(ta, tid);
+    b.template store<false>(tb, tid);
   }
 }
+
+// This lane's half of a float32 row, and its split fragments (as a B operand).  Loaded as a whole and checked once:
+// a check per fragment would wait for one load after the other (dQ of the problem below: 650 -> 770 us).
+template <int D> struct HalfRow {
+  f32x4 r[D / 8];
+  SA_DEV void load(const float* row, int h) {
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) r[i] = *reinterpret_cast<const f32x4*>(row + (i / 2) * 16 + h * 8 + (i % 2) * 4);
+  }
+  SA_DEV void split(Split8 (&f)[D / 16], bool negative) const {
+    float m = 0.0f;
+#pragma unroll
+    for (int g = 0; g < D / 16; ++g) m = magnitude8(r[2 * g], r[2 * g + 1], m);
+    auto all = [&](auto&& one) {
+#pragma unroll
+      for (int g = 0; g < D / 16; ++g) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = negative ? -r[2 * g + e / 4][e % 4] : r[2 * g + e / 4][e % 4];
+        f[g] = one(x);
+      }
+    };
+    if (any_wide(m)) all([](const float (&x)[8]) { return split8_wide(x); });
+    else all([](const float (&x)[8]) { return split8(x); });
+  }
+};
 
 // acc[row r][col c] += sum_k tile[r][k] * B[k][c] for the 32 rows of a split tile.  side(g) is vector work placed
 // behind the matrix instructions of step g: a wave that has a SIMD to itself has nothing else to fill them with.
@@ -243,8 +332,12 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
   sv.load(vbase, p.v_st, kt0 * TK, L - 1, tid);
 
   Split8 qf[D / 16];
-  load_row_split<D>(qf, reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
-                            (int64_t)(qrow < L ? qrow : L - 1) * p.q_st, h, p.scale_log2e < 0.0f);
+  {
+    HalfRow<D> qr;
+    qr.load(reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
+                (int64_t)(qrow < L ? qrow : L - 1) * p.q_st, h);
+    qr.split(qf, p.scale_log2e < 0.0f);
+  }
 
   f32x16 oacc[DB];
 #pragma unroll
@@ -253,8 +346,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
     for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
 
-  sk.store(smem, tid);
-  sv.store(smem + TILE, tid);
+  store_tiles(sk, smem, sv, smem + TILE, tid);
   __syncthreads();
 
   for (int t = kt0; t < kt1; ++t) {
@@ -314,8 +406,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
     if (more) {
       if (NST == 1) __syncthreads();   // the only stage has no reader left
       __bf16* nxt = smem + ((t + 1 - kt0) % NST) * 2 * TILE;
-      sk.store(nxt, tid);
-      sv.store(nxt + TILE, tid);
+      store_tiles(sk, nxt, sv, nxt + TILE, tid);
     }
     __syncthreads();
   }
@@ -388,20 +479,19 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
   {
     const float* gp = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh +
                       (int64_t)qr * p.do_st;
-    load_row_split<D>(qf, reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
-                              (int64_t)qr * p.q_st, h, p.scale_log2e < 0.0f);
-    load_row_split<D>(gf, gp, h, false);
+    HalfRow<D> q_row, g_row;
+    q_row.load(reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh + (int64_t)qr * p.q_st, h);
+    g_row.load(gp, h);
+    q_row.split(qf, p.scale_log2e < 0.0f);
+    g_row.split(gf, false);
     if (p.delta_out) {
-      const float* op = reinterpret_cast<const float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh +
-                        (int64_t)qr * p.o_st;
+      HalfRow<D> o_row;
+      o_row.load(reinterpret_cast<const float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh + (int64_t)qr * p.o_st, h);
       float sum = 0.0f;
 #pragma unroll
-      for (int g = 0; g < 2 * NF; ++g) {   // this lane's half of the row, as in load_row_split
-        const int d = (g >> 1) * 16 + h * 8 + (g & 1) * 4;
-        const f32x4 o4 = *reinterpret_cast<const f32x4*>(op + d), g4 = *reinterpret_cast<const f32x4*>(gp + d);
+      for (int i = 0; i < D / 8; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(o4[e], g4[e], sum);
-      }
+        for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(o_row.r[i][e], g_row.r[i][e], sum);
       delta_q = half_sum(sum);
       if (h == 0 && qrow < T_) p.delta_out[(int64_t)bh * T_ + qrow] = qrow < L ? delta_q : 0.0f;
     } else {
@@ -414,8 +504,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-  sk.store(smem, tid);
-  sv.store(smem + TILE, tid);
+  store_tiles(sk, smem, sv, smem + TILE, tid);
   __syncthreads();
 
   for (int t = kt0; t < kt1; ++t) {
@@ -449,8 +538,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     }
     if (more) {
       __bf16* nxt = smem + ((t + 1 - kt0) & 1) * 2 * TILE;
-      sk.store(nxt, tid);
-      sv.store(nxt + TILE, tid);
+      store_tiles(sk, nxt, sv, nxt + TILE, tid);
     }
     __syncthreads();
   }
@@ -525,8 +613,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
   auto stage_ptr = [&](int t) { return smem_raw + ((t - qt0) & 1) * STAGE_BYTES; };
   auto store_tile = [&](int t) {
     __bf16* st = reinterpret_cast<__bf16*>(stage_ptr(t));
-    sq.store(st, tid);
-    sg.store(st + TILE, tid);
+    store_tiles(sq, st, sg, st + TILE, tid);
     if (tid < 2 * TQ) reinterpret_cast<float*>(st + 2 * TILE)[tid] = r_row;
   };
   static_assert(2 * TQ <= NT, "one thread per staged row value");
@@ -535,10 +622,11 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
   Split8 kf[NF], vf[NF];
   {
     const int kr = valid(krow);
-    load_row_split<D>(kf, reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
-                              (int64_t)kr * p.k_st, h, p.scale_log2e < 0.0f);
-    load_row_split<D>(vf, reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
-                              (int64_t)kr * p.v_st, h, false);
+    HalfRow<D> k_row, v_row;
+    k_row.load(reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh + (int64_t)kr * p.k_st, h);
+    v_row.load(reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh + (int64_t)kr * p.v_st, h);
+    k_row.split(kf, p.scale_log2e < 0.0f);
+    v_row.split(vf, false);
   }
 
   f32x16 dk[DB], dv[DB];

@@ -36,3 +36,46 @@ def test_float32_accuracy(B, H, T, C, R, D, gain):
         assert rel <= bound, f"{name}: relative error {rel:.2e}"
     for b in range(B):
         assert not out[b, :, int(lens[b]):].any() and not qd.grad[b, :, int(lens[b]):].any()
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("B,H", [(1, 2), (8, 32)])   # both forward shapes at D=128
+def test_float32_range_ends(B, H, D):
+    """Infinities and finite values beyond bfloat16's largest give what float32 arithmetic gives, not NaN.  Chunks are
+    whole tiles, so that no masked key or query shares a tile with the planted values."""
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    T, C, R = 128, 32, 1
+    q, k, v, d_o = (t.to(dev) for t in make_inputs(B, H, T, D, seed=72))
+    lowest, inf = torch.finfo(torch.float32).min, float("inf")
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, :, 5, 0] = lowest             # score far below all others: the key has no weight
+    k[:, :, 70, 0] = -inf              # score -inf: no weight either, but 0 * inf in dQ
+    v[:, :, 33, 1], v[:, :, 34, 2] = inf, -inf
+    v[:, :, 100, 3] = lowest / 2 ** 10
+    v[:, :, 5, 4] = -lowest            # 0 * finite
+    qd, kd, vd = (t.clone().requires_grad_() for t in (q, k, v))
+    out = streaming_attention(qd, kd, vd, None, C, R)
+    want = sa_oracle.windowed(q, k, v, None, C, R, dtype=torch.float64)[0]
+    got = out.detach().double()
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and not torch.isnan(got).any()
+    assert torch.equal(got[torch.isinf(want)].sign(), want[torch.isinf(want)].sign())
+    fin = torch.isfinite(want)
+    # 32 roundings as above, relative to the largest term of the sum (position 100 dwarfs the others in element 3)
+    for d in range(D):
+        scale = want[..., d][fin[..., d]].abs().max()
+        assert ((got - want)[..., d][fin[..., d]].abs() <= 32 * 2.0 ** -24 * max(scale, 8.0)).all(), d
+
+    # an infinite dO reaches dV of every key its query sees, and no other element of dV
+    kd.data[:, :, 70, 0] = 0.0
+    vd.data.copy_(torch.where(torch.isinf(v), torch.zeros_like(v), v))
+    d_o[:, :, 40, 6] = inf
+    out = streaming_attention(qd, kd, vd, None, C, R)
+    dv = torch.autograd.grad(out, vd, d_o)[0]
+    bad = ~torch.isfinite(dv)
+    expect = torch.zeros_like(bad)
+    expect[:, :, :64, 6] = True
+    expect[:, :, 5, 6] = False         # its weight is zero: 0 * inf
+    assert torch.equal(torch.isinf(dv), expect) and torch.isnan(dv[:, :, 5, 6]).all()
+    assert torch.equal(bad.sum(), expect.sum() + B * H)
