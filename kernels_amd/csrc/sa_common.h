@@ -312,9 +312,27 @@ SA_DEV void mma_rows_n(f32x16 (&acc)[NQ][NB], const T* tile, int row0,
   static_assert(NF == G_::NF, "one register fragment per 2*VEC slice of the head dimension");
   constexpr int PITCH = G_::PITCH, VEC = Elem<T>::VEC;
   const int c = lane & 31, h = lane >> 5;
-  constexpr int N = NB * NF, G = N < 4 ? N : 4;
+  constexpr int GRP = D == 256 ? 2 : 4, N = NB * NF, G = N < GRP ? N : GRP;
   const T* base = tile + (row0 + c) * PITCH;
   const int sw = G_::swz(c);
+  if constexpr (D == 256) {
+    // Eight swizzled offsets serve all slices (those from 8 on lie 256 bytes further).  They are formed again for
+    // every block, one instruction each: kept across the loop they do not fit beside the accumulators.
+    uint32_t x = (uint32_t)(h ^ sw) * 16;
+    asm volatile("" : "+v"(x));
+    const SA_LDS char* row = (const SA_LDS char*)base;
+    pipeline<N, G>(
+        [&](int it) {
+          const int nb = it / NF, g = it % NF;
+          const SA_LDS char* p = row + (x ^ (uint32_t)((g & 7) * 32));
+          return *reinterpret_cast<const SA_LDS typename Elem<T>::Frag*>(p + (g >> 3) * 256 + nb * 32 * PITCH * 2);
+        },
+        [&](int it, const typename Elem<T>::Frag& a) {
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) mma(acc[q][it / NF], a, bf[q][it % NF]);
+        });
+    return;
+  }
   pipeline<N, G>(
       [&](int it) {
         const int nb = it / NF, g = it % NF;
@@ -396,7 +414,7 @@ SA_DEV void mma_tr_pair(f32x16 (&acc0)[NM], f32x16 (&acc1)[NM], const T* X0, con
 }
 
 // 16-bit only: acc[q][m] += X^T * B[q] for 32-row block rb of tile X, B[q] packed by pack_c.
-template <typename T, int D, int NQ, int NM, int GRP = 4>
+template <typename T, int D, int NQ, int NM, int GRP = (D == 256 ? 2 : 4)>
 SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename Elem<T>::Frag (&b)[NQ][2],
                      int lane) {
   using E = Elem<T>;
@@ -410,6 +428,25 @@ SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename E
   const int col = mb + 4 * (j & 3);
   const T* blk = X + rb * 32 * PITCH;
   constexpr int N = 2 * NM, G = N < GRP ? N : GRP;
+  if constexpr (D == 256) {   // offsets formed per block as in mma_rows_n; eight rows down flips chunk bit 1
+    uint32_t x = (uint32_t)(((col / 8) ^ G_::swz(r_lo)) * 16 + (col % 8) * 2);
+    asm volatile("" : "+v"(x));
+    const SA_LDS char* row = (const SA_LDS char*)(blk + r_lo * PITCH);
+    pipeline<N, G>(
+        [&](int it) {
+          const int half = it / NM, m = it % NM;
+          const SA_LDS char* p0 = row + (x ^ (uint32_t)((m & 3) * 64)) + (m >> 2) * 256 + half * 16 * PITCH * 2;
+          const SA_LDS char* p1 = row + (x ^ (uint32_t)((m & 3) * 64 + 32)) + (m >> 2) * 256 + (half * 16 + 8) * PITCH * 2;
+          s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS s16x4*)(p0));
+          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS s16x4*)(p1));
+          return __builtin_bit_cast(Frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        },
+        [&](int it, const Frag& a) {
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) mma(acc[q][it % NM], a, b[q][it / NM]);
+        });
+    return;
+  }
   pipeline<N, G>(
       [&](int it) {
         const int half = it / NM, m = it % NM;
@@ -453,8 +490,9 @@ template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct A
   // the last valid one come back as zeros from the hardware's range check.
   // With ASM_COPIES the copies are written as assembly: the compiler cannot tell which LDS reads a
   // copy may overlap, so for copies it knows about it waits for ALL of them (vmcnt 0) before the
-  // first transposing LDS read that follows and before every barrier.  A ring of two stages loses
-  // nothing by that (measured), a ring of three would lose its point.  Completion is the caller's
+  // first transposing LDS read that follows and before every barrier.  A ring of two stages of 64 rows loses
+  // nothing by that (head dimension 64, forward: 121 us, 127 as assembly), the 32-row tiles of head dimension 256
+  // a little (114 against 110 us), a ring of three would lose its point.  Completion is the caller's
   // business either way (wait_loads + barrier).
   u32x4 rsrc;                      // descriptor words for the assembly form
   __amdgpu_buffer_rsrc_t brsrc;    // the same descriptor for the builtin

@@ -209,7 +209,12 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
   }
 }
 
-// Forward kernel for 16-bit elements with swizzled tiles (D = 64, 128 or 256; at 256 only with 4 waves, one per SIMD, which then has all 512 registers).
+// Forward kernel for 16-bit elements with swizzled tiles (D = 32, 64, 128 or 256).
+//
+// Head dimension 256 takes tiles of 32 keys: one score block and 64 KiB of LDS leave room for two waves per SIMD, one
+// of which multiplies while the other one is at its exponentials.  With tiles of 64 keys a wave needed more than 256
+// registers and had its SIMD to itself.  B=4, H=16, T=4096, bfloat16: chunks of 128, 4 back 277 -> 221 us (728 TFLOP/s),
+// chunks of 10, 9 back 157 -> 111, one chunk of 4096 1331 -> 899 (1223 TFLOP/s); B*H=16, T=600 19.0 -> 16.5 us.
 //
 // Same algorithm as fwd_kernel, different resource balance: each wave owns QB blocks of 32
 // queries, so every K / V fragment fetched from LDS feeds QB MFMAs (the transposing V reads
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
 // to the search for its maximum.  Long windows run the plain form, whose loop is a few per cent
 // tighter (fewer registers, no per-block tests).
 template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT>
-__global__ __launch_bounds__(NW * 64) void fwd2_kernel(const FwdParams p) {
+__global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const FwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(NW * 64) void fwd2_kernel(const FwdParams p) {
   constexpr int STAGE = 2 * TILE;
   constexpr float kRescaleGap = 8.0f;
   constexpr float kSumLimit = 256.0f;
-  using Loader = AsyncTile<T, D, TK, NW>;
+  using Loader = AsyncTile<T, D, TK, NW, (D == 256)>;
   constexpr int LPT = 2 * Loader::PER_WAVE;   // async loads per wave per stage (K and V)
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];

@@ -83,10 +83,10 @@ template <int D, int NW, bool SHORT> static int fwd2_launch(FwdParams p, hipStre
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * C::FWD2_QB * 32;
   // tile stages; the epilogue's row patches (one per wave) reuse the same memory
-  constexpr size_t stages = (size_t)C::FWD2_NST * 2 * C::FWD_TK * D * sizeof(ElemT);
+  constexpr size_t stages = (size_t)C::FWD2_NST * 2 * C::fwd2_tk(D) * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
-  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, C::FWD_TK, C::FWD2_NST, SHORT>;
+  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, C::fwd2_tk(D), C::FWD2_NST, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
@@ -140,14 +140,8 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
       if (launch_choice(D, p.C, p.R).fwd == FWD_PIPELINED) return fwd3_launch<D>(p, st);
     }
     // windows of less than 1024 keys (the table's first two window classes) run the short-window form
-    // head dimension 256 exists in the 4-wave shape only: a wave then has all 512 registers of its SIMD lane
-    if constexpr (D > 128) {
-      if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
-      return fwd2_launch<D, C::NARROW_NW, false>(p, st);
-    } else {
-      if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
-      return fwd2_launch<D, C::NARROW_NW, false>(p, st);
-    }
+    if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
+    return fwd2_launch<D, C::NARROW_NW, false>(p, st);
   } else if constexpr (C::split(D)) {
     // Head dimension 128: eight waves share one workgroup's two 48 KiB stages, two waves per SIMD, once that makes a
     // workgroup per CU; smaller grids run twice as many four-wave workgroups with one stage (B*H=24, T=1024: 34

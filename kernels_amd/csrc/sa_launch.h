@@ -79,7 +79,7 @@ constexpr bool kAsmKernels = false;
 constexpr bool kAsmKernels = true;
 #endif
 inline LaunchChoice launch_choice(int D, int chunk, int back) {
-  // head dimension 256 has one shape per kernel: anything wider or deeper does not fit registers or LDS
+  // head dimension 256 has one shape per kernel
   if (D == 256) return LaunchChoice{FWD_NARROW, DQ_NARROW, DKDV_BLOCKSKIP};
   LaunchChoice c = (D == 128 ? TUNE_D128 : TUNE_D64)[chunk_class(chunk)][window_class(chunk, back)];
   const int o0 = g_tune_override[0].load(std::memory_order_relaxed);
@@ -147,6 +147,8 @@ template <typename T> struct Cfg {
 #else
   static constexpr int FWD_TK = sizeof(T) == 4 ? 32 : 64;        // keys per forward step
 #endif
+  // keys per step of fwd2_kernel: at 256 a block of 32 is what fits beside the accumulators of two waves per SIMD
+  static constexpr int fwd2_tk(int D) { return D == 256 ? 32 : FWD_TK; }
   static constexpr int DQ_TK = 32;                               // keys per dQ step
   static constexpr int DKDV_TQ = 32;                             // queries per dK/dV step
 };
