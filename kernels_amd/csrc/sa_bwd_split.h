@@ -1,5 +1,5 @@
 // dK/dV kernel whose four matrix products are split between two waves, for 16-bit elements with
-// swizzled tiles (D = 64 or 128).
+// swizzled tiles (D = 64 or 128; a form of its own for 256 at the end).
 //
 // dkdv2_kernel and dkdv3_kernel give one wave 32 keys and all four products of a block step
 // (S, dP, dV, dK): two 32 x D accumulators and the K and V fragments make more than 256
@@ -25,6 +25,15 @@
 #include "sa_common.h"
 
 namespace sa {
+
+// Shape and LDS layout of dkdv_split_wide_kernel: rings of NQ Q tiles and NG dO tiles, lse and delta rows beside the Q
+// tiles, and per pair two exchange slots of 16 floats per lane.
+template <typename T, int D> struct DkdvSplitWide {
+  static constexpr int NP = 4, TKB = NP * 32, TQ = 32, NQ = 4, NG = 3, XSLOT = 64 * 16;
+  static constexpr size_t rings = (size_t)(NQ + NG) * TQ * D * sizeof(T) + (NQ * 2 * TQ + NP * 2 * XSLOT) * sizeof(float);
+  static constexpr size_t patches = (size_t)2 * NP * RowPatch<T, D>::ELEMS * sizeof(T);
+  static constexpr size_t lds = rings > patches ? rings : patches;
+};
 
 template <typename T, int D, int NST>
 __global__ __launch_bounds__(512) void dkdv_split_kernel(const BwdParams p) {
@@ -311,6 +320,203 @@ __global__ __launch_bounds__(512) void dkdv_split_kernel(const BwdParams p) {
     if (!grad_role) store_rows_coalesced<T, D, DB>(patch, dv_base + (int64_t)row0 * D, T_ - row0, acc[0], 1.0f, lane);
     else store_rows_coalesced<T, D, DB>(patch, dk_base + (int64_t)row0 * D, T_ - row0, acc[0], -p.scale, lane);
   }
+}
+
+// The same division of labour at head dimension 256.  dkdv2_kernel holds two 32 x 256 accumulators and the K and V
+// fragments there, 400 registers, with one wave per SIMD whose products wait for its exponentials and LDS reads; a wave
+// of a pair holds half of that and two fit.  Query tiles have 32 rows, one block step each.  A Q tile is read in two
+// steps (the grad role's dK product comes one step late), a dO tile in one: rings of four and of three, two tiles ahead
+// of the compute.  P crosses in float32, 16 values per lane, so that dS has the precision that one wave would give it.
+// Bound by the LDS reads (1 KiB per matrix instruction, half of them 8-byte transposing reads); fragments requested four
+// ahead instead of two spill and measured 2 % slower.  Whole backward, B=4, H=16, T=4096, bfloat16: chunks of 128, 4 back
+// 755 -> 726 us; of 32, 1 back 401 -> 382; one chunk of 4096 3627 -> 3470; B*H=8, T=2048, chunks of 256, 6 back 184 -> 171.
+template <typename T, int D>
+__global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p) {
+  using E = Elem<T>;
+  using G = TileGeom<T, D>;
+  using Frag = typename E::Frag;
+  using S = DkdvSplitWide<T, D>;
+  static_assert(G::SWZ && D == 256, "swizzled 16-bit tiles; the LDS offsets of mma_rows_n and mma_tr_n for 256");
+  constexpr int NP = S::NP, NW = 2 * NP, TQ = S::TQ, TKB = S::TKB, NT = NW * 64;
+  constexpr int NF = G::NF, DB = G::DB, TILE = TQ * D, NQ = S::NQ, NG = S::NG;
+  constexpr int RPW = TQ / NW;   // rows of lse / delta each wave stages
+  static_assert(RPW % 4 == 0 && 2 * RPW <= 64, "lse/delta staging: one instruction per wave");
+  static_assert(NQ == 4 && NG == 3, "two tiles ahead: see issue_tile");
+  using Loader = AsyncTile<T, D, TQ, NW, true>;
+  constexpr int LPT = 2 * Loader::PER_WAVE + 1;   // asynchronous loads per wave per tile
+
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  T* const q_ring = reinterpret_cast<T*>(smem_raw);
+  T* const g_ring = q_ring + NQ * TILE;
+  float* const row_ring = reinterpret_cast<float*>(g_ring + NG * TILE);   // [NQ][NW chunks of {lse[RPW], delta[RPW]}]
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pair = wave & (NP - 1);   // waves w and w + 4 run on the same SIMD
+  const bool grad_role = wave >= NP;
+  float* const xbuf = row_ring + NQ * 2 * TQ + pair * 2 * S::XSLOT + lane * 4;   // two slots of 16 values per lane
+
+  int bh, kt, L;
+  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
+                  p.lens_stride, bh, kt, L);
+  const int hd = bh % p.H, b = bh / p.H;
+  const int T_ = p.T, C = p.C, R = p.R;
+  const int k0 = kt * TKB;
+  T* dk_base = reinterpret_cast<T*>(p.dk) + (int64_t)bh * T_ * D;
+  T* dv_base = reinterpret_cast<T*>(p.dv) + (int64_t)bh * T_ * D;
+  const int k_end = k0 + TKB < T_ ? k0 + TKB : T_;
+  if (k0 >= L) {
+    zero_rows<T, D, NT>(dk_base, k0, k_end, tid);
+    zero_rows<T, D, NT>(dv_base, k0, k_end, tid);
+    return;
+  }
+
+  auto win_lo = [&](int key) { return div_by(key, p.cdiv) * C; };
+  auto win_hi = [&](int key) {
+    const int64_t e = ((int64_t)div_by(key, p.cdiv) + R + 1) * (int64_t)C;
+    return e < (int64_t)L ? (int)e : L;
+  };
+  auto valid = [&](int key) { return key < L ? key : L - 1; };   // keys past L mimic the last valid key
+  const int krow = k0 + pair * 32 + c;
+  const int qlo = win_lo(valid(krow)), qhi = win_hi(valid(krow));
+  const int wk_first = valid(k0 + pair * 32), wk_last = valid(k0 + pair * 32 + 31);
+  const int qhi_min = win_hi(wk_first), qlo_max = win_lo(wk_last);
+  // queries that can see any key of this pair; a pair whose keys are all padding has none
+  const int qlo_min = win_lo(wk_first), qhi_max = k0 + pair * 32 < L ? win_hi(wk_last) : 0;
+  const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(valid(k0 + TKB - 1)) + TQ - 1) / TQ;
+  // both waves of a pair take the same decisions
+  auto live = [&](int t) { return t * TQ + TQ > qlo_min && t * TQ < qhi_max; };
+  auto interior = [&](int t) { return t * TQ >= qlo_max && t * TQ + TQ <= qhi_min; };
+
+  const T* qbase = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
+  const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
+  const float* row_src = (lane < RPW ? p.lse : p.delta) + (int64_t)bh * T_;
+  Loader ldq, ldg;
+  ldq.init(qbase, p.q_st, qt0 * TQ, L - 1, wave, lane);
+  ldg.init(gbase, p.do_st, qt0 * TQ, L - 1, wave, lane);
+  // Tile t goes where tile t - 4 (Q, lse, delta) and tile t - 3 (dO) were: issued at the beginning of step t - 2, when
+  // every wave has finished step t - 3, the last that reads either.
+  auto issue_tile = [&](int t, int gs) {
+    const int qs = (t - qt0) & (NQ - 1);
+    if (lane < 2 * RPW)
+      async_copy_f32<true>(row_src + valid(t * TQ + wave * RPW + lane % RPW), row_ring + (qs * NW + wave) * 2 * RPW);
+    ldq.issue(q_ring + qs * TILE, wave);
+    ldg.issue(g_ring + gs * TILE, wave);
+    ldq.advance();
+    ldg.advance();
+  };
+  issue_tile(qt0, 0);
+  if (qt0 + 1 < qt1) issue_tile(qt0 + 1, 1);
+
+  // resident fragments: K * (-scale * log2 e) for the score role, -V for the grad role (see dkdv2_kernel)
+  Frag rf[1][NF];
+  {
+    const T* rp = grad_role ? reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
+                                  (int64_t)valid(krow) * p.v_st
+                            : reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
+                                  (int64_t)valid(krow) * p.k_st;
+    const float mul = grad_role ? -1.0f : -p.scale_log2e;
+#pragma unroll
+    for (int g = 0; g < NF; ++g) {
+      rf[0][g] = *reinterpret_cast<const Frag*>(rp + (g * 2 + h) * E::VEC);
+#pragma unroll
+      for (int e = 0; e < E::VEC; ++e) rf[0][g][e] = (T)((float)rf[0][g][e] * mul);
+    }
+  }
+  f32x16 acc[1][DB];   // dV^T[d][key] (score role) or -dK^T[d][key] (grad role)
+#pragma unroll
+  for (int m = 0; m < DB; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[0][m][i] = 0.0f;
+  wait_all_loads();
+
+  // lse (which = 0) or delta (which = 1) of the 16 rows of tile t that this lane holds in a C fragment
+  auto rows16 = [&](int t, int which, f32x16& out) {
+    const float* rows = row_ring + ((t - qt0) & (NQ - 1)) * 2 * TQ + which * RPW;
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const int r = 8 * g4 + 4 * h;
+      const f32x4 v4 = *reinterpret_cast<const f32x4*>(rows + (r / RPW) * 2 * RPW + r % RPW);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[4 * g4 + e] = v4[e];
+    }
+  };
+  auto masked = [&](int t, f32x16& x) {
+    if (interior(t)) return;
+    asm volatile("");   // a real branch, not selects
+    const uint32_t rm = row_mask(qlo - t * TQ, qhi - t * TQ, h);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = keep_or_zero(x[i], keep_bits(rm, i));
+  };
+  int gs = 0;   // stage of the current dO tile
+  auto begin_step = [&](int t) {
+    if (t + 1 < qt1) wait_loads<LPT>();
+    else wait_loads<0>();
+    __syncthreads();
+    if (t + 2 < qt1) issue_tile(t + 2, gs == 0 ? 2 : gs - 1);
+  };
+
+  if (!grad_role) {
+    for (int t = qt0; t < qt1; ++t, gs = gs == NG - 1 ? 0 : gs + 1) {
+      begin_step(t);
+      if (!live(t)) continue;
+      f32x16 s[1][1];
+      rows16(t, 0, s[0][0]);
+      mma_rows_n<T, D>(s, q_ring + ((t - qt0) & (NQ - 1)) * TILE, 0, rf, lane);   // lse - S[q][key]
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[0][0][i] = fast_exp2(-s[0][0][i]);
+      masked(t, s[0][0]);
+      float* slot = xbuf + (t & 1) * S::XSLOT;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<f32x4*>(slot + g4 * 256) =
+            f32x4{s[0][0][4 * g4], s[0][0][4 * g4 + 1], s[0][0][4 * g4 + 2], s[0][0][4 * g4 + 3]};
+      Frag pf[1][2];
+      pack_c<T>(pf[0], s[0][0]);
+      mma_tr_n<T, D>(acc, g_ring + gs * TILE, 0, pf, lane);                        // dV^T[d][key] += dO^T P
+    }
+    __syncthreads();   // the grad role's last step
+  } else {
+    f32x16 dp[1][1];   // delta - dP of the step before
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dp[0][0][i] = 0.0f;
+    for (int t = qt0;; ++t, gs = gs == NG - 1 ? 0 : gs + 1) {
+      if (t < qt1) begin_step(t);
+      else __syncthreads();
+      const bool prev = t > qt0 && live(t - 1);
+      Frag df[1][2];
+      if (prev) {
+        const float* slot = xbuf + ((t - 1) & 1) * S::XSLOT;
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 p4 = *reinterpret_cast<const f32x4*>(slot + g4 * 256);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dp[0][0][4 * g4 + e] *= p4[e];   // = -dS
+        }
+        masked(t - 1, dp[0][0]);   // a masked dP may hold anything, NaN included
+        pack_c<T>(df[0], dp[0][0]);
+      }
+      if (t < qt1 && live(t)) {
+        rows16(t, 1, dp[0][0]);
+        mma_rows_n<T, D>(dp, g_ring + gs * TILE, 0, rf, lane);                      // delta - dP[q][key]
+      }
+      if (prev) mma_tr_n<T, D>(acc, q_ring + ((t - 1 - qt0) & (NQ - 1)) * TILE, 0, df, lane);   // -dK^T += Q^T (-dS)
+      if (t == qt1) break;
+    }
+  }
+
+  if (krow >= L) {
+#pragma unroll
+    for (int m = 0; m < DB; ++m)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[0][m][i] = 0.0f;
+  }
+  __syncthreads();   // the row patches lie over the rings
+  T* patch = q_ring + wave * RowPatch<T, D>::ELEMS;
+  const int row0 = k0 + pair * 32;
+  T* out = (grad_role ? dk_base : dv_base) + (int64_t)row0 * D;
+  store_rows_coalesced<T, D, DB>(patch, out, T_ - row0, acc[0], grad_role ? -p.scale : 1.0f, lane);
 }
 
 }  // namespace sa

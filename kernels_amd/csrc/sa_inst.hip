@@ -309,9 +309,23 @@ template <int D> static int dkdv_split_launch(BwdParams p, hipStream_t st) {
     return SA_ERR_HEAD_DIM;
   }
 }
+// wave pairs at head dimension 256: 8 waves (two per SIMD) own 128 keys
+template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) {
+  using S = DkdvSplitWide<ElemT, D>;
+  auto kern = dkdv_split_wide_kernel<ElemT, D>;
+  static PrepareState once;
+  if (int rc = prepare(kern, S::lds, once)) return rc;
+  p.n_tiles = (int)ceil_div(p.T, S::TKB);
+  const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * S::NP * 64), S::lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
-  if constexpr (C::fwd2(D)) {
+  if constexpr (C::fwd2(D) && D == 256) {
+    return dkdv_split_wide_launch<D>(p, st);
+  } else if constexpr (C::fwd2(D)) {
     if constexpr (D >= 64) {   // a 64-byte row splits over four waves' copies, not over eight
       if (launch_choice(D, p.C, p.R).dkdv == DKDV_SPLIT) return dkdv_split_launch<D>(p, st);
     }
