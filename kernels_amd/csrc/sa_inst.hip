@@ -59,6 +59,18 @@ template <typename K> static int prepare(K kernel, size_t lds_bytes, PrepareStat
 
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// float32, head dimensions 16 to 64: workgroups of 64 rows (two waves) instead of 128 where twice as many still find a CU
+// each and their windows are at least a tenth shorter -- such a launch takes as long as one workgroup, and that as long as
+// its tiles.  Half the threads stage a tile, which costs 3 to 8 % where the window stays the same.  Forward and backward in
+// us, 128 rows -> 64: B*H=8, T=512, D=32, chunks of 64, 2 back 12.6, 32.5 -> 9.8, 24.9; B*H=32, T=512, D=64 (128 workgroups)
+// 17.8, 47.4 -> 15.4, 40.6; B*H=4, T=300, D=64, chunks of 16, 3 back 14.7, 38.2 -> 11.2, 28.5.  On the other side of the
+// rule: chunks of 128, 1 back, B*H=8, T=1024 17.4, 46.6 -> 18.8, 48.1; 192 workgroups (B*H=48, T=512) 17.9, 48.7 -> 20.0, 49.1.
+template <typename P> static bool half_workgroups(const P& p) {
+  if ((int64_t)p.B * p.H * ceil_div(p.T, 128) > 128) return false;
+  const int64_t back = (int64_t)p.C * p.R;
+  return 10 * (back + ceil_div(64, p.C) * p.C) <= 9 * (back + ceil_div(128, p.C) * p.C);
+}
+
 // SA_DGROUP 0 holds head dimensions 16..128, SA_DGROUP 1 holds 256 (built with different
 // compiler options, see the Makefile).
 #if SA_DGROUP == 0
@@ -120,7 +132,6 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
   }
 #endif
 }
-#if SA_DTYPE_ID == 0
 template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipStream_t st) {
   constexpr size_t lds = (size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
   auto kern = fwd_split_kernel<D, NW, NST>;
@@ -132,7 +143,6 @@ template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipSt
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
-#endif
 template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D)) {
@@ -150,6 +160,7 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
       if ((int64_t)p.B * p.H * ceil_div(p.T, 256) < 256) return fwd_split_launch<D, 4, 1>(p, st);
       return fwd_split_launch<D, 8, 2>(p, st);
     } else {
+      if (half_workgroups(p)) return fwd_split_launch<D, 2, 2>(p, st);
       return fwd_split_launch<D, 4, 2>(p, st);
     }
   } else {
@@ -224,6 +235,18 @@ template <int D> static int dq3_launch(BwdParams p, hipStream_t st) {
   }
 #endif
 }
+template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st) {
+  constexpr int TQ = NW * 32;
+  constexpr size_t lds = (size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
+  auto kern = dq_split_kernel<D, NW>;
+  static PrepareState once;
+  if (int rc = prepare(kern, lds, once)) return rc;
+  p.n_tiles = (int)ceil_div(p.T, TQ);
+  const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int dq_d(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D)) {
@@ -232,16 +255,10 @@ template <int D> static int dq_d(BwdParams p, hipStream_t st) {
     }
     return dq2_launch<D, C::NARROW_NW>(p, st);
   } else if constexpr (C::split(D)) {
-    constexpr int NW = 4, TQ = NW * 32;
-    constexpr size_t lds = (size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
-    auto kern = dq_split_kernel<D, NW>;
-    static PrepareState once;
-    if (int rc = prepare(kern, lds, once)) return rc;
-    p.n_tiles = (int)ceil_div(p.T, TQ);
-    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
-    return (int)hipGetLastError();
+    if constexpr (D <= 64) {
+      if (half_workgroups(p)) return dq_split_launch<D, 2>(p, st);
+    }
+    return dq_split_launch<D, 4>(p, st);
   } else {
     if (p.delta_out) return SA_ERR_ARG;
     constexpr int TQ = C::NW * 32;
@@ -321,6 +338,18 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * S::NP * 64), S::lds, st, p);
   return (int)hipGetLastError();
 }
+template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream_t st) {
+  constexpr int TKB = NW * 32;
+  constexpr size_t lds = (size_t)2 * (2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + 2 * 32 * sizeof(float));
+  auto kern = dkdv_split_f32_kernel<D, NW>;
+  static PrepareState once;
+  if (int rc = prepare(kern, lds, once)) return rc;
+  p.n_tiles = (int)ceil_div(p.T, TKB);
+  const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D) && D == 256) {
@@ -349,16 +378,10 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::DKDV2_NW * 64), lds, st, p);
     return (int)hipGetLastError();
   } else if constexpr (C::split(D)) {
-    constexpr int NW = 4, TKB = NW * 32;
-    constexpr size_t lds = (size_t)2 * (2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + 2 * 32 * sizeof(float));
-    auto kern = dkdv_split_f32_kernel<D, NW>;
-    static PrepareState once;
-    if (int rc = prepare(kern, lds, once)) return rc;
-    p.n_tiles = (int)ceil_div(p.T, TKB);
-    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
-    return (int)hipGetLastError();
+    if constexpr (D <= 64) {
+      if (half_workgroups(p)) return dkdv_split_f32_launch<D, 2>(p, st);
+    }
+    return dkdv_split_f32_launch<D, 4>(p, st);
   } else {
     constexpr int TKB = C::NW * 32;
     constexpr size_t lds =
