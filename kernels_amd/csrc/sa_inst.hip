@@ -2,6 +2,7 @@
 // Compiled once per (SA_DTYPE_ID, SA_KIND) pair so that the families build in parallel.
 //   SA_DTYPE_ID: 0 fp32, 1 fp16, 2 bf16        SA_KIND: 0 forward, 1 delta + dQ, 2 dK/dV, 3 one-launch backward
 //   SA_DGROUP: 0 head dims 16..128, 1 head dim 256
+#include <algorithm>
 #include <mutex>
 #include "sa_launch.h"
 #include "sa_f32.h"
@@ -67,7 +68,7 @@ static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // rule: chunks of 128, 1 back, B*H=8, T=1024 17.4, 46.6 -> 18.8, 48.1; 192 workgroups (B*H=48, T=512) 17.9, 48.7 -> 20.0, 49.1.
 template <typename P> static bool half_workgroups(const P& p) {
   if ((int64_t)p.B * p.H * ceil_div(p.T, 128) > 128) return false;
-  const int64_t back = (int64_t)p.C * p.R;
+  const int64_t back = std::min((int64_t)p.C * p.R, (int64_t)1 << 32);   // ten times it stays within 64 bits
   return 10 * (back + ceil_div(64, p.C) * p.C) <= 9 * (back + ceil_div(128, p.C) * p.C);
 }
 
