@@ -225,13 +225,15 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
 // and masks are decided per 32-key block instead of per tile, and a wave's first tile goes straight
 // to the search for its maximum.  Long windows run the plain form, whose loop is a few per cent
 // tighter (fewer registers, no per-block tests).
-template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT>
+// A wave goes through a tile SB keys at a time.  At head dimension 64 half a tile instead of a whole one takes 118
+// registers instead of 143: four waves per SIMD instead of three (fwd_halves, in the launcher, says where that pays).
+template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT, int SB>
 __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const FwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ && NST >= 2 && (NST - 2) * 2 * AsyncTile<T, D, TK, NW>::PER_WAVE < 64, "swizzled 16-bit tiles; the loads of NST-2 tiles fit the load counter");
-  constexpr int WQ = QB * 32, TQ = NW * WQ, NT = NW * 64, KBN = TK / 32;
+  constexpr int WQ = QB * 32, TQ = NW * WQ, NT = NW * 64, KBN = SB / 32;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TK * D;            // elements per K or V tile
   constexpr int STAGE = 2 * TILE;
@@ -348,9 +350,11 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
 
     const T* Kt = smem + ((t - kt0) % NST) * STAGE;
     const T* Vt = Kt + TILE;
-    const int k0 = t * TK;
+#pragma unroll
+    for (int sb = 0; sb < TK; sb += SB) {
+    const int k0 = t * TK + sb;
     // the workgroup's key range is the union over its waves; skip what this wave cannot see
-    if (k0 + TK <= lo_min || k0 >= hi_max) continue;
+    if (k0 + SB <= lo_min || k0 >= hi_max) continue;
 
     // S^T[key][q] = K Q^T for the QB query blocks
     f32x16 s[QB][KBN];
@@ -365,13 +369,13 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
     bool live[KBN], inside[KBN], all_live = true;
 #pragma unroll
     for (int kb = 0; kb < KBN; ++kb) {
-      const int kb0 = SHORT ? k0 + kb * 32 : k0, kbn = SHORT ? 32 : TK;   // the block, or the whole tile
+      const int kb0 = SHORT ? k0 + kb * 32 : k0, kbn = SHORT ? 32 : SB;   // the block, or all of them
       live[kb] = !SHORT || (kb0 + kbn > lo_min && kb0 < hi_max);
       inside[kb] = kb0 >= lo_max && kb0 + kbn <= hi_min;
       all_live = all_live && live[kb];
     }
     if (all_live) {
-      mma_rows_n<T, D>(s, Kt, 0, qf, lane);
+      mma_rows_n<T, D>(s, Kt, sb, qf, lane);
     } else {
 #pragma unroll
       for (int kb = 0; kb < KBN; ++kb) {
@@ -379,7 +383,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
           f32x16 one[QB][1];
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb) one[qb][0] = s[qb][kb];
-          mma_rows_n<T, D>(one, Kt, kb * 32, qf, lane);
+          mma_rows_n<T, D>(one, Kt, sb + kb * 32, qf, lane);
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb) s[qb][kb] = one[qb][0];
         } else {
@@ -476,7 +480,8 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
       Frag bq[QB][2];
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) bq[qb][0] = pb[qb][kb][0], bq[qb][1] = pb[qb][kb][1];
-      mma_tr_n<T, D>(oacc, Vt, kb, bq, lane);
+      mma_tr_n<T, D>(oacc, Vt, sb / 32 + kb, bq, lane);
+    }
     }
   }
 
