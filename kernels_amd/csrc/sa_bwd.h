@@ -47,8 +47,9 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
   if (row < total && sub == 0) p.delta[row] = acc;
 }
 
-template <typename T, int D, int NW, int TK>
-__global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
+// One workgroup: query tile qt of (batch, head) bh.  delta(row) is rowsum(O * dO) of query `row`, below the sequence length.
+template <typename T, int D, int NW, int TK, typename Delta>
+SA_DEV void dq_rows(const BwdParams& p, int bh, int qt, int tid, Delta&& delta) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
@@ -59,12 +60,9 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
 
-  const int tid = threadIdx.x;
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
   const int hd = bh % p.H, b = bh / p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
@@ -91,6 +89,9 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
   const int wq_last = q0 + wave * 32 + 31 < L ? q0 + wave * 32 + 31 : L - 1;
   const int hi_min = (cdiv(wq_first) + 1) * C < L ? (cdiv(wq_first) + 1) * C : L;
   const int lo_max = (cdiv(wq_last) > R ? cdiv(wq_last) - R : 0) * C;
+  constexpr bool SKIP = !E::HALF && D <= 128;   // see fwd_rows
+  const int lo_min = (cdiv(wq_first) > R ? cdiv(wq_first) - R : 0) * C;
+  const int hi_max = q0 + wave * 32 >= L ? 0 : (cdiv(wq_last) + 1) * C < L ? (cdiv(wq_last) + 1) * C : L;
   const int gq_last = q0 + TQ - 1 < L ? q0 + TQ - 1 : L - 1;
   const int lo_wg = (cdiv(q0) > R ? cdiv(q0) - R : 0) * C;
   const int hi_wg = (cdiv(gq_last) + 1) * C < L ? (cdiv(gq_last) + 1) * C : L;
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
     }
     // rows past L get P = exp2(-inf) = 0
     lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qr] : INFINITY;
-    delta_q = p.delta[(int64_t)bh * T_ + qr];
+    delta_q = delta(qr);
   }
 
   const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
@@ -149,6 +150,7 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
 
 #pragma unroll
     for (int kb = 0; kb < KBN; ++kb) {
+      if (SKIP && (k0 + kb * 32 + 32 <= lo_min || k0 + kb * 32 >= hi_max)) continue;
       f32x16 s, dp;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.0f, dp[i] = 0.0f;
@@ -193,6 +195,13 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
   }
 }
 
+template <typename T, int D, int NW, int TK>
+__global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
+  int bh, qt;
+  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
+  dq_rows<T, D, NW, TK>(p, bh, qt, threadIdx.x, [&](int row) { return p.delta[(int64_t)bh * p.T + row]; });
+}
+
 // PASS selects what one launch produces: 0 both gradients, 1 dV only, 2 dK only.  Two float32 accumulators of 32 x 256
 // and the resident K and V rows are 512 registers per lane before any operand, so float32 at head dimension 256 runs
 // as two launches: the dV pass needs neither V nor dP and fits without spills; the dK pass has one accumulator and
@@ -200,7 +209,7 @@ __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
 // around the products; the form that staged both tensors at once was miscompiled (the spill code of the first tile
 // dropped a register copy), which the head-dimension parity tests catch.
 template <typename T, int D, int NW, int TQ, int PASS = 0>
-__global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
+SA_DEV void dkdv_rows(const BwdParams& p, int bh, int kt, int tid) {   // one workgroup: key tile kt of (batch, head) bh
   constexpr bool WITH_DV = PASS != 2, WITH_DK = PASS != 1;
   constexpr bool HALVES = PASS == 2;   // stage Q and dO one after the other
   static_assert(!HALVES || TQ == 32, "the two staging halves bracket a single 32-query block");
@@ -215,12 +224,9 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
 
-  const int tid = threadIdx.x;
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bh, kt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, kt);
   const int hd = bh % p.H, b = bh / p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
@@ -252,6 +258,8 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
   const int wk_first = k0 + wave * 32 < L ? k0 + wave * 32 : L - 1;
   const int wk_last = k0 + wave * 32 + 31 < L ? k0 + wave * 32 + 31 : L - 1;
   const int qhi_min = win_hi(wk_first), qlo_max = win_lo(wk_last);
+  constexpr bool SKIP = !E::HALF && D <= 128;   // see fwd_rows
+  const int qlo_min = win_lo(wk_first), qhi_max = k0 + wave * 32 < L ? win_hi(wk_last) : 0;
   const int gk_last = k0 + TKB - 1 < L ? k0 + TKB - 1 : L - 1;
   const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(gk_last) + TQ - 1) / TQ;
 
@@ -335,6 +343,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 
 #pragma unroll
     for (int qb = 0; qb < QBN; ++qb) {
+      if (SKIP && (qs + qb * 32 + 32 <= qlo_min || qs + qb * 32 >= qhi_max)) continue;
       f32x16 s, dp;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.0f, dp[i] = 0.0f;
@@ -397,6 +406,13 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
     if constexpr (WITH_DK) store_acc_T<T, D, DB>(dk_base + (int64_t)krow * D, dk, p.scale, h);
     if constexpr (WITH_DV) store_acc_T<T, D, DB>(dv_base + (int64_t)krow * D, dv, 1.0f, h);
   }
+}
+
+template <typename T, int D, int NW, int TQ, int PASS = 0>
+__global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
+  int bh, kt;
+  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, kt);
+  dkdv_rows<T, D, NW, TQ, PASS>(p, bh, kt, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------

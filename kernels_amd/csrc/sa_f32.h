@@ -1,25 +1,39 @@
 // float32 kernels on the 16-bit matrix pipe, head dimensions 16 to 128.
 //
 // v_mfma_f32_32x32x2_f32 does 64 flop per cycle and SIMD, v_mfma_f32_32x32x16_bf16 1024.  A float32
-// number is exactly the sum of three bfloat16 numbers (24 = 8 + 8 + 8 significand bits, same exponent
-// range; each part is the rounded remainder of the ones before), so a float32 product is
+// number is the sum of three bfloat16 numbers (24 = 8 + 8 + 8 significand bits; each part is the rounded
+// remainder of the ones before), so a float32 product is
 //   x*y = x1*y1 + (x1*y2 + x2*y1) + (x1*y3 + x2*y2 + x3*y1) + [x2*y3 + x3*y2 + x3*y3],
-// every term of which the bfloat16 instruction forms exactly and adds up in float32.  The bracket is
-// left out: it is below 2^-26 of |x*y|, a quarter of the 2^-24 to which float32 rounds a product (or a
-// running sum).  Six products at 16 times the rate take 6/16 of the matrix time, and the sums have fewer
-// roundings (16 contraction slots per instruction instead of 2).  Measured on problems of 200 to 4096
+// every term of which the bfloat16 instruction forms exactly and adds up in float32 (the decomposition of Henry, Tang
+// and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019).
+// The bracket is left out: it is at most 2^-24 of |x*y|, to which float32 rounds a product (or a running sum) too, and
+// 2^-27 in the root mean square.  Six products at 16 times the rate take 6/16 of the matrix time, and the
+// sums have fewer roundings (16 contraction slots per instruction instead of 2).  Measured on problems of 200 to 4096
 // positions against float64: errors of O, dQ, dK, dV at or below those of the float32 instruction
-// kernels (see the comment at each kernel for times).  Elements beyond bfloat16's range, infinities among them,
-// take a path of their own (split2_wide).
+// kernels (see the comment at each kernel for times).
+//
+// The parts reach down to 2^-133, bfloat16's smallest number, and float32 to 2^-149: every operand is multiplied by
+// kUp = 2^16 before it is split, exactly, and the products' powers of two are taken out where the result is scaled anyway.
+// What then exceeds the exponent range (elements from 2^111 on, infinities, sums and dS beyond about 2^80 to 2^96)
+// or was not a number to begin with leaves a result that is not finite, since a part of it is NaN; a workgroup
+// that sees one goes through its rows again with the float32 instruction (fwd_rows, dq_rows, dkdv_rows).
 //
 // The parts of the resident operand are formed once per wave and stay in registers; those of the streamed
 // tiles are formed once per workgroup on the way into LDS, where each part is a bfloat16 tile of its own
 // (the swizzled layout and transposing reads of the 16-bit kernels apply unchanged).  Probabilities and dS
 // are split in registers.
 #pragma once
+#include "sa_bwd.h"
 #include "sa_common.h"
+#include "sa_fwd.h"
 
 namespace sa {
+
+constexpr float kUp = 0x1p16f;                                 // of one operand
+constexpr float kUp2 = 0x1p32f, kDown2 = 0x1p-32f;             // of a product of two
+constexpr float kDown3 = 0x1p-48f;                             // of dS (a product of two) times an operand
+// A scale that times these powers of two is no normal number.
+SA_DEV bool scale_too_small(float scale_log2e) { return scale_log2e != 0.0f && fabsf(scale_log2e) < 0x1p-60f; }
 
 // Three bfloat16 fragments that add up to eight float32 values.
 struct Split8 {
@@ -48,60 +62,10 @@ SA_DEV void split_pair(Split8& s, int e, float x0, float x1) {
     s.p[k] = __builtin_bit_cast(bf16x8, w);
   }
 }
-// The same for input elements that may round to an infinite first part: the first part of a finite one is cut off
-// instead of rounded, and an infinity is (1, 0, infinity) with its sign, which the six products with another split
-// number take to what the number itself gives (x3 meets y1 only, so no remainder of y spoils the sign).
-SA_DEV void split2_wide(float x0, float x1, uint32_t (&u)[3]) {
-  uint32_t inf[2], cut[2];
-  float y[2] = {x0, x1};
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t bits = __float_as_uint(y[j]), mag = bits & 0x7FFFFFFFu;
-    inf[j] = mag == 0x7F800000u ? bits >> 16 : 0u;
-    cut[j] = mag >= 0x7F7F8000u && mag < 0x7F800000u ? bits >> 16 : 0u;
-    if (inf[j]) y[j] = __uint_as_float((bits & 0x80000000u) | 0x3F800000u);
-    if (cut[j]) y[j] = __uint_as_float(bits) - __uint_as_float(cut[j] << 16);
-  }
-  split2(y[0], y[1], u);
-  // a cut-off element is (cut, y1, y2): its y has 16 significand bits, so y3 is zero
-  const uint32_t m = (cut[0] ? 0x0000FFFFu : 0u) | (cut[1] ? 0xFFFF0000u : 0u);
-  u[2] = (u[1] & m) | (u[2] & ~m) | inf[0] | (inf[1] << 16);
-  u[1] = (u[0] & m) | (u[1] & ~m);
-  u[0] = (cut[0] | (cut[1] << 16)) | (u[0] & ~m);
-}
-// The largest magnitude among eight values and m; a NaN counts for nothing (and needs nothing).
-SA_DEV float magnitude8(const f32x4& lo, const f32x4& hi, float m) {
-  auto max3 = [](float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-  };
-  return max3(max3(lo[0], lo[1], lo[2]), max3(lo[3], hi[0], hi[1]), max3(hi[2], hi[3], m));
-}
-// Whether some lane of the wave holds elements that need split2_wide, from their largest magnitude (it gives all others
-// the same parts, so the whole wave takes one way).
-SA_DEV bool any_wide(float m) {
-  return __builtin_expect(__builtin_amdgcn_ballot_w64(m >= __uint_as_float(0x7F7F8000u)) != 0, 0);
-}
 SA_DEV Split8 split8(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int e = 0; e < 4; ++e) split_pair(s, e, x[2 * e], x[2 * e + 1]);
-  return s;
-}
-SA_DEV Split8 split8_wide(const float (&x)[8]) {
-  Split8 s;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    uint32_t u[3];
-    split2_wide(x[2 * e], x[2 * e + 1], u);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      u32x4 w = __builtin_bit_cast(u32x4, s.p[k]);
-      w[e] = u[k];
-      s.p[k] = __builtin_bit_cast(bf16x8, w);
-    }
-  }
   return s;
 }
 // The six products, smallest first.
@@ -141,51 +105,24 @@ template <int D, int ROWS, int NT> struct SplitStager {
       }
     }
   }
-  SA_DEV float magnitude(float m) const {
-#pragma unroll
-    for (int it = 0; it < N; ++it)
-      if (TOTAL % NT == 0 || (int)threadIdx.x + it * NT < TOTAL) m = magnitude8(regs[it][0], regs[it][1], m);
-    return m;
-  }
-  template <bool WIDE> SA_DEV void store(__bf16* tile, int tid) const {
+  SA_DEV void store(__bf16* tile, int tid) const {
 #pragma unroll
     for (int it = 0; it < N; ++it) {
       const int ch = tid + it * NT;
       if (TOTAL % NT == 0 || ch < TOTAL) {
-        const float x[8] = {regs[it][0][0], regs[it][0][1], regs[it][0][2], regs[it][0][3],
-                            regs[it][1][0], regs[it][1][1], regs[it][1][2], regs[it][1][3]};
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = regs[it][e / 4][e % 4] * kUp;
         __bf16* dst = tile + G::off(ch / CPR, (ch % CPR) * 8);
-        if constexpr (WIDE) {   // pair by pair, in few registers
+        const Split8 s = split8(x);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            uint32_t u[3];
-            split2_wide(x[2 * e], x[2 * e + 1], u);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) reinterpret_cast<uint32_t*>(dst + k * SplitTile<D, ROWS>::PLANE)[e] = u[k];
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        } else {
-          const Split8 s = split8(x);
-#pragma unroll
-          for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * SplitTile<D, ROWS>::PLANE) = s.p[k];
-        }
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * SplitTile<D, ROWS>::PLANE) = s.p[k];
       }
     }
   }
 };
-// Two tiles, one check for both.
-template <typename S> SA_DEV void store_tiles(const S& a, __bf16* ta, const S& b, __bf16* tb, int tid) {
-  if (any_wide(b.magnitude(a.magnitude(0.0f)))) {
-    a.template store<true>(ta, tid);
-    b.template store<true>(tb, tid);
-  } else {
-    a.template store<false>(ta, tid);
-    b.template store<false>(tb, tid);
-  }
-}
 
-// This lane's half of a float32 row, and its split fragments (as a B operand).  Loaded as a whole and checked once:
-// a check per fragment would wait for one load after the other (dQ of the problem below: 650 -> 770 us).
+// This lane's half of a float32 row, and its split fragments (as a B operand).
 template <int D> struct HalfRow {
   f32x4 r[D / 8];
   SA_DEV void load(const float* row, int h) {
@@ -193,20 +130,14 @@ template <int D> struct HalfRow {
     for (int i = 0; i < D / 8; ++i) r[i] = *reinterpret_cast<const f32x4*>(row + (i / 2) * 16 + h * 8 + (i % 2) * 4);
   }
   SA_DEV void split(Split8 (&f)[D / 16], bool negative) const {
-    float m = 0.0f;
+    const float mul = negative ? -kUp : kUp;
 #pragma unroll
-    for (int g = 0; g < D / 16; ++g) m = magnitude8(r[2 * g], r[2 * g + 1], m);
-    auto all = [&](auto&& one) {
+    for (int g = 0; g < D / 16; ++g) {
+      float x[8];
 #pragma unroll
-      for (int g = 0; g < D / 16; ++g) {
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = negative ? -r[2 * g + e / 4][e % 4] : r[2 * g + e / 4][e % 4];
-        f[g] = one(x);
-      }
-    };
-    if (any_wide(m)) all([](const float (&x)[8]) { return split8_wide(x); });
-    else all([](const float (&x)[8]) { return split8(x); });
+      for (int e = 0; e < 8; ++e) x[e] = r[2 * g + e / 4][e % 4] * mul;
+      f[g] = split8(x);
+    }
   }
 };
 
@@ -258,10 +189,44 @@ SA_DEV void mma_tr_split(f32x16 (&acc)[NM], const __bf16* X, const Split8 (&b)[N
       },
       [&](int it, const Split8& a) { mma6(acc[it % NM], a, b[it / NM]); side(it); });
 }
-// The split B operand of mma_tr_split from a whole C fragment.
-SA_DEV void split_c(Split8 (&b)[2], const f32x16& P) {
+// The split B operand of mma_tr_split from a whole C fragment, times mul (a power of two).
+SA_DEV void split_c(Split8 (&b)[2], const f32x16& P, float mul = 1.0f) {
 #pragma unroll
-  for (int i = 0; i < 16; i += 2) split_pair(b[i / 8], (i % 8) / 2, P[i], P[i + 1]);
+  for (int i = 0; i < 16; i += 2) split_pair(b[i / 8], (i % 8) / 2, P[i] * mul, P[i + 1] * mul);
+}
+
+// Whether the rows of an accumulator that stand for elements of the head dimension are finite (at 16 half of them do).
+template <int D, int NM> SA_DEV bool all_finite(const f32x16 (&acc)[NM]) {
+  float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // becomes NaN
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (m * 32 + 8 * (i >> 2) < D) z[i & 3] = __builtin_fmaf(acc[m][i], 0.0f, z[i & 3]);
+  return (z[0] + z[1]) + (z[2] + z[3]) == 0.0f;
+}
+// The same value as one that the compiler knows nothing of: what the second way through the rows derives from it is computed
+// there, not kept in registers through the loop of the first.
+SA_DEV int again_s(int x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+SA_DEV int again_v(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+// Whether some lane of the workgroup says so; smem is not read by anyone any more and free again after the call.
+template <int NW> SA_DEV bool any_in_workgroup(bool x, void* smem, int wave, int lane) {
+  volatile SA_LDS uint32_t* flags = (volatile SA_LDS uint32_t*)smem;
+  const bool mine = __builtin_amdgcn_ballot_w64(x) != 0;
+  if (lane == 0) flags[wave] = mine;
+  __syncthreads();
+  uint32_t any = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) any |= flags[w];
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return false;
+  __syncthreads();
+  return true;
 }
 
 // The windows of a wave's 32 queries, of one lane's query, and of the workgroup.
@@ -286,7 +251,7 @@ struct QueryWindow {
 // bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back: D=128 685 us with the float32 instruction, 425 here;
 // D=64 (ragged) 266 -> 153; D=32 147 -> 92; D=16 116 -> 73.
 template <int D, int NW, int NST>
-__global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p) {
+__global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
   constexpr float kRescaleGap = 8.0f;
@@ -323,7 +288,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
   const QueryWindow w(q0, wave, TQ, qrow, L, p.C, p.R, p.cdiv);
   const int kt0 = w.lo_wg / TK, kt1 = (w.hi_wg + TK - 1) / TK;
   // never exactly 0, so that a masked score of -inf stays -inf after scaling
-  const float sl2e = fmaxf(fabsf(p.scale_log2e), 1e-30f);
+  const float sl2e = fmaxf(fabsf(p.scale_log2e) * kDown2, 0x1p-126f);
 
   const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
@@ -346,7 +311,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
     for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
 
-  store_tiles(sk, smem, sv, smem + TILE, tid);
+  sk.store(smem, tid);
+  sv.store(smem + TILE, tid);
   __syncthreads();
 
   for (int t = kt0; t < kt1; ++t) {
@@ -400,21 +366,27 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_split_kernel(const FwdParams p
       }
       l_run += rs0 + rs1;
       Split8 pb[2];
-      split_c(pb, pr);
+      split_c(pb, pr, kUp);
       mma_tr_split<D, TK>(oacc, Vt, pb, lane);   // O^T[d][q] += V^T P^T
     }
     if (more) {
       if (NST == 1) __syncthreads();   // the only stage has no reader left
       __bf16* nxt = smem + ((t + 1 - kt0) % NST) * 2 * TILE;
-      store_tiles(sk, nxt, sv, nxt + TILE, tid);
+      sk.store(nxt, tid);
+      sv.store(nxt + TILE, tid);
     }
     __syncthreads();
   }
 
   const float l_tot = half_sum(l_run);
+  const bool odd = q0 + wave * 32 < L && (!(l_tot > 0.0f) || !all_finite<D>(oacc) || scale_too_small(p.scale_log2e));
+  if (any_in_workgroup<NW>(odd, smem_raw, wave, lane)) {
+    fwd_rows<float, D, NW, TK>(p, again_s(bh), again_s(qt), again_v(tid));
+    return;
+  }
   const bool valid = qrow < L;
   if (qrow < T_) {
-    const float inv = valid ? 1.0f / l_tot : 0.0f;
+    const float inv = valid ? 1.0f / l_tot * kDown2 : 0.0f;
     if (!valid) {
 #pragma unroll
       for (int m = 0; m < DB; ++m)
@@ -464,7 +436,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
   const int qrow = q0 + wave * 32 + c;
   const QueryWindow w(q0, wave, TQ, qrow, L, p.C, p.R, p.cdiv);
   const int kt0 = w.lo_wg / TK, kt1 = (w.hi_wg + TK - 1) / TK;
-  const float sl2e = fabsf(p.scale_log2e);
+  const float sl2e = fabsf(p.scale_log2e) * kDown2;
 
   const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
@@ -499,12 +471,15 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     }
   }
 
+  const float dinit = -delta_q * kUp2;
+
   f32x16 acc[DB];
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-  store_tiles(sk, smem, sv, smem + TILE, tid);
+  sk.store(smem, tid);
+  sv.store(smem + TILE, tid);
   __syncthreads();
 
   for (int t = kt0; t < kt1; ++t) {
@@ -519,7 +494,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     if (k0 + TK > w.lo_min && k0 < w.hi_max) {
       f32x16 s, dp;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = 0.0f, dp[i] = -delta_q;
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f, dp[i] = dinit;
       mma_rows_split<D, TK>(s, Kt, qf, lane);
       mma_rows_split<D, TK>(dp, Vt, gf, lane, [&](int g) {
 #pragma unroll
@@ -538,11 +513,16 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     }
     if (more) {
       __bf16* nxt = smem + ((t + 1 - kt0) & 1) * 2 * TILE;
-      store_tiles(sk, nxt, sv, nxt + TILE, tid);
+      sk.store(nxt, tid);
+      sv.store(nxt + TILE, tid);
     }
     __syncthreads();
   }
 
+  if (any_in_workgroup<NW>(!all_finite<D>(acc) || scale_too_small(p.scale_log2e), smem_raw, wave, lane)) {
+    dq_rows<float, D, NW, TK>(p, again_s(bh), again_s(qt), again_v(tid), [&](int) { return delta_q; });   // this lane's query
+    return;
+  }
   if (qrow < T_) {
     if (qrow >= L) {
 #pragma unroll
@@ -550,7 +530,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
     }
-    store_acc_T<float, D, DB>(dq_base + (int64_t)qrow * D, acc, p.scale, h);
+    store_acc_T<float, D, DB>(dq_base + (int64_t)qrow * D, acc, p.scale * kDown3, h);
   }
 }
 
@@ -598,7 +578,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
   const int qhi_min = win_hi(wk_first), qlo_max = win_lo(wk_last);
   const int qlo_min = win_lo(wk_first), qhi_max = k0 + wave * 32 < L ? win_hi(wk_last) : 0;
   const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(valid(k0 + TKB - 1)) + TQ - 1) / TQ;
-  const float sl2e = fabsf(p.scale_log2e);
+  const float sl2e = fabsf(p.scale_log2e) * kDown2;
 
   const float* qbase = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
   const float* gbase = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
@@ -613,8 +593,9 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
   auto stage_ptr = [&](int t) { return smem_raw + ((t - qt0) & 1) * STAGE_BYTES; };
   auto store_tile = [&](int t) {
     __bf16* st = reinterpret_cast<__bf16*>(stage_ptr(t));
-    store_tiles(sq, st, sg, st + TILE, tid);
-    if (tid < 2 * TQ) reinterpret_cast<float*>(st + 2 * TILE)[tid] = r_row;
+    sq.store(st, tid);
+    sg.store(st + TILE, tid);
+    if (tid < 2 * TQ) reinterpret_cast<float*>(st + 2 * TILE)[tid] = tid < TQ ? r_row : r_row * kUp2;
   };
   static_assert(2 * TQ <= NT, "one thread per staged row value");
   load_tile(qt0);
@@ -663,7 +644,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
           s[i] = fast_exp2(__builtin_fmaf(s[i], sl2e, -lse_r[i]));
           s[i + 1] = fast_exp2(__builtin_fmaf(s[i + 1], sl2e, -lse_r[i + 1]));
           if (!interior) s[i] = keep_or_zero(s[i], keep_bits(rm, i)), s[i + 1] = keep_or_zero(s[i + 1], keep_bits(rm, i + 1));
-          split_pair(pb[i / 8], (i % 8) / 2, s[i], s[i + 1]);
+          split_pair(pb[i / 8], (i % 8) / 2, s[i] * kUp, s[i + 1] * kUp);
         }
       });
       mma_tr_split<D, TQ>(dv, Gt, pb, lane, [&](int it) {    // dV^T[d][key] += dO^T P
@@ -681,6 +662,11 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
     __syncthreads();
   }
 
+  const bool odd = !all_finite<D>(dk) || !all_finite<D>(dv) || scale_too_small(p.scale_log2e);
+  if (any_in_workgroup<NW>(odd, smem_raw, wave, lane)) {
+    dkdv_rows<float, D, NW, TQ>(p, again_s(bh), again_s(kt), again_v(tid));
+    return;
+  }
   if (krow < T_) {
     if (krow >= L) {
 #pragma unroll
@@ -688,8 +674,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
 #pragma unroll
         for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
     }
-    store_acc_T<float, D, DB>(dk_base + (int64_t)krow * D, dk, p.scale, h);
-    store_acc_T<float, D, DB>(dv_base + (int64_t)krow * D, dv, 1.0f, h);
+    store_acc_T<float, D, DB>(dk_base + (int64_t)krow * D, dk, p.scale * kDown3, h);
+    store_acc_T<float, D, DB>(dv_base + (int64_t)krow * D, dv, kDown2, h);
   }
 }
 

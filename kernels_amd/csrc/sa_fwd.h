@@ -11,8 +11,9 @@
 
 namespace sa {
 
+// One workgroup: query tile qt of (batch, head) bh.
 template <typename T, int D, int NW, int TK>
-__global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
+SA_DEV void fwd_rows(const FwdParams& p, int bh, int qt, int tid) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
@@ -24,12 +25,9 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);  // [stage][K|V][TK][PITCH]
 
-  const int tid = threadIdx.x;
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
   const int hd = bh % p.H, b = bh / p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
@@ -62,6 +60,10 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
   const int wq_last = q0 + wave * 32 + 31 < L ? q0 + wave * 32 + 31 : L - 1;
   const int hi_min = (cdiv(wq_first) + 1) * C < L ? (cdiv(wq_first) + 1) * C : L;
   const int lo_max = (cdiv(wq_last) > R ? cdiv(wq_last) - R : 0) * C;
+  // float32 up to head dimension 128 runs after fwd_split_kernel, which leaves out the tiles that no query of a wave sees
+  constexpr bool SKIP = !E::HALF && D <= 128;
+  const int lo_min = (cdiv(wq_first) > R ? cdiv(wq_first) - R : 0) * C;
+  const int hi_max = q0 + wave * 32 >= L ? 0 : (cdiv(wq_last) + 1) * C < L ? (cdiv(wq_last) + 1) * C : L;
   // union over the workgroup decides which tiles are visited
   const int gq_last = q0 + TQ - 1 < L ? q0 + TQ - 1 : L - 1;
   const int lo_wg = (cdiv(q0) > R ? cdiv(q0) - R : 0) * C;
@@ -112,6 +114,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
       sv.load(vbase, p.v_st, (t + 1) * TK, L - 1, tid);
     }
     const int k0 = t * TK;
+    if (!SKIP || (k0 + TK > lo_min && k0 < hi_max)) {
 
     // S^T[key][q] = K Q^T
     f32x16 s[KBN];
@@ -184,6 +187,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
     // O^T[d][q] += V^T P^T
 #pragma unroll
     for (int kb = 0; kb < KBN; ++kb) mma_tr<T, D>(oacc, Vt, kb, s[kb], lane);
+    }
 
     if (more) {
       T* nxt = smem + (cur ^ 1) * 2 * TILE;
@@ -207,6 +211,13 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
     store_acc_T<T, D, DB>(o_base + (int64_t)qrow * D, oacc, inv, h);
     if (lse_base && h == 0) lse_base[qrow] = valid ? m_run + __builtin_amdgcn_logf(l_tot) : 0.0f;
   }
+}
+
+template <typename T, int D, int NW, int TK>
+__global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
+  int bh, qt;
+  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
+  fwd_rows<T, D, NW, TK>(p, bh, qt, threadIdx.x);
 }
 
 // Forward kernel for 16-bit elements with swizzled tiles (D = 32, 64, 128 or 256).

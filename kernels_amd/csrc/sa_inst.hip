@@ -60,6 +60,10 @@ template <typename K> static int prepare(K kernel, size_t lds_bytes, PrepareStat
 
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// LDS of a float32 kernel on the 16-bit matrix pipe: its split tiles, or the float32 tiles of the rows it goes through again.
+constexpr size_t split_lds(size_t split_bytes, size_t rows_bytes) { return split_bytes > rows_bytes ? split_bytes : rows_bytes; }
+template <int D> constexpr size_t float_tiles = (size_t)2 * 2 * 32 * TileGeom<float, D>::PITCH * sizeof(float);   // two stages
+
 // float32, head dimensions 16 to 64: workgroups of 64 rows (two waves) instead of 128 where twice as many still find a CU
 // each and their windows are at least a tenth shorter -- such a launch takes as long as one workgroup, and that as long as
 // its tiles.  Half the threads stage a tile, which costs 3 to 8 % where the window stays the same.  Forward and backward in
@@ -140,7 +144,7 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
 #endif
 }
 template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipStream_t st) {
-  constexpr size_t lds = (size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
+  constexpr size_t lds = split_lds((size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>);
   auto kern = fwd_split_kernel<D, NW, NST>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
@@ -247,7 +251,7 @@ template <int D> static int dq3_launch(BwdParams p, hipStream_t st) {
 }
 template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st) {
   constexpr int TQ = NW * 32;
-  constexpr size_t lds = (size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16);
+  constexpr size_t lds = split_lds((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>);
   auto kern = dq_split_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
@@ -350,7 +354,8 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
 }
 template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream_t st) {
   constexpr int TKB = NW * 32;
-  constexpr size_t lds = (size_t)2 * (2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + 2 * 32 * sizeof(float));
+  constexpr size_t rows = (size_t)2 * 2 * 32 * sizeof(float);   // lse and delta
+  constexpr size_t lds = split_lds((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + rows, float_tiles<D> + rows);
   auto kern = dkdv_split_f32_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;

@@ -79,3 +79,50 @@ def test_float32_range_ends(B, H, D):
     expect[:, :, 5, 6] = False         # its weight is zero: 0 * inf
     assert torch.equal(torch.isinf(dv), expect) and torch.isnan(dv[:, :, 5, 6]).all()
     assert torch.equal(bad.sum(), expect.sum() + B * H)
+
+
+# magnitudes whose bfloat16 parts fall below or above bfloat16's range: tiny and huge operands that balance each other, and tiny
+# values or upstream gradients by themselves (dS is tiny then too)
+@pytest.mark.parametrize("B,H,T,C,R", [(2, 2, 129, 32, 2), (1, 2, 415, 100, 1), (8, 32, 260, 48, 2)])   # 64, 128 and 256 rows
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("gq,gv,gd", [(1e33, 1e-33, 1e33), (1e36, 1e-36, 1e36), (1e-36, 1e36, 1e-36), (1.0, 1.0, 1e-36),
+                                      (1.0, 1e-36, 1.0), (1.0, 1e18, 1e-36)])
+def test_float32_accuracy_at_the_ends_of_the_range(B, H, T, D, C, R, gq, gv, gd):
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    q, k, v, d_o = (t.to(dev) for t in make_inputs(B, H, T, D, seed=73))
+    q, k, v, d_o = q * gq, k / gq, v * gv, d_o * gd
+    lens = torch.tensor([T - (b * 37) % (T // 2) for b in range(B)], dtype=torch.int32, device=dev)
+    qd, kd, vd = (t.clone().requires_grad_() for t in (q, k, v))
+    out, lse = streaming_attention(qd, kd, vd, lens, C, R, return_lse=True)
+    out.backward(d_o)
+    want = sa_oracle.windowed(q, k, v, lens, C, R, d_out=d_o, dtype=torch.float64)
+    for name, got, ref in zip(("O", "LSE", "dQ", "dK", "dV"), (out, lse, qd.grad, kd.grad, vd.grad), want):
+        rel = ((got.detach().double() - ref).norm() / ref.norm()).item()
+        assert rel <= 32 * 2.0 ** -24, f"{name}: relative error {rel:.2e}"   # as in test_float32_accuracy
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("B", [1, 8, 33])   # 64-row workgroups up to head dimension 64, 128-row ones, more than one round of them
+@pytest.mark.parametrize("dp", [float("inf"), 2.0 ** 128 * (1 - 2.0 ** -10)])   # the latter rounds to an infinite bfloat16
+def test_float32_ds_at_the_end_of_the_range(B, D, dp):
+    """An infinite dS gives signed infinities (NaN against a zero), a finite one that rounds to an infinite bfloat16 finite
+    gradients, as float32 arithmetic does."""
+    dev = torch.device("cuda:0")
+    H, T, C, q0, j0 = 4, 128, 32, 37, 50   # one key tile per chunk; query 37 and key 50 share one
+    g = torch.Generator().manual_seed(3)
+    q, k, v, o, d_o = (torch.zeros(B, H, T, D, device=dev) for _ in range(5))
+    q[..., 0] = (torch.rand(B, H, T, generator=g) + 0.5).to(dev) * 2.0 ** -10   # scores are zero: q and k are orthogonal
+    k[..., 1:] = torch.randn(B, H, T, D - 1, generator=g).to(dev) * 2.0 ** -10
+    v[:, :, j0, 0], d_o[:, :, q0, 0] = 2.0 ** 100, dp * 2.0 ** -100 if dp < float("inf") else 2.0 ** 30
+    lse = torch.zeros(B, H, T, device=dev)   # every probability is one
+    dq, dk, dv = torch.ops.alexdremov_streaming_attention.backward(q, k, v, None, o, lse, d_o, C, 0, 1.0, False, False, "ieee")
+    ds = torch.tensor(dp)
+    want_q, want_k = ds * k[:, :, j0].cpu(), ds * q[:, :, q0].cpu()
+    torch.testing.assert_close(dq[:, :, q0].cpu(), want_q, rtol=2.0 ** -20, atol=0, equal_nan=True)
+    torch.testing.assert_close(dk[:, :, j0].cpu(), want_k, rtol=2.0 ** -20, atol=0, equal_nan=True)
+    rest_q, rest_k = dq.clone(), dk.clone()
+    rest_q[:, :, q0], rest_k[:, :, j0] = 0.0, 0.0
+    assert not rest_q.any() and not rest_k.any()
+    assert torch.equal(dv[:, :, 32:64, 0], d_o[:, :, q0, :1].expand(B, H, 32)) and not dv[:, :, :32].any()
