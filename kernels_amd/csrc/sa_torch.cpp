@@ -230,12 +230,13 @@ const c10::TypedOperatorHandle<BackwardOp>& backward_op() {
 }
 
 // Autograd glue of the forward op (src/streaming_attention/kernel.py:1467-1530): saves q, k, v, O, LSE and lens, hands dO to
-// the backward op, lets no gradient flow through the log-sum-exp output (kernel.py:1498).
+// the backward op, lets no gradient flow through the log-sum-exp (kernel.py:1498): it leaves through lse_out, beside the
+// node's one output.  An output marked as not differentiable would be refused by compiled autograd, which takes native
+// nodes without such marks only.
 struct StreamingAttention : torch::autograd::Function<StreamingAttention> {
-  static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k,
-                                                const Tensor& v, const OptTensor& lens, SymInt context_size,
-                                                SymInt back_contexts, double sm_scale, bool autotune, bool return_lse,
-                                                bool prescale_qk, std::string precision) {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                        const OptTensor& lens, SymInt context_size, SymInt back_contexts, double sm_scale, bool autotune,
+                        bool return_lse, bool prescale_qk, std::string precision, Tensor* lse_out) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [o, lse] = forward_op().call(q, k, v, lens, context_size, back_contexts, sm_scale, autotune, return_lse,
                                       prescale_qk, precision);
@@ -245,13 +246,13 @@ struct StreamingAttention : torch::autograd::Function<StreamingAttention> {
     ctx->saved_data["sm_scale"] = sm_scale;
     ctx->saved_data["flags"] = (int64_t)(autotune ? 1 : 0) | (prescale_qk ? 2 : 0);
     ctx->saved_data["precision"] = std::move(precision);
-    ctx->mark_non_differentiable({lse});
-    ctx->set_materialize_grads(false);   // the log-sum-exp never has a gradient: no zeros for it; O's are made in backward
-    return {o, lse};
+    ctx->set_materialize_grads(false);   // a missing gradient of O is made in backward, in O's own type and layout
+    *lse_out = std::move(lse);
+    return o;
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
-    torch::autograd::variable_list out(11);
+    torch::autograd::variable_list out(12);   // one per argument of forward
     const auto saved = ctx->get_saved_variables();
     const Tensor d_o = grads[0].defined() ? grads[0] : at::zeros_like(saved[3]);
     const int64_t flags = ctx->saved_data["flags"].toInt();
@@ -289,9 +290,10 @@ std::tuple<Tensor, Tensor> forward_autograd(const Tensor& q, const Tensor& k, co
     return forward_op().call(q, k, v, lens, std::move(context_size), std::move(back_contexts), sm_scale, autotune, return_lse,
                              prescale_qk, precision);
   }
-  auto r = StreamingAttention::apply(q, k, v, lens, std::move(context_size), std::move(back_contexts), sm_scale, autotune,
-                                     return_lse, prescale_qk, std::string(precision));
-  return {std::move(r[0]), std::move(r[1])};
+  Tensor lse;
+  Tensor o = StreamingAttention::apply(q, k, v, lens, std::move(context_size), std::move(back_contexts), sm_scale, autotune,
+                                       return_lse, prescale_qk, std::string(precision), &lse);
+  return {std::move(o), std::move(lse)};
 }
 
 // Marks the outputs of the backward op as not differentiable a second time: the reference registers no autograd formula

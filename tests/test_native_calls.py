@@ -58,3 +58,14 @@ def test_dense_is_forward_only():
     assert out.requires_grad
     with pytest.raises(RuntimeError, match="no autograd formula"):
         torch.autograd.grad(out.sum(), q)
+
+
+def test_backward_runs_under_compiled_autograd():
+    from torch._dynamo import compiled_autograd
+
+    q = _meta(True)
+    out, lse = _call(q, return_lse=True)
+    assert not lse.requires_grad and lse.grad_fn is None
+    with compiled_autograd._enable(torch.compile(backend="eager")):
+        out.sum().backward()
+    assert q.grad.shape == q.shape

@@ -137,3 +137,22 @@ def test_inside_a_compiled_function():
     assert_close("O", out, 2.0 * ref["O"], torch.float32)
     assert_close("dQ", qd.grad, ref["dQ"], torch.float32)
     assert_close("dV", vd.grad, ref["dV"], torch.float32)
+
+
+def test_compiled_autograd_gives_the_eager_gradients():
+    """The native node under compiled autograd, one graph after another: other values, windows and lengths each time."""
+    from torch._dynamo import compiled_autograd
+
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    for seed, (C, R, lens) in enumerate([(16, 2, None), (16, 2, None), (10, 1, None), (16, 2, [100, 37]), (16, 2, [5, 100])]):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        q, k, v = (torch.randn(2, 3, 100, 64, generator=g, device=dev, requires_grad=True) for _ in range(3))
+        d_o = torch.randn(2, 3, 100, 64, generator=g, device=dev)
+        le = None if lens is None else torch.tensor(lens, dtype=torch.int32, device=dev)
+        want = torch.autograd.grad(streaming_attention(q, k, v, le, C, R), (q, k, v), d_o)
+        out = streaming_attention(q, k, v, le, C, R)
+        with compiled_autograd._enable(torch.compile(backend="eager")):
+            out.backward(d_o)
+        assert all(torch.equal(t.grad, w) for t, w in zip((q, k, v), want))
