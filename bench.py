@@ -108,8 +108,9 @@ def make_inputs(name, device, zeros=False):
                 lens_list=lens_list, B=B, H=H, T=T, D=D, C=C, R=R, dtype=dtype_name)
 
 
-def time_kernels(w, iters, only=None):
-    """Average duration of each kernel (or of those named in `only`) launched on its own through the C ABI, in ms."""
+def time_kernels(w, iters, only=("fwd", "delta", "dq", "dkdv")):
+    """Average duration of each kernel (or of those named in `only`) launched on its own through the C ABI, in ms.  `bwd` is
+    the whole of sa_backward."""
     import torch
     from streaming_attention import _lib
 
@@ -143,9 +144,14 @@ def time_kernels(w, iters, only=None):
                                delta.data_ptr(), dk.data_ptr(), dv.data_ptr(), s4(q), s4(k), s4(v), s4(d_o),
                                B, H, T, D, C, R, scale, dt, st)
 
+    def bwd():
+        return lib.sa_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), lp, ls, o.data_ptr(), d_o.data_ptr(),
+                               lse.data_ptr(), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), s4(q),
+                               s4(k), s4(v), s4(o), s4(d_o), B, H, T, D, C, R, scale, dt, st)
+
     out = {}
-    for name, fn in (("fwd", fwd), ("delta", dlt), ("dq", dqf), ("dkdv", dkv)):
-        if only is not None and name not in only:
+    for name, fn in (("fwd", fwd), ("delta", dlt), ("dq", dqf), ("dkdv", dkv), ("bwd", bwd)):
+        if name not in only:
             continue
         _lib.check(fn(), name)
         torch.cuda.synchronize()
@@ -352,8 +358,7 @@ def tune_sweep(device, iters=10):
 
 def path_sweep(device, iters=10):
     """Per-kernel times of every (dtype, head dimension) family the library serves, on one shape
-    (B=4, H=16, T=4096, context_size=128, back_contexts=4, lens=None): the 16-bit D in {64, 128, 256}
-    kernels next to the first-generation kernels that serve float32 and D in {16, 32}
+    (B=4, H=16, T=4096, context_size=128, back_contexts=4, lens=None), each launched on its own
     (the reference covers the same range from one tuned kernel, src/streaming_attention/kernel.py:196-203,
     1288-1290).  Rates are executed flop (S and dP are computed by both backward kernels) and
     algorithmic HBM bytes."""
@@ -385,6 +390,20 @@ def path_sweep(device, iters=10):
 
 
 VARIANT_NAMES = {"fwd": ["narrow", "pipelined"], "dq": ["narrow", "pipelined"], "dkdv": ["blockskip", "pipelined", "split"]}
+
+
+def step_kernels(lib, dtype, D, C, R):
+    """{kernel: variant} of the launches of one step (`bwd`: one launch for the whole backward pass)."""
+    if dtype == "float32":
+        kind = "float32 instruction" if D == 256 else "bfloat16 parts"
+        return dict.fromkeys(("fwd", "dq", "dkdv") if D <= 128 else ("fwd", "delta", "dq", "dkdv"), kind)
+    if D == 16:
+        return dict.fromkeys(("fwd", "delta", "dq", "dkdv"), "first generation")
+    if D == 256:
+        return {"fwd": "narrow", "dq": "narrow", "dkdv": "split"}
+    variants = {kn: "narrow" if kn != "dkdv" else "blockskip" for kn in ("fwd", "dq", "dkdv")} if D == 32 else \
+        {kn: VARIANT_NAMES[kn][lib.sa_launch_choice(D, C, R, ki)] for ki, kn in enumerate(("fwd", "dq", "dkdv"))}
+    return {"fwd": variants["fwd"], "bwd": "one launch"} if lib.sa_launch_choice(D, C, R, 3) == 1 else variants
 
 
 def measure_workload(name, dev, steps, warmup, kernel_iters, zeros=False, compiled=False):
@@ -467,13 +486,11 @@ def measure_workload(name, dev, steps, warmup, kernel_iters, zeros=False, compil
             torch.cuda.synchronize()
             compiled_ms = (time.perf_counter() - t1) * 1e3 / steps
 
-    kt = time_kernels(w, kernel_iters)
-    lib = _lib.load()
-    variants = {kn: (VARIANT_NAMES[kn][lib.sa_launch_choice(D, C, R, ki)] if w["dtype"] != "float32" and D >= 64
-                     else "first generation")
-                for ki, kn in enumerate(("fwd", "dq", "dkdv"))}
-    # GEMMs each kernel performs per unmasked pair: fwd S,PV; dq S,dP,dQ; dkdv S,dP,dV,dK
-    kernel_flops = {"fwd": 4.0 * D * H * P, "dq": 6.0 * D * H * P, "dkdv": 8.0 * D * H * P}
+    variants = step_kernels(_lib.load(), w["dtype"], D, C, R)
+    # the launches of the step; without the one-launch backward also the delta pass, which most steps do without
+    kt = time_kernels(w, kernel_iters, only={"fwd", "bwd"} if "bwd" in variants else {"fwd", "delta", "dq", "dkdv"})
+    # GEMMs each kernel performs per unmasked pair: fwd S,PV; dq S,dP,dQ; dkdv S,dP,dV,dK; bwd those of dq and dkdv
+    kernel_flops = {"fwd": 4.0 * D * H * P, "dq": 6.0 * D * H * P, "dkdv": 8.0 * D * H * P, "bwd": 14.0 * D * H * P}
     es = 4 if w["dtype"] == "float32" else 2
     N = B * H * T
     tensor = float(N) * D * es
@@ -483,7 +500,9 @@ def measure_workload(name, dev, steps, warmup, kernel_iters, zeros=False, compil
     valid = sum(min(int(L), T) for L in w["lens_list"]) / float(B * T)
     rd, rows = tensor * valid, 4.0 * N
     kernel_bytes = {"fwd": 3.0 * rd + tensor + rows, "delta": 2.0 * tensor + rows,
-                    "dq": 4.0 * rd + 2.0 * rows * valid + tensor, "dkdv": 4.0 * rd + 2.0 * rows * valid + 2.0 * tensor}
+                    "dq": 4.0 * rd + 2.0 * rows * valid + tensor, "dkdv": 4.0 * rd + 2.0 * rows * valid + 2.0 * tensor,
+                    "bwd": 5.0 * rd + rows * valid + 3.0 * tensor + rows}
+    kernel_flops, kernel_bytes = ({n: x for n, x in d.items() if n in kt} for d in (kernel_flops, kernel_bytes))
     # per step every tensor once: forward reads q, k, v and writes O; backward reads q, k, v, O, dO and
     # writes dQ, dK, dV; lse and delta are written and read once each
     step_bytes = 8.0 * rd + 4.0 * tensor + 4.0 * rows
@@ -587,9 +606,10 @@ def main():
                        "hbm_gbs": PEAK_HBM_GBS},
         "kernel_ms": kt,
         "kernel_variants": m["kernel_variants"],
-        "kernel_ms_note": ("each kernel launched on its own through the C ABI; for this dtype and head dimension the step's "
-                           "backward forms delta inside the dQ kernel and does not launch the delta pass timed here"
-                           if w["dtype"] != "float32" and D >= 64 else "each kernel launched on its own through the C ABI"),
+        "kernel_ms_note": ("each kernel launched on its own through the C ABI; the step's backward forms delta inside the dQ "
+                           "kernel and does not launch the delta pass timed here"
+                           if "delta" in kt and "delta" not in m["kernel_variants"] else
+                           "each kernel launched on its own through the C ABI"),
         "kernel_tflops": m["kernel_tflops"],
         "kernel_gbs": m["kernel_gbs"],
         "roofline": m["roofline"],

@@ -283,6 +283,10 @@ int sa_query(int what) {
 }
 
 int sa_launch_choice(int D, int context_size, int back_contexts, int kernel) {
+  if (kernel == 3) {
+    if (!fused_backward_exists<__bf16>(D) || context_size < 1 || back_contexts < 0) return -1;
+    return fused_backward(D, context_size, back_contexts) ? 1 : 0;
+  }
   if ((D != 64 && D != 128 && D != 256) || context_size < 1 || back_contexts < 0 || kernel < 0 || kernel > 2) return -1;
   const LaunchChoice c = launch_choice(D, context_size, back_contexts);
   return kernel == 0 ? c.fwd : kernel == 1 ? c.dq : c.dkdv;

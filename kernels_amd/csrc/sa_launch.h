@@ -79,7 +79,7 @@ constexpr bool kAsmKernels = false;
 constexpr bool kAsmKernels = true;
 #endif
 inline LaunchChoice launch_choice(int D, int chunk, int back) {
-  // head dimension 256 has one shape per kernel
+  // head dimension 256 has one shape per kernel, variant 0 whatever it is called elsewhere (dK/dV: dkdv_split_wide_kernel)
   if (D == 256) return LaunchChoice{FWD_NARROW, DQ_NARROW, DKDV_BLOCKSKIP};
   LaunchChoice c = (D == 128 ? TUNE_D128 : TUNE_D64)[chunk_class(chunk)][window_class(chunk, back)];
   const int o0 = g_tune_override[0].load(std::memory_order_relaxed);

@@ -68,6 +68,25 @@ def test_query_and_error_strings(lib):
         assert len(lib.sa_error_string(code)) > 10
 
 
+def test_launch_choice_names_the_one_launch_backward(lib):
+    """Kernel 3 answers for sa_backward: short windows run one launch unless a variant of the launches it replaces is pinned."""
+    def rows(C, R):   # query rows that a workgroup of 128 keys goes through, in tiles of 64, over all positions of the pattern
+        return max(64 * (-(-((128 * i + 127) // C + R + 1) * C // 64) - 128 * i // C * C // 64) for i in range(C))
+
+    for C in [*range(1, 34), 50, 64, 65, 100, 112, 127, 128, 129, 160, 256, 319, 320, 321]:
+        for R in range(33):
+            few = rows(C, R) if C * (R + 1) <= 320 else 1 << 30
+            assert lib.sa_launch_choice(64, C, R, 3) == (few <= 320), (C, R)
+            assert lib.sa_launch_choice(32, C, R, 3) == (few <= 256), (C, R)
+    assert lib.sa_launch_choice(64, 1, 2 ** 31 - 1, 3) == 0 and lib.sa_launch_choice(64, 2 ** 31 - 1, 2 ** 31 - 1, 3) == 0
+    assert lib.sa_launch_choice(256, 32, 2, 3) == -1 and lib.sa_launch_choice(64, 0, 2, 3) == -1
+    assert lib.sa_launch_choice(64, 32, -1, 3) == -1
+    for kernel in (1, 2):
+        assert lib.sa_tune_override(kernel, 0) == 0
+        assert lib.sa_launch_choice(64, 32, 2, 3) == 0
+        assert lib.sa_tune_override(kernel, -1) == 0
+
+
 def test_validation_codes_without_gpu(lib):
     """Bad arguments are rejected on the host, before any HIP call."""
     st = (ctypes.c_int64 * 4)(8 * 16 * 64, 16 * 64, 64, 1)
