@@ -6,10 +6,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype,eps", [(torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)])
-@pytest.mark.parametrize("B,H,T,C,R", [(513, 1, 129, 1000, 1), (257, 1, 511, 33, 31), (16, 8, 1100, 1100, 0)])
+# windows of at least 1024 keys after both have been limited to T: shorter ones take whole tiles.  Lengths of 129 (one row past a
+# workgroup) and 1100 end in the first half of a 64-key tile, 511 in the second.
+@pytest.mark.parametrize("B,H,T,C,R", [(513, 1, 129, 33, 31), (513, 1, 129, 1000, 1000), (257, 1, 511, 33, 31), (16, 8, 1100, 1100, 0)])
 def test_forward_halves(B, H, T, C, R, dtype, eps):
     from streaming_attention import streaming_attention
 
+    assert min(C, T) * (min(R, T) + 1) >= 1024 and B * H * -(-T // 128) > 1024
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(5)
     q, k, v = (torch.randn(B, H, T, 64, generator=g, device=dev).to(dtype) for _ in range(3))

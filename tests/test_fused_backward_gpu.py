@@ -9,16 +9,18 @@ from tests.helpers import assert_close, make_inputs
 pytestmark = pytest.mark.gpu
 
 
-# rows that a workgroup walks: 128, 192, 256, 320 (all chosen at D=64; the last not at D=32); a chunk that ends far beyond the
-# workgroup's rows (the own key rows are then read from memory again); 384: the two launches
-@pytest.mark.parametrize("C,R", [(128, 0), (32, 2), (64, 2), (10, 9), (100, 0), (50, 2)])
+# query rows that a workgroup walks: up to 320 are chosen at D=64, up to 256 at D=32, 384 run the two launches.  Chunks of 112 and
+# 256 end more than a tile beyond a workgroup's rows, whose own key rows are then read from memory again.
+@pytest.mark.parametrize("C,R,rows", [(128, 0, 128), (32, 2, 192), (64, 2, 256), (256, 0, 256), (10, 9, 320), (112, 0, 320),
+                                      (100, 0, 384), (50, 2, 384)])
 @pytest.mark.parametrize("T,lens", [(1, [1, 1]), (64, [64, 3]), (129, [129, 128]), (193, [0, 65]), (700, [700, 385])])
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
-def test_one_launch_backward(dtype, D, T, lens, C, R):
+def test_one_launch_backward(dtype, D, T, lens, C, R, rows):
     from streaming_attention import _lib
 
     lib = _lib.load()
+    assert lib.sa_launch_choice(D, C, R, 3) == (rows <= (320 if D == 64 else 256))
     dev = torch.device("cuda:0")
     B, H = 2, 3
     q, k, v, d_o = make_inputs(B, H, T, D, seed=81, dtype=dtype)
