@@ -220,12 +220,30 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
   fwd_rows<T, D, NW, TK>(p, bh, qt, threadIdx.x);
 }
 
+// LDS of the form that goes through a tile of 64 keys half a tile at a time with both halves of K at hand (the first
+// half's step looks for a maximum in the second half's scores): five slots of 32 rows.  Step 0 of a tile uses K0, V0 and K1
+// and sends for the tile's V1 and the next tile's K1; step 1 uses K1 and V1 and sends for the next tile's K0 and V0.  A slot
+// is sent for once the barrier at the beginning of a step shows that every wave is past its last use.
+struct Fwd2Slots {
+  static constexpr int ROWS = 5 * 32, K0 = 0, V0 = 1;
+  int k1 = 2, v1 = 3;
+  SA_DEV int free() const { return 9 - k1 - v1; }   // the V1 of the tile before
+  SA_DEV void advance() {
+    const int next = free();
+    v1 = k1;
+    k1 = next;
+  }
+};
+
 // Forward kernel for 16-bit elements with swizzled tiles (D = 32, 64, 128 or 256).
 //
-// Head dimension 256 takes tiles of 32 keys: one score block and 64 KiB of LDS leave room for two waves per SIMD, one
-// of which multiplies while the other one is at its exponentials.  With tiles of 64 keys a wave needed more than 256
-// registers and had its SIMD to itself.  B=4, H=16, T=4096, bfloat16: chunks of 128, 4 back 277 -> 221 us (728 TFLOP/s),
-// chunks of 10, 9 back 157 -> 111, one chunk of 4096 1331 -> 899 (1223 TFLOP/s); B*H=16, T=600 19.0 -> 16.5 us.
+// Head dimension 256 goes through a tile of 64 keys half a tile at a time: one score block and 80 KiB of LDS (Fwd2Slots)
+// leave room for two waves per SIMD, one of which multiplies while the other one is at its exponentials; on whole tiles a
+// wave needed more than 256 registers and had its SIMD to itself.  The maximum stays that of the whole tile, so that the
+// largest probability of a row's first tile is exactly 1 in the element type and the results are those of whole tiles, bit
+// for bit unless a later tile moves a maximum.  (A maximum of each half's own took O 0.2 to 1.5 % further from the
+// exact result.)  B=4, H=16, T=4096, bfloat16: chunks of 128, 4 back 266 -> 217 us (743 TFLOP/s), chunks of 10, 9 back,
+// ragged 150 -> 105; 2 x 16, one chunk of 4096, ragged 475 -> 339; with each half's own maximum 218, 104, 326.
 //
 // Same algorithm as fwd_kernel, different resource balance: each wave owns QB blocks of 32
 // queries, so every K / V fragment fetched from LDS feeds QB MFMAs (the transposing V reads
@@ -236,25 +254,28 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
 // and masks are decided per 32-key block instead of per tile, and a wave's first tile goes straight
 // to the search for its maximum.  Long windows run the plain form, whose loop is a few per cent
 // tighter (fewer registers, no per-block tests).
-// A wave goes through a tile SB keys at a time.  At head dimension 64 half a tile instead of a whole one takes 118
-// registers instead of 143: four waves per SIMD instead of three (fwd_halves, in the launcher, says where that pays).
-template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT, int SB>
+// Half tiles at head dimension 64 (four waves per SIMD instead of three) are up to 6 % slower than whole ones; with each half's
+// own maximum they were up to 6 % faster on full grids, 15 % slower where half the workgroups were padding, and less exact.
+template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT>
 __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const FwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ && NST >= 2 && (NST - 2) * 2 * AsyncTile<T, D, TK, NW>::PER_WAVE < 64, "swizzled 16-bit tiles; the loads of NST-2 tiles fit the load counter");
+  constexpr bool HALVES = D == 256;
+  constexpr int SB = HALVES ? 32 : TK;     // keys that a wave goes through at a time
   constexpr int WQ = QB * 32, TQ = NW * WQ, NT = NW * 64, KBN = SB / 32;
   constexpr int NF = G::NF, DB = G::DB;
+  static_assert(!HALVES || TK == 64, "a half continues the sums of the one before");
   constexpr int TILE = TK * D;            // elements per K or V tile
   constexpr int STAGE = 2 * TILE;
   constexpr float kRescaleGap = 8.0f;
   constexpr float kSumLimit = 256.0f;
-  using Loader = AsyncTile<T, D, TK, NW, (D == 256)>;
+  using Loader = AsyncTile<T, D, SB, NW, HALVES>;
   constexpr int LPT = 2 * Loader::PER_WAVE;   // async loads per wave per stage (K and V)
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  T* smem = reinterpret_cast<T*>(smem_raw);  // [stage][K|V][TK][D]
+  T* smem = reinterpret_cast<T*>(smem_raw);  // [stage][K|V][TK][D], or the slots
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
@@ -322,9 +343,24 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
     ldv.advance();
   };
   // prologue: NST-1 tiles in flight
+  if constexpr (!HALVES) {
 #pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (kt0 + i < kt1) issue_tile(kt0 + i);
+    for (int i = 0; i < NST - 1; ++i)
+      if (kt0 + i < kt1) issue_tile(kt0 + i);
+  }
+  // Fwd2Slots: a block that no query of the workgroup sees is not sent for
+  Fwd2Slots slots;
+  auto seen = [&](int k0) { return k0 + SB > lo_wg && k0 < hi_wg; };
+  auto send = [&](const Loader& ld, int blocks_ahead, int slot) {
+    Loader at = ld;
+    at.soff += blocks_ahead * ld.tstep;
+    at.issue(smem + slot * SB * D, wave);
+  };
+  if constexpr (HALVES) {   // ldk and ldv stay at the first block of the next tile
+    if (seen(kt0 * TK)) send(ldk, 0, Fwd2Slots::K0), send(ldv, 0, Fwd2Slots::V0);
+    if (seen(kt0 * TK + SB)) send(ldk, 1, slots.k1);
+    ldk.soff += 2 * ldk.tstep, ldv.soff += 2 * ldv.tstep;
+  }
 
   Frag qf[QB][NF];
 #pragma unroll
@@ -353,79 +389,147 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   wait_all_loads();   // Q fragments (and, as loads complete in order, the first tiles)
 
   for (int t = kt0; t < kt1; ++t) {
-    // tile t has landed once at most the loads of the younger tiles are outstanding: NST-2 of them, fewer
-    // near the end of the window
-    wait_tiles<LPT, NST - 2>(kt1 - 1 - t);
-    __syncthreads();   // every wave's share is visible; stage (t-1) % NST is free again
-    if (t + NST - 1 < kt1) issue_tile(t + NST - 1);
-
-    const T* Kt = smem + ((t - kt0) % NST) * STAGE;
-    const T* Vt = Kt + TILE;
+    if constexpr (!HALVES) {
+      // tile t has landed once at most the loads of the younger tiles are outstanding: NST-2 of them, fewer
+      // near the end of the window
+      wait_tiles<LPT, NST - 2>(kt1 - 1 - t);
+      __syncthreads();   // every wave's share is visible; stage (t-1) % NST is free again
+      if (t + NST - 1 < kt1) issue_tile(t + NST - 1);
+    }
+    auto key_block = [&](int sb) {
+      if constexpr (HALVES) return smem + (sb == 0 ? Fwd2Slots::K0 : slots.k1) * SB * D;
+      else return smem + ((t - kt0) % NST) * STAGE + sb * D;
+    };
+    auto value_block = [&](int sb) {
+      if constexpr (HALVES) return smem + (sb == 0 ? Fwd2Slots::V0 : slots.v1) * SB * D;
+      else return smem + ((t - kt0) % NST) * STAGE + TILE + sb * D;
+    };
+    float rs[QB][2];   // sums of the tile's probabilities
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) rs[qb][0] = rs[qb][1] = 0.0f;
 #pragma unroll
     for (int sb = 0; sb < TK; sb += SB) {
+    if constexpr (HALVES) {
+      const bool k1_next = t + 1 < kt1 && seen((t + 1) * TK + SB);
+      if (sb != 0 && k1_next) wait_loads<Loader::PER_WAVE>();   // V1 was sent for before it
+      else wait_loads<0>();
+      __syncthreads();
+      if (sb == 0) {
+        if (seen(t * TK + SB)) send(ldv, -1, slots.v1);
+        if (k1_next) send(ldk, 1, slots.free());
+      } else if (t + 1 < kt1) {
+        send(ldk, 0, Fwd2Slots::K0);
+        send(ldv, 0, Fwd2Slots::V0);
+        ldk.soff += 2 * ldk.tstep, ldv.soff += 2 * ldv.tstep;
+      }
+    }
     const int k0 = t * TK + sb;
     // the workgroup's key range is the union over its waves; skip what this wave cannot see
     if (k0 + SB <= lo_min || k0 >= hi_max) continue;
 
     // S^T[key][q] = K Q^T for the QB query blocks
     f32x16 s[QB][KBN];
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int kb = 0; kb < KBN; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[qb][kb][i] = 0.0f;
     // Short windows end inside a tile: a 32-key block that no query of this wave can see is left
     // out of both products and of the arithmetic, one that every query sees in full needs no mask.
-    bool live[KBN], inside[KBN], all_live = true;
+    bool live[KBN];
+    auto scores = [&](int sb, int k0) {
 #pragma unroll
-    for (int kb = 0; kb < KBN; ++kb) {
-      const int kb0 = SHORT ? k0 + kb * 32 : k0, kbn = SHORT ? 32 : SB;   // the block, or all of them
-      live[kb] = !SHORT || (kb0 + kbn > lo_min && kb0 < hi_max);
-      inside[kb] = kb0 >= lo_max && kb0 + kbn <= hi_min;
-      all_live = all_live && live[kb];
-    }
-    if (all_live) {
-      mma_rows_n<T, D>(s, Kt, sb, qf, lane);
-    } else {
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int kb = 0; kb < KBN; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[qb][kb][i] = 0.0f;
+      bool inside[KBN], all_live = true;
 #pragma unroll
       for (int kb = 0; kb < KBN; ++kb) {
-        if (live[kb]) {
-          f32x16 one[QB][1];
+        const int kb0 = SHORT ? k0 + kb * 32 : k0, kbn = SHORT ? 32 : SB;   // the block, or all of them
+        live[kb] = !SHORT || HALVES || (kb0 + kbn > lo_min && kb0 < hi_max);
+        inside[kb] = kb0 >= lo_max && kb0 + kbn <= hi_min;
+        all_live = all_live && live[kb];
+      }
+      if (all_live) {
+        mma_rows_n<T, D>(s, key_block(sb), 0, qf, lane);
+      } else {
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) one[qb][0] = s[qb][kb];
-          mma_rows_n<T, D>(one, Kt, sb + kb * 32, qf, lane);
+        for (int kb = 0; kb < KBN; ++kb) {
+          if (live[kb]) {
+            f32x16 one[QB][1];
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) s[qb][kb] = one[qb][0];
-        } else {
+            for (int qb = 0; qb < QB; ++qb) one[qb][0] = s[qb][kb];
+            mma_rows_n<T, D>(one, key_block(sb), kb * 32, qf, lane);
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb)
+            for (int qb = 0; qb < QB; ++qb) s[qb][kb] = one[qb][0];
+          } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[qb][kb][i] = -INFINITY;
+            for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) s[qb][kb][i] = -INFINITY;
+          }
         }
+      }
+      // keys outside [lo, hi) score -inf (whatever the product gave, NaN from padding included)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int kb = 0; kb < KBN; ++kb) {
+          if (live[kb] && !inside[kb]) {
+            const uint32_t rm = row_mask(lo[qb] - (k0 + kb * 32), hi[qb] - (k0 + kb * 32), h);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[qb][kb][i] = keep_or_neg_inf(s[qb][kb][i], keep_bits(rm, i));
+          }
+        }
+    };
+    auto largest = [&](int qb) {
+      float mk[KBN], mx = -INFINITY;   // one chain per key block, so that consecutive instructions are independent
+#pragma unroll
+      for (int kb = 0; kb < KBN; ++kb) mk[kb] = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 16; i += 2)
+#pragma unroll
+        for (int kb = 0; kb < KBN; ++kb) mk[kb] = fast_max3(mk[kb], s[qb][kb][i], s[qb][kb][i + 1]);
+#pragma unroll
+      for (int kb = 0; kb < KBN; ++kb) mx = fast_max(mx, mk[kb]);
+      return mx;
+    };
+
+    // A wave none of whose lanes has a maximum yet (its first visible tile) goes straight to the
+    // search: the speculative pass would be thrown away, and short windows are all first tiles.
+    bool fresh = SHORT || HALVES;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) fresh = fresh && __builtin_amdgcn_ballot_w64(m_run[qb] != -INFINITY) == 0;
+    // A maximum is that of a tile.  Half a tile at a time, the first half looks for it in the second half's scores too,
+    // formed once more for that; a wave without a maximum sets it beforehand and needs no search.
+    const bool other = HALVES && sb == 0 && k0 + SB < hi_max;
+    float mx_other[QB];
+    if (HALVES && fresh) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) mx_other[qb] = -INFINITY;
+      if (other) {
+        scores(SB, k0 + SB);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) mx_other[qb] = largest(qb);
+      }
+    }
+    scores(sb, k0);
+    if (HALVES && fresh) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float mx = half_max(fast_max(mx_other[qb], largest(qb))) * sl2e;
+        m_run[qb] = mx > -INFINITY ? mx : -INFINITY;   // NaN: none
       }
     }
 
     Frag pb[QB][KBN][2];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      // keys outside [lo, hi) score -inf (whatever the product gave, NaN from padding included)
-#pragma unroll
-      for (int kb = 0; kb < KBN; ++kb) {
-        if (live[kb] && !inside[kb]) {
-          const uint32_t rm = row_mask(lo[qb] - (k0 + kb * 32), hi[qb] - (k0 + kb * 32), h);
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s[qb][kb][i] = keep_or_neg_inf(s[qb][kb][i], keep_bits(rm, i));
-        }
-      }
       // Probabilities relative to the running maximum as it stands.  The maximum is only looked
       // for when they show that it has been left behind: a tile whose probabilities of one half
       // row add up to at most kSumLimit holds no score more than log2(kSumLimit) above it, which
       // is harmless in fp32 and in the 16-bit operand (the result does not depend on which
       // maximum is subtracted).  Lanes without a maximum yet always look for one.
-      float rs[2];
+      float before[2] = {rs[qb][0], rs[qb][1]};   // the sums of the tile's first half
       auto probabilities = [&](float m_use) {
-        rs[0] = rs[1] = 0.0f;
+        rs[qb][0] = before[0], rs[qb][1] = before[1];
 #pragma unroll
         for (int kb = 0; kb < KBN; ++kb) {
           if (!live[kb]) continue;   // never multiplied
@@ -433,38 +537,24 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
 #pragma unroll
           for (int i = 0; i < 16; ++i) pr[i] = fast_exp2(__builtin_fmaf(s[qb][kb][i], sl2e, -m_use));
           pack_c<T>(pb[qb][kb], pr);
-#ifdef SA_FWD2_DOT_SUMS
-          rs[0] = sum_frag(pb[qb][kb][0], rs[0]);
-          rs[1] = sum_frag(pb[qb][kb][1], rs[1]);
-#else
           // plain float32 additions in two chains: the two-element dot products that could add up the rounded
           // values at half the instruction count stall against the MFMAs in flight
 #pragma unroll
-          for (int i = 0; i < 16; i += 2) rs[0] += pr[i], rs[1] += pr[i + 1];
-#endif
+          for (int i = 0; i < 16; i += 2) rs[qb][0] += pr[i], rs[qb][1] += pr[i + 1];
         }
       };
-      // A wave none of whose lanes has a maximum yet (its first visible tile) goes straight to the
-      // search: the speculative pass would be thrown away, and short windows are all first tiles.
-      const bool fresh = SHORT && __builtin_amdgcn_ballot_w64(m_run[qb] != -INFINITY) == 0;
-      bool search = fresh;
-      if (!fresh) {
+      bool search = !HALVES && fresh;
+      if (HALVES || !fresh) {
         probabilities(m_run[qb] == -INFINITY ? 0.0f : m_run[qb]);
-        const bool behind = !(rs[0] + rs[1] <= kSumLimit) || m_run[qb] == -INFINITY;   // true for NaN too
-        search = __builtin_amdgcn_ballot_w64(behind) != 0;
+        const bool behind = !(rs[qb][0] + rs[qb][1] <= kSumLimit) || m_run[qb] == -INFINITY;   // true for NaN too
+        search = __builtin_amdgcn_ballot_w64(behind) != 0 && !(HALVES && fresh);
       }
       if (search) {
-        float mx = -INFINITY;
-        {
-          float mk[KBN];   // one chain per key block, so that consecutive instructions are independent
-#pragma unroll
-          for (int kb = 0; kb < KBN; ++kb) mk[kb] = -INFINITY;
-#pragma unroll
-          for (int i = 0; i < 16; i += 2)
-#pragma unroll
-            for (int kb = 0; kb < KBN; ++kb) mk[kb] = fast_max3(mk[kb], s[qb][kb][i], s[qb][kb][i + 1]);
-#pragma unroll
-          for (int kb = 0; kb < KBN; ++kb) mx = fast_max(mx, mk[kb]);
+        float mx = largest(qb);
+        if (other) {
+          scores(SB, k0 + SB);
+          mx = fast_max(mx, largest(qb));
+          scores(sb, k0);
         }
         mx = half_max(mx) * sl2e;
         const bool move = mx > m_run[qb] + kRescaleGap;   // false for mx = -inf or NaN
@@ -473,6 +563,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
           m_run[qb] = move ? mx : m_run[qb];
           l_run[qb] *= alpha;
           if (!fresh) {   // a fresh wave has accumulated nothing yet
+            if (HALVES) before[0] *= alpha, before[1] *= alpha;
 #pragma unroll
             for (int m = 0; m < DB; ++m)
 #pragma unroll
@@ -481,7 +572,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
           probabilities(m_run[qb] == -INFINITY ? 0.0f : m_run[qb]);
         }
       }
-      l_run[qb] += rs[0] + rs[1];
+      if (!HALVES) l_run[qb] += rs[qb][0] + rs[qb][1];
     }
 
     // O^T[d][q] += V^T P^T
@@ -491,9 +582,13 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
       Frag bq[QB][2];
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) bq[qb][0] = pb[qb][kb][0], bq[qb][1] = pb[qb][kb][1];
-      mma_tr_n<T, D>(oacc, Vt, sb / 32 + kb, bq, lane);
+      mma_tr_n<T, D>(oacc, value_block(sb), kb, bq, lane);
     }
     }
+    if (HALVES)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) l_run[qb] += rs[qb][0] + rs[qb][1];
+    if constexpr (HALVES) slots.advance();
   }
 
   // ---- epilogue --------------------------------------------------------------------

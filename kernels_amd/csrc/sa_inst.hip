@@ -96,20 +96,14 @@ template <typename P> static bool half_workgroups(const P& p) {
 #endif
 
 #if SA_KIND == 0
-// Head dimension 64: half a tile at a time, four waves per SIMD, where the grid has more workgroups than three per SIMD
-// take at once; below that a launch is as long as one of its waves, which is faster on whole tiles.  Whole -> half, us.
-// Long windows: 1152 workgroups, T=1500 dense, ragged 42.6 -> 41.6; 2048 of 512 and 1 back 69.4 -> 67.8; 3072, T=2048 dense
-// 136.3 -> 135.7; 2 x 8 x T=16384, 300 and 6 back 174.0 -> 170.6; on the other side 576 46.8 -> 46.3, 432 29.5 -> 30.1, 192
-// 28.1 -> 30.2, 80 19.0 -> 20.3.  Short windows keep whole tiles: chunks of 32, 2 back, T=3000 427 -> 439.
-static bool fwd_halves(const FwdParams& p) { return (int64_t)p.B * p.H * ceil_div(p.T, 128) > 1024; }
-template <int D, int NW, bool SHORT, bool HALVES = false> static int fwd2_launch(FwdParams p, hipStream_t st) {
+template <int D, int NW, bool SHORT> static int fwd2_launch(FwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * C::FWD2_QB * 32;
   // tile stages; the epilogue's row patches (one per wave) reuse the same memory
-  constexpr size_t stages = (size_t)C::FWD2_NST * 2 * C::fwd2_tk(D) * D * sizeof(ElemT);
+  constexpr size_t stages = (D == 256 ? (size_t)Fwd2Slots::ROWS : (size_t)C::FWD2_NST * 2 * C::FWD_TK) * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
-  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, C::fwd2_tk(D), C::FWD2_NST, SHORT, HALVES ? 32 : C::fwd2_tk(D)>;
+  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, C::FWD_TK, C::FWD2_NST, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
@@ -162,9 +156,6 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
     }
     // windows of less than 1024 keys (the table's first two window classes) run the short-window form
     if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
-    if constexpr (D == 64) {
-      if (fwd_halves(p)) return fwd2_launch<D, C::NARROW_NW, false, true>(p, st);
-    }
     return fwd2_launch<D, C::NARROW_NW, false>(p, st);
   } else if constexpr (C::split(D)) {
     // Head dimension 128: eight waves share one workgroup's two 48 KiB stages, two waves per SIMD, once that makes a

@@ -147,8 +147,6 @@ template <typename T> struct Cfg {
 #else
   static constexpr int FWD_TK = sizeof(T) == 4 ? 32 : 64;        // keys per forward step
 #endif
-  // keys per step of fwd2_kernel: at 256 a block of 32 is what fits beside the accumulators of two waves per SIMD
-  static constexpr int fwd2_tk(int D) { return D == 256 ? 32 : FWD_TK; }
   static constexpr int DQ_TK = 32;                               // keys per dQ step
   static constexpr int DKDV_TQ = 32;                             // queries per dK/dV step
 };
