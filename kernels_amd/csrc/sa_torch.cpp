@@ -446,6 +446,16 @@ PyObject* py_self_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// kernel_layout(tensor): what the kernels get for it.
+PyObject* py_kernel_layout(PyObject*, PyObject* t) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(THPVariable_Check(t), "kernel_layout takes a tensor");
+  const Tensor& x = THPVariable_Unpack(t);
+  TORCH_CHECK_VALUE(x.dim() == 4, "kernel_layout takes a [B, H, T, D] tensor");
+  return THPVariable_Wrap(kernel_layout(x));
+  END_HANDLE_TH_ERRORS
+}
+
 // Whether the environment routes calls through the compiled wrapper (read on every call: it may change at run time).
 PyObject* py_env_asks_for_wrapper(PyObject*, PyObject*) {
   const char* compiled = getenv("STREAMING_ATTENTION_COMPILED");
@@ -454,6 +464,7 @@ PyObject* py_env_asks_for_wrapper(PyObject*, PyObject*) {
 }
 
 PyMethodDef methods[] = {
+    {"kernel_layout", py_kernel_layout, METH_O, nullptr},
     {"env_asks_for_wrapper", py_env_asks_for_wrapper, METH_NOARGS, nullptr},
     {"streaming_attention", (PyCFunction)(void (*)())py_streaming_attention, METH_FASTCALL, nullptr},
     {"self_attention", (PyCFunction)(void (*)())py_self_attention, METH_FASTCALL, nullptr},

@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 
 try:
-    from . import _native  # noqa: F401  (registers the ops)
+    from ._native import kernel_layout as _kernel_layout  # noqa: F401  (the module registers the ops)
 except ImportError as e:
     raise ImportError(
         "streaming_attention._native cannot be loaded: build it with `make -C kernels_amd/csrc` "
@@ -25,29 +25,6 @@ except ImportError as e:
     ) from e
 
 _HEAD_DIMS = (16, 32, 64, 128, 256)
-_VEC_BYTES = 16
-
-
-def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
-    """The layout rule of the native code, in Python: ``t`` itself when the kernels can read it in place (unit stride along the head
-    dimension, every other stride and the base address a multiple of 16 bytes, a non-zero stride
-    along T), otherwise a contiguous copy.  The 16-bit kernels for head dimensions 32 and up
-    address the rows of one (batch, head) slice with 32-bit byte offsets (a contiguous tensor is
-    within that range up to tens of millions of positions); the other kernels have no such limit."""
-    es = t.element_size()
-    offsets32 = es == 2 and t.shape[-1] >= 32
-    if t.is_contiguous() and t.data_ptr() % _VEC_BYTES == 0 and t.shape[-1] * es % _VEC_BYTES == 0 \
-            and (not offsets32 or (t.shape[-2] + 1024) * t.shape[-1] * es < 2**32):
-        return t          # the common case, without looking at every stride
-    vec = _VEC_BYTES // es
-    ok = (
-        t.stride(-1) == 1
-        and all(s % vec == 0 for s in t.stride()[:-1])
-        and (t.stride(-2) > 0 or t.shape[-2] <= 1)
-        and t.data_ptr() % _VEC_BYTES == 0
-        and (not offsets32 or (t.shape[-2] + 1024) * t.stride(-2) * es < 2**32)
-    )
-    return t if ok else t.contiguous()
 
 
 def _validate_placement(q, k, v, lens, *others):

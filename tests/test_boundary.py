@@ -231,6 +231,37 @@ def test_kernel_layout_rule():
     assert _kernel_layout(odd).is_contiguous()
 
 
+def test_kernel_layout_is_the_native_rule():
+    """The rule that calls run, not a second one beside it, at the limits of what is read in place."""
+    from streaming_attention import _native, ops
+
+    layout = ops._kernel_layout
+    assert layout is _native.kernel_layout
+    for dtype in (torch.float16, torch.bfloat16, torch.float32):
+        vec = 16 // torch.empty(0, dtype=dtype).element_size()
+        flat = torch.arange(4 * 4 * 16 * 96, dtype=torch.float32).to(dtype)
+        in_place = [flat.as_strided((2, 3, 16, 64), (4 * 16 * 64 + vec, 16 * 64 + vec, 64 + vec, 1)),
+                    flat.as_strided((2, 3, 16, 64), (0, 0, 64, 1)),                    # expanded batches and heads
+                    flat.as_strided((2, 3, 1, 64), (64, 64, 0, 1)),                    # a single row, whatever its stride
+                    flat[vec:].as_strided((2, 3, 16, 64), (4096, 1024, 64, 1), vec)]
+        copied = [flat.as_strided((2, 3, 16, 64), (4 * 16 * 64, 16 * 64, 64 + vec // 2, 1)),
+                  flat.as_strided((2, 3, 16, 64), (4 * 16 * 64, 16 * 64 + 1, 64, 1)),
+                  flat.as_strided((2, 3, 16, 64), (4 * 16 * 64 + 1, 16 * 64, 64, 1)),
+                  flat.as_strided((2, 3, 16, 64), (4 * 16 * 64, 16 * 64, 0, 1)),       # one row for all positions
+                  flat.as_strided((2, 3, 16, 64), (4096, 1024, 64, 1), vec // 2)]      # contiguous, base 8 bytes off
+        for x in in_place:
+            assert layout(x) is x
+        for x in copied:
+            y = layout(x)
+            assert y.is_contiguous() and y.data_ptr() % 16 == 0 and y.data_ptr() != x.data_ptr() and torch.equal(y, x)
+    # 32-bit byte offsets, with 1024 rows to spare: 16-bit types from head dimension 32 on
+    step = 2 ** 31 // 1026 // 8 * 8
+    wide = torch.empty(2 * (step + 8), dtype=torch.float16)
+    assert layout(x := wide.as_strided((1, 1, 2, 32), (8, 8, step, 1))) is x
+    assert layout(x := wide.as_strided((1, 1, 2, 16), (8, 8, step + 8, 1))) is x
+    assert layout(wide.as_strided((1, 1, 2, 32), (8, 8, step + 8, 1))).is_contiguous()
+
+
 def test_bench_rejects_more_than_one_gpu():
     out = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True,
                          text=True, timeout=300)
