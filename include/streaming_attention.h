@@ -34,7 +34,8 @@
  *     operator passed: their probabilities differ from the forward's by about |score| * 2^-9 (bf16) /
  *     2^-12 (fp16) relative, inside the 16-bit accuracy bar.  Forward and dQ scale in float32.
  *   - float32 at D <= 128: every product is formed from three bfloat16 parts per operand, which hold all 24
- *     significand bits, and summed in float32; a non-finite input element gives NaN wherever it is used.
+ *     significand bits, and summed in float32.  What leaves the range of that (infinities, elements or sums beyond
+ *     about 2^80) is computed with the float32 instruction, so it gives what float32 arithmetic gives.
  */
 #ifndef STREAMING_ATTENTION_H
 #define STREAMING_ATTENTION_H
