@@ -6,9 +6,10 @@
 // is going to see (its own and the neighbours' in reach, whose O and dO rows the neighbouring
 // workgroups of the same XCD read at about the same time), walks the key tiles of its queries (dq2_kernel's
 // loop, three stages), picks up its own K and V rows from the tiles that are still in LDS, and walks the query tiles of
-// its keys (dkdv2_kernel's loop).  A row that is read again ten microseconds later has left the 4 MiB L2 of its XCD
-// at this rate, which is why the pick-up counts: with two stages and the rows read again the kernel fetched
-// ten tensors instead of five (counters) and gained half as much.
+// its keys (dkdv2_kernel's loop).  A row that is read again ten microseconds later has mostly left the 4 MiB L2 of its XCD
+// at this rate, which is why the pick-up counts: with two stages and the rows read again the kernel gained half as
+// much.  Counters on the first problem below: 8.0 tensors fetched where five are needed and three written (192 rows in reach
+// make the loads of a workgroup 11 tensors' worth); the two launches fetched 10.9 and wrote 3.1.
 //
 // B=128, H=12, T=3000, D=64, chunks of 32, 2 back (float16): 1370 us in two launches, 1083 here, 4.4 TB/s of the eight tensors
 // (a copy reaches 4.9); the same without the products 946.  B=8, H=16, T=4096, D=64, one chunk of 128: 160 -> 127 us.

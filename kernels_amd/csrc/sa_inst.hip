@@ -66,10 +66,12 @@ template <int D> constexpr size_t float_tiles = (size_t)2 * 2 * 32 * TileGeom<fl
 
 // float32, head dimensions 16 to 64: workgroups of 64 rows (two waves) instead of 128 where twice as many still find a CU
 // each and their windows are at least a tenth shorter -- such a launch takes as long as one workgroup, and that as long as
-// its tiles.  Half the threads stage a tile, which costs 3 to 8 % where the window stays the same.  Forward and backward in
-// us, 128 rows -> 64: B*H=8, T=512, D=32, chunks of 64, 2 back 12.6, 32.5 -> 9.8, 24.9; B*H=32, T=512, D=64 (128 workgroups)
-// 17.8, 47.4 -> 15.4, 40.6; B*H=4, T=300, D=64, chunks of 16, 3 back 14.7, 38.2 -> 11.2, 28.5.  On the other side of the
-// rule: chunks of 128, 1 back, B*H=8, T=1024 17.4, 46.6 -> 18.8, 48.1; 192 workgroups (B*H=48, T=512) 17.9, 48.7 -> 20.0, 49.1.
+// its tiles.  Forward and backward in us, 128 rows -> 64, at D=16; 32; 64.  Chunks of 64, 2 back, B*H=8, T=512 11.2, 27.7 ->
+// 9.3, 22.2; 12.6, 33.0 -> 10.3, 25.9; 17.4, 47.5 -> 15.1, 39.3, and with 128 workgroups (B*H=32) 11.3, 28.0 -> 9.5, 22.8; 12.8,
+// 33.7 -> 10.5, 26.7; 17.7, 48.8 -> 15.5, 41.0; chunks of 10, 9 back, 128 workgroups 12.6, 29.0 -> 10.7, 25.6; 15.1, 35.9 -> 12.5,
+// 30.1; 20.4, 51.3 -> 18.1, 45.7.  On the other side of the rule: the same window (chunks of 128, 1 back, B*H=8, T=1024) 11.6, 28.7 ->
+// 11.4, 27.9; 12.9, 34.1 -> 12.6, 32.1; 17.4, 48.1 -> 18.9, 49.2 (half the threads stage a tile); 192 workgroups (B*H=48, T=512)
+// 11.5, 28.3 -> 11.9, 30.5; 13.0, 34.0 -> 13.7, 37.8; 17.9, 49.3 -> 20.6, 50.3.
 template <typename P> static bool half_workgroups(const P& p) {
   if ((int64_t)p.B * p.H * ceil_div(p.T, 128) > 128) return false;
   const int64_t back = std::min((int64_t)p.C * p.R, (int64_t)1 << 32);   // ten times it stays within 64 bits
