@@ -141,17 +141,6 @@ SA_DEV float fast_max3(float a, float b, float c) {
   return r;
 }
 
-// acc + the sum of the eight 16-bit values of a fragment: four dot products with (1, 1), i.e.
-// half a vector instruction per element, and the sum is over the rounded values that the
-// following matrix product consumes.
-SA_DEV float sum_frag(bf16x8 f, float acc) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    acc = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{f[2 * j], f[2 * j + 1]}, one, acc, false);
-  return acc;
-}
 // acc + the dot product of two fragments, two elements per instruction, products and sums in float32
 SA_DEV float dot_frag(bf16x8 a, bf16x8 b, float acc) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -165,14 +154,6 @@ SA_DEV float dot_frag(f16x8 a, f16x8 b, float acc) {
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     acc = __builtin_amdgcn_fdot2(f16x2{a[2 * j], a[2 * j + 1]}, f16x2{b[2 * j], b[2 * j + 1]}, acc, false);
-  return acc;
-}
-SA_DEV float sum_frag(f16x8 f, float acc) {
-  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-  const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    acc = __builtin_amdgcn_fdot2(f16x2{f[2 * j], f[2 * j + 1]}, one, acc, false);
   return acc;
 }
 
