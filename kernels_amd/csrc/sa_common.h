@@ -678,16 +678,23 @@ template <typename T> SA_DEV void store4(T* dst, float a, float b, float c, floa
   *reinterpret_cast<typename Elem<T>::Quad*>(dst) = q;
 }
 
+// Whole rows of a result are stored past the caches (the non-temporal hint): nothing of the launch reads them again, and
+// kept in the 4 MiB L2 of an XCD they push out the rows of Q, K, V and dO that neighbouring workgroups are about to read.
+// Forward and backward in us, plain -> non-temporal: B=16, H=8, T<=2048, D=128, chunks of 64, 1 back, strongly ragged (half
+// of the stores are zeros of padding) 137 -> 119; B=225, H=4, T<=993, D=32, chunks of 16, 2 back 129 -> 121; B=128, H=12,
+// T=3000, D=64, chunks of 32, 2 back 1535 -> 1495 (with O kept in the caches for the backward pass 1508); B=8, H=16, T=4096,
+// D=64, chunks of 128, 4 back 440 -> 430; B=4, H=16, D=128, T<=16384 3365 -> 3340.  Not for stores of part of a row: the float32
+// kernels' 16 bytes per lane with the hint 2040 -> 2170, and not for loads (rows of Q and O, a quarter per instruction: 251 -> 266,
+// 1495 -> 1548).
+SA_DEV void store_streaming(void* dst, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst)); }
+
 // Zero rows [row0, row1) of a contiguous [*, D] matrix with the whole workgroup.
 template <typename T, int D, int NT> SA_DEV void zero_rows(T* base, int row0, int row1, int tid) {
   using E = Elem<T>;
   constexpr int CPR = D / E::VEC;
   const int total = (row1 - row0) * CPR;
-  typename E::Frag z;
-#pragma unroll
-  for (int e = 0; e < E::VEC; ++e) z[e] = (T)0.0f;
   for (int ch = tid; ch < total; ch += NT)
-    *reinterpret_cast<typename E::Frag*>(base + (int64_t)row0 * D + (int64_t)ch * E::VEC) = z;
+    store_streaming(base + (int64_t)row0 * D + (int64_t)ch * E::VEC, u32x4{0, 0, 0, 0});
 }
 
 // Transposed store of DB accumulator blocks holding X^T[d][row] into X[row][d]:
@@ -733,7 +740,7 @@ SA_DEV void store_rows_coalesced(T* patch, T* out_rows, int rows_valid, const f3
   for (int j = 0; j < 32 / P::RPI; ++j) {
     const int row = j * P::RPI + rr;
     const u32x4 v16 = *reinterpret_cast<const u32x4*>(patch + row * P::PITCH + ch * 8);
-    if (row < rows_valid) *reinterpret_cast<u32x4*>(out_rows + (int64_t)row * D + ch * 8) = v16;
+    if (row < rows_valid) store_streaming(out_rows + (int64_t)row * D + ch * 8, v16);
   }
 }
 
