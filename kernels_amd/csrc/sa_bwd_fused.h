@@ -14,6 +14,8 @@
 // B=128, H=12, T=3000, D=64, chunks of 32, 2 back (float16): 1370 us in two launches, 1083 here, 4.4 TB/s of the eight tensors
 // (a copy reaches 4.9); the same without the products 946.  B=8, H=16, T=4096, D=64, one chunk of 128: 160 -> 127 us.
 // B=16, H=8, T=2048 ragged, D=64, chunks of 64, 1 back: 46 -> 39.  B=225, H=4, T=993 ragged, D=32, chunks of 16, 2 back: 94 -> 92.
+// Two waves and 32-row tiles instead of four and 64 where that reads no more rows per row of its own (and at D = 32 on
+// windows that lie across the 32-row blocks): fused_backward_in_two_waves in sa_launch.h has the rule and both sides' times.
 // A form that slides along a sequence and reads every row once (scores formed once, dS handed over in LDS) took 967 us
 // on the first problem and up to twice as long on windows of more than four 32-row blocks: one workgroup per CU, steps
 // in lockstep.
@@ -22,8 +24,8 @@
 
 namespace sa {
 
-struct BwdFused {
-  static constexpr int NW = 4, ROWS = NW * 32, TT = 64, NST = 3;
+template <int NW_, int TT_> struct BwdFused {
+  static constexpr int NW = NW_, ROWS = NW * 32, TT = TT_, NST = 3;
   // two stages, then the third or the row patches of the dQ store, then lse and delta of `rows` query rows
   template <typename T, int D> static constexpr int rows_offset() {
     constexpr int stage = 2 * TT * D * (int)sizeof(T), patches = NW * RowPatch<T, D>::ELEMS * (int)sizeof(T);
@@ -32,21 +34,22 @@ struct BwdFused {
   template <typename T, int D> static constexpr size_t lds_bytes(int rows) { return rows_offset<T, D>() + 2 * rows * sizeof(float); }
 };
 
-template <typename T, int D>
-__global__ __launch_bounds__(256, (D == 64 ? 3 : 1)) void bwd_fused_kernel(const BwdParams p) {
+template <typename T, int D, int NW, int TT>
+__global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(const BwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ, "swizzled 16-bit tiles");
-  constexpr int NW = BwdFused::NW, ROWS = BwdFused::ROWS, TT = BwdFused::TT, NT = NW * 64;
+  using Shape = BwdFused<NW, TT>;
+  constexpr int ROWS = Shape::ROWS, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB, TILE = TT * D, STAGE = 2 * TILE;
   constexpr int PG = D == 64 ? 2 : 4;   // see dkdv2_kernel
   using Loader = AsyncTile<T, D, TT, NW, true>;
-  constexpr int NST = BwdFused::NST, LPT = 2 * Loader::PER_WAVE;
+  constexpr int NST = Shape::NST, LPT = 2 * Loader::PER_WAVE;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
-  float* lse_s = reinterpret_cast<float*>(smem_raw + BwdFused::rows_offset<T, D>());
+  float* lse_s = reinterpret_cast<float*>(smem_raw + Shape::template rows_offset<T, D>());
   float* delta_s = lse_s + p.fused_rows;
 
   const int tid = threadIdx.x;
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 3 : 1)) void bwd_fused_kernel(const
   // ---- lse and delta of the query rows in reach, at their places in the tiles from qt0 on (rows beside them are masked) --
   const int d0 = qt0 * TT;
   {
-    constexpr int LPR = D / 8, RPP = NT / LPR, U = 256 / RPP;   // lanes per row, rows per pass, passes in flight
+    constexpr int LPR = D / 8, RPP = NT / LPR, U = 256 / RPP < 8 ? 256 / RPP : 8;   // lanes per row, rows per pass, passes in flight
     const int sub = tid % LPR, nd = q_hi(g_last) - d0;
     for (int base = 0; base < nd; base += RPP * U) {
       Frag of[U], gf[U];
@@ -169,13 +172,13 @@ __global__ __launch_bounds__(256, (D == 64 ? 3 : 1)) void bwd_fused_kernel(const
       dq2_tile<T, D, TT>(acc, Kt, Kt + TILE, t * TT, wq, qf, gf, sl2e, lse_q, dinit, lane);
     }
     // the last three key tiles are still in LDS: as a rule the workgroup's own rows are among them
-    if (kt1 * TT <= r0 + ROWS + TT) {
+    if (kt1 * TT <= r0 + NST * TT) {
       const int own = (r0 + wave * 32) / TT;                       // this wave's tile, from one to three back
       const int back = kt1 - own;
       int s2 = st - back;                                           // st is one past the last tile's stage
       s2 = s2 < 0 ? s2 + NST : s2;
       if (wave_live) {
-        const T* Kt = smem + s2 * STAGE + (wave & 1) * 32 * D;
+        const T* Kt = smem + s2 * STAGE + wave * 32 % TT * D;
 #pragma unroll
         for (int g = 0; g < NF; ++g) {
           kf[g] = *reinterpret_cast<const Frag*>(Kt + G::off(c, (g * 2 + h) * E::VEC));

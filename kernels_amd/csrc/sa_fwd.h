@@ -254,6 +254,12 @@ struct Fwd2Slots {
 // and masks are decided per 32-key block instead of per tile, and a wave's first tile goes straight
 // to the search for its maximum.  Long windows run the plain form, whose loop is a few per cent
 // tighter (fewer registers, no per-block tests).
+// SHORT with tiles of 32 keys and two waves: windows of about a hundred keys are bound by what surrounds the products (the
+// tile set-up, edge masks, waits at barriers for tiles that a wave does not see), and 119 registers (D = 64; 90 at D = 32) and
+// 16 KiB of LDS let twice as many waves hide it (forward_in_two_waves in sa_launch.h: the rule, and both sides' times).
+// B=128, H=12, T=1354, D=64, chunks of 10, 9 back: 248 -> 229 us (4.65 TB/s of its four tensors; without products 220, without
+// tile loads 220 before).  The same with three stages 253, with one wave 262; tiles of 64 and two waves 281.  O is 0.4 to 4 % nearer
+// to the exact result (float16 2.774e-4 -> 2.742e-4 there), as the second tile's maximum is taken too.
 // Half tiles at head dimension 64 (four waves per SIMD instead of three) are up to 6 % slower than whole ones; with each half's
 // own maximum they were up to 6 % faster on full grids, 15 % slower where half the workgroups were padding, and less exact.
 template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT>
@@ -262,7 +268,8 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
   static_assert(G::SWZ && NST >= 2 && (NST - 2) * 2 * AsyncTile<T, D, TK, NW>::PER_WAVE < 64, "swizzled 16-bit tiles; the loads of NST-2 tiles fit the load counter");
-  constexpr bool HALVES = D == 256;
+  constexpr bool HALVES = D == 256, BLOCKS = SHORT && TK == 32;
+  static_assert(BLOCKS || TK == 64, "whole tiles of 64 keys, or of 32 on short windows");
   constexpr int SB = HALVES ? 32 : TK;     // keys that a wave goes through at a time
   constexpr int WQ = QB * 32, TQ = NW * WQ, NT = NW * 64, KBN = SB / 32;
   constexpr int NF = G::NF, DB = G::DB;
@@ -388,6 +395,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   }
   wait_all_loads();   // Q fragments (and, as loads complete in order, the first tiles)
 
+  int tiles_seen = 0;   // BLOCKS: tiles that this wave has gone through
   for (int t = kt0; t < kt1; ++t) {
     if constexpr (!HALVES) {
       // tile t has landed once at most the loads of the younger tiles are outstanding: NST-2 of them, fewer
@@ -497,6 +505,11 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
     bool fresh = SHORT || HALVES;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) fresh = fresh && __builtin_amdgcn_ballot_w64(m_run[qb] != -INFINITY) == 0;
+    // Tiles of 32 keys: the first maximum is that of few keys, so the second tile that a wave sees always looks for its
+    // own, and moves to it by however little; the largest probability of each is then exactly 1 in the element type, as on
+    // tiles of 64.  (Without this O came out up to 1 % further from the exact result.)
+    const bool settle = BLOCKS && !fresh && tiles_seen == 1;
+    if (BLOCKS) ++tiles_seen;
     // A maximum is that of a tile.  Half a tile at a time, the first half looks for it in the second half's scores too,
     // formed once more for that; a wave without a maximum sets it beforehand and needs no search.
     const bool other = HALVES && sb == 0 && k0 + SB < hi_max;
@@ -543,8 +556,8 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
           for (int i = 0; i < 16; i += 2) rs[qb][0] += pr[i], rs[qb][1] += pr[i + 1];
         }
       };
-      bool search = !HALVES && fresh;
-      if (HALVES || !fresh) {
+      bool search = !HALVES && (fresh || settle);
+      if (HALVES || !search) {
         probabilities(m_run[qb] == -INFINITY ? 0.0f : m_run[qb]);
         const bool behind = !(rs[qb][0] + rs[qb][1] <= kSumLimit) || m_run[qb] == -INFINITY;   // true for NaN too
         search = __builtin_amdgcn_ballot_w64(behind) != 0 && !(HALVES && fresh);
@@ -557,12 +570,12 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
           scores(sb, k0);
         }
         mx = half_max(mx) * sl2e;
-        const bool move = mx > m_run[qb] + kRescaleGap;   // false for mx = -inf or NaN
-        if (fresh || __builtin_amdgcn_ballot_w64(move) != 0) {
+        const bool move = mx > m_run[qb] + (settle ? 0.0f : kRescaleGap);   // false for mx = -inf or NaN
+        if (fresh || settle || __builtin_amdgcn_ballot_w64(move) != 0) {
           const float alpha = move ? fast_exp2(m_run[qb] - mx) : 1.0f;
           m_run[qb] = move ? mx : m_run[qb];
           l_run[qb] *= alpha;
-          if (!fresh) {   // a fresh wave has accumulated nothing yet
+          if (!fresh && (!settle || __builtin_amdgcn_ballot_w64(move) != 0)) {   // a fresh wave has accumulated nothing yet
             if (HALVES) before[0] *= alpha, before[1] *= alpha;
 #pragma unroll
             for (int m = 0; m < DB; ++m)

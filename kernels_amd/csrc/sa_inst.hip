@@ -98,14 +98,14 @@ template <typename P> static bool half_workgroups(const P& p) {
 #endif
 
 #if SA_KIND == 0
-template <int D, int NW, bool SHORT> static int fwd2_launch(FwdParams p, hipStream_t st) {
+template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * C::FWD2_QB * 32;
   // tile stages; the epilogue's row patches (one per wave) reuse the same memory
-  constexpr size_t stages = (D == 256 ? (size_t)Fwd2Slots::ROWS : (size_t)C::FWD2_NST * 2 * C::FWD_TK) * D * sizeof(ElemT);
+  constexpr size_t stages = (D == 256 ? (size_t)Fwd2Slots::ROWS : (size_t)C::FWD2_NST * 2 * TK) * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
-  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, C::FWD_TK, C::FWD2_NST, SHORT>;
+  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, TK, C::FWD2_NST, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
@@ -157,8 +157,13 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
       if (launch_choice(D, p.C, p.R).fwd == FWD_PIPELINED) return fwd3_launch<D>(p, st);
     }
     // windows of less than 1024 keys (the table's first two window classes) run the short-window form
-    if (window_class(p.C, p.R) <= 1) return fwd2_launch<D, C::NARROW_NW, true>(p, st);
-    return fwd2_launch<D, C::NARROW_NW, false>(p, st);
+    if (window_class(p.C, p.R) <= 1) {
+      if constexpr (D <= 64) {
+        if (forward_in_two_waves(D, p.C, p.R, (int64_t)p.B * p.H * ceil_div(p.T, 128))) return fwd2_launch<D, 2, 32, true>(p, st);
+      }
+      return fwd2_launch<D, C::NARROW_NW, C::FWD_TK, true>(p, st);
+    }
+    return fwd2_launch<D, C::NARROW_NW, C::FWD_TK, false>(p, st);
   } else if constexpr (C::split(D)) {
     // Head dimension 128: eight waves share one workgroup's two 48 KiB stages, two waves per SIMD, once that makes a
     // workgroup per CU; smaller grids run twice as many four-wave workgroups with one stage (B*H=24, T=1024: 34
@@ -423,18 +428,23 @@ template <> int launch_dkdv<ElemT, SA_DGROUP>(const BwdParams& p, int D, hipStre
 #undef X
 }
 #else
+template <int D, int NW, int TT> static int bwd_fused_launch(BwdParams p, hipStream_t st) {
+  using S = BwdFused<NW, TT>;
+  p.fused_rows = rows_in_reach(p.C, p.R, S::ROWS, TT);
+  const size_t lds = S::template lds_bytes<ElemT, D>(p.fused_rows);
+  auto kern = bwd_fused_kernel<ElemT, D, NW, TT>;
+  static PrepareState once;
+  if (int rc = prepare(kern, S::template lds_bytes<ElemT, D>(BWD_FUSED_MAX_ROWS), once)) return rc;
+  p.n_tiles = (int)ceil_div(p.T, S::ROWS);
+  const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int bwd_fused_d(BwdParams p, hipStream_t st) {
   if constexpr (fused_backward_exists<ElemT>(D)) {
-    p.fused_rows = fused_rows(p.C, p.R);
-    const size_t lds = BwdFused::lds_bytes<ElemT, D>(p.fused_rows);
-    auto kern = bwd_fused_kernel<ElemT, D>;
-    static PrepareState once;
-    if (int rc = prepare(kern, BwdFused::lds_bytes<ElemT, D>(BWD_FUSED_MAX_ROWS), once)) return rc;
-    p.n_tiles = (int)ceil_div(p.T, BwdFused::ROWS);
-    const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(BwdFused::NW * 64), lds, st, p);
-    return (int)hipGetLastError();
+    if (fused_backward_in_two_waves(D, p.C, p.R)) return bwd_fused_launch<D, 2, 32>(p, st);
+    return bwd_fused_launch<D, 4, 64>(p, st);
   } else {
     return SA_ERR_HEAD_DIM;
   }

@@ -95,30 +95,61 @@ inline LaunchChoice launch_choice(int D, int chunk, int back) {
   return c;
 }
 
-// The one-launch backward (sa_bwd_fused.h), 16-bit elements.
-template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 32 || D == 64); }
-// Query rows that a workgroup of 128 rows goes through for dK and dV, in whole 64-row tiles: the most over all positions.
-constexpr int BWD_FUSED_MAX_ROWS = 320;
-inline int fused_rows(int chunk, int back) {
-  int period = chunk;   // the pattern repeats after chunk / gcd(chunk, 128) workgroups
-  while (period % 2 == 0 && period > chunk / 128) period /= 2;
+// Rows that a workgroup of `rows` rows goes through for its windows, in whole tiles: the most over all positions.
+inline int rows_in_reach(int chunk, int back, int rows, int tile) {
+  int period = chunk;   // the pattern repeats after chunk / gcd(chunk, rows) workgroups
+  while (period % 2 == 0 && period > chunk / rows) period /= 2;
   int most = 0;
   for (int i = 0; i < period; ++i) {
-    const int first = 128 * i / chunk * chunk / 64, last = ((128 * i + 127) / chunk + back + 1) * chunk;
-    most = (last + 63) / 64 - first > most ? (last + 63) / 64 - first : most;
+    const int first = rows * i / chunk * chunk / tile, last = ((rows * i + rows - 1) / chunk + back + 1) * chunk;
+    most = (last + tile - 1) / tile - first > most ? (last + tile - 1) / tile - first : most;
   }
-  return most * 64;
+  return most * tile;
 }
-// Used while those rows are few: beyond its own 128 a workgroup reads and multiplies rows that belong to its neighbours.
-// Measured against the two launches (B=8, H=16, T=4096, D=64 and batches of the sizes in sa_bwd_fused.h), rows: gain --
-// 128: 1.27; 192: 1.27, 1.17; 256: 1.13; 320: 1.07, 1.01; 384: 0.94; 448: 0.91.  D=32 -- 192: 1.02, 1.05; 320: 0.98; 384: 0.91.
+// Short windows, head dimensions 32 and 64: workgroups of two waves (64 rows, tiles of 32) instead of four (128 rows,
+// tiles of 64).  In the large workgroup every wave waits at the barriers of about twice as many tiles as it sees itself,
+// and half as many waves are resident; the small one goes through more rows per row of its own unless the windows begin and
+// end where its rows do.  So it is taken where that costs nothing (chunks divide 32 or are divided by it, and the
+// rows in reach are no more per row), and where the windows lie across the 32-row blocks, so that the kernel is bound by
+// what it computes, not by what it reads.
+inline bool aligned_chunks(int chunk) { return 32 % chunk == 0 || chunk % 32 == 0; }
+inline bool two_waves_read_no_more(int chunk, int back) {
+  return aligned_chunks(chunk) && 2 * rows_in_reach(chunk, back, 64, 32) <= rows_in_reach(chunk, back, 128, 64);
+}
+// The forward in us, four waves -> two.  D=32, B=225, H=4, T<=993: chunks of 16, 2 back 37.5 -> 29.5; 10, 9 back 48.7 -> 38.1; 64, 1 back
+// 36.8 -> 32.1; 64, 7 back 54.7 -> 52.9; on the other side 128, none back 34.4 -> 32.6 (64 x 8 x 1024: 26.6 -> 26.5), 128, 3 back
+// 53.0 -> 55.5, 10, 40 back 61 -> 55.  D=64, B=128, H=12, T=1354: 10, 9 back 248 -> 229; 50, 1 back 254 -> 228; 10, 20 back 313 -> 307; 16, 2
+// back 189 -> 182; 32, 1 back 188 -> 181; on the other side 32, 2 back 193 -> 197 (64 x 8 x 1024: 55.5 -> 58.0), 64, 2 back 65.9 ->
+// 74.6, 128, none back 53.8 -> 62.2, 10, 40 back 406 -> 424.  Up to 1024 workgroups of 128 rows more of them count for more (16 x 8 x 1024
+// ragged): 32, 2 back 14.1 -> 13.0; 128, none back 14.1 -> 12.2; 64, 2 back 16.1 -> 15.6; but 64, 1 back 14.6 -> 15.4.
+inline bool forward_in_two_waves(int D, int chunk, int back, int64_t workgroups_of_128) {
+  const long long window = (long long)chunk * ((long long)back + 1);
+  if (D == 32) return chunk < 128 && window <= 512;
+  if (D != 64 || window > 256) return false;
+  return workgroups_of_128 <= 1024 || !aligned_chunks(chunk) || two_waves_read_no_more(chunk, back);
+}
+
+// The one-launch backward (sa_bwd_fused.h), 16-bit elements.
+template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 32 || D == 64); }
+// Used while the query rows that a workgroup of 128 rows goes through for dK and dV are few: beyond its own 128 it reads and
+// multiplies rows that belong to its neighbours.  Measured against the two launches (B=8, H=16, T=4096, D=64 and batches of
+// the sizes in sa_bwd_fused.h), rows: gain -- 128: 1.27; 192: 1.27, 1.17; 256: 1.13; 320: 1.07, 1.01; 384: 0.94; 448: 0.91.
+// D=32 -- 192: 1.02, 1.05; 320: 0.98 (1.02 to 1.05 of the whole step at B=225, H=4, T<=993); 384: 0.91.
+constexpr int BWD_FUSED_MAX_ROWS = 320;
 inline bool fused_backward(int D, int chunk, int back) {
   if (!fused_backward_exists<__bf16>(D)) return false;
   // a pinned dQ or dK/dV variant asks for the launches of their own
   if (g_tune_override[1].load(std::memory_order_relaxed) >= 0 || g_tune_override[2].load(std::memory_order_relaxed) >= 0)
     return false;
   if ((long long)chunk * ((long long)back + 1) > BWD_FUSED_MAX_ROWS) return false;
-  return fused_rows(chunk, back) <= (D == 64 ? BWD_FUSED_MAX_ROWS : 256);
+  return rows_in_reach(chunk, back, 128, 64) <= (D == 64 ? BWD_FUSED_MAX_ROWS : 256);
+}
+// Forward and backward in us, four waves -> two.  D=32, B=225, H=4, T<=993: chunks of 16, 2 back 125.4 -> 119.2; 40, 2 back 158.0 -> 148.9;
+// 10, 9 back 157.5 -> 151.7; on the other side 32, 3 back 130.1 -> 128.1 (64 x 8 x 1024: 104.9 -> 111.0), 64, 1 back 124.7 -> 122.2 (98.8 ->
+// 102.4), 128, none back 116.5 -> 122.4.  D=64, B=64, H=12, T=1354: 8, 3 back 339 -> 324; 16, 2 back 335 -> 323; 64, none back 306 -> 293; on the
+// other side 10, 9 back 463 -> 465, 32, 2 back 348 -> 347 (64 x 8 x 1024: 182 -> 189), 32, 3 back 390 -> 396, 128, none back 344 -> 365.
+inline bool fused_backward_in_two_waves(int D, int chunk, int back) {
+  return (D == 32 && !aligned_chunks(chunk)) || two_waves_read_no_more(chunk, back);
 }
 
 template <typename T> struct Cfg {
