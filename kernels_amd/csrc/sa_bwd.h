@@ -580,47 +580,48 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
     ldk.advance();
     ldv.advance();
   };
-#pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (kt0 + i < kt1) issue_tile(kt0 + i);
+  // This wave's Q rows go where the second tile will be; its dO rows beside the stages or, where a third stage's worth
+  // of LDS would cost a resident workgroup, where the first tile will be, which is then sent for once they have been read.
+  using Rows = OwnRows<T, D>;
+  static_assert(NST == 2 && NW * 32 == 2 * TK, "the rows of a workgroup fill a stage");
+  constexpr bool OVER = D >= 128;
+  const int wrow0 = q0 + wave * 32;
+  T* const q_area = smem + STAGE + wave * Rows::ELEMS;
+  T* const g_area = smem + (OVER ? 0 : NST * STAGE) + wave * Rows::ELEMS;
+  const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
+  Rows::send(reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh, p.q_st, wrow0, L - 1, q_area, lane);
+  Rows::send(gbase, p.do_st, wrow0, L - 1, g_area, lane);
+  // delta = rowsum(O * dO) is formed here when the caller has not run the delta kernel
+  // (no branch around the loads: a value defined on one side only is copied where the sides join, and the copy
+  // waits for the load; without a row of O to read, the dO row is read)
+  RowDots<T, D> dots;
+  dots.load(p.delta_out ? reinterpret_cast<const T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh : gbase,
+            p.delta_out ? p.o_st : p.do_st, wrow0, L - 1, lane);
+  const float lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qrow] : INFINITY;   // rows past L: P = exp2(-inf) = 0
+  if (!OVER) issue_tile(kt0);
 
   Frag qf[NF], gf[NF];
-  float lse_q, delta_q;
-  {
-    const int qr = qrow < L ? qrow : L - 1;
-    const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
-                  (int64_t)qr * p.q_st;
-    const T* gp = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh +
-                  (int64_t)qr * p.do_st;
-    // delta = rowsum(O * dO) is formed here when the caller has not run the delta kernel: this lane holds half
-    // of its query's dO row, so the forward output is fetched in the same pattern, in flight together with the
-    // other rows, and the two halves are added across lanes
-    // (no branch around the loads: a value defined on one side only is copied where the sides join, and the copy
-    // waits for the load; without a row of O to read, the dO row is read twice)
-    Frag of[NF];
-    const T* op = p.delta_out ? reinterpret_cast<const T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh +
-                                    (int64_t)qr * p.o_st
-                              : gp;
+  float delta_q;
+  landed();
 #pragma unroll
-    for (int g = 0; g < NF; ++g) of[g] = *reinterpret_cast<const Frag*>(op + (g * 2 + h) * E::VEC);
-#pragma unroll
-    for (int g = 0; g < NF; ++g) {
-      qf[g] = *reinterpret_cast<const Frag*>(qp + (g * 2 + h) * E::VEC);
-      if (neg) qf[g] = negate<T>(qf[g]);
-      // dO enters negated: the dP accumulator starts at delta and ends at delta - dP, which
-      // saves the subtraction per element; the sign is put back by the scale of the store
-      gf[g] = negate<T>(*reinterpret_cast<const Frag*>(gp + (g * 2 + h) * E::VEC));
-    }
-    lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qr] : INFINITY;   // rows past L: P = exp2(-inf) = 0
-    float osum = 0.0f;
-#pragma unroll
-    for (int g = 0; g < NF; ++g) osum = dot_frag(of[g], gf[g], osum);
-    delta_q = -half_sum(osum);
-    if (p.delta_out) {
-      if (h == 0 && qrow < T_) p.delta_out[(int64_t)bh * T_ + qrow] = qrow < L ? delta_q : 0.0f;
-    } else {
-      delta_q = p.delta[(int64_t)bh * T_ + qr];
-    }
+  for (int g = 0; g < NF; ++g) {
+    qf[g] = Rows::read(q_area, g, lane);
+    if (neg) qf[g] = negate<T>(qf[g]);
+    // dO enters negated: the dP accumulator starts at delta and ends at delta - dP, which
+    // saves the subtraction per element; the sign is put back by the scale of the store
+    gf[g] = negate<T>(Rows::read(g_area, g, lane));
+  }
+  float* const sums = reinterpret_cast<float*>(q_area);
+  dots.partial(g_area, sums, lane);
+  if (OVER) {
+    __syncthreads();
+    issue_tile(kt0);
+  }
+  if (p.delta_out) {
+    delta_q = RowDots<T, D>::total(sums, lane);
+    if (h == 0 && qrow < T_) p.delta_out[(int64_t)bh * T_ + qrow] = qrow < L ? delta_q : 0.0f;
+  } else {
+    delta_q = p.delta[(int64_t)bh * T_ + qe];
   }
   f32x16 dinit;
 #pragma unroll
@@ -748,27 +749,27 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
     ldq.advance();
     ldg.advance();
   };
-#pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (qt0 + i < qt1) issue_tile(qt0 + i);
+  // This wave's K rows go where the second tile will be, its V rows beside the stages.
+  using Rows = OwnRows<T, D>;
+  static_assert(NST == 2 && NW * 32 == 2 * TQ, "the rows of a workgroup fill a stage");
+  T* const k_area = reinterpret_cast<T*>(smem_raw + STAGE_BYTES) + wave * Rows::ELEMS;
+  T* const v_area = reinterpret_cast<T*>(smem_raw + NST * STAGE_BYTES) + wave * Rows::ELEMS;
+  const int wrow0 = k0 + wave * 32;
+  Rows::send(reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh, p.k_st, wrow0, L - 1, k_area, lane);
+  Rows::send(reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh, p.v_st, wrow0, L - 1, v_area, lane);
+  issue_tile(qt0);
 
   Frag kf[NF], vf[NF];
-  {
-    const int kr = krow < L ? krow : L - 1;
-    const T* kp = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
-                  (int64_t)kr * p.k_st;
-    const T* vp = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
-                  (int64_t)kr * p.v_st;
+  landed();
 #pragma unroll
-    for (int g = 0; g < NF; ++g) {
-      // K enters multiplied by -scale*log2(e), rounded to the element type: the score accumulator
-      // starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability
-      kf[g] = *reinterpret_cast<const Frag*>(kp + (g * 2 + h) * E::VEC);
+  for (int g = 0; g < NF; ++g) {
+    // K enters multiplied by -scale*log2(e), rounded to the element type: the score accumulator
+    // starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability
+    kf[g] = Rows::read(k_area, g, lane);
 #pragma unroll
-      for (int e = 0; e < E::VEC; ++e) kf[g][e] = (T)((float)kf[g][e] * kmul);
-      // V enters negated: the dP accumulator starts at delta and ends at delta - dP
-      vf[g] = negate<T>(*reinterpret_cast<const Frag*>(vp + (g * 2 + h) * E::VEC));
-    }
+    for (int e = 0; e < E::VEC; ++e) kf[g][e] = (T)((float)kf[g][e] * kmul);
+    // V enters negated: the dP accumulator starts at delta and ends at delta - dP
+    vf[g] = negate<T>(Rows::read(v_area, g, lane));
   }
 
   f32x16 dk[DB], dv[DB];

@@ -123,32 +123,35 @@ __global__ __launch_bounds__(512) void dkdv_split_kernel(const BwdParams p) {
     ldq.advance();
     ldg.advance();
   };
+  // this wave's rows go where the third tile and the exchange slots will be
+  using Rows = OwnRows<T, D>;
+  T* const area = reinterpret_cast<T*>(smem_raw + (NST - 1) * STAGE_BYTES) + wave * Rows::ELEMS;
+  if (!grad_role)
+    Rows::send(reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh, p.k_st, k0 + pair * 32, L - 1, area, lane);
+  else
+    Rows::send(reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh, p.v_st, k0 + pair * 32, L - 1, area, lane);
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
     if (qt0 + i < qt1) issue_tile(qt0 + i, i * STAGE_BYTES);
 
   // resident fragments: K for the score role, V for the grad role
   Frag rf[NF];
+  landed();
   {
-    const int kr = krow < L ? krow : L - 1;
     const float kmul = -p.scale_log2e;
     if (!grad_role) {
-      const T* kp = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
-                    (int64_t)kr * p.k_st;
 #pragma unroll
       for (int g = 0; g < NF; ++g) {
         // K enters multiplied by -scale*log2(e), rounded to the element type: the score accumulator
         // starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability
-        rf[g] = *reinterpret_cast<const Frag*>(kp + (g * 2 + h) * E::VEC);
+        rf[g] = Rows::read(area, g, lane);
 #pragma unroll
         for (int e = 0; e < E::VEC; ++e) rf[g][e] = (T)((float)rf[g][e] * kmul);
       }
     } else {
-      const T* vp = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
-                    (int64_t)kr * p.v_st;
       // V enters negated: the dP accumulator starts at delta and ends at delta - dP
 #pragma unroll
-      for (int g = 0; g < NF; ++g) rf[g] = negate<T>(*reinterpret_cast<const Frag*>(vp + (g * 2 + h) * E::VEC));
+      for (int g = 0; g < NF; ++g) rf[g] = negate<T>(Rows::read(area, g, lane));
     }
   }
 
@@ -406,30 +409,35 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
     ldq.advance();
     ldg.advance();
   };
-  issue_tile(qt0, 0);
-  if (qt0 + 1 < qt1) issue_tile(qt0 + 1, 1);
+  // this wave's rows first, over the rings
+  using Rows = OwnRows<T, D>;
+  static_assert(NW * Rows::ELEMS * sizeof(T) <= S::lds, "rows of all waves");
+  T* const area = q_ring + wave * Rows::ELEMS;
+  if (grad_role)
+    Rows::send(reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh, p.v_st, k0 + pair * 32, L - 1, area, lane);
+  else
+    Rows::send(reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh, p.k_st, k0 + pair * 32, L - 1, area, lane);
+  landed();
 
   // resident fragments: K * (-scale * log2 e) for the score role, -V for the grad role (see dkdv2_kernel)
   Frag rf[1][NF];
   {
-    const T* rp = grad_role ? reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh +
-                                  (int64_t)valid(krow) * p.v_st
-                            : reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh +
-                                  (int64_t)valid(krow) * p.k_st;
     const float mul = grad_role ? -1.0f : -p.scale_log2e;
 #pragma unroll
     for (int g = 0; g < NF; ++g) {
-      rf[0][g] = *reinterpret_cast<const Frag*>(rp + (g * 2 + h) * E::VEC);
+      rf[0][g] = Rows::read(area, g, lane);
 #pragma unroll
       for (int e = 0; e < E::VEC; ++e) rf[0][g][e] = (T)((float)rf[0][g][e] * mul);
     }
   }
+  __syncthreads();
+  issue_tile(qt0, 0);
+  if (qt0 + 1 < qt1) issue_tile(qt0 + 1, 1);
   f32x16 acc[1][DB];   // dV^T[d][key] (score role) or -dK^T[d][key] (grad role)
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[0][m][i] = 0.0f;
-  wait_all_loads();
 
   // lse (which = 0) or delta (which = 1) of the 16 rows of tile t that this lane holds in a C fragment
   auto rows16 = [&](int t, int which, f32x16& out) {

@@ -555,6 +555,65 @@ template <int LPT, int MAXA> SA_DEV void wait_tiles(int ahead) {
   }
 }
 
+// The 32 rows that a wave keeps as operand fragments, through 32 * D elements of LDS of its own.  Fragment g of a lane is
+// sixteen bytes of its row, so a load straight from memory touches 32 rows and a quarter of a cache line of each; the lines come
+// in four times over once the waves of a CU have more of them in flight than the 32 KiB first-level cache holds.  Here
+// the rows arrive as copies of whole rows and are read from LDS.  Cycles from the first load to the last fragment at
+// D = 256: Q, dO and O of dq2_kernel 18800 of the 82500 of a workgroup, K and V of dkdv_split_wide_kernel 14600 of 95200.
+// Rows past the last valid one come as zeros.  The copies are assembly: the caller waits (landed) before it reads.
+template <typename T, int D> struct OwnRows {
+  using G_ = TileGeom<T, D>;
+  using Frag = typename Elem<T>::Frag;
+  using Copy = AsyncTile<T, D, 32, 1, true>;
+  static constexpr int ELEMS = 32 * D;
+  SA_DEV static void send(const T* base, int64_t row_stride, int row0, int last_row, T* area, int lane) {
+    Copy rows;
+    rows.init(base, row_stride, row0, last_row, 0, lane);
+    rows.issue(area, 0);
+  }
+  SA_DEV static Frag read(const T* area, int g, int lane) {
+    return *reinterpret_cast<const Frag*>(area + G_::off(lane & 31, (g * 2 + (lane >> 5)) * Elem<T>::VEC));
+  }
+};
+// every load and copy of this wave has arrived, and the compiler reads no LDS ahead of that
+SA_DEV void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// this wave's LDS reads are done; a barrier may follow after which others overwrite what it read
+SA_DEV void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// Row sums of the products of 32 rows of O, from memory in whole rows, with those of dO in the layout of OwnRows.
+template <typename T, int D> struct RowDots {
+  using G_ = TileGeom<T, D>;
+  using Frag = typename Elem<T>::Frag;
+  static constexpr int CPR = G_::CPR, RPI = 64 / CPR, N = 32 / RPI, PITCH = CPR + 4;
+  static_assert(32 * PITCH * sizeof(float) <= OwnRows<T, D>::ELEMS * sizeof(T), "the scratch fits where the rows were");
+  Frag of[N];
+  SA_DEV void load(const T* base, int64_t row_stride, int row0, int last_row, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int r = row0 + i * RPI + lane / CPR;
+      r = r < last_row ? r : last_row;
+      of[i] = *reinterpret_cast<const Frag*>(base + (int64_t)r * row_stride + lane % CPR * 8);
+    }
+  }
+  // partial sums into 32 * PITCH floats of LDS of this wave's own
+  SA_DEV void partial(const T* g_area, float* scratch, int lane) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = i * RPI + lane / CPR, ch = lane % CPR;
+      const Frag gf = *reinterpret_cast<const Frag*>(g_area + G_::off(r, ch * 8));
+      scratch[r * PITCH + ch] = dot_frag(of[i], gf, 0.0f);
+    }
+  }
+  // the sum of row lane % 32
+  SA_DEV static float total(const float* scratch, int lane) {
+    const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * (CPR / 2);
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CPR / 2; ++j) sum += row[j];
+    return half_sum(sum);
+  }
+};
+
 // Cooperative copy of a [ROWS][D] row-major global tile into registers and on into an
 // LDS tile.  Rows are clamped to `last_row` so that a ragged final tile reads valid
 // memory (the values are masked by the caller).

@@ -210,7 +210,8 @@ template <> int launch_delta<ElemT, SA_DGROUP>(const DeltaParams& p, int D, hipS
 template <int D, int NW> static int dq2_launch(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * 32;
-  constexpr size_t stages = (size_t)C::DQ2_NST * 2 * C::DQ2_TK * D * sizeof(ElemT);
+  // beside the stages up to head dimension 64: a workgroup's dO rows
+  constexpr size_t stages = (size_t)(C::DQ2_NST + (D <= 64 ? 1 : 0)) * 2 * C::DQ2_TK * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
   auto kern = dq2_kernel<ElemT, D, NW, C::DQ2_TK, C::DQ2_NST>;
@@ -325,7 +326,8 @@ template <int D> static int dkdv_split_launch(BwdParams p, hipStream_t st) {
     constexpr size_t stages = (size_t)NST * (2 * TQ * D * sizeof(ElemT) + 2 * TQ * sizeof(float));
     constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
     static_assert(patches <= stages, "row patches must not reach the exchange slots");
-    constexpr size_t lds = stages + (size_t)4 * 2 * 2048;
+    constexpr size_t rows = stages / NST * (NST - 1) + (size_t)NW * OwnRows<ElemT, D>::ELEMS * sizeof(ElemT);
+    constexpr size_t lds = std::max(stages + (size_t)4 * 2 * 2048, rows);
     auto kern = dkdv_split_kernel<ElemT, D, NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
@@ -379,7 +381,8 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     }
     constexpr int TKB = C::DKDV2_NW * 32;
     constexpr size_t stages =
-        (size_t)C::DKDV2_NST * (2 * C::DKDV2_TQ * D * sizeof(ElemT) + 2 * C::DKDV2_TQ * sizeof(float));
+        (size_t)C::DKDV2_NST * (2 * C::DKDV2_TQ * D * sizeof(ElemT) + 2 * C::DKDV2_TQ * sizeof(float)) +
+        (size_t)C::DKDV2_NW * OwnRows<ElemT, D>::ELEMS * sizeof(ElemT);   // a workgroup's V rows
     constexpr size_t patches = (size_t)C::DKDV2_NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
     constexpr size_t lds = stages > patches ? stages : patches;
     auto kern = dkdv2_kernel<ElemT, D, C::DKDV2_NW, C::DKDV2_TQ, C::DKDV2_NST>;
