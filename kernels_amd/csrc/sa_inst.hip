@@ -232,7 +232,7 @@ template <int D> static int dq3_launch(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D) && D == 128) {
     constexpr int NW = 4, TQ = NW * 64, NST = 4;
-    constexpr size_t stages = (size_t)NST * 2 * 64 * D * sizeof(ElemT);
+    constexpr size_t stages = (size_t)(NST + 1) * 2 * 64 * D * sizeof(ElemT);   // one for half of the dO rows
     constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
     constexpr size_t lds = stages > patches ? stages : patches;
     auto kern = dq3_kernel<ElemT, D, NST>;
@@ -301,7 +301,8 @@ template <int D> static int dkdv3_launch(BwdParams p, hipStream_t st) {
   if constexpr (C::fwd2(D) && D == 128) {
     constexpr int TKB = 128, TQ = 64;
     // tile stages; the epilogue's row patches (one per wave) reuse the same memory
-    constexpr size_t stages = (size_t)C::DKDV3_NST * (2 * TQ * D * sizeof(ElemT) + 2 * TQ * sizeof(float));
+    constexpr size_t stages = (size_t)C::DKDV3_NST * (2 * TQ * D * sizeof(ElemT) + 2 * TQ * sizeof(float)) +
+                              (size_t)4 * OwnRows<ElemT, D>::ELEMS * sizeof(ElemT);   // a workgroup's V rows
     constexpr size_t patches = (size_t)4 * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
     constexpr size_t lds = stages > patches ? stages : patches;
     auto kern = dkdv3_kernel<ElemT, D, C::DKDV3_NST>;
