@@ -108,8 +108,14 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   };
   ld0.init(kbase, p.k_st, kt0 * TT, L - 1, wave, lane);
   ld1.init(vbase, p.v_st, kt0 * TT, L - 1, wave, lane);
+  // this wave's Q and dO rows go where the third and the second tile will be
+  using Rows = OwnRows<T, D>;
+  static_assert(NW * Rows::ELEMS == STAGE, "the rows of a workgroup fill a stage");
+  T* const q_area = smem + 2 * STAGE + wave * Rows::ELEMS;
+  T* const g_area = smem + STAGE + wave * Rows::ELEMS;
+  Rows::send(qbase, p.q_st, r0 + wave * 32, L - 1, q_area, lane);
+  Rows::send(gbase, p.do_st, r0 + wave * 32, L - 1, g_area, lane);
   issue_tile(0);
-  if (kt0 + 1 < kt1) issue_tile(1);
 
   // ---- lse and delta of the query rows in reach, at their places in the tiles from qt0 on (rows beside them are masked) --
   const int d0 = qt0 * TT;
@@ -142,15 +148,15 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   {
     const float sl2e = fabsf(p.scale_log2e);
     Frag qf[NF], gf[NF];
-    const T* qp = qbase + (int64_t)valid(row) * p.q_st;
-    const T* gp = gbase + (int64_t)valid(row) * p.do_st;
+    landed();
 #pragma unroll
     for (int g = 0; g < NF; ++g) {
-      qf[g] = *reinterpret_cast<const Frag*>(qp + (g * 2 + h) * E::VEC);
+      qf[g] = Rows::read(q_area, g, lane);
       if (p.scale_log2e < 0.0f) qf[g] = negate<T>(qf[g]);
-      gf[g] = negate<T>(*reinterpret_cast<const Frag*>(gp + (g * 2 + h) * E::VEC));
+      gf[g] = negate<T>(Rows::read(g_area, g, lane));
     }
-    __syncthreads();   // lse_s, delta_s
+    __syncthreads();   // lse_s, delta_s; the rows have been read
+    if (kt0 + 1 < kt1) issue_tile(1);
     if (tid < ROWS && r0 + tid < T_) p.delta_out[out_row + r0 + tid] = r0 + tid < L ? delta_s[r0 + tid - d0] : 0.0f;
     const float lse_q = row < L ? lse_s[row - d0] : INFINITY;   // rows past L: P = exp2(-inf) = 0
     f32x16 dinit, acc[DB];

@@ -349,8 +349,14 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
     ldk.advance();
     ldv.advance();
   };
+  // This wave's Q rows go where the second tile will be.
+  using Rows = OwnRows<T, D>;
+  static_assert(HALVES || (NST == 2 && QB == 1 && NW * 32 == 2 * TK), "the rows of a workgroup fill a stage");
+  T* const q_area = smem + STAGE + wave * Rows::ELEMS;
+  const T* qbase = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
   // prologue: NST-1 tiles in flight
   if constexpr (!HALVES) {
+    Rows::send(qbase, p.q_st, q0 + wave * WQ, L - 1, q_area, lane);
 #pragma unroll
     for (int i = 0; i < NST - 1; ++i)
       if (kt0 + i < kt1) issue_tile(kt0 + i);
@@ -372,14 +378,18 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   Frag qf[QB][NF];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    const int qr = qrow[qb] < L ? qrow[qb] : L - 1;
-    const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
-                  (int64_t)qr * p.q_st;
+    if constexpr (HALVES) {
+      const T* qp = qbase + (int64_t)(qrow[qb] < L ? qrow[qb] : L - 1) * p.q_st;
 #pragma unroll
-    for (int g = 0; g < NF; ++g) {
-      qf[qb][g] = *reinterpret_cast<const Frag*>(qp + (g * 2 + h) * E::VEC);
-      if (neg) qf[qb][g] = negate<T>(qf[qb][g]);
+      for (int g = 0; g < NF; ++g) qf[qb][g] = *reinterpret_cast<const Frag*>(qp + (g * 2 + h) * E::VEC);
+    } else {
+      landed();
+#pragma unroll
+      for (int g = 0; g < NF; ++g) qf[qb][g] = Rows::read(q_area, g, lane);
     }
+#pragma unroll
+    for (int g = 0; g < NF; ++g)
+      if (neg) qf[qb][g] = negate<T>(qf[qb][g]);
   }
 
   f32x16 oacc[QB][DB];
