@@ -511,12 +511,11 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
-  static_assert(G::SWZ && (NST == 2 || NST == 3), "swizzled 16-bit tiles, 2 or 3 stages");
+  static_assert(G::SWZ, "swizzled 16-bit tiles");
   constexpr int TQ = NW * 32, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TK * D, STAGE = 2 * TILE;
   using Loader = AsyncTile<T, D, TK, NW>;
-  constexpr int LPT = 2 * Loader::PER_WAVE;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
@@ -573,17 +572,16 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   Loader ldk, ldv;
   ldk.init(kbase, p.k_st, kt0 * TK, L - 1, wave, lane);
   ldv.init(vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
-  auto issue_tile = [&](int t) {   // tiles are issued in ascending order
-    T* st = smem + ((t - kt0) % NST) * STAGE;
-    ldk.issue(st, wave);
-    ldv.issue(st + TILE, wave);
-    ldk.advance();
-    ldv.advance();
+  const TileOrder order(kt0, kt1, p.period, p.pdiv);
+  auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
+    T* st = smem + (it & 1) * STAGE;
+    ldk.at(t - kt0).issue(st, wave);
+    ldv.at(t - kt0).issue(st + TILE, wave);
   };
   // This wave's Q rows go where the second tile will be; its dO rows beside the stages or, where a third stage's worth
   // of LDS would cost a resident workgroup, where the first tile will be, which is then sent for once they have been read.
   using Rows = OwnRows<T, D>;
-  static_assert(NST == 2 && NW * 32 == 2 * TK, "the rows of a workgroup fill a stage");
+  static_assert(NST == 2 && NW * 32 == 2 * TK, "two stages; the rows of a workgroup fill one");
   constexpr bool OVER = D >= 128;
   const int wrow0 = q0 + wave * 32;
   T* const q_area = smem + STAGE + wave * Rows::ELEMS;
@@ -598,7 +596,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   dots.load(p.delta_out ? reinterpret_cast<const T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh : gbase,
             p.delta_out ? p.o_st : p.do_st, wrow0, L - 1, lane);
   const float lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qrow] : INFINITY;   // rows past L: P = exp2(-inf) = 0
-  if (!OVER) issue_tile(kt0);
+  if (!OVER) issue_tile(order.first, 0);
 
   Frag qf[NF], gf[NF];
   float delta_q;
@@ -615,7 +613,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   dots.partial(g_area, sums, lane);
   if (OVER) {
     __syncthreads();
-    issue_tile(kt0);
+    issue_tile(order.first, 0);
   }
   if (p.delta_out) {
     delta_q = RowDots<T, D>::total(sums, lane);
@@ -634,13 +632,12 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
     for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
   wait_all_loads();
 
-  for (int t = kt0; t < kt1; ++t) {
-    if (NST == 3 && t + 1 < kt1) wait_loads<LPT>();
-    else wait_loads<0>();
+  for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    wait_loads<0>();
     __syncthreads();
-    if (t + NST - 1 < kt1) issue_tile(t + NST - 1);
+    if (order.next(t) != order.first) issue_tile(order.next(t), it + 1);
 
-    const T* Kt = smem + ((t - kt0) % NST) * STAGE;
+    const T* Kt = smem + (it & 1) * STAGE;
     const T* Vt = Kt + TILE;
     const int k0 = t * TK;
     if (k0 + TK <= win.lo_min || k0 >= win.hi_max) continue;   // outside this wave's windows
@@ -673,7 +670,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   constexpr int PG = D == 64 ? 2 : 4;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
-  static_assert(G::SWZ && (NST == 2 || NST == 3), "swizzled 16-bit tiles, 2 or 3 stages");
+  static_assert(G::SWZ, "swizzled 16-bit tiles");
   constexpr int TKB = NW * 32, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TQ * D;
@@ -682,7 +679,6 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   // stage layout: [Q tile][dO tile][NW chunks of {lse[RPW], delta[RPW]}]
   constexpr int STAGE_BYTES = 2 * TILE * (int)sizeof(T) + 2 * TQ * (int)sizeof(float);
   using Loader = AsyncTile<T, D, TQ, NW>;
-  constexpr int LPT = 2 * Loader::PER_WAVE + 1;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
 
@@ -730,34 +726,33 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
   const float* lse_base = p.lse + (int64_t)bh * T_;
   const float* delta_base = p.delta + (int64_t)bh * T_;
-  auto stage_ptr = [&](int t) { return smem_raw + ((t - qt0) % NST) * STAGE_BYTES; };
+  const TileOrder order(qt0, qt1, p.period, p.pdiv);
   Loader ldq, ldg;
   ldq.init(qbase, p.q_st, qt0 * TQ, L - 1, wave, lane);
   ldg.init(gbase, p.do_st, qt0 * TQ, L - 1, wave, lane);
-  auto issue_tile = [&](int t) {   // tiles are issued in ascending order
-    T* st = reinterpret_cast<T*>(stage_ptr(t));
+  auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
+    char* const stage = smem_raw + (it & 1) * STAGE_BYTES;
+    T* st = reinterpret_cast<T*>(stage);
     // lanes [0, RPW) fetch lse, lanes [RPW, 2*RPW) fetch delta of this wave's RPW rows
     if (lane < 2 * RPW) {
       int r = t * TQ + wave * RPW + (lane % RPW);
       r = r < L ? r : L - 1;
       const float* src = (lane < RPW ? lse_base : delta_base) + r;
-      float* dst = reinterpret_cast<float*>(stage_ptr(t) + 2 * TILE * sizeof(T)) + wave * 2 * RPW;
+      float* dst = reinterpret_cast<float*>(stage + 2 * TILE * sizeof(T)) + wave * 2 * RPW;
       async_copy_f32(src, dst);
     }
-    ldq.issue(st, wave);
-    ldg.issue(st + TILE, wave);
-    ldq.advance();
-    ldg.advance();
+    ldq.at(t - qt0).issue(st, wave);
+    ldg.at(t - qt0).issue(st + TILE, wave);
   };
   // This wave's K rows go where the second tile will be, its V rows beside the stages.
   using Rows = OwnRows<T, D>;
-  static_assert(NST == 2 && NW * 32 == 2 * TQ, "the rows of a workgroup fill a stage");
+  static_assert(NST == 2 && NW * 32 == 2 * TQ, "two stages; the rows of a workgroup fill one");
   T* const k_area = reinterpret_cast<T*>(smem_raw + STAGE_BYTES) + wave * Rows::ELEMS;
   T* const v_area = reinterpret_cast<T*>(smem_raw + NST * STAGE_BYTES) + wave * Rows::ELEMS;
   const int wrow0 = k0 + wave * 32;
   Rows::send(reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh, p.k_st, wrow0, L - 1, k_area, lane);
   Rows::send(reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh, p.v_st, wrow0, L - 1, v_area, lane);
-  issue_tile(qt0);
+  issue_tile(order.first, 0);
 
   Frag kf[NF], vf[NF];
   landed();
@@ -779,15 +774,15 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
     for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
   wait_all_loads();
 
-  for (int t = qt0; t < qt1; ++t) {
-    if (NST == 3 && t + 1 < qt1) wait_loads<LPT>();
-    else wait_loads<0>();
+  for (int t = order.first, it = 0; it < qt1 - qt0; ++it, t = order.next(t)) {
+    wait_loads<0>();
     __syncthreads();
-    if (t + NST - 1 < qt1) issue_tile(t + NST - 1);
+    if (order.next(t) != order.first) issue_tile(order.next(t), it + 1);
 
-    const T* Qt = reinterpret_cast<const T*>(stage_ptr(t));
+    const char* const stage = smem_raw + (it & 1) * STAGE_BYTES;
+    const T* Qt = reinterpret_cast<const T*>(stage);
     const T* Gt = Qt + TILE;
-    const float* ld_t = reinterpret_cast<const float*>(stage_ptr(t) + 2 * TILE * sizeof(T));
+    const float* ld_t = reinterpret_cast<const float*>(stage + 2 * TILE * sizeof(T));
     const int qs = t * TQ;
     if (qs + TQ <= win.lo_min || qs >= win.hi_max) continue;   // outside this wave's windows
 

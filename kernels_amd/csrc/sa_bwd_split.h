@@ -398,16 +398,17 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
   Loader ldq, ldg;
   ldq.init(qbase, p.q_st, qt0 * TQ, L - 1, wave, lane);
   ldg.init(gbase, p.do_st, qt0 * TQ, L - 1, wave, lane);
-  // Tile t goes where tile t - 4 (Q, lse, delta) and tile t - 3 (dO) were: issued at the beginning of step t - 2, when
-  // every wave has finished step t - 3, the last that reads either.
-  auto issue_tile = [&](int t, int gs) {
-    const int qs = (t - qt0) & (NQ - 1);
+  const TileOrder order(qt0, qt1, p.period, p.pdiv);
+  const int n = qt1 - qt0;
+  auto tile = [&](int it) { return order.first + it < qt1 ? order.first + it : order.first + it - n; };   // of step it
+  // The tile of step `it` goes where those of steps it - 4 (Q, lse, delta) and it - 3 (dO) were: issued at the beginning of
+  // step it - 2, when every wave has finished step it - 3, the last that reads either.
+  auto issue_tile = [&](int it, int gs) {
+    const int qs = it & (NQ - 1), t = tile(it);
     if (lane < 2 * RPW)
       async_copy_f32<true>(row_src + valid(t * TQ + wave * RPW + lane % RPW), row_ring + (qs * NW + wave) * 2 * RPW);
-    ldq.issue(q_ring + qs * TILE, wave);
-    ldg.issue(g_ring + gs * TILE, wave);
-    ldq.advance();
-    ldg.advance();
+    ldq.at(t - qt0).issue(q_ring + qs * TILE, wave);
+    ldg.at(t - qt0).issue(g_ring + gs * TILE, wave);
   };
   // this wave's rows first, over the rings
   using Rows = OwnRows<T, D>;
@@ -431,17 +432,17 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
     }
   }
   __syncthreads();
-  issue_tile(qt0, 0);
-  if (qt0 + 1 < qt1) issue_tile(qt0 + 1, 1);
+  issue_tile(0, 0);
+  if (n > 1) issue_tile(1, 1);
   f32x16 acc[1][DB];   // dV^T[d][key] (score role) or -dK^T[d][key] (grad role)
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[0][m][i] = 0.0f;
 
-  // lse (which = 0) or delta (which = 1) of the 16 rows of tile t that this lane holds in a C fragment
-  auto rows16 = [&](int t, int which, f32x16& out) {
-    const float* rows = row_ring + ((t - qt0) & (NQ - 1)) * 2 * TQ + which * RPW;
+  // lse (which = 0) or delta (which = 1) of the 16 rows of step it's tile that this lane holds in a C fragment
+  auto rows16 = [&](int it, int which, f32x16& out) {
+    const float* rows = row_ring + (it & (NQ - 1)) * 2 * TQ + which * RPW;
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
       const int r = 8 * g4 + 4 * h;
@@ -458,24 +459,25 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
     for (int i = 0; i < 16; ++i) x[i] = keep_or_zero(x[i], keep_bits(rm, i));
   };
   int gs = 0;   // stage of the current dO tile
-  auto begin_step = [&](int t) {
-    if (t + 1 < qt1) wait_loads<LPT>();
+  auto begin_step = [&](int it) {
+    if (it + 1 < n) wait_loads<LPT>();
     else wait_loads<0>();
     __syncthreads();
-    if (t + 2 < qt1) issue_tile(t + 2, gs == 0 ? 2 : gs - 1);
+    if (it + 2 < n) issue_tile(it + 2, gs == 0 ? 2 : gs - 1);
   };
 
   if (!grad_role) {
-    for (int t = qt0; t < qt1; ++t, gs = gs == NG - 1 ? 0 : gs + 1) {
-      begin_step(t);
+    for (int it = 0; it < n; ++it, gs = gs == NG - 1 ? 0 : gs + 1) {
+      begin_step(it);
+      const int t = tile(it);
       if (!live(t)) continue;
       f32x16 s[1][1];
-      rows16(t, 0, s[0][0]);
-      mma_rows_n<T, D>(s, q_ring + ((t - qt0) & (NQ - 1)) * TILE, 0, rf, lane);   // lse - S[q][key]
+      rows16(it, 0, s[0][0]);
+      mma_rows_n<T, D>(s, q_ring + (it & (NQ - 1)) * TILE, 0, rf, lane);          // lse - S[q][key]
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[0][0][i] = fast_exp2(-s[0][0][i]);
       masked(t, s[0][0]);
-      float* slot = xbuf + (t & 1) * S::XSLOT;
+      float* slot = xbuf + (it & 1) * S::XSLOT;
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4)
         *reinterpret_cast<f32x4*>(slot + g4 * 256) =
@@ -489,28 +491,28 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
     f32x16 dp[1][1];   // delta - dP of the step before
 #pragma unroll
     for (int i = 0; i < 16; ++i) dp[0][0][i] = 0.0f;
-    for (int t = qt0;; ++t, gs = gs == NG - 1 ? 0 : gs + 1) {
-      if (t < qt1) begin_step(t);
+    for (int it = 0;; ++it, gs = gs == NG - 1 ? 0 : gs + 1) {
+      if (it < n) begin_step(it);
       else __syncthreads();
-      const bool prev = t > qt0 && live(t - 1);
+      const bool prev = it > 0 && live(tile(it - 1));
       Frag df[1][2];
       if (prev) {
-        const float* slot = xbuf + ((t - 1) & 1) * S::XSLOT;
+        const float* slot = xbuf + ((it - 1) & 1) * S::XSLOT;
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
           const f32x4 p4 = *reinterpret_cast<const f32x4*>(slot + g4 * 256);
 #pragma unroll
           for (int e = 0; e < 4; ++e) dp[0][0][4 * g4 + e] *= p4[e];   // = -dS
         }
-        masked(t - 1, dp[0][0]);   // a masked dP may hold anything, NaN included
+        masked(tile(it - 1), dp[0][0]);   // a masked dP may hold anything, NaN included
         pack_c<T>(df[0], dp[0][0]);
       }
-      if (t < qt1 && live(t)) {
-        rows16(t, 1, dp[0][0]);
+      if (it < n && live(tile(it))) {
+        rows16(it, 1, dp[0][0]);
         mma_rows_n<T, D>(dp, g_ring + gs * TILE, 0, rf, lane);                      // delta - dP[q][key]
       }
-      if (prev) mma_tr_n<T, D>(acc, q_ring + ((t - 1 - qt0) & (NQ - 1)) * TILE, 0, df, lane);   // -dK^T += Q^T (-dS)
-      if (t == qt1) break;
+      if (prev) mma_tr_n<T, D>(acc, q_ring + ((it - 1) & (NQ - 1)) * TILE, 0, df, lane);   // -dK^T += Q^T (-dS)
+      if (it == n) break;
     }
   }
 

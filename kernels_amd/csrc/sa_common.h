@@ -523,6 +523,11 @@ template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct A
   }
   SA_DEV void issue(T* tile, int wave) const { issue_part<0, PER_WAVE>(tile, wave); }
   SA_DEV void advance() { soff += tstep; }
+  SA_DEV AsyncTile at(int tiles_ahead) const {
+    AsyncTile a = *this;
+    a.soff += (uint32_t)tiles_ahead * tstep;
+    return a;
+  }
 };
 
 // Asynchronous copy of one float per active lane to consecutive LDS words starting at dst
@@ -543,16 +548,6 @@ template <bool ASM_COPIES = false> SA_DEV void async_copy_f32(const float* src, 
 template <int N> SA_DEV void wait_loads() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-// Waits until at most min(ahead, MAXA) tiles of LPT loads each are outstanding (ahead is wave-uniform).
-template <int LPT, int MAXA> SA_DEV void wait_tiles(int ahead) {
-  if constexpr (MAXA <= 0) {
-    wait_loads<0>();
-  } else {
-    if (ahead >= MAXA) wait_loads<MAXA * LPT>();
-    else wait_tiles<LPT, MAXA - 1>(ahead);
-  }
 }
 
 // The 32 rows that a wave keeps as operand fragments, through 32 * D elements of LDS of its own.  Fragment g of a lane is
@@ -824,6 +819,24 @@ static_assert(div_by(2999, chunk_div(10)) == 299 && div_by(3000, chunk_div(10)) 
               div_by(0x7fffffff, chunk_div(3)) == 715827882 && div_by(0x7fffffff, chunk_div(641)) == 3350208 &&
               div_by(65535, chunk_div(256)) == 255 && div_by(0x7fffffff, chunk_div(10000)) == 214748, "samples");
 
+// Where a workgroup begins to go through the tiles [t0, t1) of its window: at the multiple of `period`, the number of tiles of
+// a full window, among them, and round to the tile before it.  Neighbouring workgroups of an XCD, whose windows
+// overlap, then read the same tile at the same time and it crosses into their L2 once; each from its own first tile on, they read it
+// several steps apart, when it has left the 4 MiB again.  The last tiles of a sequence and the windows that still grow begin
+// where they can.  MB fetched by forward, dQ
+// and dK/dV at B=4, H=16, T=4096, D=256, chunks of 128, 4 back (q, k, v, dO and O of 134 MB each): 1285, 1111, 1029 -> 461,
+// 733, 599, forward and backward 929 -> 898 us; B=8, H=16, T=4096, D=64: 229, 444, 360 -> 215, 354, 293, 418 -> 414.
+struct TileOrder {
+  int t0, t1, first;
+  SA_DEV TileOrder(int t0_, int t1_, int period, ChunkDiv pdiv) : t0(t0_), t1(t1_), first(t0_) {
+    if (period > 1) {
+      const int f = div_by(t0 + period - 1, pdiv) * period;
+      first = f < t1 ? f : t0;
+    }
+  }
+  SA_DEV int next(int t) const { return t + 1 == t1 ? t0 : t + 1; }   // `first` again after the last one
+};
+
 struct FwdParams {
   const void *q, *k, *v;
   void* o;          // contiguous [B,H,T,D]
@@ -835,6 +848,8 @@ struct FwdParams {
   float scale_log2e;  // sm_scale * log2(e); sign carried separately
   int n_tiles;        // query tiles per (b,h)
   ChunkDiv cdiv;      // division by C
+  int period;         // TileOrder; 0: ascending
+  ChunkDiv pdiv;      // division by period
 };
 
 struct BwdParams {
@@ -853,6 +868,8 @@ struct BwdParams {
   int64_t o_sb, o_sh, o_st;
   float* delta_out;
   ChunkDiv cdiv;      // division by C
+  int period;         // TileOrder; 0: ascending
+  ChunkDiv pdiv;      // division by period
   int fused_rows;     // one-launch backward only: query rows whose lse and delta a workgroup keeps
 };
 

@@ -249,7 +249,7 @@ struct Fwd2Slots {
 // queries, so every K / V fragment fetched from LDS feeds QB MFMAs (the transposing V reads
 // are 8-byte LDS reads and would otherwise cap the second product well below the MFMA
 // rate); K and V tiles are brought in by asynchronous global->LDS copies into a ring of NST
-// stages, NST-1 tiles ahead of the compute, with one barrier per key tile.
+// stages, one tile ahead of the compute, with one barrier per key tile.
 // SHORT selects the form for short windows (a handful of key tiles per workgroup): work is skipped
 // and masks are decided per 32-key block instead of per tile, and a wave's first tile goes straight
 // to the search for its maximum.  Long windows run the plain form, whose loop is a few per cent
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   using E = Elem<T>;
   using G = TileGeom<T, D>;
   using Frag = typename E::Frag;
-  static_assert(G::SWZ && NST >= 2 && (NST - 2) * 2 * AsyncTile<T, D, TK, NW>::PER_WAVE < 64, "swizzled 16-bit tiles; the loads of NST-2 tiles fit the load counter");
+  static_assert(G::SWZ, "swizzled 16-bit tiles");
   constexpr bool HALVES = D == 256, BLOCKS = SHORT && TK == 32;
   static_assert(BLOCKS || TK == 64, "whole tiles of 64 keys, or of 32 on short windows");
   constexpr int SB = HALVES ? 32 : TK;     // keys that a wave goes through at a time
@@ -279,7 +279,6 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   constexpr float kRescaleGap = 8.0f;
   constexpr float kSumLimit = 256.0f;
   using Loader = AsyncTile<T, D, SB, NW, HALVES>;
-  constexpr int LPT = 2 * Loader::PER_WAVE;   // async loads per wave per stage (K and V)
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);  // [stage][K|V][TK][D], or the slots
@@ -342,37 +341,31 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   Loader ldk, ldv;
   ldk.init(kbase, p.k_st, kt0 * TK, L - 1, wave, lane);
   ldv.init(vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
-  auto issue_tile = [&](int t) {   // tiles are issued in ascending order
-    T* st = smem + ((t - kt0) % NST) * STAGE;
-    ldk.issue(st, wave);
-    ldv.issue(st + TILE, wave);
-    ldk.advance();
-    ldv.advance();
+  const TileOrder order(kt0, kt1, p.period, p.pdiv);
+  auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
+    T* st = smem + (it & 1) * STAGE;
+    ldk.at(t - kt0).issue(st, wave);
+    ldv.at(t - kt0).issue(st + TILE, wave);
   };
   // This wave's Q rows go where the second tile will be.
   using Rows = OwnRows<T, D>;
-  static_assert(HALVES || (NST == 2 && QB == 1 && NW * 32 == 2 * TK), "the rows of a workgroup fill a stage");
+  static_assert(NST == 2 && (HALVES || (QB == 1 && NW * 32 == 2 * TK)), "two stages; the rows of a workgroup fill one");
   T* const q_area = smem + STAGE + wave * Rows::ELEMS;
   const T* qbase = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
-  // prologue: NST-1 tiles in flight
   if constexpr (!HALVES) {
     Rows::send(qbase, p.q_st, q0 + wave * WQ, L - 1, q_area, lane);
-#pragma unroll
-    for (int i = 0; i < NST - 1; ++i)
-      if (kt0 + i < kt1) issue_tile(kt0 + i);
+    issue_tile(order.first, 0);
   }
   // Fwd2Slots: a block that no query of the workgroup sees is not sent for
   Fwd2Slots slots;
   auto seen = [&](int k0) { return k0 + SB > lo_wg && k0 < hi_wg; };
-  auto send = [&](const Loader& ld, int blocks_ahead, int slot) {
-    Loader at = ld;
-    at.soff += blocks_ahead * ld.tstep;
-    at.issue(smem + slot * SB * D, wave);
+  auto send = [&](const Loader& ld, int t, int block, int slot) { ld.at((t - kt0) * 2 + block).issue(smem + slot * SB * D, wave); };
+  auto send_first_blocks = [&](int t) {
+    if (seen(t * TK)) send(ldk, t, 0, Fwd2Slots::K0), send(ldv, t, 0, Fwd2Slots::V0);
   };
-  if constexpr (HALVES) {   // ldk and ldv stay at the first block of the next tile
-    if (seen(kt0 * TK)) send(ldk, 0, Fwd2Slots::K0), send(ldv, 0, Fwd2Slots::V0);
-    if (seen(kt0 * TK + SB)) send(ldk, 1, slots.k1);
-    ldk.soff += 2 * ldk.tstep, ldv.soff += 2 * ldv.tstep;
+  if constexpr (HALVES) {
+    send_first_blocks(order.first);
+    if (seen(order.first * TK + SB)) send(ldk, order.first, 1, slots.k1);
   }
 
   Frag qf[QB][NF];
@@ -406,21 +399,21 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   wait_all_loads();   // Q fragments (and, as loads complete in order, the first tiles)
 
   int tiles_seen = 0;   // BLOCKS: tiles that this wave has gone through
-  for (int t = kt0; t < kt1; ++t) {
+  for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    const int t_next = order.next(t);
+    const bool more = t_next != order.first;
     if constexpr (!HALVES) {
-      // tile t has landed once at most the loads of the younger tiles are outstanding: NST-2 of them, fewer
-      // near the end of the window
-      wait_tiles<LPT, NST - 2>(kt1 - 1 - t);
-      __syncthreads();   // every wave's share is visible; stage (t-1) % NST is free again
-      if (t + NST - 1 < kt1) issue_tile(t + NST - 1);
+      wait_loads<0>();
+      __syncthreads();   // every wave's share of tile t is visible; the other stage is free again
+      if (more) issue_tile(t_next, it + 1);
     }
     auto key_block = [&](int sb) {
       if constexpr (HALVES) return smem + (sb == 0 ? Fwd2Slots::K0 : slots.k1) * SB * D;
-      else return smem + ((t - kt0) % NST) * STAGE + sb * D;
+      else return smem + (it & 1) * STAGE + sb * D;
     };
     auto value_block = [&](int sb) {
       if constexpr (HALVES) return smem + (sb == 0 ? Fwd2Slots::V0 : slots.v1) * SB * D;
-      else return smem + ((t - kt0) % NST) * STAGE + TILE + sb * D;
+      else return smem + (it & 1) * STAGE + TILE + sb * D;
     };
     float rs[QB][2];   // sums of the tile's probabilities
 #pragma unroll
@@ -428,17 +421,15 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
 #pragma unroll
     for (int sb = 0; sb < TK; sb += SB) {
     if constexpr (HALVES) {
-      const bool k1_next = t + 1 < kt1 && seen((t + 1) * TK + SB);
+      const bool k1_next = more && seen(t_next * TK + SB);
       if (sb != 0 && k1_next) wait_loads<Loader::PER_WAVE>();   // V1 was sent for before it
       else wait_loads<0>();
       __syncthreads();
       if (sb == 0) {
-        if (seen(t * TK + SB)) send(ldv, -1, slots.v1);
-        if (k1_next) send(ldk, 1, slots.free());
-      } else if (t + 1 < kt1) {
-        send(ldk, 0, Fwd2Slots::K0);
-        send(ldv, 0, Fwd2Slots::V0);
-        ldk.soff += 2 * ldk.tstep, ldv.soff += 2 * ldv.tstep;
+        if (seen(t * TK + SB)) send(ldv, t, 1, slots.v1);
+        if (k1_next) send(ldk, t_next, 1, slots.free());
+      } else if (more) {
+        send_first_blocks(t_next);
       }
     }
     const int k0 = t * TK + sb;

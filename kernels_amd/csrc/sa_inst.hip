@@ -109,6 +109,7 @@ template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p,
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
+  set_tile_order(p, TQ, TK);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -218,6 +219,7 @@ template <int D, int NW> static int dq2_launch(BwdParams p, hipStream_t st) {
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
+  set_tile_order(p, TQ, C::DQ2_TK);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -348,6 +350,7 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
   static PrepareState once;
   if (int rc = prepare(kern, S::lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, S::TKB);
+  set_tile_order(p, S::TKB, S::TQ);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * S::NP * 64), S::lds, st, p);
@@ -390,6 +393,7 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
     p.n_tiles = (int)ceil_div(p.T, TKB);
+    set_tile_order(p, TKB, C::DKDV2_TQ);
     const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::DKDV2_NW * 64), lds, st, p);

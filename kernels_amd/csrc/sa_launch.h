@@ -106,6 +106,19 @@ inline int rows_in_reach(int chunk, int back, int rows, int tile) {
   }
   return most * tile;
 }
+// The tiles of a full window of a workgroup of `rows` rows, for TileOrder; 0 where the order has nothing to gain: a window
+// that covers the sequence (every workgroup begins at the first tile anyway).
+inline int tiles_of_window(int T, int chunk, int back, int rows, int tile) {
+  const long long chunks = chunk % rows == 0 ? 1 : rows % chunk == 0 ? rows / chunk : (rows + chunk - 2) / chunk + 1;
+  const long long span = (chunks + back) * chunk;
+  if (span >= T) return 0;
+  const bool aligned = chunk % tile == 0 || (rows % chunk == 0 && (long long)chunk * back % tile == 0);
+  return (int)((span + tile - 1 + (aligned ? 0 : tile - 1)) / tile);
+}
+template <typename P> void set_tile_order(P& p, int rows, int tile) {
+  p.period = tiles_of_window(p.T, p.C, p.R, rows, tile);
+  p.pdiv = chunk_div(p.period > 0 ? p.period : 1);
+}
 // Short windows, head dimensions 32 and 64: workgroups of two waves (64 rows, tiles of 32) instead of four (128 rows,
 // tiles of 64).  In the large workgroup every wave waits at the barriers of about twice as many tiles as it sees itself,
 // and half as many waves are resident; the small one goes through more rows per row of its own unless the windows begin and
