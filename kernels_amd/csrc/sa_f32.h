@@ -122,12 +122,99 @@ template <int D, int ROWS, int NT> struct SplitStager {
   }
 };
 
+// The 32 rows that a wave keeps, as copies of whole rows through 32 * D floats of LDS of its own (see OwnRows in sa_common.h,
+// whose swizzle of rows of as many bytes this is).  The addresses are formed per lane, in 64 bits: float32 tensors have no
+// limit on their row stride.  Rows past the last valid one mimic it.
+template <int D> struct OwnRows32 {
+  using G = TileGeom<__bf16, 2 * D>;
+  static constexpr int ELEMS = 32 * D, CPR = D / 4, RPI = 64 / CPR, N = 32 / RPI;
+  SA_DEV static int off(int row, int chunk) { return G::off(row, chunk * 8) / 2; }   // of sixteen bytes, in floats
+  SA_DEV static void send(const float* base, int64_t row_stride, int row0, int last_row, float* area, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = i * RPI + lane / CPR, gr = row0 + r < last_row ? row0 + r : last_row;
+      const float* src = base + (int64_t)gr * row_stride + ((lane % CPR) ^ G::swz(r)) * 4;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (SA_LDS void*)(area + i * 256), 16, 0, 0);
+    }
+  }
+};
+// Not where a row is a sixteenth of a kilobyte (D = 16: B=8, H=16, T=1000, chunks of 20, 4 back, forward and backward 88.1 us, 91.5
+// this way) nor in the workgroups of two waves, whose grids take as long as one workgroup's chain of latencies (see
+// half_workgroups; B=2, H=4, T=512, D=64 forward 15.0, 15.4 this way): there a lane loads its half row itself, stores its
+// row itself, and the tiles come in ascending order.
+constexpr bool direct_rows(int D, int NW) { return D == 16 || NW == 2; }
+// Row sums of the products of a wave's rows of O, read whole from memory, with those of dO in LDS (see RowDots).
+template <int D> struct RowDots32 {
+  using Rows = OwnRows32<D>;
+  static constexpr int CPR = Rows::CPR, RPI = Rows::RPI, N = Rows::N, PITCH = CPR + 4;
+  f32x4 of[N];
+  SA_DEV void load(const float* base, int64_t row_stride, int row0, int last_row, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = row0 + i * RPI + lane / CPR;
+      of[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)(r < last_row ? r : last_row) * row_stride + lane % CPR * 4);
+    }
+  }
+  SA_DEV void partial(const float* g_area, float* scratch, int lane) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = i * RPI + lane / CPR, ch = lane % CPR;
+      const f32x4 gf = *reinterpret_cast<const f32x4*>(g_area + Rows::off(r, ch));
+      scratch[r * PITCH + ch] = __builtin_fmaf(of[i][0], gf[0], of[i][1] * gf[1]) + __builtin_fmaf(of[i][2], gf[2], of[i][3] * gf[3]);
+    }
+  }
+  SA_DEV static float total(const float* scratch, int lane) {
+    const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * (CPR / 2);
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CPR / 2; ++j) sum += row[j];
+    return half_sum(sum);
+  }
+};
+
+// Whole rows from the accumulators (X^T: a lane owns a row), 64 columns at a time through a patch of LDS of the wave's own, so
+// that a store instruction writes whole cache lines and may pass the caches (store_streaming).
+template <int D> struct RowPatch32 {
+  static constexpr int W = D < 64 ? D : 64, PITCH = W + 4, ELEMS = 32 * PITCH, CPR = W / 4, RPI = 64 / CPR;
+};
+template <int D, bool DIRECT, int DB>
+SA_DEV void store_rows_f32(float* patch, float* out_rows, int rows_valid, const f32x16 (&acc)[DB], float mul, int lane) {
+  using P = RowPatch32<D>;
+  const int c = lane & 31, h = lane >> 5;
+  if constexpr (DIRECT) {
+    if (c < rows_valid) store_acc_T<float, D, DB>(out_rows + (int64_t)c * D, acc, mul, h);
+    return;
+  }
+#pragma unroll
+  for (int col = 0; col < D; col += P::W) {
+#pragma unroll
+    for (int m = col / 32; m < DB && m * 32 < col + P::W; ++m)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = m * 32 - col + 8 * g + 4 * h;
+        store4<float>(patch + c * P::PITCH + d, acc[m][4 * g] * mul, acc[m][4 * g + 1] * mul, acc[m][4 * g + 2] * mul,
+                      acc[m][4 * g + 3] * mul);
+      }
+#pragma unroll
+    for (int j = 0; j < 32 / P::RPI; ++j) {
+      const int row = j * P::RPI + lane / P::CPR, ch = lane % P::CPR;
+      const u32x4 v16 = *reinterpret_cast<const u32x4*>(patch + row * P::PITCH + ch * 4);
+      if (row < rows_valid) store_streaming(out_rows + (int64_t)row * D + col + ch * 4, v16);
+    }
+  }
+}
+
 // This lane's half of a float32 row, and its split fragments (as a B operand).
 template <int D> struct HalfRow {
   f32x4 r[D / 8];
   SA_DEV void load(const float* row, int h) {
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) r[i] = *reinterpret_cast<const f32x4*>(row + (i / 2) * 16 + h * 8 + (i % 2) * 4);
+  }
+  SA_DEV void read(const float* area, int lane) {
+    const int c = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) r[i] = *reinterpret_cast<const f32x4*>(area + OwnRows32<D>::off(c, (i / 2) * 4 + h * 2 + i % 2));
   }
   SA_DEV void split(Split8 (&f)[D / 16], bool negative) const {
     const float mul = negative ? -kUp : kUp;
@@ -229,6 +316,11 @@ template <int NW> SA_DEV bool any_in_workgroup(bool x, void* smem, int wave, int
   return true;
 }
 
+// A wave's row patch after any_in_workgroup, whose flags other waves may still read.
+template <int D> SA_DEV float* row_patch(char* smem, int wave) {
+  return reinterpret_cast<float*>(smem + 64) + wave * RowPatch32<D>::ELEMS;
+}
+
 // The windows of a wave's 32 queries, of one lane's query, and of the workgroup.
 struct QueryWindow {
   int lo, hi;            // this lane's keys
@@ -293,17 +385,27 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
 
   const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
+  float* const q_area = reinterpret_cast<float*>(smem_raw) + wave * OwnRows32<D>::ELEMS;
+  const float* qbase = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
+  constexpr bool DIRECT = direct_rows(D, NW);
+  if (!DIRECT) OwnRows32<D>::send(qbase, p.q_st, q0 + wave * 32, L - 1, q_area, lane);
+  const TileOrder order(kt0, kt1, DIRECT ? 0 : p.period, p.pdiv);
   SplitStager<D, TK, NT> sk, sv;
-  sk.load(kbase, p.k_st, kt0 * TK, L - 1, tid);
-  sv.load(vbase, p.v_st, kt0 * TK, L - 1, tid);
+  sk.load(kbase, p.k_st, order.first * TK, L - 1, tid);
+  sv.load(vbase, p.v_st, order.first * TK, L - 1, tid);
 
   Split8 qf[D / 16];
   {
     HalfRow<D> qr;
-    qr.load(reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh +
-                (int64_t)(qrow < L ? qrow : L - 1) * p.q_st, h);
+    if (DIRECT) {
+      qr.load(qbase + (int64_t)(qrow < L ? qrow : L - 1) * p.q_st, h);
+    } else {
+      landed();
+      qr.read(q_area, lane);
+    }
     qr.split(qf, p.scale_log2e < 0.0f);
   }
+  if (!DIRECT) __syncthreads();   // the tiles go where the rows were
 
   f32x16 oacc[DB];
 #pragma unroll
@@ -316,13 +418,13 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
   sv.store(smem + TILE, tid);
   __syncthreads();
 
-  for (int t = kt0; t < kt1; ++t) {
-    const __bf16* Kt = smem + ((t - kt0) % NST) * 2 * TILE;
+  for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    const __bf16* Kt = smem + (it % NST) * 2 * TILE;
     const __bf16* Vt = Kt + TILE;
-    const bool more = t + 1 < kt1;
+    const bool more = order.next(t) != order.first;
     if (more) {
-      sk.load(kbase, p.k_st, (t + 1) * TK, L - 1, tid);
-      sv.load(vbase, p.v_st, (t + 1) * TK, L - 1, tid);
+      sk.load(kbase, p.k_st, order.next(t) * TK, L - 1, tid);
+      sv.load(vbase, p.v_st, order.next(t) * TK, L - 1, tid);
     }
     const int k0 = t * TK;
     if (k0 + TK > w.lo_min && k0 < w.hi_max) {   // some query of this wave sees the tile
@@ -372,7 +474,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
     }
     if (more) {
       if (NST == 1) __syncthreads();   // the only stage has no reader left
-      __bf16* nxt = smem + ((t + 1 - kt0) % NST) * 2 * TILE;
+      __bf16* nxt = smem + ((it + 1) % NST) * 2 * TILE;
       sk.store(nxt, tid);
       sv.store(nxt + TILE, tid);
     }
@@ -386,17 +488,16 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
     return;
   }
   const bool valid = qrow < L;
-  if (qrow < T_) {
-    const float inv = valid ? 1.0f / l_tot * kDown2 : 0.0f;
-    if (!valid) {
+  const float inv = valid ? 1.0f / l_tot * kDown2 : 0.0f;
+  if (!valid) {
 #pragma unroll
-      for (int m = 0; m < DB; ++m)
+    for (int m = 0; m < DB; ++m)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
-    }
-    store_acc_T<float, D, DB>(o_base + (int64_t)qrow * D, oacc, inv, h);
-    if (lse_base && h == 0) lse_base[qrow] = valid ? m_run + __builtin_amdgcn_logf(l_tot) : 0.0f;
+      for (int i = 0; i < 16; ++i) oacc[m][i] = 0.0f;
   }
+  const int row0 = q0 + wave * 32;
+  store_rows_f32<D, DIRECT>(row_patch<D>(smem_raw, wave), o_base + (int64_t)row0 * D, T_ - row0, oacc, inv, lane);
+  if (lse_base && h == 0 && qrow < T_) lse_base[qrow] = valid ? m_run + __builtin_amdgcn_logf(l_tot) : 0.0f;
 }
 
 // dQ, one wave per 32 queries, tiles of 32 keys, two stages.  delta = rowsum(O * dO) is formed in the prologue (the
@@ -442,36 +543,63 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
 
   const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
+  using Rows = OwnRows32<D>;
+  const int row0 = q0 + wave * 32;
+  float* const q_area = reinterpret_cast<float*>(smem_raw) + wave * Rows::ELEMS;
+  float* const g_area = q_area + NW * Rows::ELEMS;
+  const float* gbase = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
+  const float* qbase = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
+  // (no branch around the loads: without a row of O to read, the dO row is read; see dq2_kernel)
+  const float* obase = p.delta_out ? reinterpret_cast<const float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh : gbase;
+  const int64_t o_st = p.delta_out ? p.o_st : p.do_st;
+  constexpr bool DIRECT = direct_rows(D, NW);
+  RowDots32<D> dots;
+  if (!DIRECT) {
+    Rows::send(qbase, p.q_st, row0, L - 1, q_area, lane);
+    Rows::send(gbase, p.do_st, row0, L - 1, g_area, lane);
+    dots.load(obase, o_st, row0, L - 1, lane);
+  }
+  const TileOrder order(kt0, kt1, DIRECT ? 0 : p.period, p.pdiv);
   SplitStager<D, TK, NT> sk, sv;
-  sk.load(kbase, p.k_st, kt0 * TK, L - 1, tid);
-  sv.load(vbase, p.v_st, kt0 * TK, L - 1, tid);
+  sk.load(kbase, p.k_st, order.first * TK, L - 1, tid);
+  sv.load(vbase, p.v_st, order.first * TK, L - 1, tid);
 
   Split8 qf[NF], gf[NF];
   const int qr = qrow < L ? qrow : L - 1;
   const float lse_q = qrow < L ? p.lse[(int64_t)bh * T_ + qr] : INFINITY;   // rows past L: P = exp2(-inf) = 0
   float delta_q;
   {
-    const float* gp = reinterpret_cast<const float*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh +
-                      (int64_t)qr * p.do_st;
-    HalfRow<D> q_row, g_row;
-    q_row.load(reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh + (int64_t)qr * p.q_st, h);
-    g_row.load(gp, h);
-    q_row.split(qf, p.scale_log2e < 0.0f);
-    g_row.split(gf, false);
-    if (p.delta_out) {
-      HalfRow<D> o_row;
-      o_row.load(reinterpret_cast<const float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh + (int64_t)qr * p.o_st, h);
-      float sum = 0.0f;
+    float sum = 0.0f;
+    if (DIRECT) {
+      HalfRow<D> q_row, g_row, o_row;
+      q_row.load(qbase + (int64_t)qr * p.q_st, h);
+      g_row.load(gbase + (int64_t)qr * p.do_st, h);
+      o_row.load(obase + (int64_t)qr * o_st, h);
+      q_row.split(qf, p.scale_log2e < 0.0f);
+      g_row.split(gf, false);
 #pragma unroll
       for (int i = 0; i < D / 8; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(o_row.r[i][e], g_row.r[i][e], sum);
-      delta_q = half_sum(sum);
+      sum = half_sum(sum);
+    } else {
+      HalfRow<D> row;
+      landed();
+      row.read(g_area, lane);
+      row.split(gf, false);
+      row.read(q_area, lane);
+      row.split(qf, p.scale_log2e < 0.0f);
+      dots.partial(g_area, q_area, lane);
+      sum = RowDots32<D>::total(q_area, lane);
+    }
+    if (p.delta_out) {
+      delta_q = sum;
       if (h == 0 && qrow < T_) p.delta_out[(int64_t)bh * T_ + qrow] = qrow < L ? delta_q : 0.0f;
     } else {
       delta_q = p.delta[(int64_t)bh * T_ + qr];
     }
   }
+  if (!DIRECT) __syncthreads();   // the tiles go where the rows were
 
   const float dinit = -delta_q * kUp2;
 
@@ -484,13 +612,13 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
   sv.store(smem + TILE, tid);
   __syncthreads();
 
-  for (int t = kt0; t < kt1; ++t) {
-    const __bf16* Kt = smem + ((t - kt0) & 1) * 2 * TILE;
+  for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    const __bf16* Kt = smem + (it & 1) * 2 * TILE;
     const __bf16* Vt = Kt + TILE;
-    const bool more = t + 1 < kt1;
+    const bool more = order.next(t) != order.first;
     if (more) {
-      sk.load(kbase, p.k_st, (t + 1) * TK, L - 1, tid);
-      sv.load(vbase, p.v_st, (t + 1) * TK, L - 1, tid);
+      sk.load(kbase, p.k_st, order.next(t) * TK, L - 1, tid);
+      sv.load(vbase, p.v_st, order.next(t) * TK, L - 1, tid);
     }
     const int k0 = t * TK;
     if (k0 + TK > w.lo_min && k0 < w.hi_max) {
@@ -514,7 +642,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
       mma_tr_split<D, TK>(acc, Kt, sb, lane);   // dQ^T[d][q] += K^T dS^T
     }
     if (more) {
-      __bf16* nxt = smem + ((t + 1 - kt0) & 1) * 2 * TILE;
+      __bf16* nxt = smem + (~it & 1) * 2 * TILE;
       sk.store(nxt, tid);
       sv.store(nxt + TILE, tid);
     }
@@ -525,15 +653,13 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     dq_rows<float, D, NW, TK>(p, again_s(bh), again_s(qt), again_v(tid), [&](int) { return delta_q; });   // this lane's query
     return;
   }
-  if (qrow < T_) {
-    if (qrow >= L) {
+  if (qrow >= L) {
 #pragma unroll
-      for (int m = 0; m < DB; ++m)
+    for (int m = 0; m < DB; ++m)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-    }
-    store_acc_T<float, D, DB>(dq_base + (int64_t)qrow * D, acc, p.scale * kDown3, h);
+      for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
   }
+  store_rows_f32<D, DIRECT>(row_patch<D>(smem_raw, wave), dq_base + (int64_t)row0 * D, T_ - row0, acc, p.scale * kDown3, lane);
 }
 
 // dK and dV, one wave per 32 keys, tiles of 32 queries, two stages.  Four products per tile; the vector work sits behind
@@ -593,40 +719,57 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
     sg.load(gbase, p.do_st, t * TQ, L - 1, tid);
     if (tid < 2 * TQ) r_row = row_base[valid(t * TQ + tid % TQ)];
   };
-  auto stage_ptr = [&](int t) { return smem_raw + ((t - qt0) & 1) * STAGE_BYTES; };
-  auto store_tile = [&](int t) {
-    __bf16* st = reinterpret_cast<__bf16*>(stage_ptr(t));
+  constexpr bool DIRECT = direct_rows(D, NW);
+  const TileOrder order(qt0, qt1, DIRECT ? 0 : p.period, p.pdiv);
+  auto store_tile = [&](int it) {
+    __bf16* st = reinterpret_cast<__bf16*>(smem_raw + (it & 1) * STAGE_BYTES);
     sq.store(st, tid);
     sg.store(st + TILE, tid);
     if (tid < 2 * TQ) reinterpret_cast<float*>(st + 2 * TILE)[tid] = tid < TQ ? r_row : r_row * kUp2;
   };
   static_assert(2 * TQ <= NT, "one thread per staged row value");
-  load_tile(qt0);
+  using Rows = OwnRows32<D>;
+  const int row0 = k0 + wave * 32;
+  float* const k_area = reinterpret_cast<float*>(smem_raw) + wave * Rows::ELEMS;
+  float* const v_area = k_area + NW * Rows::ELEMS;
+  const float* kbase = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
+  const float* vbase = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
+  if (!DIRECT) {
+    Rows::send(kbase, p.k_st, row0, L - 1, k_area, lane);
+    Rows::send(vbase, p.v_st, row0, L - 1, v_area, lane);
+  }
+  load_tile(order.first);
 
   Split8 kf[NF], vf[NF];
   {
-    const int kr = valid(krow);
     HalfRow<D> k_row, v_row;
-    k_row.load(reinterpret_cast<const float*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh + (int64_t)kr * p.k_st, h);
-    v_row.load(reinterpret_cast<const float*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh + (int64_t)kr * p.v_st, h);
+    if (DIRECT) {
+      k_row.load(kbase + (int64_t)valid(krow) * p.k_st, h);
+      v_row.load(vbase + (int64_t)valid(krow) * p.v_st, h);
+    } else {
+      landed();
+      k_row.read(k_area, lane);
+      v_row.read(v_area, lane);
+    }
     k_row.split(kf, p.scale_log2e < 0.0f);
     v_row.split(vf, false);
   }
+  if (!DIRECT) __syncthreads();   // the tiles go where the rows were
 
   f32x16 dk[DB], dv[DB];
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
-  store_tile(qt0);
+  store_tile(0);
   __syncthreads();
 
-  for (int t = qt0; t < qt1; ++t) {
-    const __bf16* Qt = reinterpret_cast<const __bf16*>(stage_ptr(t));
+  for (int t = order.first, it = 0; it < qt1 - qt0; ++it, t = order.next(t)) {
+    const __bf16* Qt = reinterpret_cast<const __bf16*>(smem_raw + (it & 1) * STAGE_BYTES);
     const __bf16* Gt = Qt + TILE;
     const float* rows = reinterpret_cast<const float*>(Qt + 2 * TILE);
-    const bool more = t + 1 < qt1;
-    if (more) load_tile(t + 1);
+    const bool more = order.next(t) != order.first;
+    if (more) load_tile(order.next(t));
     const int qs = t * TQ;
     if (qs + TQ > qlo_min && qs < qhi_max) {
       const bool interior = qs >= qlo_max && qs + TQ <= qhi_min;
@@ -661,7 +804,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
       });
       mma_tr_split<D, TQ>(dk, Qt, sb, lane);                 // dK^T[d][key] += Q^T dS
     }
-    if (more) store_tile(t + 1);
+    if (more) store_tile(it + 1);
     __syncthreads();
   }
 
@@ -670,16 +813,15 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
     dkdv_rows<float, D, NW, TQ>(p, again_s(bh), again_s(kt), again_v(tid));
     return;
   }
-  if (krow < T_) {
-    if (krow >= L) {
+  if (krow >= L) {
 #pragma unroll
-      for (int m = 0; m < DB; ++m)
+    for (int m = 0; m < DB; ++m)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
-    }
-    store_acc_T<float, D, DB>(dk_base + (int64_t)krow * D, dk, p.scale * kDown3, h);
-    store_acc_T<float, D, DB>(dv_base + (int64_t)krow * D, dv, kDown2, h);
+      for (int i = 0; i < 16; ++i) dk[m][i] = 0.0f, dv[m][i] = 0.0f;
   }
+  float* const patch = row_patch<D>(smem_raw, wave);
+  store_rows_f32<D, DIRECT>(patch, dk_base + (int64_t)row0 * D, T_ - row0, dk, p.scale * kDown3, lane);
+  store_rows_f32<D, DIRECT>(patch, dv_base + (int64_t)row0 * D, T_ - row0, dv, kDown2, lane);
 }
 
 }  // namespace sa

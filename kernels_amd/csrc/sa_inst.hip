@@ -61,7 +61,11 @@ template <typename K> static int prepare(K kernel, size_t lds_bytes, PrepareStat
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // LDS of a float32 kernel on the 16-bit matrix pipe: its split tiles, or the float32 tiles of the rows it goes through again.
-constexpr size_t split_lds(size_t split_bytes, size_t rows_bytes) { return split_bytes > rows_bytes ? split_bytes : rows_bytes; }
+// (or the own rows of its waves, `own` sets of them, or their row patches: whichever is most)
+template <int D, int NW> constexpr size_t split_lds(size_t split_bytes, size_t rows_bytes, int own) {
+  return std::max({split_bytes, rows_bytes, direct_rows(D, NW) ? 0 : (size_t)own * NW * OwnRows32<D>::ELEMS * sizeof(float),
+                   64 + (size_t)NW * RowPatch32<D>::ELEMS * sizeof(float)});
+}
 template <int D> constexpr size_t float_tiles = (size_t)2 * 2 * 32 * TileGeom<float, D>::PITCH * sizeof(float);   // two stages
 
 // float32, head dimensions 16 to 64: workgroups of 64 rows (two waves) instead of 128 where twice as many still find a CU
@@ -141,11 +145,12 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
 #endif
 }
 template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipStream_t st) {
-  constexpr size_t lds = split_lds((size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>);
+  constexpr size_t lds = split_lds<D, NW>((size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>, 1);
   auto kern = fwd_split_kernel<D, NW, NST>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, NW * 32);
+  set_tile_order(p, NW * 32, 32);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -252,11 +257,12 @@ template <int D> static int dq3_launch(BwdParams p, hipStream_t st) {
 }
 template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st) {
   constexpr int TQ = NW * 32;
-  constexpr size_t lds = split_lds((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>);
+  constexpr size_t lds = split_lds<D, NW>((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>, 2);
   auto kern = dq_split_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TQ);
+  set_tile_order(p, TQ, 32);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -359,11 +365,12 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
 template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream_t st) {
   constexpr int TKB = NW * 32;
   constexpr size_t rows = (size_t)2 * 2 * 32 * sizeof(float);   // lse and delta
-  constexpr size_t lds = split_lds((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + rows, float_tiles<D> + rows);
+  constexpr size_t lds = split_lds<D, NW>((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16) + rows, float_tiles<D> + rows, 2);
   auto kern = dkdv_split_f32_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   p.n_tiles = (int)ceil_div(p.T, TKB);
+  set_tile_order(p, TKB, 32);
   const int64_t blocks = (int64_t)p.B * p.H * p.n_tiles;
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
