@@ -63,7 +63,7 @@ SA_DEV void dq_rows(const BwdParams& p, int bh, int qt, int tid, Delta&& delta) 
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  const int hd = bh % p.H, b = bh / p.H;
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
 
@@ -198,7 +198,7 @@ SA_DEV void dq_rows(const BwdParams& p, int bh, int qt, int tid, Delta&& delta) 
 template <typename T, int D, int NW, int TK>
 __global__ __launch_bounds__(NW * 64) void dq_kernel(const BwdParams p) {
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
   dq_rows<T, D, NW, TK>(p, bh, qt, threadIdx.x, [&](int row) { return p.delta[(int64_t)bh * p.T + row]; });
 }
 
@@ -227,7 +227,7 @@ SA_DEV void dkdv_rows(const BwdParams& p, int bh, int kt, int tid) {   // one wo
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  const int hd = bh % p.H, b = bh / p.H;
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
 
@@ -411,7 +411,7 @@ SA_DEV void dkdv_rows(const BwdParams& p, int bh, int kt, int tid) {   // one wo
 template <typename T, int D, int NW, int TQ, int PASS = 0>
 __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
   int bh, kt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, kt);
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, kt);
   dkdv_rows<T, D, NW, TQ, PASS>(p, bh, kt, threadIdx.x);
 }
 
@@ -525,8 +525,8 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, growing_tiles(p.C, p.R, p.T, NW * 32));
-  const int hd = bh % p.H, b = bh / p.H;
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
 
@@ -687,9 +687,8 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, kt, L;
-  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
-                  p.lens_stride, bh, kt, L);
-  const int hd = bh % p.H, b = bh / p.H;
+  key_tile_coords(blockIdx.x, gridDim.x, p.tiles, TKB, p.T, p.lens, p.lens_stride, bh, kt, L);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
   const int k0 = kt * TKB;

@@ -57,8 +57,8 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, rt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, rt);
-  const int hd = bh % p.H, b = bh / p.H;
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, rt);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
   int L = T_;

@@ -66,9 +66,8 @@ __global__ __launch_bounds__(512) void dkdv_split_kernel(const BwdParams p) {
   const bool grad_role = wave >= NP;
 
   int bh, kt, L;
-  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
-                  p.lens_stride, bh, kt, L);
-  const int hd = bh % p.H, b = bh / p.H;
+  key_tile_coords(blockIdx.x, gridDim.x, p.tiles, TKB, p.T, p.lens, p.lens_stride, bh, kt, L);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
   const int k0 = kt * TKB;
@@ -361,9 +360,8 @@ __global__ __launch_bounds__(512) void dkdv_split_wide_kernel(const BwdParams p)
   float* const xbuf = row_ring + NQ * 2 * TQ + pair * 2 * S::XSLOT + lane * 4;   // two slots of 16 values per lane
 
   int bh, kt, L;
-  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
-                  p.lens_stride, bh, kt, L);
-  const int hd = bh % p.H, b = bh / p.H;
+  key_tile_coords(blockIdx.x, gridDim.x, p.tiles, TKB, p.T, p.lens, p.lens_stride, bh, kt, L);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   const int k0 = kt * TKB;
   T* dk_base = reinterpret_cast<T*>(p.dk) + (int64_t)bh * T_ * D;

@@ -645,6 +645,28 @@ template <typename T, int D, int ROWS, int NT> struct Stager {
   }
 };
 
+// Division of a number below 2^31 by a divisor that the host knows (the chunk size, the tiles of a sequence, the heads) without
+// the 30-instruction emulation of an integer division:
+// with l = ceil(log2(d)) and m = ceil(2^(31+l) / d) (m < 2^32), n / d == (n * m) >> (31 + l) for every
+// 0 <= n < 2^31 (Granlund and Montgomery, "Division by invariant integers using multiplication", 1994).
+struct ChunkDiv {
+  uint32_t mul, shift;
+};
+constexpr ChunkDiv chunk_div(int d) {   // d >= 1
+  uint32_t l = 0;
+  while ((1ull << l) < (unsigned long long)d) ++l;
+  const unsigned long long two = 1ull << (31 + l);
+  return ChunkDiv{(uint32_t)((two + (unsigned long long)d - 1) / (unsigned long long)d), 31 + l};
+}
+constexpr int div_by(int n, ChunkDiv c) { return (int)(((unsigned long long)(uint32_t)n * c.mul) >> c.shift); }
+static_assert(div_by(0x7fffffff, chunk_div(1)) == 0x7fffffff && div_by(12345, chunk_div(1)) == 12345, "d = 1");
+static_assert(div_by(0x7fffffff, chunk_div(2)) == 0x3fffffff && div_by(0x7ffffffe, chunk_div(0x7fffffff)) == 0 &&
+              div_by(0x7fffffff, chunk_div(0x7fffffff)) == 1, "extremes");
+static_assert(div_by(2999, chunk_div(10)) == 299 && div_by(3000, chunk_div(10)) == 300 && div_by(95, chunk_div(96)) == 0 &&
+              div_by(96, chunk_div(96)) == 1 && div_by(0x7fffffff, chunk_div(10)) == 214748364 &&
+              div_by(0x7fffffff, chunk_div(3)) == 715827882 && div_by(0x7fffffff, chunk_div(641)) == 3350208 &&
+              div_by(65535, chunk_div(256)) == 255 && div_by(0x7fffffff, chunk_div(10000)) == 214748, "samples");
+
 // Hardware hands workgroup i to XCD i % 8 (each XCD has its own L2).  Map block ids so that
 // all tiles of one (batch, head) run on one XCD, in consecutive dispatch slots -- neighbouring
 // tiles then share that L2 for the keys and values they have in common -- and so that the
@@ -658,71 +680,66 @@ template <typename T, int D, int ROWS, int NT> struct Stager {
 // B=4, H=16, T=16384, D=128 and 3-4 % on small problems; the long-window forward kernel loses 1 % (tiles
 // of one sequence that share keys in L2 no longer run side by side) and passes n_start = 0.  A tail that
 // keeps the tiles of a (batch, head) pair together measured slower than either.
-SA_DEV void tile_coords(int bid, int n_blocks, int n_tiles, int& bh, int& tile, int n_start = 0) {
-  const int nbh = n_blocks / n_tiles;
+// All divisors are the host's (three emulated divisions, one after the other, before a workgroup's first load): 0.6 to 1.3 % on
+// windows of about a hundred keys, whose workgroups live for three tiles (B=225, H=4, T<=993, D=32 110.8 -> 109.1 us).
+struct TileMap {
+  int n_tiles, nbh;   // tiles of a (batch, head) pair, pairs
+  int n_tail;         // cheap tiles of every pair that are dispatched last
+  ChunkDiv by_tiles, by_lead, by_pairs, by_heads;   // n_tiles, n_tiles - n_tail, nbh / 8, H
+};
+SA_DEV void tile_coords(int bid, int n_blocks, const TileMap& m, int& bh, int& tile) {
   int logical;
-  if ((nbh & 7) == 0) {
-    const int x = bid & 7, idx = bid >> 3;
-    const int nb = nbh >> 3;
-    const int ns = 2 * n_start <= n_tiles ? n_start : 0;
-    const int nl = n_tiles - ns;
+  const int x = bid & 7, idx = bid >> 3;
+  if ((m.nbh & 7) == 0) {
+    const int nb = m.nbh >> 3, nl = m.n_tiles - m.n_tail;
     if (idx < nb * nl) {
-      bh = (idx / nl) * 8 + x;
-      logical = idx % nl;
+      const int pair = div_by(idx, m.by_lead);
+      bh = pair * 8 + x;
+      logical = idx - pair * nl;
     } else {
-      const int r = idx - nb * nl;
-      bh = (r % nb) * 8 + x;
-      logical = nl + r / nb;
+      const int r = idx - nb * nl, t = div_by(r, m.by_pairs);
+      bh = (r - t * nb) * 8 + x;
+      logical = nl + t;
     }
   } else {
     const int per = n_blocks >> 3, rem = n_blocks & 7;
-    const int x = bid & 7, idx = bid >> 3;
     const int l = x * per + (x < rem ? x : rem) + idx;
-    bh = l / n_tiles;
-    logical = l % n_tiles;
+    bh = div_by(l, m.by_tiles);
+    logical = l - bh * m.n_tiles;
   }
-  tile = n_tiles - 1 - logical;
+  tile = m.n_tiles - 1 - logical;
 }
 // The same for key tiles of ROWS keys.  There the short tiles are the last n_end ones below a sequence's length
 // L (the queries that see those keys stop at L), so the order depends on L: tiles below them and the empty
 // tiles beyond L come first, then, tile by tile over the XCD's (batch, head) pairs, the n_end tiles that lead up to L.
 // Returns the clamped length of the pair's sequence as well.
-#ifndef SA_ORDER_KEYS
-#define SA_ORDER_KEYS 1
-#endif
-SA_DEV void key_tile_coords(int bid, int n_blocks, int n_tiles, int n_end, int ROWS, int H, int T,
-                            const int32_t* lens, int64_t lens_stride, int& bh, int& tile, int& L) {
-  const int nbh = n_blocks / n_tiles;
-  const int ns = (SA_ORDER_KEYS && (nbh & 7) == 0 && 2 * n_end <= n_tiles) ? n_end : 0;
+SA_DEV void key_tile_coords(int bid, int n_blocks, const TileMap& m, int ROWS, int T, const int32_t* lens, int64_t lens_stride,
+                            int& bh, int& tile, int& L) {
+  const int ns = m.n_tail;
   if (ns == 0) {
-    tile_coords(bid, n_blocks, n_tiles, bh, tile);
+    tile_coords(bid, n_blocks, m, bh, tile);
   } else {
-    const int x = bid & 7, idx = bid >> 3, nb = nbh >> 3, nl = n_tiles - ns;
+    const int x = bid & 7, idx = bid >> 3, nb = m.nbh >> 3, nl = m.n_tiles - ns;
     if (idx < nb * nl) {
-      bh = (idx / nl) * 8 + x;
-      tile = nl - 1 - idx % nl;      // position among the tiles that are not in the tail
+      const int pair = div_by(idx, m.by_lead);
+      bh = pair * 8 + x;
+      tile = nl - 1 - (idx - pair * nl);   // position among the tiles that are not in the tail
     } else {
-      const int r = idx - nb * nl;
-      bh = (r % nb) * 8 + x;
-      tile = -1 - r / nb;            // -1 - j: tail tile j, counted towards L
+      const int r = idx - nb * nl, t = div_by(r, m.by_pairs);
+      bh = (r - t * nb) * 8 + x;
+      tile = -1 - t;                       // -1 - j: tail tile j, counted towards L
     }
   }
   L = T;
   if (lens) {
-    L = lens[(int64_t)(bh / H) * lens_stride];
+    L = lens[(int64_t)div_by(bh, m.by_heads) * lens_stride];
     L = L < 0 ? 0 : (L > T ? T : L);
   }
   if (ns != 0) {
-    const int live = (L + ROWS - 1) / ROWS < n_tiles ? (L + ROWS - 1) / ROWS : n_tiles;   // tiles with a key below L
-    const int a = live > ns ? live - ns : 0;                                               // tiles before the tail
+    const int live = (L + ROWS - 1) / ROWS < m.n_tiles ? (L + ROWS - 1) / ROWS : m.n_tiles;   // tiles with a key below L
+    const int a = live > ns ? live - ns : 0;                                                   // tiles before the tail
     tile = tile < 0 ? a + (-1 - tile) : (tile < a ? tile : tile + ns);
   }
-}
-
-// Number of leading query tiles of ROWS rows whose windows are still growing: rows below back_contexts chunks.
-SA_DEV int growing_tiles(int C, int R, int T, int ROWS) {
-  const int64_t rows = (int64_t)C * (int64_t)R;
-  return rows >= (int64_t)T ? 0x3fffffff : (int)((rows + ROWS - 1) / ROWS);
 }
 
 // Write four consecutive fp32 values as four elements of T.
@@ -798,27 +815,6 @@ SA_DEV void store_rows_coalesced(T* patch, T* out_rows, int rows_valid, const f3
   }
 }
 
-// Division of a position below 2^31 by the chunk size without the hardware's 30-instruction emulation:
-// with l = ceil(log2(d)) and m = ceil(2^(31+l) / d) (m < 2^32), n / d == (n * m) >> (31 + l) for every
-// 0 <= n < 2^31 (Granlund and Montgomery, "Division by invariant integers using multiplication", 1994).
-struct ChunkDiv {
-  uint32_t mul, shift;
-};
-constexpr ChunkDiv chunk_div(int d) {   // d >= 1
-  uint32_t l = 0;
-  while ((1ull << l) < (unsigned long long)d) ++l;
-  const unsigned long long two = 1ull << (31 + l);
-  return ChunkDiv{(uint32_t)((two + (unsigned long long)d - 1) / (unsigned long long)d), 31 + l};
-}
-constexpr int div_by(int n, ChunkDiv c) { return (int)(((unsigned long long)(uint32_t)n * c.mul) >> c.shift); }
-static_assert(div_by(0x7fffffff, chunk_div(1)) == 0x7fffffff && div_by(12345, chunk_div(1)) == 12345, "d = 1");
-static_assert(div_by(0x7fffffff, chunk_div(2)) == 0x3fffffff && div_by(0x7ffffffe, chunk_div(0x7fffffff)) == 0 &&
-              div_by(0x7fffffff, chunk_div(0x7fffffff)) == 1, "extremes");
-static_assert(div_by(2999, chunk_div(10)) == 299 && div_by(3000, chunk_div(10)) == 300 && div_by(95, chunk_div(96)) == 0 &&
-              div_by(96, chunk_div(96)) == 1 && div_by(0x7fffffff, chunk_div(10)) == 214748364 &&
-              div_by(0x7fffffff, chunk_div(3)) == 715827882 && div_by(0x7fffffff, chunk_div(641)) == 3350208 &&
-              div_by(65535, chunk_div(256)) == 255 && div_by(0x7fffffff, chunk_div(10000)) == 214748, "samples");
-
 // Where a workgroup begins to go through the tiles [t0, t1) of its window: at the multiple of `period`, the number of tiles of
 // a full window, among them, and round to the tile before it.  Neighbouring workgroups of an XCD, whose windows
 // overlap, then read the same tile at the same time and it crosses into their L2 once; each from its own first tile on, they read it
@@ -846,7 +842,7 @@ struct FwdParams {
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st;  // element strides
   int B, H, T, C, R;
   float scale_log2e;  // sm_scale * log2(e); sign carried separately
-  int n_tiles;        // query tiles per (b,h)
+  TileMap tiles;
   ChunkDiv cdiv;      // division by C
   int period;         // TileOrder; 0: ascending
   ChunkDiv pdiv;      // division by period
@@ -861,7 +857,7 @@ struct BwdParams {
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, do_sb, do_sh, do_st;
   int B, H, T, C, R;
   float scale, scale_log2e;
-  int n_tiles;
+  TileMap tiles;
   // Set only for a dQ kernel that forms the row sums itself (delta_out != null): the forward output, its
   // element strides, and where the sums go for the dK/dV kernel that runs after it.  `delta` is then unused.
   const void* o;

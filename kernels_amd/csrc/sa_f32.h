@@ -358,8 +358,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, growing_tiles(p.C, p.R, p.T, TQ));
-  const int hd = bh % p.H, b = bh / p.H;
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T;
   int L = T_;
   if (p.lens) {
@@ -518,8 +518,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, growing_tiles(p.C, p.R, p.T, TQ));
-  const int hd = bh % p.H, b = bh / p.H;
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T;
   int L = T_;
   if (p.lens) {
@@ -680,9 +680,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, kt, L;
-  key_tile_coords(blockIdx.x, gridDim.x, p.n_tiles, growing_tiles(p.C, p.R, p.T, TKB), TKB, p.H, p.T, p.lens,
-                  p.lens_stride, bh, kt, L);
-  const int hd = bh % p.H, b = bh / p.H;
+  key_tile_coords(blockIdx.x, gridDim.x, p.tiles, TKB, p.T, p.lens, p.lens_stride, bh, kt, L);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   const int k0 = kt * TKB;
   float* dk_base = reinterpret_cast<float*>(p.dk) + (int64_t)bh * T_ * D;

@@ -28,7 +28,7 @@ SA_DEV void fwd_rows(const FwdParams& p, int bh, int qt, int tid) {
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  const int hd = bh % p.H, b = bh / p.H;
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
 
@@ -216,7 +216,7 @@ SA_DEV void fwd_rows(const FwdParams& p, int bh, int qt, int tid) {
 template <typename T, int D, int NW, int TK>
 __global__ __launch_bounds__(NW * 64) void fwd_kernel(const FwdParams p) {
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt);
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
   fwd_rows<T, D, NW, TK>(p, bh, qt, threadIdx.x);
 }
 
@@ -288,8 +288,8 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.n_tiles, bh, qt, SHORT ? growing_tiles(p.C, p.R, p.T, NW * QB * 32) : 0);
-  const int hd = bh % p.H, b = bh / p.H;
+  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
   const int T_ = p.T, C = p.C, R = p.R;
   auto cdiv = [&](int x) { return div_by(x, p.cdiv); };   // x / C
 

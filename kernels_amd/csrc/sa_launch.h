@@ -115,6 +115,21 @@ inline int tiles_of_window(int T, int chunk, int back, int rows, int tile) {
   const bool aligned = chunk % tile == 0 || (rows % chunk == 0 && (long long)chunk * back % tile == 0);
   return (int)((span + tile - 1 + (aligned ? 0 : tile - 1)) / tile);
 }
+// The workgroups of a launch, `rows` rows each, and how they are dispatched (tile_coords): with `tail`, those whose windows
+// are still growing (query tiles: the first R chunks of a sequence) or already shrinking (key tiles: the last) come last, where
+// the pairs divide over the XCDs and they are no more than half.
+template <typename P> int64_t set_tiles(P& p, int rows, bool tail) {
+  TileMap& m = p.tiles;
+  m.n_tiles = (int)(((int64_t)p.T + rows - 1) / rows);
+  const int64_t nbh = (int64_t)p.B * p.H, growing = ((int64_t)p.C * p.R + rows - 1) / rows;
+  m.nbh = (int)nbh;
+  m.n_tail = tail && nbh % 8 == 0 && (int64_t)p.C * p.R < p.T && 2 * growing <= m.n_tiles ? (int)growing : 0;
+  m.by_tiles = chunk_div(m.n_tiles);
+  m.by_lead = chunk_div(m.n_tiles - m.n_tail);
+  m.by_pairs = chunk_div(nbh >= 16 && nbh <= 0x7fffffff ? (int)(nbh >> 3) : 1);
+  m.by_heads = chunk_div(p.H);
+  return nbh * m.n_tiles;
+}
 template <typename P> void set_tile_order(P& p, int rows, int tile) {
   p.period = tiles_of_window(p.T, p.C, p.R, rows, tile);
   p.pdiv = chunk_div(p.period > 0 ? p.period : 1);
