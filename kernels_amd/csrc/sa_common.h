@@ -684,14 +684,17 @@ static_assert(div_by(2999, chunk_div(10)) == 299 && div_by(3000, chunk_div(10)) 
 // windows of about a hundred keys, whose workgroups live for three tiles (B=225, H=4, T<=993, D=32 110.8 -> 109.1 us).
 struct TileMap {
   int n_tiles, nbh;   // tiles of a (batch, head) pair, pairs
-  int n_tail;         // cheap tiles of every pair that are dispatched last
+  int n_tail;         // cheap tiles of every pair that are dispatched last, or first
+  int tail_first;     // workgroups of those (of one XCD) if first, else 0
   ChunkDiv by_tiles, by_lead, by_pairs, by_heads;   // n_tiles, n_tiles - n_tail, nbh / 8, H
 };
 SA_DEV void tile_coords(int bid, int n_blocks, const TileMap& m, int& bh, int& tile) {
   int logical;
-  const int x = bid & 7, idx = bid >> 3;
+  const int x = bid & 7;
+  int idx = bid >> 3;
   if ((m.nbh & 7) == 0) {
     const int nb = m.nbh >> 3, nl = m.n_tiles - m.n_tail;
+    idx = idx < m.tail_first ? nb * nl + idx : idx - m.tail_first;
     if (idx < nb * nl) {
       const int pair = div_by(idx, m.by_lead);
       bh = pair * 8 + x;
@@ -719,7 +722,9 @@ SA_DEV void key_tile_coords(int bid, int n_blocks, const TileMap& m, int ROWS, i
   if (ns == 0) {
     tile_coords(bid, n_blocks, m, bh, tile);
   } else {
-    const int x = bid & 7, idx = bid >> 3, nb = m.nbh >> 3, nl = m.n_tiles - ns;
+    const int x = bid & 7, nb = m.nbh >> 3, nl = m.n_tiles - ns;
+    int idx = bid >> 3;
+    idx = idx < m.tail_first ? nb * nl + idx : idx - m.tail_first;
     if (idx < nb * nl) {
       const int pair = div_by(idx, m.by_lead);
       bh = pair * 8 + x;

@@ -112,7 +112,7 @@ template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p,
   auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, TK, C::FWD2_NST, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TQ, SHORT);
+  const int64_t blocks = set_tiles(p, TQ, !SHORT ? PLAIN : D == 256 ? SHORT_FIRST : SHORT_LAST);
   set_tile_order(p, TQ, TK);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -133,7 +133,7 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
     auto kern = fwd3_kernel<ElemT, D, NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, false);
+    const int64_t blocks = set_tiles(p, TQ, PLAIN);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
@@ -147,7 +147,7 @@ template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipSt
   auto kern = fwd_split_kernel<D, NW, NST>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, NW * 32, true);
+  const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
   set_tile_order(p, NW * 32, 32);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -184,7 +184,7 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
     auto kern = fwd_kernel<ElemT, D, C::NW, C::FWD_TK>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, false);
+    const int64_t blocks = set_tiles(p, TQ, PLAIN);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
     return (int)hipGetLastError();
@@ -219,7 +219,7 @@ template <int D, int NW> static int dq2_launch(BwdParams p, hipStream_t st) {
   auto kern = dq2_kernel<ElemT, D, NW, C::DQ2_TK, C::DQ2_NST>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TQ, true);
+  const int64_t blocks = set_tiles(p, TQ, D == 256 ? SHORT_FIRST : SHORT_LAST);
   set_tile_order(p, TQ, C::DQ2_TK);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -240,7 +240,7 @@ template <int D> static int dq3_launch(BwdParams p, hipStream_t st) {
     auto kern = dq3_kernel<ElemT, D, NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, true);
+    const int64_t blocks = set_tiles(p, TQ, SHORT_LAST);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
@@ -255,7 +255,7 @@ template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st)
   auto kern = dq_split_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TQ, true);
+  const int64_t blocks = set_tiles(p, TQ, SHORT_LAST);
   set_tile_order(p, TQ, 32);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -280,7 +280,7 @@ template <int D> static int dq_d(BwdParams p, hipStream_t st) {
     auto kern = dq_kernel<ElemT, D, C::NW, C::DQ_TK>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, false);
+    const int64_t blocks = set_tiles(p, TQ, PLAIN);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
     return (int)hipGetLastError();
@@ -308,7 +308,7 @@ template <int D> static int dkdv3_launch(BwdParams p, hipStream_t st) {
     auto kern = dkdv3_kernel<ElemT, D, C::DKDV3_NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TKB, true);
+    const int64_t blocks = set_tiles(p, TKB, SHORT_LAST);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, st, p);
     return (int)hipGetLastError();
@@ -331,7 +331,7 @@ template <int D> static int dkdv_split_launch(BwdParams p, hipStream_t st) {
     auto kern = dkdv_split_kernel<ElemT, D, NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TKB, true);
+    const int64_t blocks = set_tiles(p, TKB, SHORT_FIRST);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
@@ -345,7 +345,7 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
   auto kern = dkdv_split_wide_kernel<ElemT, D>;
   static PrepareState once;
   if (int rc = prepare(kern, S::lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, S::TKB, true);
+  const int64_t blocks = set_tiles(p, S::TKB, SHORT_FIRST);
   set_tile_order(p, S::TKB, S::TQ);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * S::NP * 64), S::lds, st, p);
@@ -358,7 +358,7 @@ template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream
   auto kern = dkdv_split_f32_kernel<D, NW>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TKB, true);
+  const int64_t blocks = set_tiles(p, TKB, SHORT_LAST);
   set_tile_order(p, TKB, 32);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -387,7 +387,7 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     auto kern = dkdv2_kernel<ElemT, D, C::DKDV2_NW, C::DKDV2_TQ, C::DKDV2_NST>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TKB, true);
+    const int64_t blocks = set_tiles(p, TKB, SHORT_LAST);
     set_tile_order(p, TKB, C::DKDV2_TQ);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::DKDV2_NW * 64), lds, st, p);
@@ -401,7 +401,7 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     constexpr int TKB = C::NW * 32;
     constexpr size_t lds =
         (size_t)2 * (2 * C::DKDV_TQ * TileGeom<ElemT, D>::PITCH * sizeof(ElemT) + 2 * C::DKDV_TQ * sizeof(float));
-    const int64_t blocks = set_tiles(p, TKB, false);
+    const int64_t blocks = set_tiles(p, TKB, PLAIN);
     if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
     if constexpr (sizeof(ElemT) == 4 && D == 256) {
       // both accumulators and both resident rows do not fit a lane's registers: one launch per gradient
@@ -436,7 +436,7 @@ template <int D, int NW, int TT> static int bwd_fused_launch(BwdParams p, hipStr
   auto kern = bwd_fused_kernel<ElemT, D, NW, TT>;
   static PrepareState once;
   if (int rc = prepare(kern, S::template lds_bytes<ElemT, D>(BWD_FUSED_MAX_ROWS), once)) return rc;
-  const int64_t blocks = set_tiles(p, S::ROWS, false);
+  const int64_t blocks = set_tiles(p, S::ROWS, PLAIN);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();

@@ -115,15 +115,24 @@ inline int tiles_of_window(int T, int chunk, int back, int rows, int tile) {
   const bool aligned = chunk % tile == 0 || (rows % chunk == 0 && (long long)chunk * back % tile == 0);
   return (int)((span + tile - 1 + (aligned ? 0 : tile - 1)) / tile);
 }
-// The workgroups of a launch, `rows` rows each, and how they are dispatched (tile_coords): with `tail`, those whose windows
-// are still growing (query tiles: the first R chunks of a sequence) or already shrinking (key tiles: the last) come last, where
-// the pairs divide over the XCDs and they are no more than half.
-template <typename P> int64_t set_tiles(P& p, int rows, bool tail) {
+// The workgroups of a launch, `rows` rows each, and how they are dispatched (tile_coords).  Those whose windows are still growing
+// (query tiles: the first R chunks of a sequence) or already shrinking (key tiles: the last) come last with SHORT_LAST, where
+// the pairs divide over the XCDs and they are no more than half.  SHORT_FIRST, for kernels with one workgroup per CU: equal
+// workgroups that start together stay in step, all CUs fetch their rows at the same time and the memory idles while all
+// multiply (a fifth of dQ at head dimension 256 went by at full memory rate); short workgroups at the beginning leave the CUs at
+// different points.  Only from 512 workgroups on: a last round of long workgroups on a few CUs costs more.  Forward and
+// backward in us, short last -> first: D=256, chunks of 128, 4 back, B*H=64, T=4096 884 -> 865, ragged 647 -> 628; 64, 3 back, B*H=32,
+// T=2000 143 -> 139; B*H=16, T=3000 (384 workgroups) 187 -> 185, ragged 137 -> 151.  dkdv_split_kernel, D=128, B*H=128, T=2048, 64, 1 back ragged
+// 164 -> 158, 50, 3 back, B*H=96, T=2000 215 -> 206.  Two or three workgroups per CU keep each other busy and lose: D=64, 128, 4 back
+// 422 -> 431.  The other kernels of head dimension 128 gain on some windows and lose as much on others.
+enum Tail { PLAIN, SHORT_LAST, SHORT_FIRST };
+template <typename P> int64_t set_tiles(P& p, int rows, Tail tail) {
   TileMap& m = p.tiles;
   m.n_tiles = (int)(((int64_t)p.T + rows - 1) / rows);
   const int64_t nbh = (int64_t)p.B * p.H, growing = ((int64_t)p.C * p.R + rows - 1) / rows;
   m.nbh = (int)nbh;
-  m.n_tail = tail && nbh % 8 == 0 && (int64_t)p.C * p.R < p.T && 2 * growing <= m.n_tiles ? (int)growing : 0;
+  m.n_tail = tail != PLAIN && nbh % 8 == 0 && (int64_t)p.C * p.R < p.T && 2 * growing <= m.n_tiles ? (int)growing : 0;
+  m.tail_first = tail == SHORT_FIRST && nbh * m.n_tiles >= 512 ? (int)(nbh / 8) * m.n_tail : 0;
   m.by_tiles = chunk_div(m.n_tiles);
   m.by_lead = chunk_div(m.n_tiles - m.n_tail);
   m.by_pairs = chunk_div(nbh >= 16 && nbh <= 0x7fffffff ? (int)(nbh >> 3) : 1);
