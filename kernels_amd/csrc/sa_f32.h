@@ -341,8 +341,9 @@ struct QueryWindow {
 
 // Forward.  One wave per 32 queries, tiles of 32 keys in NST stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
 // bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back, us with the float32 instruction -> here: D=128 720 -> 455,
-// D=64 392 -> 220, D=32 200 -> 125, D=16 167 -> 107.  The register limits (four waves per SIMD up to 32, three at 64, two at
-// 128) make D=64 and 128 spill 20 and 25 registers per lane, 71 in the four-wave form of 128, around the products.
+// D=64 392 -> 220, D=32 200 -> 125, D=16 167 -> 107 (with OwnRows32, whole-row stores and TileOrder 456 -> 432, 223 -> 218, 129 -> 128
+// on one box).  The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 31
+// registers per lane, 82 in the four-wave form of 128, around the products.
 template <int D, int NW, int NST>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D>::DB;
@@ -665,7 +666,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
 // dK and dV, one wave per 32 keys, tiles of 32 queries, two stages.  Four products per tile; the vector work sits behind
 // their matrix instructions (the exponentials and the parts of P behind dP, dS and its parts behind dV): from head
 // dimension 64 on a wave has its SIMD to itself.  Held to 256 registers for a second wave, D=64 spilled and measured
-// the same or slower.  Same problem as above: D=128 1470 -> 883 us (40 registers spilled), D=64 665 -> 476, D=32 351 -> 245,
+// the same or slower.  Same problem as above: D=128 1470 -> 883 us (42 registers spilled), D=64 665 -> 476, D=32 351 -> 245,
 // D=16 261 -> 194.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_kernel(const BwdParams p) {
