@@ -243,7 +243,8 @@ struct Fwd2Slots {
 // largest probability of a row's first tile is exactly 1 in the element type and the results are those of whole tiles, bit
 // for bit unless a later tile moves a maximum.  (A maximum of each half's own took O 0.2 to 1.5 % further from the
 // exact result.)  B=4, H=16, T=4096, bfloat16: chunks of 128, 4 back 266 -> 217 us (743 TFLOP/s), chunks of 10, 9 back,
-// ragged 150 -> 105; 2 x 16, one chunk of 4096, ragged 475 -> 339; with each half's own maximum 218, 104, 326.
+// ragged 150 -> 105; 2 x 16, one chunk of 4096, ragged 475 -> 339; with each half's own maximum 218, 104, 326.  Chunks of 128,
+// 4 back in TileOrder, short windows first: 215 -> 181.
 //
 // Same algorithm as fwd_kernel, different resource balance: each wave owns QB blocks of 32
 // queries, so every K / V fragment fetched from LDS feeds QB MFMAs (the transposing V reads
