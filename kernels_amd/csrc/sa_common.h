@@ -443,6 +443,17 @@ SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename E
       });
 }
 
+// One buffer_load_dwordx4 ... lds written as assembly.  The compiler pads no hazard inside the statement or at its edge, and any
+// of the scalars may come out of a vector instruction right before it (a readfirstlane, the readlane of a spilled
+// scalar): a vector memory instruction may read such a scalar five wait states later at the earliest.  The move to
+// M0 and the four states of the s_nop are those five; the copy may use M0 one state after the move.
+SA_DEV void copy_rows_asm(const u32x4& rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory", "m0");
+}
+
 // Asynchronous copy of [ROWS][D] row-major global tiles into swizzled LDS tiles with
 // buffer_load_dwordx4 ... lds: the data never passes through registers.  One instruction moves
 // 1 KiB (64 lanes x 16 bytes) to consecutive LDS addresses, i.e. 1024/(2*D) whole rows; lane l
@@ -511,10 +522,7 @@ template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct A
         // both scalars are wave-uniform by construction; readfirstlane makes that known to the compiler
         const uint32_t lds_addr = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(SA_LDS void*)dst);
         const uint32_t so = (uint32_t)__builtin_amdgcn_readfirstlane((int)(soff + (uint32_t)i * istep));
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     :
-                     : "s"(lds_addr), "v"(voff[i % NVO]), "s"(rsrc), "s"(so)
-                     : "memory", "m0");
+        copy_rows_asm(rsrc, voff[i % NVO], so, lds_addr);
       } else {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (SA_LDS void*)dst, 16, (int)voff[i % NVO],
                                                  (int)(soff + (uint32_t)i * istep), 0, 0);
