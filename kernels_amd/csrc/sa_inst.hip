@@ -162,7 +162,7 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
     // windows of less than 1024 keys (the table's first two window classes) run the short-window form
     if (window_class(p.C, p.R) <= 1) {
       if constexpr (D <= 64) {
-        if (forward_in_two_waves(D, p.C, p.R, (int64_t)p.B * p.H * ceil_div(p.T, 128))) return fwd2_launch<D, 2, 32, true>(p, st);
+        if (forward_in_two_waves(D, p.C, p.R)) return fwd2_launch<D, 2, 32, true>(p, st);
       }
       return fwd2_launch<D, C::NARROW_NW, C::FWD_TK, true>(p, st);
     }

@@ -153,17 +153,19 @@ inline bool aligned_chunks(int chunk) { return 32 % chunk == 0 || chunk % 32 == 
 inline bool two_waves_read_no_more(int chunk, int back) {
   return aligned_chunks(chunk) && 2 * rows_in_reach(chunk, back, 64, 32) <= rows_in_reach(chunk, back, 128, 64);
 }
+// The windows alone decide, not the size of the grid: the two forms look for the maximum of a row in tiles of different
+// size, and a sequence has the same bits alone and in any batch.
 // The forward in us, four waves -> two.  D=32, B=225, H=4, T<=993: chunks of 16, 2 back 37.5 -> 29.5; 10, 9 back 48.7 -> 38.1; 64, 1 back
-// 36.8 -> 32.1; 64, 7 back 54.7 -> 52.9; on the other side 128, none back 34.4 -> 32.6 (64 x 8 x 1024: 26.6 -> 26.5), 128, 3 back
-// 53.0 -> 55.5, 10, 40 back 61 -> 55.  D=64, B=128, H=12, T=1354: 10, 9 back 248 -> 229; 50, 1 back 254 -> 228; 10, 20 back 313 -> 307; 16, 2
-// back 189 -> 182; 32, 1 back 188 -> 181; on the other side 32, 2 back 193 -> 197 (64 x 8 x 1024: 55.5 -> 58.0), 64, 2 back 65.9 ->
-// 74.6, 128, none back 53.8 -> 62.2, 10, 40 back 406 -> 424.  Up to 1024 workgroups of 128 rows more of them count for more (16 x 8 x 1024
-// ragged): 32, 2 back 14.1 -> 13.0; 128, none back 14.1 -> 12.2; 64, 2 back 16.1 -> 15.6; but 64, 1 back 14.6 -> 15.4.
-inline bool forward_in_two_waves(int D, int chunk, int back, int64_t workgroups_of_128) {
+// 36.8 -> 32.1; 64, 7 back 54.7 -> 52.9; 10, 40 back (410 keys) 61 -> 55; on the other side 128, none back 34.4 -> 32.6 (64 x 8 x
+// 1024: 26.6 -> 26.5), 128, 3 back 53.0 -> 55.5.  D=64, B=128, H=12, T=1354: 10, 9 back 248 -> 229; 50, 1 back 254 -> 228; 10, 20 back
+// 313 -> 307; 16, 2 back 189 -> 182; 32, 1 back 188 -> 181; on the other side 32, 2 back 193 -> 197 (64 x 8 x 1024: 55.5 -> 58.0),
+// 64, 2 back 65.9 -> 74.6, 128, none back 53.8 -> 62.2, 10, 40 back 406 -> 424.  On grids of up to 1024 workgroups of 128 rows the
+// other side differs less, either way (16 x 8 x 1024 ragged): 32, 2 back 14.1 -> 13.0; 128, none back 14.1 -> 12.2; 64, 2 back 16.1
+// -> 15.6; 64, 1 back 14.6 -> 15.4.
+inline bool forward_in_two_waves(int D, int chunk, int back) {
   const long long window = (long long)chunk * ((long long)back + 1);
   if (D == 32) return chunk < 128 && window <= 512;
-  if (D != 64 || window > 256) return false;
-  return workgroups_of_128 <= 1024 || !aligned_chunks(chunk) || two_waves_read_no_more(chunk, back);
+  return D == 64 && window <= 256 && (!aligned_chunks(chunk) || two_waves_read_no_more(chunk, back));
 }
 
 // The one-launch backward (sa_bwd_fused.h), 16-bit elements.

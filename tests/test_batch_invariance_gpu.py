@@ -1,0 +1,34 @@
+"""A sequence has the same bits alone and in a batch of any size: where the size of the grid picks the workgroups, their results
+do not differ.  16-bit elements: batches around 1024 workgroups of 128 rows."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def bits_alone_and_in_batches(dtype, H, T, D, C, R, batches):
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(31)
+    B = max(batches)
+    q, k, v, d_o = (torch.randn(B, H, T, D, generator=g, device=dev).to(dtype) for _ in range(4))
+    lens = torch.randint(T // 2, T + 1, (B,), generator=g, device=dev, dtype=torch.int32)
+    lens[:2] = torch.tensor([T, T // 3])
+
+    def step(n0, n1):
+        x = [t[n0:n1].clone().requires_grad_() for t in (q, k, v)]
+        o, lse = streaming_attention(*x, lens[n0:n1], C, R, return_lse=True)
+        return [o.detach(), lse.detach(), *torch.autograd.grad(o, x, d_o[n0:n1])]
+
+    alone = [torch.cat(pair) for pair in zip(step(0, 1), step(1, 2))]
+    for n in batches:
+        for name, one, many in zip(("O", "LSE", "dQ", "dK", "dV"), alone, step(0, n)):
+            assert torch.equal(one, many[:2]), (name, n, int((one != many[:2]).sum()))
+
+
+@pytest.mark.parametrize("C,R", [(32, 2), (64, 1), (64, 2), (128, 0), (128, 1), (16, 2), (10, 9), (50, 3), (200, 0)])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+def test_16_bit_short_windows(dtype, D, C, R):
+    bits_alone_and_in_batches(dtype, 8, 300, D, C, R, (2, 42, 43))   # 1008 and 1032 workgroups of 128 rows
