@@ -140,10 +140,13 @@ template <int D> struct OwnRows32 {
 };
 // Not where a row is a sixteenth of a kilobyte (D = 16: B=8, H=16, T=1000, chunks of 20, 4 back, forward and backward 88.1 us, 91.5
 // this way) nor in the workgroups of two waves, whose grids take as long as one workgroup's chain of latencies (see
-// half_workgroups; B=2, H=4, T=512, D=64 forward 15.0, 15.4 this way): there a lane loads its half row itself, stores its
-// row itself, and the tiles come in ascending order.
+// half_workgroups; B=2, H=4, T=512, D=64 forward 15.0, 15.4 this way): there a lane loads its half row itself and stores its
+// row itself.  The size of the grid picks the workgroups of a head dimension, so all of them add up in the same order and a
+// sequence has the same bits in any batch: row sums as dot_half_row, tiles in the order of the largest workgroup's
+// windows (tile_order_f32 in sa_inst.hip).
 constexpr bool direct_rows(int D, int NW) { return D == 16 || NW == 2; }
 // Row sums of the products of a wave's rows of O, read whole from memory, with those of dO in LDS (see RowDots).
+SA_DEV float dot4(const f32x4& a, const f32x4& b) { return __builtin_fmaf(a[0], b[0], a[1] * b[1]) + __builtin_fmaf(a[2], b[2], a[3] * b[3]); }
 template <int D> struct RowDots32 {
   using Rows = OwnRows32<D>;
   static constexpr int CPR = Rows::CPR, RPI = Rows::RPI, N = Rows::N, PITCH = CPR + 4;
@@ -160,14 +163,14 @@ template <int D> struct RowDots32 {
     for (int i = 0; i < N; ++i) {
       const int r = i * RPI + lane / CPR, ch = lane % CPR;
       const f32x4 gf = *reinterpret_cast<const f32x4*>(g_area + Rows::off(r, ch));
-      scratch[r * PITCH + ch] = __builtin_fmaf(of[i][0], gf[0], of[i][1] * gf[1]) + __builtin_fmaf(of[i][2], gf[2], of[i][3] * gf[3]);
+      scratch[r * PITCH + ch] = dot4(of[i], gf);
     }
   }
   SA_DEV static float total(const float* scratch, int lane) {
-    const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * (CPR / 2);
+    const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * 2;
     float sum = 0.0f;
 #pragma unroll
-    for (int j = 0; j < CPR / 2; ++j) sum += row[j];
+    for (int i = 0; i < CPR / 2; ++i) sum += row[(i / 2) * 4 + i % 2];   // the chunks of HalfRow
     return half_sum(sum);
   }
 };
@@ -215,6 +218,12 @@ template <int D> struct HalfRow {
     const int c = lane & 31, h = lane >> 5;
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) r[i] = *reinterpret_cast<const f32x4*>(area + OwnRows32<D>::off(c, (i / 2) * 4 + h * 2 + i % 2));
+  }
+  SA_DEV float dot_half_row(const HalfRow& other) const {   // RowDots32 adds up the same numbers in the same order
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) sum += dot4(r[i], other.r[i]);
+    return half_sum(sum);
   }
   SA_DEV void split(Split8 (&f)[D / 16], bool negative) const {
     const float mul = negative ? -kUp : kUp;
@@ -390,7 +399,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
   const float* qbase = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
   constexpr bool DIRECT = direct_rows(D, NW);
   if (!DIRECT) OwnRows32<D>::send(qbase, p.q_st, q0 + wave * 32, L - 1, q_area, lane);
-  const TileOrder order(kt0, kt1, DIRECT ? 0 : p.period, p.pdiv);
+  const TileOrder order(kt0, kt1, p.period, p.pdiv);
   SplitStager<D, TK, NT> sk, sv;
   sk.load(kbase, p.k_st, order.first * TK, L - 1, tid);
   sv.load(vbase, p.v_st, order.first * TK, L - 1, tid);
@@ -560,7 +569,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
     Rows::send(gbase, p.do_st, row0, L - 1, g_area, lane);
     dots.load(obase, o_st, row0, L - 1, lane);
   }
-  const TileOrder order(kt0, kt1, DIRECT ? 0 : p.period, p.pdiv);
+  const TileOrder order(kt0, kt1, p.period, p.pdiv);
   SplitStager<D, TK, NT> sk, sv;
   sk.load(kbase, p.k_st, order.first * TK, L - 1, tid);
   sv.load(vbase, p.v_st, order.first * TK, L - 1, tid);
@@ -578,11 +587,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(co
       o_row.load(obase + (int64_t)qr * o_st, h);
       q_row.split(qf, p.scale_log2e < 0.0f);
       g_row.split(gf, false);
-#pragma unroll
-      for (int i = 0; i < D / 8; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(o_row.r[i][e], g_row.r[i][e], sum);
-      sum = half_sum(sum);
+      sum = o_row.dot_half_row(g_row);
     } else {
       HalfRow<D> row;
       landed();
@@ -720,7 +725,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_ker
     if (tid < 2 * TQ) r_row = row_base[valid(t * TQ + tid % TQ)];
   };
   constexpr bool DIRECT = direct_rows(D, NW);
-  const TileOrder order(qt0, qt1, DIRECT ? 0 : p.period, p.pdiv);
+  const TileOrder order(qt0, qt1, p.period, p.pdiv);
   auto store_tile = [&](int it) {
     __bf16* st = reinterpret_cast<__bf16*>(smem_raw + (it & 1) * STAGE_BYTES);
     sq.store(st, tid);

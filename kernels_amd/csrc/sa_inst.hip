@@ -82,6 +82,13 @@ template <typename P> static bool half_workgroups(const P& p) {
   return 10 * (back + ceil_div(64, p.C) * p.C) <= 9 * (back + ceil_div(128, p.C) * p.C);
 }
 
+// TileOrder of the float32 kernels, with the period of the largest workgroup that a kernel has at this head dimension, whatever
+// the grid picks: no window holds two multiples of it, so the windows of a smaller workgroup start at the same tile or have none of
+// them, and every row goes through its tiles in the same order.  At head dimension 16 the order gained nothing.
+template <int D, typename P> static void tile_order_f32(P& p, int largest) {
+  if (D > 16) set_tile_order(p, largest, 32);
+}
+
 // SA_DGROUP 0 holds head dimensions 16..128, SA_DGROUP 1 holds 256 (built with different
 // compiler options, see the Makefile).
 #if SA_DGROUP == 0
@@ -148,7 +155,7 @@ template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipSt
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
-  set_tile_order(p, NW * 32, 32);
+  tile_order_f32<D>(p, D == 128 ? 256 : 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
@@ -256,7 +263,7 @@ template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st)
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, TQ, SHORT_LAST);
-  set_tile_order(p, TQ, 32);
+  tile_order_f32<D>(p, 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
@@ -359,7 +366,7 @@ template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, TKB, SHORT_LAST);
-  set_tile_order(p, TKB, 32);
+  tile_order_f32<D>(p, 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();

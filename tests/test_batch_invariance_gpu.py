@@ -1,5 +1,5 @@
 """A sequence has the same bits alone and in a batch of any size: where the size of the grid picks the workgroups, their results
-do not differ.  16-bit elements: batches around 1024 workgroups of 128 rows."""
+do not differ.  Batches on both sides of every such rule (up to 1024 and 128 workgroups of 128 rows, 256 of 256 rows)."""
 import pytest
 import torch
 
@@ -32,3 +32,15 @@ def bits_alone_and_in_batches(dtype, H, T, D, C, R, batches):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
 def test_16_bit_short_windows(dtype, D, C, R):
     bits_alone_and_in_batches(dtype, 8, 300, D, C, R, (2, 42, 43))   # 1008 and 1032 workgroups of 128 rows
+
+
+@pytest.mark.parametrize("C,R", [(64, 2), (50, 1), (10, 9), (32, 2), (128, 1), (24, 5)])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_float32(D, C, R):
+    """Two, four and eight waves to a workgroup go through the tiles of a row's window in one order and form its row sum in one order."""
+    bits_alone_and_in_batches(torch.float32, 8, 600, D, C, R, (2, 3, 4, 10, 11))   # 120 and 160 workgroups of 128 rows, 240 and 264 of 256
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_float32_long_windows(D):
+    bits_alone_and_in_batches(torch.float32, 8, 1500, D, 96, 4, (2, 4, 6))   # 192 workgroups of 128 rows, 288 of 256

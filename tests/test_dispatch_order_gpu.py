@@ -1,6 +1,6 @@
 """The order in which workgroups are dispatched (short windows first from 512 workgroups on, last below; pairs that do and do not
 divide over the eight XCDs) changes no bit of any result: a large grid against the same sequences one at a time.  16-bit elements;
-the float32 kernels take another shape on a small grid, and with it another order of sums."""
+float32, whose workgroups are of another size on a small grid, in test_batch_invariance_gpu.py."""
 import pytest
 import torch
 
