@@ -582,6 +582,13 @@ template <typename T, int D> struct OwnRows {
 SA_DEV void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // this wave's LDS reads are done; a barrier may follow after which others overwrite what it read
 SA_DEV void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// What lanes of this wave have written to LDS, other lanes of it may read now, and what they have read they may overwrite.  A wave's
+// LDS accesses are performed in order, so this is no instruction: it keeps the compiler from exchanging them.
+SA_DEV void wave_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // Row sums of the products of 32 rows of O, from memory in whole rows, with those of dO in the layout of OwnRows.
 template <typename T, int D> struct RowDots {
@@ -598,8 +605,9 @@ template <typename T, int D> struct RowDots {
       of[i] = *reinterpret_cast<const Frag*>(base + (int64_t)r * row_stride + lane % CPR * 8);
     }
   }
-  // partial sums into 32 * PITCH floats of LDS of this wave's own
+  // partial sums into 32 * PITCH floats of LDS of this wave's own, which may have held rows
   SA_DEV void partial(const T* g_area, float* scratch, int lane) const {
+    wave_exchange();
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int r = i * RPI + lane / CPR, ch = lane % CPR;
@@ -609,6 +617,7 @@ template <typename T, int D> struct RowDots {
   }
   // the sum of row lane % 32
   SA_DEV static float total(const float* scratch, int lane) {
+    wave_exchange();
     const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * (CPR / 2);
     float sum = 0.0f;
 #pragma unroll
@@ -813,12 +822,14 @@ SA_DEV void store_rows_coalesced(T* patch, T* out_rows, int rows_valid, const f3
   using P = RowPatch<T, D>;
   static_assert(Elem<T>::HALF && DB * 32 == D, "16-bit types, one accumulator block per 32 columns");
   const int c = lane & 31, h = lane >> 5;
+  wave_exchange();
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
     for (int g = 0; g < 4; ++g)
       store4<T>(patch + c * P::PITCH + m * 32 + 8 * g + 4 * h, acc[m][4 * g] * mul, acc[m][4 * g + 1] * mul,
                 acc[m][4 * g + 2] * mul, acc[m][4 * g + 3] * mul);
+  wave_exchange();
   const int rr = lane / P::CPR, ch = lane % P::CPR;
 #pragma unroll
   for (int j = 0; j < 32 / P::RPI; ++j) {

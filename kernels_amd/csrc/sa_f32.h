@@ -159,6 +159,7 @@ template <int D> struct RowDots32 {
     }
   }
   SA_DEV void partial(const float* g_area, float* scratch, int lane) const {
+    wave_exchange();
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int r = i * RPI + lane / CPR, ch = lane % CPR;
@@ -167,6 +168,7 @@ template <int D> struct RowDots32 {
     }
   }
   SA_DEV static float total(const float* scratch, int lane) {
+    wave_exchange();
     const float* row = scratch + (lane & 31) * PITCH + (lane >> 5) * 2;
     float sum = 0.0f;
 #pragma unroll
@@ -190,6 +192,7 @@ SA_DEV void store_rows_f32(float* patch, float* out_rows, int rows_valid, const 
   }
 #pragma unroll
   for (int col = 0; col < D; col += P::W) {
+    wave_exchange();
 #pragma unroll
     for (int m = col / 32; m < DB && m * 32 < col + P::W; ++m)
 #pragma unroll
@@ -198,6 +201,7 @@ SA_DEV void store_rows_f32(float* patch, float* out_rows, int rows_valid, const 
         store4<float>(patch + c * P::PITCH + d, acc[m][4 * g] * mul, acc[m][4 * g + 1] * mul, acc[m][4 * g + 2] * mul,
                       acc[m][4 * g + 3] * mul);
       }
+    wave_exchange();
 #pragma unroll
     for (int j = 0; j < 32 / P::RPI; ++j) {
       const int row = j * P::RPI + lane / P::CPR, ch = lane % P::CPR;
