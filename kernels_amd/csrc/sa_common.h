@@ -26,6 +26,7 @@
 namespace sa {
 
 #define SA_DEV __device__ __forceinline__
+#define SA_BOTH __host__ __device__ __forceinline__   // the maps of workgroups and tiles, which tests evaluate on the host
 #define SA_LDS __attribute__((address_space(3)))
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -705,7 +706,7 @@ struct TileMap {
   int tail_first;     // workgroups of those (of one XCD) if first, else 0
   ChunkDiv by_tiles, by_lead, by_pairs, by_heads;   // n_tiles, n_tiles - n_tail, nbh / 8, H
 };
-SA_DEV void tile_coords(int bid, int n_blocks, const TileMap& m, int& bh, int& tile) {
+SA_BOTH void tile_coords(int bid, int n_blocks, const TileMap& m, int& bh, int& tile) {
   int logical;
   const int x = bid & 7;
   int idx = bid >> 3;
@@ -733,8 +734,8 @@ SA_DEV void tile_coords(int bid, int n_blocks, const TileMap& m, int& bh, int& t
 // L (the queries that see those keys stop at L), so the order depends on L: tiles below them and the empty
 // tiles beyond L come first, then, tile by tile over the XCD's (batch, head) pairs, the n_end tiles that lead up to L.
 // Returns the clamped length of the pair's sequence as well.
-SA_DEV void key_tile_coords(int bid, int n_blocks, const TileMap& m, int ROWS, int T, const int32_t* lens, int64_t lens_stride,
-                            int& bh, int& tile, int& L) {
+SA_BOTH void key_tile_coords(int bid, int n_blocks, const TileMap& m, int ROWS, int T, const int32_t* lens, int64_t lens_stride,
+                             int& bh, int& tile, int& L) {
   const int ns = m.n_tail;
   if (ns == 0) {
     tile_coords(bid, n_blocks, m, bh, tile);
@@ -848,13 +849,13 @@ SA_DEV void store_rows_coalesced(T* patch, T* out_rows, int rows_valid, const f3
 // 733, 599, forward and backward 929 -> 898 us; B=8, H=16, T=4096, D=64: 229, 444, 360 -> 215, 354, 293, 418 -> 414.
 struct TileOrder {
   int t0, t1, first;
-  SA_DEV TileOrder(int t0_, int t1_, int period, ChunkDiv pdiv) : t0(t0_), t1(t1_), first(t0_) {
+  SA_BOTH TileOrder(int t0_, int t1_, int period, ChunkDiv pdiv) : t0(t0_), t1(t1_), first(t0_) {
     if (period > 1) {
       const int f = div_by(t0 + period - 1, pdiv) * period;
       first = f < t1 ? f : t0;
     }
   }
-  SA_DEV int next(int t) const { return t + 1 == t1 ? t0 : t + 1; }   // `first` again after the last one
+  SA_BOTH int next(int t) const { return t + 1 == t1 ? t0 : t + 1; }   // `first` again after the last one
 };
 
 struct FwdParams {
