@@ -417,7 +417,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 
 // ---------------------------------------------------------------------------------------
 // Variants for 16-bit elements with swizzled tiles (D = 32, 64, 128; dQ also 256): tiles arrive by
-// asynchronous global->LDS copies into a ring of NST stages, one barrier per tile.
+// asynchronous global->LDS copies into a ring of two stages, one barrier per tile.
 // ---------------------------------------------------------------------------------------
 
 // The window of one lane's row (a query's keys, or a key's queries), of all rows of its wave and of any of them.
@@ -506,7 +506,7 @@ SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T*
   }
 }
 
-template <typename T, int D, int NW, int TK, int NST>
+template <typename T, int D, int NW, int TK>
 __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
@@ -581,11 +581,11 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   // This wave's Q rows go where the second tile will be; its dO rows beside the stages or, where a third stage's worth
   // of LDS would cost a resident workgroup, where the first tile will be, which is then sent for once they have been read.
   using Rows = OwnRows<T, D>;
-  static_assert(NST == 2 && NW * 32 == 2 * TK, "two stages; the rows of a workgroup fill one");
+  static_assert(NW * 32 == 2 * TK, "the rows of a workgroup fill a stage");
   constexpr bool OVER = D >= 128;
   const int wrow0 = q0 + wave * 32;
   T* const q_area = smem + STAGE + wave * Rows::ELEMS;
-  T* const g_area = smem + (OVER ? 0 : NST * STAGE) + wave * Rows::ELEMS;
+  T* const g_area = smem + (OVER ? 0 : RING * STAGE) + wave * Rows::ELEMS;
   const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
   Rows::send(reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh, p.q_st, wrow0, L - 1, q_area, lane);
   Rows::send(gbase, p.do_st, wrow0, L - 1, g_area, lane);
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   }
 }
 
-template <typename T, int D, int NW, int TQ, int NST>
+template <typename T, int D, int NW, int TQ>
 // At head dimension 64 the kernel needs 174 registers, six more than three waves per SIMD may have; held to 168 it
 // reloads a few values per tile and runs 5 % faster with three workgroups per CU instead of two (measured at B=8,
 // H=16, T=4096).  At 128 the same step (290 -> 256 registers) spills inside the products and is 40 % slower.
@@ -745,9 +745,9 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   };
   // This wave's K rows go where the second tile will be, its V rows beside the stages.
   using Rows = OwnRows<T, D>;
-  static_assert(NST == 2 && NW * 32 == 2 * TQ, "two stages; the rows of a workgroup fill one");
+  static_assert(NW * 32 == 2 * TQ, "the rows of a workgroup fill a stage");
   T* const k_area = reinterpret_cast<T*>(smem_raw + STAGE_BYTES) + wave * Rows::ELEMS;
-  T* const v_area = reinterpret_cast<T*>(smem_raw + NST * STAGE_BYTES) + wave * Rows::ELEMS;
+  T* const v_area = reinterpret_cast<T*>(smem_raw + RING * STAGE_BYTES) + wave * Rows::ELEMS;
   const int wrow0 = k0 + wave * 32;
   Rows::send(reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh, p.k_st, wrow0, L - 1, k_area, lane);
   Rows::send(reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh, p.v_st, wrow0, L - 1, v_area, lane);

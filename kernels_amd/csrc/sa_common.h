@@ -553,6 +553,8 @@ template <bool ASM_COPIES = false> SA_DEV void async_copy_f32(const float* src, 
   }
 }
 
+constexpr int RING = 2;   // tile stages of fwd2_kernel, dq2_kernel and dkdv2_kernel: one read, one on its way
+
 // s_waitcnt vmcnt(N), other counters untouched (gfx9 encoding: vmcnt in bits 3:0 and 15:14).
 template <int N> SA_DEV void wait_loads() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");

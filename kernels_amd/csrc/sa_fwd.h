@@ -249,7 +249,7 @@ struct Fwd2Slots {
 // Same algorithm as fwd_kernel, different resource balance: each wave owns QB blocks of 32
 // queries, so every K / V fragment fetched from LDS feeds QB MFMAs (the transposing V reads
 // are 8-byte LDS reads and would otherwise cap the second product well below the MFMA
-// rate); K and V tiles are brought in by asynchronous global->LDS copies into a ring of NST
+// rate); K and V tiles are brought in by asynchronous global->LDS copies into a ring of two
 // stages, one tile ahead of the compute, with one barrier per key tile.
 // SHORT selects the form for short windows (a handful of key tiles per workgroup): work is skipped
 // and masks are decided per 32-key block instead of per tile, and a wave's first tile goes straight
@@ -263,7 +263,7 @@ struct Fwd2Slots {
 // to the exact result (float16 2.774e-4 -> 2.742e-4 there), as the second tile's maximum is taken too.
 // Half tiles at head dimension 64 (four waves per SIMD instead of three) are up to 6 % slower than whole ones; with each half's
 // own maximum they were up to 6 % faster on full grids, 15 % slower where half the workgroups were padding, and less exact.
-template <typename T, int D, int QB, int NW, int TK, int NST, bool SHORT>
+template <typename T, int D, int QB, int NW, int TK, bool SHORT>
 __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const FwdParams p) {
   using E = Elem<T>;
   using G = TileGeom<T, D>;
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   };
   // This wave's Q rows go where the second tile will be.
   using Rows = OwnRows<T, D>;
-  static_assert(NST == 2 && (HALVES || (QB == 1 && NW * 32 == 2 * TK)), "two stages; the rows of a workgroup fill one");
+  static_assert(HALVES || (QB == 1 && NW * 32 == 2 * TK), "the rows of a workgroup fill a stage");
   T* const q_area = smem + STAGE + wave * Rows::ELEMS;
   const T* qbase = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
   if constexpr (!HALVES) {

@@ -113,10 +113,10 @@ template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p,
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * C::FWD2_QB * 32;
   // tile stages; the epilogue's row patches (one per wave) reuse the same memory
-  constexpr size_t stages = (D == 256 ? (size_t)Fwd2Slots::ROWS : (size_t)C::FWD2_NST * 2 * TK) * D * sizeof(ElemT);
+  constexpr size_t stages = (D == 256 ? (size_t)Fwd2Slots::ROWS : (size_t)RING * 2 * TK) * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
-  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, TK, C::FWD2_NST, SHORT>;
+  auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, TK, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, TQ, !SHORT ? PLAIN : D == 256 ? SHORT_FIRST : SHORT_LAST);
@@ -220,10 +220,10 @@ template <int D, int NW> static int dq2_launch(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   constexpr int TQ = NW * 32;
   // beside the stages up to head dimension 64: a workgroup's dO rows
-  constexpr size_t stages = (size_t)(C::DQ2_NST + (D <= 64 ? 1 : 0)) * 2 * C::DQ2_TK * D * sizeof(ElemT);
+  constexpr size_t stages = (size_t)(RING + (D <= 64 ? 1 : 0)) * 2 * C::DQ2_TK * D * sizeof(ElemT);
   constexpr size_t patches = (size_t)NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
   constexpr size_t lds = stages > patches ? stages : patches;
-  auto kern = dq2_kernel<ElemT, D, NW, C::DQ2_TK, C::DQ2_NST>;
+  auto kern = dq2_kernel<ElemT, D, NW, C::DQ2_TK>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, TQ, D == 256 ? SHORT_FIRST : SHORT_LAST);
@@ -387,11 +387,11 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     }
     constexpr int TKB = C::DKDV2_NW * 32;
     constexpr size_t stages =
-        (size_t)C::DKDV2_NST * (2 * C::DKDV2_TQ * D * sizeof(ElemT) + 2 * C::DKDV2_TQ * sizeof(float)) +
+        (size_t)RING * (2 * C::DKDV2_TQ * D * sizeof(ElemT) + 2 * C::DKDV2_TQ * sizeof(float)) +
         (size_t)C::DKDV2_NW * OwnRows<ElemT, D>::ELEMS * sizeof(ElemT);   // a workgroup's V rows
     constexpr size_t patches = (size_t)C::DKDV2_NW * RowPatch<ElemT, D>::ELEMS * sizeof(ElemT);
     constexpr size_t lds = stages > patches ? stages : patches;
-    auto kern = dkdv2_kernel<ElemT, D, C::DKDV2_NW, C::DKDV2_TQ, C::DKDV2_NST>;
+    auto kern = dkdv2_kernel<ElemT, D, C::DKDV2_NW, C::DKDV2_TQ>;
     static PrepareState once;
     if (int rc = prepare(kern, lds, once)) return rc;
     const int64_t blocks = set_tiles(p, TKB, SHORT_LAST);

@@ -23,23 +23,14 @@ template <typename T> int launch_bwd_fused(const BwdParams& p, int D, hipStream_
 #ifndef SA_DQ2_TK
 #define SA_DQ2_TK 64
 #endif
-#ifndef SA_DQ2_NST
-#define SA_DQ2_NST 2
-#endif
 #ifndef SA_DKDV2_NW
 #define SA_DKDV2_NW 4
 #endif
 #ifndef SA_DKDV2_TQ
 #define SA_DKDV2_TQ 64
 #endif
-#ifndef SA_DKDV2_NST
-#define SA_DKDV2_NST 2
-#endif
 #ifndef SA_DKDV3_NST
 #define SA_DKDV3_NST 3
-#endif
-#ifndef SA_FWD2_NST
-#define SA_FWD2_NST 2
 #endif
 // ---- launch-configuration table -------------------------------------------------------------------
 // The 16-bit kernels for head dimensions 64 and 128 exist in several shapes (256 in one); which one runs is read
@@ -193,18 +184,17 @@ inline bool fused_backward_in_two_waves(int D, int chunk, int back) {
 
 template <typename T> struct Cfg {
   static constexpr int NW = 4;                                   // waves per workgroup
-  // 16-bit, D in {64, 128, 256}: forward kernel with QB query blocks per wave and NST LDS stages.
+  // 16-bit, D in {64, 128, 256}: forward kernel with QB query blocks per wave.
   // The compiler-scheduled forward and dQ kernels run 4 waves (128 queries) per workgroup, two workgroups
   // per CU (an 8-wave shape measured slower or equal in every cell of the tuning sweep and was removed).
   static constexpr int NARROW_NW = 4;
-  static constexpr int DQ2_TK = SA_DQ2_TK, DQ2_NST = SA_DQ2_NST;
-  static constexpr int DKDV2_NW = SA_DKDV2_NW, DKDV2_TQ = SA_DKDV2_TQ, DKDV2_NST = SA_DKDV2_NST;
+  static constexpr int DQ2_TK = SA_DQ2_TK;
+  static constexpr int DKDV2_NW = SA_DKDV2_NW, DKDV2_TQ = SA_DKDV2_TQ;
   // The software-pipelined dK/dV kernel exists at head dimension 128 only: at 64 a block step has
   // half the MFMAs for the same softmax arithmetic, the loop is bound by its vector work and dkdv2
   // is faster (0.23 against 0.30 ms at B=8, H=16, T=4096, chunk 128).
   static constexpr int DKDV3_NST = SA_DKDV3_NST;
   static constexpr int FWD2_QB = SA_FWD2_QB;
-  static constexpr int FWD2_NST = SA_FWD2_NST;
 #ifdef SA_FWD2_DISABLE
   static constexpr bool fwd2(int) { return false; }
 #else
