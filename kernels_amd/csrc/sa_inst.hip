@@ -119,7 +119,7 @@ template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p,
   auto kern = fwd2_kernel<ElemT, D, C::FWD2_QB, NW, TK, SHORT>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TQ, !SHORT ? PLAIN : D == 256 ? SHORT_FIRST : SHORT_LAST);
+  const int64_t blocks = set_tiles(p, TQ, SHORT ? SHORT_LAST : PLAIN);
   set_tile_order(p, TQ, TK);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -226,7 +226,7 @@ template <int D, int NW> static int dq2_launch(BwdParams p, hipStream_t st) {
   auto kern = dq2_kernel<ElemT, D, NW, C::DQ2_TK>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, TQ, D == 256 ? SHORT_FIRST : SHORT_LAST);
+  const int64_t blocks = set_tiles(p, TQ, D == 256 ? backward_tail_256(p.lens) : SHORT_LAST);
   set_tile_order(p, TQ, C::DQ2_TK);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -352,7 +352,7 @@ template <int D> static int dkdv_split_wide_launch(BwdParams p, hipStream_t st) 
   auto kern = dkdv_split_wide_kernel<ElemT, D>;
   static PrepareState once;
   if (int rc = prepare(kern, S::lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, S::TKB, SHORT_FIRST);
+  const int64_t blocks = set_tiles(p, S::TKB, backward_tail_256(p.lens));
   set_tile_order(p, S::TKB, S::TQ);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(2 * S::NP * 64), S::lds, st, p);

@@ -111,12 +111,18 @@ inline int tiles_of_window(int T, int chunk, int back, int rows, int tile) {
 // the pairs divide over the XCDs and they are no more than half.  SHORT_FIRST, for kernels with one workgroup per CU: equal
 // workgroups that start together stay in step, all CUs fetch their rows at the same time and the memory idles while all
 // multiply (a fifth of dQ at head dimension 256 went by at full memory rate); short workgroups at the beginning leave the CUs at
-// different points.  Only from 512 workgroups on: a last round of long workgroups on a few CUs costs more.  Forward and
-// backward in us, short last -> first: D=256, chunks of 128, 4 back, B*H=64, T=4096 884 -> 865, ragged 647 -> 628; 64, 3 back, B*H=32,
-// T=2000 143 -> 139; B*H=16, T=3000 (384 workgroups) 187 -> 185, ragged 137 -> 151.  dkdv_split_kernel, D=128, B*H=128, T=2048, 64, 1 back ragged
-// 164 -> 158, 50, 3 back, B*H=96, T=2000 215 -> 206.  Two or three workgroups per CU keep each other busy and lose: D=64, 128, 4 back
-// 422 -> 431.  The other kernels of head dimension 128 gain on some windows and lose as much on others.
+// different points.  Only from 512 workgroups on: with few rounds the long ones that come last show (256 at D=256: 73.4 -> 73.8).
+// Forward and backward in us, short last -> first, dkdv_split_kernel, D=128: 64, 1 back, T=2048, 1280 workgroups 140 -> 137, ragged 94 ->
+// 89; 50, 3 back, T=3000, 1536 workgroups 218 -> 208, ragged 178 -> 174; on large grids within 1 % (8192, ragged 710 -> 724 at the
+// worst).  Two or three workgroups per CU keep each other busy and lose: D=64, 128, 4 back 422 -> 431; the forward at D=256, whole
+// lengths -2 to +10 %, ragged up to +21 % (200, 2 back, 640 workgroups 52.4 -> 63.6).  The other kernels of head dimension 128 gain on
+// some windows and lose as much on others.
 enum Tail { PLAIN, SHORT_LAST, SHORT_FIRST };
+// The backward at D=256: first where every sequence has its whole length (64, 3 back, T=2048, 640 workgroups 202 -> 196, T=4096, 2048
+// workgroups 567 -> 550; 128, 4 back 886 -> 869; 200, 2 back, T=1000 223 -> 218).  Of ragged lengths a part of the workgroups is
+// empty, fewer rounds are left and the long ones that come last show: any lengths in [1, T], 200, 2 back, T=1000 162 -> 186, T=2048
+// 600 -> 659; 128, 4 back 133 -> 151, 531 -> 583; short chunks would gain (64, 3 back 200 -> 195, 714 -> 699) less than those lose.
+inline Tail backward_tail_256(const void* lens) { return lens ? SHORT_LAST : SHORT_FIRST; }
 template <typename P> int64_t set_tiles(P& p, int rows, Tail tail) {
   TileMap& m = p.tiles;
   m.n_tiles = (int)(((int64_t)p.T + rows - 1) / rows);

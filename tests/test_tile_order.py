@@ -103,6 +103,8 @@ int main() {
 DISPATCH = HEAD + r"""
 int main() {
   int grids = 0;
+  int32_t some_lengths = 1;   // head dimension 256: short windows first only where no sequence is shorter than T
+  CHECK(backward_tail_256(nullptr) == SHORT_FIRST && backward_tail_256(&some_lengths) == SHORT_LAST, "order at head dimension 256");
   for (int B : {1, 2, 3, 8, 17})
     for (int H : {1, 4, 8})
       for (int T : {1, 127, 128, 129, 1000, 2048, 5000})
