@@ -226,7 +226,14 @@ template <int D> struct HalfRow {
   SA_DEV float dot_half_row(const HalfRow& other) const {   // RowDots32 adds up the same numbers in the same order
     float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < D / 8; ++i) sum += dot4(r[i], other.r[i]);
+    for (int i = 0; i < D / 8; ++i) {
+      if constexpr (D == 16) {   // every workgroup reads its rows directly: one chain, as near as any order
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(r[i][e], other.r[i][e], sum);
+      } else {
+        sum += dot4(r[i], other.r[i]);
+      }
+    }
     return half_sum(sum);
   }
   SA_DEV void split(Split8 (&f)[D / 16], bool negative) const {
