@@ -12,7 +12,8 @@
 // make the loads of a workgroup 11 tensors' worth; 5.4 TB/s, a copy reaches 6.25); the two launches fetched 10.9 and wrote 3.1.
 //
 // B=128, H=12, T=3000, D=64, chunks of 32, 2 back (float16): 1370 us in two launches, 1083 here; the same without the products
-// 946; with results past the caches and the Q and dO rows of a wave through LDS 1031, 4.6 TB/s of the eight tensors.  B=8, H=16, T=4096, D=64, one chunk of 128: 160 -> 127 us.
+// 946; with results past the caches and the Q and dO rows of a wave through LDS 1031, 4.6 TB/s of the eight tensors.  When it came also B=8, H=16, T=4096, D=64, one
+// chunk of 128: 160 -> 127 us.
 // B=16, H=8, T=2048 ragged, D=64, chunks of 64, 1 back: 46 -> 39.  B=225, H=4, T=993 ragged, D=32, chunks of 16, 2 back: 94 -> 92.
 // Two waves and 32-row tiles instead of four and 64 where that reads no more rows per row of its own (and at D = 32 on
 // windows that lie across the 32-row blocks): fused_backward_in_two_waves in sa_launch.h has the rule and both sides' times.

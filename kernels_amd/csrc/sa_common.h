@@ -462,8 +462,9 @@ SA_DEV void copy_rows_asm(const u32x4& rsrc, uint32_t voff, uint32_t soff, uint3
 // maps there.  The NW waves of a workgroup interleave instruction by instruction.  Completion
 // is tracked by vmcnt; visibility to the other waves needs a barrier after the wait.
 //
-// Tiles are issued in ascending order.  Offsets are 32-bit byte offsets inside one (batch, head)
-// slice: the host checks that T * row_stride * sizeof(T) fits.
+// issue() and advance() go through ascending tiles (the hand-scheduled kernels, dkdv_split_kernel, the one-launch backward);
+// at() names any tile (TileOrder).  Offsets are 32-bit byte offsets inside one (batch, head)
+// slice: the host checks that (T + 1024) * row_stride * sizeof(T) fits.
 template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct AsyncTile {
   using G_ = TileGeom<T, D>;
   static_assert(G_::SWZ, "asynchronous tiles use the swizzled layout");
@@ -776,12 +777,13 @@ template <typename T> SA_DEV void store4(T* dst, float a, float b, float c, floa
 
 // Whole rows of a result are stored past the caches (the non-temporal hint): nothing of the launch reads them again, and
 // kept in the 4 MiB L2 of an XCD they push out the rows of Q, K, V and dO that neighbouring workgroups are about to read.
-// Forward and backward in us, plain -> non-temporal: B=16, H=8, T<=2048, D=128, chunks of 64, 1 back, strongly ragged (half
-// of the stores are zeros of padding) 137 -> 119; B=225, H=4, T<=993, D=32, chunks of 16, 2 back 129 -> 121; B=128, H=12,
-// T=3000, D=64, chunks of 32, 2 back 1535 -> 1495 (with O kept in the caches for the backward pass 1508); B=8, H=16, T=4096,
-// D=64, chunks of 128, 4 back 440 -> 430; B=4, H=16, D=128, T<=16384 3365 -> 3340.  Not for stores of part of a row: the float32
-// kernels' 16 bytes per lane with the hint 2040 -> 2170, and not for loads (rows of Q and O, a quarter per instruction: 251 -> 266,
-// 1495 -> 1548).
+// Forward and backward in us, plain -> non-temporal, on tensors that change from pass to pass (in brackets on the same ones, whose
+// cached part then grows by what the results leave free): B=16, H=8, T<=2048, D=128, chunks of 64, 1 back, strongly ragged (half of
+// the stores are zeros of padding) 129 -> 117 (115 -> 105); B=225, H=4, T<=993, D=32, chunks of 16, 2 back 118 -> 112 (107 -> 100);
+// B=128, H=12, T=3000, D=64, chunks of 32, 2 back 1476 -> 1439; B=8, H=16, T=4096, D=64, chunks of 128, 4 back 418 -> 409 (415 -> 396);
+// B=4, H=16, D=128, T<=16384 3294 -> 3267.  (O kept in the caches for the backward pass cost 13 of the gain of the third.)  Not for
+// stores of part of a row: the float32 kernels' 16 bytes per lane with the hint 2040 -> 2170, and not for loads (rows of Q and O, a
+// quarter per instruction: 251 -> 266, 1495 -> 1548).
 SA_DEV void store_streaming(void* dst, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst)); }
 
 // Zero rows [row0, row1) of a contiguous [*, D] matrix with the whole workgroup.

@@ -124,7 +124,7 @@ template <int D, int ROWS, int NT> struct SplitStager {
 
 // The 32 rows that a wave keeps, as copies of whole rows through 32 * D floats of LDS of its own (see OwnRows in sa_common.h,
 // whose swizzle of rows of as many bytes this is).  The addresses are formed per lane, in 64 bits: float32 tensors have no
-// limit on their row stride.  Rows past the last valid one mimic it.
+// limit on their row stride.  Rows past the last valid one have its values.
 template <int D> struct OwnRows32 {
   using G = TileGeom<__bf16, 2 * D>;
   static constexpr int ELEMS = 32 * D, CPR = D / 4, RPI = 64 / CPR, N = 32 / RPI;
@@ -138,6 +138,10 @@ template <int D> struct OwnRows32 {
     }
   }
 };
+// What own rows through LDS, whole-row stores past the caches and the tile order give each, us with the other two in place, without ->
+// with: forward and backward B=4, H=8, T<=2000, chunks of 50, 3 back, D=128 285, 281, 277 -> 275, D=64 151, 150, 148 -> 147, D=32 91, 90, 91 ->
+// 88; B=4, H=16, T=4096, chunks of 128, 4 back, D=128 1965, 1966, 1969 -> 1954 (spread 16); the stores lose on D=128, lengths in [1, 4096],
+// chunks of 32, 2 back 782 -> 795.  The copies' addresses cost registers: see the spills at the kernels.
 // Not where a row is a sixteenth of a kilobyte (D = 16: B=8, H=16, T=1000, chunks of 20, 4 back, forward and backward 88.1 us, 91.5
 // this way) nor in the workgroups of two waves, whose grids take as long as one workgroup's chain of latencies (see
 // half_workgroups; B=2, H=4, T=512, D=64 forward 15.0, 15.4 this way): there a lane loads its half row itself and stores its

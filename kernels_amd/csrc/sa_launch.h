@@ -168,9 +168,10 @@ inline bool forward_in_two_waves(int D, int chunk, int back) {
 // The one-launch backward (sa_bwd_fused.h), 16-bit elements.
 template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 32 || D == 64); }
 // Used while the query rows that a workgroup of 128 rows goes through for dK and dV are few: beyond its own 128 it reads and
-// multiplies rows that belong to its neighbours.  Measured against the two launches (B=8, H=16, T=4096, D=64 and batches of
-// the sizes in sa_bwd_fused.h), rows: gain -- 128: 1.27; 192: 1.27, 1.17; 256: 1.13; 320: 1.07, 1.01; 384: 0.94; 448: 0.91.
-// D=32 -- 192: 1.02, 1.05; 320: 0.98 (1.02 to 1.05 of the whole step at B=225, H=4, T<=993); 384: 0.91.
+// multiplies rows that belong to its neighbours.  Forward and backward against the two launches, rows: gain -- D=64, B=8, H=16,
+// T=4096 128: 1.12 to 1.24; 192: 1.06 to 1.17; 256: 1.01 to 1.05; 320: 0.95 to 0.99; B=64, H=12, T=1354 1.17 to 1.31; 1.11 to 1.27; 1.04
+// to 1.06; 1.00 to 1.02; the backward alone, when it came, 384: 0.94; 448: 0.91.  D=32, B=225, H=4, T=993 and B=16, H=16, T=4096 128:
+// 1.06 to 1.22; 192: 1.06 to 1.19; 256: 1.02 to 1.04; the backward alone, when it came, 320: 0.98; 384: 0.91.
 constexpr int BWD_FUSED_MAX_ROWS = 320;
 inline bool fused_backward(int D, int chunk, int back) {
   if (!fused_backward_exists<__bf16>(D)) return false;
