@@ -207,8 +207,10 @@ template <typename T> struct Cfg {
 #else
   static constexpr bool fwd2(int D) { return sizeof(T) == 2 && (D == 32 || D == 64 || D == 128 || D == 256); }
 #endif
-  // float32 on the 16-bit matrix pipe (sa_f32.h); at 256 the parts of the resident rows exceed the registers
+  // float32 on the 16-bit matrix pipe; at 256 the parts of the resident rows exceed the registers
   static constexpr bool split(int D) { return sizeof(T) == 4 && D <= 128; }
+  // which has kernels with two float16 parts per number (sa_f32h.h), and up to 64 with three bfloat16 parts (sa_f32.h)
+  static constexpr bool halves(int D) { return split(D) && D >= 32; }
 #ifdef SA_FWD_TK16
   static constexpr int FWD_TK = sizeof(T) == 4 ? 32 : SA_FWD_TK16;
 #else
