@@ -24,12 +24,8 @@
 
 namespace sa {
 
-// Magnitudes are compared as whole numbers (the bits of a float without its sign).
-SA_DEV uint32_t magnitude(float x) { return __float_as_uint(x) & 0x7FFFFFFFu; }
+// Magnitudes of several lanes are compared as whole numbers, the bits of a float without a sign.
 SA_DEV uint32_t larger(uint32_t a, uint32_t b) { return a > b ? a : b; }
-SA_DEV uint32_t larger4(uint32_t m, const f32x4& x) {
-  return larger(larger(larger(larger(m, magnitude(x[0])), magnitude(x[1])), magnitude(x[2])), magnitude(x[3]));
-}
 // The largest over groups of N neighbouring lanes (4, 8 or 16), left in all of them.
 template <int N> SA_DEV uint32_t lanes_max(uint32_t x) {
   auto step = [](uint32_t a, auto ctrl) {
@@ -50,6 +46,8 @@ SA_DEV float abs_max3(float m, float a, float b) {
   asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
   return r;
 }
+// m and the magnitudes of four elements, the largest that is a number: NaN keeps its place in the parts, whatever the factor
+SA_DEV float abs_max4(float m, const f32x4& x) { return abs_max3(abs_max3(m, x[0], x[1]), x[2], x[3]); }
 // Powers of two for a row whose largest magnitude is m: times `to` it is in [2^14, 2^15) (less below 2^-112), from = 1 / to.
 struct RowScale {
   float to = 0.0f, from = 0.0f;
@@ -119,7 +117,7 @@ template <int D, int NT> struct HalfStager {
   SA_DEV void step(int x, _Float16* tile, float* factors, int tid, float mul = 1.0f) {   // mul: of the factors
     const int it = x / 6, e = x % 6 - 1;
     if (e < 0) {
-      scale = RowScale(lanes_max<CPR>(larger4(larger4(0, regs[it][0]), regs[it][1])));
+      scale = RowScale(lanes_max<CPR>(__float_as_uint(abs_max4(abs_max4(0.0f, regs[it][0]), regs[it][1]))));
       most = fast_max(most, scale.from);
     } else if (e < 4) {
       halve_pair(parts, e, regs[it][e / 2][2 * (e % 2)], scale.to, regs[it][e / 2][2 * (e % 2) + 1], scale.to);
@@ -140,10 +138,10 @@ template <int D, int NT> struct HalfStager {
 
 // The parts of this lane's half of a row.
 template <int D> SA_DEV RowScale halve_row(Half8 (&f)[D / 16], const HalfRow<D>& row) {
-  uint32_t m = 0;
+  float m = 0.0f;
 #pragma unroll
-  for (int i = 0; i < D / 8; ++i) m = larger4(m, row.r[i]);
-  const RowScale sc(halves_max(m));
+  for (int i = 0; i < D / 8; ++i) m = abs_max4(m, row.r[i]);
+  const RowScale sc(halves_max(__float_as_uint(m)));
 #pragma unroll
   for (int g = 0; g < D / 16; ++g)
 #pragma unroll
@@ -160,6 +158,16 @@ SA_DEV void row_factors(float (&f)[16], const float* factors, int h) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) f[4 * g4 + e] = v[e];
   }
+}
+
+// Keeps fragments that every step multiplies in accumulation registers, where the matrix instruction reads them.  Left alone the
+// compiler copies those that it has put there back for every use: 127 copies among the 960 instructions of a dQ step at D=128, 430 of
+1500 in dK/dV.  Counted over the 4k case below, with the masks by bits alone and the factors by v_max3: vector instructions of dQ 108 -> 86
+million, of dK/dV 182 -> 124, cycles 269 -> 254 and 393 -> 334; the clock follows the power, so the times less (two kernels 1220 -> 1125
+us).  Not where two waves share the registers of a SIMD (forward in eight waves: 80 registers spilled instead of 29).
+template <int N> SA_DEV void keep_in_agprs(Half8 (&f)[N]) {
+#pragma unroll
+  for (int g = 0; g < N; ++g) asm("" : "+a"(f[g].p[0]), "+a"(f[g].p[1]));
 }
 
 // acc[row r][col c] += sum_k tile[r][k] * B[k][c] for the 32 rows of a tile; side(g) is vector work placed behind step g.
@@ -357,6 +365,7 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && NW == 4 ? 1 : 2)) void fwd_ha
   __syncthreads();
 
   for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    if constexpr (D == 128 && NW == 4) keep_in_agprs(qf);
     const _Float16* Kt = smem + (it & 1) * 2 * TILE;
     const _Float16* Vt = Kt + TILE;
     const float* kv = factors + (it & 1) * 2 * TK;
@@ -457,8 +466,10 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && NW == 4 ? 1 : 2)) void fwd_ha
 SA_DEV bool too_large(float factor) { return factor >= 0x1p45f; }
 
 // dQ, one wave per 32 queries, tiles of 32 keys, two stages, delta as in dq_split_kernel.  The next tile's parts are formed behind the
-// products of S and the exponentials behind those of dP.  Same problem as above, dQ and dK/dV together, us: D=128 1562 -> 1229 (traced
-// alone 713 -> 563; one wave per SIMD, whose vector work is what is left between products), D=64 812 -> 644, D=32 430 -> 386.
+// products of S and the exponentials behind those of dP.  Same problem as above, dQ and dK/dV together, us: D=128 1562 -> 1125 (traced
+// alone 713 -> 563; one wave per SIMD, whose vector work is what is left between products), D=64 812 -> 590, D=32 430 -> 350.
+// Tried at D=128: dS formed behind the products of the next tile and dQ added a step later, from three stages: 269 -> 277 million cycles;
+// the loads of the next tile right behind its predecessor's parts instead of at the end of a step: 254 -> 269.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_halves_kernel(const BwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<_Float16, D>::DB;
@@ -570,6 +581,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_halves_kernel(c
   __syncthreads();
 
   for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+    if constexpr (D == 128) {
+      keep_in_agprs(qf);
+      keep_in_agprs(gf);
+    }
     const _Float16* Kt = smem + (it & 1) * 2 * TILE;
     const _Float16* Vt = Kt + TILE;
     const float* kv = factors + (it & 1) * 2 * TK;
@@ -643,7 +658,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_halves_kernel(c
 }
 
 // dK and dV, one wave per 32 keys, tiles of 32 queries, two stages, the vector work behind the products as in dkdv_split_f32_kernel
-// (times above; D=128 traced alone 881 -> 807, 26 registers spilled).  Held to 256 registers for a second wave per SIMD D=64 spills and
+// (times above; D=128 traced alone 881 -> 775).  Every tile is masked: a mask that is all ones costs two instructions per element, one that is
+// left out of inner tiles by a branch three, as the compiler makes a select of it (D=128 1210 -> 1087 vector instructions, no spills at 32);
+// two bodies, with and without, cost 240 copies of registers each.  The next tile's elements held in LDS on their way, to free 32
+// registers: no difference.  Held to 256 registers for a second wave per SIMD D=64 spills and
 // is slower.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_halves_kernel(const BwdParams p) {
@@ -750,6 +768,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_halves_kernel
   __syncthreads();
 
   for (int t = order.first, it = 0; it < qt1 - qt0; ++it, t = order.next(t)) {
+    if constexpr (D >= 64) {
+      keep_in_agprs(kf);
+      keep_in_agprs(vf);
+    }
     const _Float16* Qt = reinterpret_cast<const _Float16*>(smem_raw + (it & 1) * STAGE_BYTES);
     const _Float16* Gt = Qt + TILE;
     const float* rows = reinterpret_cast<const float*>(Qt + 2 * TILE);
@@ -783,7 +805,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_halves_kernel
 #pragma unroll
           for (int e = i; e < i + 2; ++e) {
             s[e] = fast_exp2(__builtin_fmaf(s[e], of_row(Q_FACTOR, e) * ck, -of_row(LSE, e)));
-            if (!interior) s[e] = keep_or_zero(s[e], keep_bits(rm, e));
+            s[e] = keep_or_zero(s[e], keep_bits(rm, e));
           }
           v_unit.pair(pb, i, s[i], of_row(G_FACTOR, i), s[i + 1], of_row(G_FACTOR, i + 1), most);
         }
@@ -803,7 +825,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_halves_kernel
         for (int i = it * 8 / DB; i < (it + 1) * 8 / DB; ++i) {
           s[i] *= __builtin_fmaf(dp[i], of_row(G_FACTOR, i), -of_row(DELTA, i) * v_scale.to);
           // a masked dP may hold anything (NaN included): P = 0 does not clear it
-          if (!interior) s[i] = keep_or_zero(s[i], keep_bits(rm, i));
+          s[i] = keep_or_zero(s[i], keep_bits(rm, i));
         }
       });
       float fq[16];
