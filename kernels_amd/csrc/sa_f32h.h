@@ -162,9 +162,9 @@ SA_DEV void row_factors(float (&f)[16], const float* factors, int h) {
 
 // Keeps fragments that every step multiplies in accumulation registers, where the matrix instruction reads them.  Left alone the
 // compiler copies those that it has put there back for every use: 127 copies among the 960 instructions of a dQ step at D=128, 430 of
-1500 in dK/dV.  Counted over the 4k case below, with the masks by bits alone and the factors by v_max3: vector instructions of dQ 108 -> 86
-million, of dK/dV 182 -> 124, cycles 269 -> 254 and 393 -> 334; the clock follows the power, so the times less (two kernels 1220 -> 1125
-us).  Not where two waves share the registers of a SIMD (forward in eight waves: 80 registers spilled instead of 29).
+// 1500 in dK/dV.  Counted over the 4k case below, with the masks by bits alone and the factors by v_max3: vector instructions of dQ
+// 108 -> 86 million, of dK/dV 182 -> 124, cycles 269 -> 254 and 393 -> 334; the clock follows the power, so the times less (two kernels
+// 1220 -> 1125 us).  Not where two waves share the registers of a SIMD (forward in eight waves: 80 registers spilled instead of 29).
 template <int N> SA_DEV void keep_in_agprs(Half8 (&f)[N]) {
 #pragma unroll
   for (int g = 0; g < N; ++g) asm("" : "+a"(f[g].p[0]), "+a"(f[g].p[1]));
