@@ -397,11 +397,9 @@ def step_kernels(lib, dtype, D, C, R):
     if dtype == "float32":
         kind = "float32 instruction" if D == 256 else "16-bit parts"
         return dict.fromkeys(("fwd", "dq", "dkdv") if D <= 128 else ("fwd", "delta", "dq", "dkdv"), kind)
-    if D == 16:
-        return dict.fromkeys(("fwd", "delta", "dq", "dkdv"), "first generation")
     if D == 256:
         return {"fwd": "narrow", "dq": "narrow", "dkdv": "split"}
-    variants = {kn: "narrow" if kn != "dkdv" else "blockskip" for kn in ("fwd", "dq", "dkdv")} if D == 32 else \
+    variants = {kn: "narrow" if kn != "dkdv" else "blockskip" for kn in ("fwd", "dq", "dkdv")} if D <= 32 else \
         {kn: VARIANT_NAMES[kn][lib.sa_launch_choice(D, C, R, ki)] for ki, kn in enumerate(("fwd", "dq", "dkdv"))}
     return {"fwd": variants["fwd"], "bwd": "one launch"} if lib.sa_launch_choice(D, C, R, 3) == 1 else variants
 

@@ -175,11 +175,11 @@ int sa_query(int what);
  *   kernel = 1: dQ        variant 0 = 4 waves (128 queries), 1 = software-pipelined kernel (D = 128)
  *   kernel = 2: dK/dV     variant 0 = block-skipping kernel, 1 = software-pipelined kernel (D = 128),
  *                         2 = wave pairs (two waves per SIMD share 32 keys: one forms S and dV, the other dP and dK)
- *   kernel = 3: sa_backward (D in {32, 64})   0 = dQ and dK/dV as launches of their own, 1 = one launch for all three
+ *   kernel = 3: sa_backward (D in {16, 32, 64})   0 = dQ and dK/dV as launches of their own, 1 = one launch for all three
  *                         gradients, of neither of the variants above (short windows)
  * sa_launch_choice() returns the variant a call with these sizes runs (context_size and back_contexts at most T; longer
  * ones count as T).  At D = 256 every kernel exists in one shape, which is variant 0 (for dK/dV that is a wave-pair kernel).
- * -1 for a D outside {64, 128, 256} (kernels 0..2) or {32, 64} (3), another kernel id, context_size < 1 or
+ * -1 for a D outside {64, 128, 256} (kernels 0..2) or {16, 32, 64} (3), another kernel id, context_size < 1 or
  * back_contexts < 0.  Every variant computes the same function. */
 int sa_launch_choice(int D, int context_size, int back_contexts, int kernel);
 

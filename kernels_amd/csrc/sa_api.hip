@@ -34,7 +34,7 @@ int check_layout(const void* p, const int64_t* s, int dtype, int T, int D) {
     if (s[i] % vec != 0) return SA_ERR_LAYOUT;
   if (s[2] < 0 || (s[2] == 0 && T > 1)) return SA_ERR_LAYOUT;
   const bool offsets32 = dtype != SA_DTYPE_F32 && D >= 32;
-  if (offsets32 && ((int64_t)T + 1024) * s[2] * 2 >= (int64_t(1) << 32)) return SA_ERR_TOO_LARGE;
+  if (offsets32 && !offsets_fit(T, s[2])) return SA_ERR_TOO_LARGE;
   return SA_OK;
 }
 
@@ -180,10 +180,10 @@ int sa_bwd_dkdv(const void* q, const void* k, const void* v, const int32_t* lens
     return D == 256 ? launch_dkdv<E, 1>(p, D, (hipStream_t)stream) : launch_dkdv<E, 0>(p, D, (hipStream_t)stream); });
 }
 
-// Most dQ kernels hold each query's dO row and form delta = rowsum(O * dO) in their prologue; the separate pass
-// over O and dO is then launched only for 16-bit elements at head dimension 16 and float32 at 256.
-static bool delta_inside_dq(int D, int dtype) {
-  return dtype == SA_DTYPE_F32 ? Cfg<float>::split(D) : Cfg<__bf16>::fwd2(D);
+// Most dQ kernels hold each query's dO row and form delta = rowsum(O * dO) in their prologue; the separate pass over O and dO is
+// then launched only for float32 at head dimension 256 and, at 16, for 16-bit elements in slices beyond 32-bit offsets.
+static bool delta_inside_dq(const BwdParams& p, int D, int dtype) {
+  return dtype == SA_DTYPE_F32 ? Cfg<float>::split(D) : Cfg<__bf16>::fwd2(D) && slices_fit(p);
 }
 
 // The launches behind sa_backward and sa_backward_static: delta, dK/dV, dQ -- or dQ (forming delta), dK/dV -- or one for all.
@@ -193,6 +193,7 @@ static int backward_launches(const void* q, const void* k, const void* v, const 
                              const int64_t* gs, int B, int H, int T, int D, int context_size, int back_contexts,
                              float sm_scale, int dtype, void* stream) {
   if (int rc = check_common(B, H, T, D, dtype)) return rc;
+  bool delta_inside = false;
   if (B > 0 && H > 0 && T > 0) {
     // every output is checked before the first launch: nothing is enqueued for a call that is going to fail
     if (!dq || !dk || !dv || !delta) return SA_ERR_ARG;
@@ -202,7 +203,8 @@ static int backward_launches(const void* q, const void* k, const void* v, const 
     if (int rc = fill_bwd(p, q, k, v, lens, lens_stride, d_o, lse, delta, qs, ks, vs, gs, B, H, T, D, context_size,
                           back_contexts, sm_scale, dtype))
       return rc;
-    if (dtype != SA_DTYPE_F32 && fused_backward(D, p.C, p.R)) {
+    delta_inside = delta_inside_dq(p, D, dtype);
+    if (dtype != SA_DTYPE_F32 && slices_fit(p) && fused_backward(D, p.C, p.R)) {
       p.dq = dq; p.dk = dk; p.dv = dv;
       p.o = o; p.o_sb = os[0]; p.o_sh = os[1]; p.o_st = os[2];
       p.delta_out = delta;
@@ -210,7 +212,7 @@ static int backward_launches(const void* q, const void* k, const void* v, const 
                                    : launch_bwd_fused<__bf16>(p, D, (hipStream_t)stream);
     }
   }
-  if (delta_inside_dq(D, dtype) && B > 0 && H > 0 && T > 0) {
+  if (delta_inside) {
     if (int rc = run_dq(q, k, v, lens, lens_stride, d_o, lse, delta, dq, qs, ks, vs, gs, B, H, T, D, context_size,
                         back_contexts, sm_scale, dtype, stream, o, os))
       return rc;

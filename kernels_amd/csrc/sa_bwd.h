@@ -458,19 +458,31 @@ SA_DEV void dq2_tile(f32x16 (&acc)[DB], const T* Kt, const T* Vt, int k0, const 
   }
 }
 
+// A fragment of K as dkdv2_tile wants it: multiplied by -scale*log2(e) and rounded to the element type, so that the score accumulator
+// starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability.  At head dimension 16 the scores are
+// scaled in float32, which costs a multiplication per score of a kernel that is bound by memory and latency.
+constexpr bool scaled_scores(int D) { return D < 32; }
+template <typename T, int D> SA_DEV typename Elem<T>::Frag dkdv2_keys(typename Elem<T>::Frag k, float scale_log2e) {
+  if constexpr (!scaled_scores(D)) {
+    const float kmul = -scale_log2e;
+#pragma unroll
+    for (int e = 0; e < Elem<T>::VEC; ++e) k[e] = (T)((float)k[e] * kmul);
+  }
+  return k;
+}
 // dV^T += dO^T P and -dK^T += Q^T (-dS) for the TQ queries from qs on.  rows(r) gives the four lse and the four delta
-// values of the tile's rows r to r+3.  kf holds K * (-scale * log2 e), vf holds -V.
+// values of the tile's rows r to r+3.  kf holds K * (-scale * log2 e), or K where the scores are scaled instead, vf holds -V.
 template <typename T, int D, int TQ, int PG, int NF, int DB, typename Rows>
 SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T* Gt, int qs, const WaveWindow& win,
-                       const typename Elem<T>::Frag (&kf)[NF], const typename Elem<T>::Frag (&vf)[NF], Rows&& rows,
-                       int lane) {
+                       const typename Elem<T>::Frag (&kf)[NF], const typename Elem<T>::Frag (&vf)[NF], float scale_log2e,
+                       Rows&& rows, int lane) {
   const int h = lane >> 5;
 #pragma unroll
   for (int qb = 0; qb < TQ / 32; ++qb) {
     const int qb0 = qs + qb * 32;
     if (qb0 + 32 <= win.lo_min || qb0 >= win.hi_max) continue;
     const bool interior = (qb0 >= win.lo_max) && (qb0 + 32 <= win.hi_min);
-    f32x16 s[1], dp[1];
+    f32x16 s[1], dp[1], lse;   // lse: scaled scores
     // lse / delta of the 16 rows this lane holds, fetched ahead of the products and read
     // straight into the score and dP accumulators
 #pragma unroll
@@ -478,7 +490,10 @@ SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T*
       f32x4 l4, d4;
       rows(qb * 32 + 8 * g4 + 4 * h, l4, d4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[0][4 * g4 + e] = l4[e], dp[0][4 * g4 + e] = d4[e];
+      for (int e = 0; e < 4; ++e) {
+        s[0][4 * g4 + e] = scaled_scores(D) ? 0.0f : l4[e], dp[0][4 * g4 + e] = d4[e];
+        if constexpr (scaled_scores(D)) lse[4 * g4 + e] = l4[e];
+      }
     }
     // S[q][key] = Q K^T and dP[q][key] = dO V^T
     mma_rows_pair<T, D, NF, PG>(s[0], dp[0], Qt, Gt, qb * 32, kf, vf, lane);
@@ -487,7 +502,9 @@ SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T*
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * g4 + e;
-        const float pr = fast_exp2(-s[0][i]);
+        float pr;
+        if constexpr (scaled_scores(D)) pr = fast_exp2(__builtin_fmaf(s[0][i], scale_log2e, -lse[i]));
+        else pr = fast_exp2(-s[0][i]);
         s[0][i] = pr;
         dp[0][i] = pr * dp[0][i];   // = -dS
       }
@@ -515,7 +532,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB;
   constexpr int TILE = TK * D, STAGE = 2 * TILE;
-  using Loader = AsyncTile<T, D, TK, NW>;
+  using Loader = TilePair<T, D, TK, NW, false>;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
@@ -569,14 +586,11 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
 
   const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const T* vbase = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
-  Loader ldk, ldv;
-  ldk.init(kbase, p.k_st, kt0 * TK, L - 1, wave, lane);
-  ldv.init(vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
+  Loader tiles;
+  tiles.init(kbase, p.k_st, vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
   const TileOrder order(kt0, kt1, p.period, p.pdiv);
   auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
-    T* st = smem + (it & 1) * STAGE;
-    ldk.at(t - kt0).issue(st, wave);
-    ldv.at(t - kt0).issue(st + TILE, wave);
+    tiles.issue(smem + (it & 1) * STAGE, wave, t - kt0);
   };
   // This wave's Q rows go where the second tile will be; its dO rows beside the stages or, where a third stage's worth
   // of LDS would cost a resident workgroup, where the first tile will be, which is then sent for once they have been read.
@@ -678,7 +692,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   static_assert(TQ % NW == 0 && RPW % 4 == 0 && 2 * RPW <= 64, "lse/delta staging: one instruction per wave");
   // stage layout: [Q tile][dO tile][NW chunks of {lse[RPW], delta[RPW]}]
   constexpr int STAGE_BYTES = 2 * TILE * (int)sizeof(T) + 2 * TQ * (int)sizeof(float);
-  using Loader = AsyncTile<T, D, TQ, NW>;
+  using Loader = TilePair<T, D, TQ, NW, false>;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
 
@@ -719,16 +733,14 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   const int gk_last = k0 + TKB - 1 < L ? k0 + TKB - 1 : L - 1;
   const int qt0 = win_lo(k0) / TQ, qt1 = (win_hi(gk_last) + TQ - 1) / TQ;
 
-  const float kmul = -p.scale_log2e;
 
   const T* qbase = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)hd * p.q_sh;
   const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
   const float* lse_base = p.lse + (int64_t)bh * T_;
   const float* delta_base = p.delta + (int64_t)bh * T_;
   const TileOrder order(qt0, qt1, p.period, p.pdiv);
-  Loader ldq, ldg;
-  ldq.init(qbase, p.q_st, qt0 * TQ, L - 1, wave, lane);
-  ldg.init(gbase, p.do_st, qt0 * TQ, L - 1, wave, lane);
+  Loader tiles;
+  tiles.init(qbase, p.q_st, gbase, p.do_st, qt0 * TQ, L - 1, wave, lane);
   auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
     char* const stage = smem_raw + (it & 1) * STAGE_BYTES;
     T* st = reinterpret_cast<T*>(stage);
@@ -740,8 +752,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
       float* dst = reinterpret_cast<float*>(stage + 2 * TILE * sizeof(T)) + wave * 2 * RPW;
       async_copy_f32(src, dst);
     }
-    ldq.at(t - qt0).issue(st, wave);
-    ldg.at(t - qt0).issue(st + TILE, wave);
+    tiles.issue(st, wave, t - qt0);
   };
   // This wave's K rows go where the second tile will be, its V rows beside the stages.
   using Rows = OwnRows<T, D>;
@@ -757,11 +768,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
   landed();
 #pragma unroll
   for (int g = 0; g < NF; ++g) {
-    // K enters multiplied by -scale*log2(e), rounded to the element type: the score accumulator
-    // starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability
-    kf[g] = Rows::read(k_area, g, lane);
-#pragma unroll
-    for (int e = 0; e < E::VEC; ++e) kf[g][e] = (T)((float)kf[g][e] * kmul);
+    kf[g] = dkdv2_keys<T, D>(Rows::read(k_area, g, lane), p.scale_log2e);
     // V enters negated: the dP accumulator starts at delta and ends at delta - dP
     vf[g] = negate<T>(Rows::read(v_area, g, lane));
   }
@@ -785,7 +792,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
     const int qs = t * TQ;
     if (qs + TQ <= win.lo_min || qs >= win.hi_max) continue;   // outside this wave's windows
 
-    dkdv2_tile<T, D, TQ, PG>(dk, dv, Qt, Gt, qs, win, kf, vf, [&](int r, f32x4& l4, f32x4& d4) {
+    dkdv2_tile<T, D, TQ, PG>(dk, dv, Qt, Gt, qs, win, kf, vf, p.scale_log2e, [&](int r, f32x4& l4, f32x4& d4) {
       const float* chunk = ld_t + (r / RPW) * 2 * RPW + (r % RPW);
       l4 = *reinterpret_cast<const f32x4*>(chunk);
       d4 = *reinterpret_cast<const f32x4*>(chunk + RPW);

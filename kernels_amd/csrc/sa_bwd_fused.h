@@ -1,4 +1,4 @@
-// The whole backward pass in one launch, for windows of about a hundred keys (16-bit elements, head dimensions 32 and 64).
+// The whole backward pass in one launch, for windows of about a hundred keys (16-bit elements, head dimensions 16 to 64).
 //
 // On such windows the two backward kernels are bound by memory: dQ reads q, k, v, O, dO and writes dQ, dK/dV
 // reads q, k, v, dO again and writes two tensors -- twelve passes, of which eight are needed.  Here one
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   constexpr int ROWS = Shape::ROWS, NT = NW * 64;
   constexpr int NF = G::NF, DB = G::DB, TILE = TT * D, STAGE = 2 * TILE;
   constexpr int PG = D == 64 ? 2 : 4;   // see dkdv2_kernel
-  using Loader = AsyncTile<T, D, TT, NW, true>;
-  constexpr int NST = Shape::NST, LPT = 2 * Loader::PER_WAVE;
+  using Loader = TilePair<T, D, TT, NW, true>;
+  constexpr int NST = Shape::NST, LPT = Loader::PER_WAVE;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
@@ -100,15 +100,12 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   const T* obase = reinterpret_cast<const T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)hd * p.o_sh;
   const T* gbase = reinterpret_cast<const T*>(p.d_o) + (int64_t)b * p.do_sb + (int64_t)hd * p.do_sh;
 
-  Loader ld0, ld1;
+  Loader tiles;
   auto issue_tile = [&](int stage) {
-    ld0.issue(smem + stage * STAGE, wave);
-    ld1.issue(smem + stage * STAGE + TILE, wave);
-    ld0.advance();
-    ld1.advance();
+    tiles.issue(smem + stage * STAGE, wave);
+    tiles.advance();
   };
-  ld0.init(kbase, p.k_st, kt0 * TT, L - 1, wave, lane);
-  ld1.init(vbase, p.v_st, kt0 * TT, L - 1, wave, lane);
+  tiles.init(kbase, p.k_st, vbase, p.v_st, kt0 * TT, L - 1, wave, lane);
   // this wave's Q and dO rows go where the third and the second tile will be
   using Rows = OwnRows<T, D>;
   static_assert(NW * Rows::ELEMS == STAGE, "the rows of a workgroup fill a stage");
@@ -202,8 +199,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
       }
     }
     __syncthreads();   // no wave reads a stage any more: the first query tiles go to stages 0 and 1, the row patches over stage 2
-    ld0.init(qbase, p.q_st, qt0 * TT, L - 1, wave, lane);
-    ld1.init(gbase, p.do_st, qt0 * TT, L - 1, wave, lane);
+    tiles.init(qbase, p.q_st, gbase, p.do_st, qt0 * TT, L - 1, wave, lane);
     issue_tile(0);
     if (qt0 + 1 < qt1) issue_tile(1);
     if (row >= L) {
@@ -218,14 +214,10 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
   }
 
   // ---- dK, dV ---------------------------------------------------------------------------------------------
-  {
-    const float kmul = -p.scale_log2e;   // see dkdv2_kernel
 #pragma unroll
-    for (int g = 0; g < NF; ++g) {
-#pragma unroll
-      for (int e = 0; e < E::VEC; ++e) kf[g][e] = (T)((float)kf[g][e] * kmul);
-      vf[g] = negate<T>(vf[g]);
-    }
+  for (int g = 0; g < NF; ++g) {
+    kf[g] = dkdv2_keys<T, D>(kf[g], p.scale_log2e);
+    vf[g] = negate<T>(vf[g]);
   }
   f32x16 dk[DB], dv[DB];
 #pragma unroll
@@ -243,7 +235,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
     if (t * TT + TT <= wk.lo_min || t * TT >= wk.hi_max) continue;
     const float* l = lse_s + (t - qt0) * TT;
     const float* d = delta_s + (t - qt0) * TT;
-    dkdv2_tile<T, D, TT, PG>(dk, dv, Qt, Qt + TILE, t * TT, wk, kf, vf, [&](int r, f32x4& l4, f32x4& d4) {
+    dkdv2_tile<T, D, TT, PG>(dk, dv, Qt, Qt + TILE, t * TT, wk, kf, vf, p.scale_log2e, [&](int r, f32x4& l4, f32x4& d4) {
       l4 = *reinterpret_cast<const f32x4*>(l + r);
       d4 = *reinterpret_cast<const f32x4*>(d + r);
     }, lane);

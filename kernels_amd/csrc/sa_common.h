@@ -64,12 +64,12 @@ template <> struct Elem<float> {
 };
 
 // LDS tile geometry.  Two layouts:
-//  * swizzled (16-bit types, D >= 32): rows are stored unpadded and the 16-byte chunk index
+//  * swizzled (16-bit types): rows are stored unpadded and the 16-byte chunk index
 //    inside a row is XOR-ed with a permutation of the low row bits, chosen so that both access
 //    patterns of the kernels spread over all 64 banks: 16 lanes reading the same chunk of 16
 //    consecutive rows (row-major fragments), and 32 lanes reading a 4-row x 64-byte patch
 //    (transposing reads).
-//  * padded (everything else): the head dimension (at least one 32-wide block, so that
+//  * padded (float32, and the parts of float32 numbers at D = 16): the head dimension (at least one 32-wide block, so that
 //    transposed reads of a D=16 tile stay inside the row) plus one 16-byte pad.
 #ifndef SA_PAD_VECS
 #define SA_PAD_VECS 1
@@ -77,10 +77,10 @@ template <> struct Elem<float> {
 #ifndef SA_SWIZZLE
 #define SA_SWIZZLE 1
 #endif
-template <typename T, int D> struct TileGeom {
+template <typename T, int D, bool PADDED = false> struct TileGeom {
   static constexpr int VEC = Elem<T>::VEC;
   static constexpr int DP = D < 32 ? 32 : D;
-  static constexpr bool SWZ = SA_SWIZZLE && Elem<T>::HALF && D >= 32;
+  static constexpr bool SWZ = SA_SWIZZLE && Elem<T>::HALF && !PADDED;
   static constexpr int PITCH = SWZ ? D : DP + SA_PAD_VECS * VEC;
   static constexpr int NF = D / (2 * VEC);   // row fragments per lane
   static constexpr int DB = DP / 32;         // 32-wide blocks along D
@@ -91,7 +91,8 @@ template <typename T, int D> struct TileGeom {
     if constexpr (!SWZ) return 0;
     else if constexpr (CPR >= 16) return ((row & 3) << 2) | ((row >> 2) & 3);
     else if constexpr (CPR == 8) return ((row >> 2) & 1) | (((row >> 3) & 1) << 1) | (((row >> 1) & 1) << 2);
-    else return (row >> 2) & 3;   // CPR == 4: four rows fill the 64 banks, rows 4 apart must differ
+    else if constexpr (CPR == 4) return (row >> 2) & 3;   // four rows fill the 64 banks, rows 4 apart must differ
+    else return (row >> 3) & 1;                           // CPR == 2: eight rows fill them
   }
   // element offset of (row, element col) inside a tile
   SA_DEV static int off(int row, int col) {
@@ -248,7 +249,7 @@ SA_DEV void mma_tr(f32x16 (&acc)[NM], const T* X, int rb, const f32x16& P, int l
   if constexpr (E::HALF) {
     using Frag = typename E::Frag;
     const int g16 = lane >> 4, j = lane & 15;
-    const int h = g16 >> 1, mb = (g16 & 1) * 16;
+    const int h = g16 >> 1, mb = D < 32 ? 0 : (g16 & 1) * 16;   // D = 16: the rows from 16 on of the product repeat the first
     // This lane's source address for the transposing read: row (j/4) of a 4-row run, the
     // 4 columns starting at 4*(j%4); the instruction hands lane j column j of the 4x16
     // block, i.e. 4 consecutive rows of one column.  Two runs, 8 rows apart, make the
@@ -373,7 +374,7 @@ SA_DEV void mma_tr_pair(f32x16 (&acc0)[NM], f32x16 (&acc1)[NM], const T* X0, con
   constexpr int PITCH = G_::PITCH;
   const int g16 = lane >> 4, j = lane & 15;
   const int r_lo = 4 * (g16 >> 1) + (j >> 2);
-  const int col = (g16 & 1) * 16 + 4 * (j & 3);
+  const int col = (D < 32 ? 0 : (g16 & 1) * 16) + 4 * (j & 3);
   Frag b0[2], b1[2];
   pack_c<T>(b0, P0);
   pack_c<T>(b1, P1);
@@ -405,7 +406,7 @@ SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename E
   static_assert(E::HALF && NM == G_::DB, "transposing reads exist for 16-bit elements only");
   constexpr int PITCH = G_::PITCH;
   const int g16 = lane >> 4, j = lane & 15;
-  const int h = g16 >> 1, mb = (g16 & 1) * 16;
+  const int h = g16 >> 1, mb = D < 32 ? 0 : (g16 & 1) * 16;
   const int r_lo = 4 * h + (j >> 2);
   const int col = mb + 4 * (j & 3);
   const T* blk = X + rb * 32 * PITCH;
@@ -537,6 +538,43 @@ template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct A
     AsyncTile a = *this;
     a.soff += (uint32_t)tiles_ahead * tstep;
     return a;
+  }
+};
+
+// The copies of two tiles that a step reads together (K and V, or Q and dO), one behind the other in a stage.  Head dimension 16:
+// one instruction moves 32 rows, so a stage of 32 rows per pair of waves is one instruction per wave, half of the waves to a tile.
+// That, tiles without padding and the kernels of the wider heads instead of tiles staged through registers, float16, forward and with
+// backward in us: B=225, H=4, T<=993, chunks of 16, 2 back 67.4, 164.5 -> 21.1, 73.3; 64 x 8 x 1024, 40, 3 back 97.7, 225.9 -> 31.4, 112.9;
+// 64, 5 back 68.9, 218.4 -> 41.7, 145.5; one chunk, 8 x 8 x 1500 39.9, 143.7 -> 34.5, 121.1.  Bound by latency and the masks' vector work
+// (the first at 2.7 TB/s of its eight tensors).
+template <typename T, int D, int ROWS, int NW, bool ASM_COPIES> struct TilePair {
+  static constexpr bool ONE_EACH = D < 32;
+  static_assert(!ONE_EACH || 2 * ROWS == 32 * NW, "one instruction per wave");
+  using Copy = AsyncTile<T, D, ONE_EACH ? 32 : ROWS, ONE_EACH ? 1 : NW, ASM_COPIES>;
+  static constexpr int PER_WAVE = ONE_EACH ? 1 : 2 * Copy::PER_WAVE;
+  Copy a, b;   // ONE_EACH: a is this wave's
+
+  SA_DEV void init(const T* base_a, int64_t stride_a, const T* base_b, int64_t stride_b, int first_row, int last_row, int wave, int lane) {
+    if constexpr (ONE_EACH) {
+      const bool second = wave >= NW / 2;
+      a.init(second ? base_b : base_a, second ? stride_b : stride_a, first_row + wave % (NW / 2) * 32, last_row, 0, lane);
+      a.tstep *= ROWS / 32;
+    } else {
+      a.init(base_a, stride_a, first_row, last_row, wave, lane);
+      b.init(base_b, stride_b, first_row, last_row, wave, lane);
+    }
+  }
+  SA_DEV void issue(T* stage, int wave, int tiles_ahead = 0) const {
+    if constexpr (ONE_EACH) {
+      a.at(tiles_ahead).issue(stage + wave * 32 * D, 0);   // the second tile follows the first
+    } else {
+      a.at(tiles_ahead).issue(stage, wave);
+      b.at(tiles_ahead).issue(stage + ROWS * D, wave);
+    }
+  }
+  SA_DEV void advance() {
+    a.advance();
+    if constexpr (!ONE_EACH) b.advance();
   }
 };
 
@@ -825,13 +863,13 @@ template <typename T, int D, int DB>
 SA_DEV void store_rows_coalesced(T* patch, T* out_rows, int rows_valid, const f32x16 (&acc)[DB], float mul,
                                  int lane) {
   using P = RowPatch<T, D>;
-  static_assert(Elem<T>::HALF && DB * 32 == D, "16-bit types, one accumulator block per 32 columns");
+  static_assert(Elem<T>::HALF && DB == TileGeom<T, D>::DB, "16-bit types, one accumulator block per 32 columns");
   const int c = lane & 31, h = lane >> 5;
   wave_exchange();
 #pragma unroll
   for (int m = 0; m < DB; ++m)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < (D < 32 ? D / 8 : 4); ++g)
       store4<T>(patch + c * P::PITCH + m * 32 + 8 * g + 4 * h, acc[m][4 * g] * mul, acc[m][4 * g + 1] * mul,
                 acc[m][4 * g + 2] * mul, acc[m][4 * g + 3] * mul);
   wave_exchange();

@@ -81,7 +81,7 @@ SA_DEV void mma6(f32x16& acc, const Split8& a, const Split8& b) {
 
 // One LDS tile of ROWS rows: three bfloat16 tiles, one per part.
 template <int D, int ROWS> struct SplitTile {
-  using G = TileGeom<__bf16, D>;
+  using G = TileGeom<__bf16, D, D == 16>;
   static constexpr int PLANE = ROWS * G::PITCH;   // elements
   static constexpr int ELEMS = 3 * PLANE;
 };
@@ -89,7 +89,7 @@ template <int D, int ROWS> struct SplitTile {
 // Copy of a [ROWS][D] float32 tile through registers into a SplitTile, eight elements per thread and step.
 // Rows are clamped to last_row (the values are masked by the caller).
 template <int D, int ROWS, int NT> struct SplitStager {
-  using G = TileGeom<__bf16, D>;
+  using G = TileGeom<__bf16, D, D == 16>;
   static constexpr int CPR = D / 8, TOTAL = ROWS * CPR, N = (TOTAL + NT - 1) / NT;
   f32x4 regs[N][2];
 
@@ -260,7 +260,7 @@ struct NoSide {
 };
 template <int D, int ROWS, typename Side = NoSide>
 SA_DEV void mma_rows_split(f32x16& acc, const __bf16* tile, const Split8 (&b)[D / 16], int lane, Side&& side = Side()) {
-  using G = TileGeom<__bf16, D>;
+  using G = TileGeom<__bf16, D, D == 16>;
   const int c = lane & 31, h = lane >> 5;
   const __bf16* base = tile + c * G::PITCH;
   const int sw = G::swz(c);
@@ -280,7 +280,7 @@ SA_DEV void mma_rows_split(f32x16& acc, const __bf16* tile, const Split8 (&b)[D 
 template <int D, int ROWS, int NM, int NH, typename Side = NoSide>
 SA_DEV void mma_tr_split(f32x16 (&acc)[NM], const __bf16* X, const Split8 (&b)[NH], int lane, Side&& side = Side(),
                          int half0 = 0) {
-  using G = TileGeom<__bf16, D>;
+  using G = TileGeom<__bf16, D, D == 16>;
   static_assert(NM == G::DB, "one accumulator per 32-wide block of the head dimension");
   const int g16 = lane >> 4, j = lane & 15;
   const int r_lo = 4 * (g16 >> 1) + (j >> 2);
@@ -370,7 +370,7 @@ struct QueryWindow {
 // The register limits (four waves per SIMD up to 32, three at 64) make D=64 spill 19 registers per lane around the products.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
-  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
   constexpr float kRescaleGap = 8.0f;
   constexpr float kSumLimit = 256.0f;
@@ -530,7 +530,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_
 // delta here saves a pass over O and dO (40 us at D=128).
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void dq_split_kernel(const BwdParams p) {
-  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_split_kernel(const BwdParams p)
 // the same or slower.  Same problem as above: D=64 665 -> 476 us, D=32 351 -> 245, D=16 261 -> 194.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_kernel(const BwdParams p) {
-  constexpr int TKB = NW * 32, NT = NW * 64, TQ = 32, NF = D / 16, DB = TileGeom<__bf16, D>::DB;
+  constexpr int TKB = NW * 32, NT = NW * 64, TQ = 32, NF = D / 16, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TQ>::ELEMS;
   constexpr int STAGE_BYTES = 2 * TILE * 2 + 2 * TQ * 4;   // [Q][dO][lse, delta]
 

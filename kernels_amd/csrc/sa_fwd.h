@@ -279,7 +279,7 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   constexpr int STAGE = 2 * TILE;
   constexpr float kRescaleGap = 8.0f;
   constexpr float kSumLimit = 256.0f;
-  using Loader = AsyncTile<T, D, SB, NW, HALVES>;
+  using Loader = TilePair<T, D, SB, NW, HALVES>;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);  // [stage][K|V][TK][D], or the slots
@@ -339,14 +339,11 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
 
   const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)hd * p.k_sh;
   const T* vbase = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)hd * p.v_sh;
-  Loader ldk, ldv;
-  ldk.init(kbase, p.k_st, kt0 * TK, L - 1, wave, lane);
-  ldv.init(vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
+  Loader tiles;
+  tiles.init(kbase, p.k_st, vbase, p.v_st, kt0 * TK, L - 1, wave, lane);
   const TileOrder order(kt0, kt1, p.period, p.pdiv);
   auto issue_tile = [&](int t, int it) {   // tile t, the it-th that the workgroup goes through
-    T* st = smem + (it & 1) * STAGE;
-    ldk.at(t - kt0).issue(st, wave);
-    ldv.at(t - kt0).issue(st + TILE, wave);
+    tiles.issue(smem + (it & 1) * STAGE, wave, t - kt0);
   };
   // This wave's Q rows go where the second tile will be.
   using Rows = OwnRows<T, D>;
@@ -360,13 +357,13 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
   // Fwd2Slots: a block that no query of the workgroup sees is not sent for
   Fwd2Slots slots;
   auto seen = [&](int k0) { return k0 + SB > lo_wg && k0 < hi_wg; };
-  auto send = [&](const Loader& ld, int t, int block, int slot) { ld.at((t - kt0) * 2 + block).issue(smem + slot * SB * D, wave); };
+  auto send = [&](const typename Loader::Copy& ld, int t, int block, int slot) { ld.at((t - kt0) * 2 + block).issue(smem + slot * SB * D, wave); };
   auto send_first_blocks = [&](int t) {
-    if (seen(t * TK)) send(ldk, t, 0, Fwd2Slots::K0), send(ldv, t, 0, Fwd2Slots::V0);
+    if (seen(t * TK)) send(tiles.a, t, 0, Fwd2Slots::K0), send(tiles.b, t, 0, Fwd2Slots::V0);
   };
   if constexpr (HALVES) {
     send_first_blocks(order.first);
-    if (seen(order.first * TK + SB)) send(ldk, order.first, 1, slots.k1);
+    if (seen(order.first * TK + SB)) send(tiles.a, order.first, 1, slots.k1);
   }
 
   Frag qf[QB][NF];
@@ -423,12 +420,12 @@ __global__ __launch_bounds__(NW * 64, (D == 256 ? 2 : 1)) void fwd2_kernel(const
     for (int sb = 0; sb < TK; sb += SB) {
     if constexpr (HALVES) {
       const bool k1_next = more && seen(t_next * TK + SB);
-      if (sb != 0 && k1_next) wait_loads<Loader::PER_WAVE>();   // V1 was sent for before it
+      if (sb != 0 && k1_next) wait_loads<Loader::Copy::PER_WAVE>();   // V1 was sent for before it
       else wait_loads<0>();
       __syncthreads();
       if (sb == 0) {
-        if (seen(t * TK + SB)) send(ldv, t, 1, slots.v1);
-        if (k1_next) send(ldk, t_next, 1, slots.free());
+        if (seen(t * TK + SB)) send(tiles.b, t, 1, slots.v1);
+        if (k1_next) send(tiles.a, t_next, 1, slots.free());
       } else if (more) {
         send_first_blocks(t_next);
       }

@@ -186,9 +186,24 @@ template <int D, int NW> static int fwd_halves_launch(FwdParams p, hipStream_t s
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
+template <int D> static int fwd_first_launch(FwdParams p, hipStream_t st) {
+  using C = Cfg<ElemT>;
+  constexpr int TQ = C::NW * 32;
+  constexpr size_t lds = (size_t)2 * 2 * C::FWD_TK * TileGeom<ElemT, D>::PITCH * sizeof(ElemT);
+  auto kern = fwd_kernel<ElemT, D, C::NW, C::FWD_TK>;
+  static PrepareState once;
+  if (int rc = prepare(kern, lds, once)) return rc;
+  const int64_t blocks = set_tiles(p, TQ, PLAIN);
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D)) {
+    if constexpr (D == 16) {
+      if (!slices_fit(p)) return fwd_first_launch<D>(p, st);
+    }
     if constexpr (D == 128) {
       if (launch_choice(D, p.C, p.R).fwd == FWD_PIPELINED) return fwd3_launch<D>(p, st);
     }
@@ -220,15 +235,7 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
       return fwd_split_launch<D, 4>(p, st);
     }
   } else {
-    constexpr int TQ = C::NW * 32;
-    constexpr size_t lds = (size_t)2 * 2 * C::FWD_TK * TileGeom<ElemT, D>::PITCH * sizeof(ElemT);
-    auto kern = fwd_kernel<ElemT, D, C::NW, C::FWD_TK>;
-    static PrepareState once;
-    if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, PLAIN);
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
-    return (int)hipGetLastError();
+    return fwd_first_launch<D>(p, st);
   }
 }
 template <> int launch_fwd<ElemT, SA_DGROUP>(const FwdParams& p, int D, hipStream_t st) {
@@ -313,9 +320,25 @@ template <int D, int NW> static int dq_halves_launch(BwdParams p, hipStream_t st
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
+template <int D> static int dq_first_launch(BwdParams p, hipStream_t st) {
+  using C = Cfg<ElemT>;
+  if (p.delta_out) return SA_ERR_ARG;
+  constexpr int TQ = C::NW * 32;
+  constexpr size_t lds = (size_t)2 * 2 * C::DQ_TK * TileGeom<ElemT, D>::PITCH * sizeof(ElemT);
+  auto kern = dq_kernel<ElemT, D, C::NW, C::DQ_TK>;
+  static PrepareState once;
+  if (int rc = prepare(kern, lds, once)) return rc;
+  const int64_t blocks = set_tiles(p, TQ, PLAIN);
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
+  return (int)hipGetLastError();
+}
 template <int D> static int dq_d(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D)) {
+    if constexpr (D == 16) {
+      if (!slices_fit(p)) return dq_first_launch<D>(p, st);
+    }
     if constexpr (D == 128) {
       if (launch_choice(D, p.C, p.R).dq == DQ_PIPELINED) return dq3_launch<D>(p, st);
     }
@@ -334,16 +357,7 @@ template <int D> static int dq_d(BwdParams p, hipStream_t st) {
       return dq_split_launch<D, 4>(p, st);
     }
   } else {
-    if (p.delta_out) return SA_ERR_ARG;
-    constexpr int TQ = C::NW * 32;
-    constexpr size_t lds = (size_t)2 * 2 * C::DQ_TK * TileGeom<ElemT, D>::PITCH * sizeof(ElemT);
-    auto kern = dq_kernel<ElemT, D, C::NW, C::DQ_TK>;
-    static PrepareState once;
-    if (int rc = prepare(kern, lds, once)) return rc;
-    const int64_t blocks = set_tiles(p, TQ, PLAIN);
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
-    return (int)hipGetLastError();
+    return dq_first_launch<D>(p, st);
   }
 }
 template <> int launch_dq<ElemT, SA_DGROUP>(const BwdParams& p, int D, hipStream_t st) {
@@ -436,11 +450,40 @@ template <int D, int NW> static int dkdv_halves_launch(BwdParams p, hipStream_t 
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
+template <int D> static int dkdv_first_launch(BwdParams p, hipStream_t st) {
+  using C = Cfg<ElemT>;
+  constexpr int TKB = C::NW * 32;
+  constexpr size_t lds =
+      (size_t)2 * (2 * C::DKDV_TQ * TileGeom<ElemT, D>::PITCH * sizeof(ElemT) + 2 * C::DKDV_TQ * sizeof(float));
+  const int64_t blocks = set_tiles(p, TKB, PLAIN);
+  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
+  if constexpr (sizeof(ElemT) == 4 && D == 256) {
+    // both accumulators and both resident rows do not fit a lane's registers: one launch per gradient
+    auto kern_dv = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ, 1>;
+    auto kern_dk = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ, 2>;
+    static PrepareState once_dv, once_dk;
+    if (int rc = prepare(kern_dv, lds, once_dv)) return rc;
+    if (int rc = prepare(kern_dk, lds, once_dk)) return rc;
+    hipLaunchKernelGGL(kern_dv, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(kern_dk, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
+    return (int)hipGetLastError();
+  } else {
+    auto kern = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ>;
+    static PrepareState once;
+    if (int rc = prepare(kern, lds, once)) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
+    return (int)hipGetLastError();
+  }
+}
 template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if constexpr (C::fwd2(D) && D == 256) {
     return dkdv_split_wide_launch<D>(p, st);
   } else if constexpr (C::fwd2(D)) {
+    if constexpr (D == 16) {
+      if (!slices_fit(p)) return dkdv_first_launch<D>(p, st);
+    }
     if constexpr (D >= 64) {   // a 64-byte row splits over four waves' copies, not over eight
       if (launch_choice(D, p.C, p.R).dkdv == DKDV_SPLIT) return dkdv_split_launch<D>(p, st);
     }
@@ -478,29 +521,7 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
       return dkdv_split_f32_launch<D, 4>(p, st);
     }
   } else {
-    constexpr int TKB = C::NW * 32;
-    constexpr size_t lds =
-        (size_t)2 * (2 * C::DKDV_TQ * TileGeom<ElemT, D>::PITCH * sizeof(ElemT) + 2 * C::DKDV_TQ * sizeof(float));
-    const int64_t blocks = set_tiles(p, TKB, PLAIN);
-    if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-    if constexpr (sizeof(ElemT) == 4 && D == 256) {
-      // both accumulators and both resident rows do not fit a lane's registers: one launch per gradient
-      auto kern_dv = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ, 1>;
-      auto kern_dk = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ, 2>;
-      static PrepareState once_dv, once_dk;
-      if (int rc = prepare(kern_dv, lds, once_dv)) return rc;
-      if (int rc = prepare(kern_dk, lds, once_dk)) return rc;
-      hipLaunchKernelGGL(kern_dv, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
-      if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
-      hipLaunchKernelGGL(kern_dk, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
-      return (int)hipGetLastError();
-    } else {
-      auto kern = dkdv_kernel<ElemT, D, C::NW, C::DKDV_TQ>;
-      static PrepareState once;
-      if (int rc = prepare(kern, lds, once)) return rc;
-      hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NW * 64), lds, st, p);
-      return (int)hipGetLastError();
-    }
+    return dkdv_first_launch<D>(p, st);
   }
 }
 template <> int launch_dkdv<ElemT, SA_DGROUP>(const BwdParams& p, int D, hipStream_t st) {

@@ -159,19 +159,31 @@ inline bool two_waves_read_no_more(int chunk, int back) {
 // 64, 2 back 65.9 -> 74.6, 128, none back 53.8 -> 62.2, 10, 40 back 406 -> 424.  On grids of up to 1024 workgroups of 128 rows the
 // other side differs less, either way (16 x 8 x 1024 ragged): 32, 2 back 14.1 -> 13.0; 128, none back 14.1 -> 12.2; 64, 2 back 16.1
 // -> 15.6; 64, 1 back 14.6 -> 15.4.
+// D=16, B=225, H=4, T<=993; 64 x 8 x 1024: 16, 2 back 29.4 -> 21.4; 24.4 -> 18.7; 10, 9 back 40.7 -> 30.0; 35.5 -> 28.5; 64, 1 back 27.3 ->
+// 23.1; 23.2 -> 20.2; 64, 7 back 45.7 -> 44.0; 44.9 -> 44.3; on the other side 128, none back 26.8 -> 24.0; 19.5 -> 20.3; 128, 3 back
+// 43.1 -> 45.0; 42.7 -> 45.6.
 inline bool forward_in_two_waves(int D, int chunk, int back) {
   const long long window = (long long)chunk * ((long long)back + 1);
-  if (D == 32) return chunk < 128 && window <= 512;
+  if (D <= 32) return chunk < 128 && window <= 512;
   return D == 64 && window <= 256 && (!aligned_chunks(chunk) || two_waves_read_no_more(chunk, back));
 }
 
+// The kernels with copies into LDS address the rows of a (batch, head) slice with 32-bit byte offsets.  At head dimension 16
+// slices that are longer go to the first kernels (sa_fwd.h, sa_bwd.h), which have no such limit.
+inline bool offsets_fit(int T, int64_t row_stride) { return ((int64_t)T + 1024) * row_stride * 2 < (int64_t(1) << 32); }
+inline bool slices_fit(const FwdParams& p) { return offsets_fit(p.T, p.q_st) && offsets_fit(p.T, p.k_st) && offsets_fit(p.T, p.v_st); }
+inline bool slices_fit(const BwdParams& p) {
+  return offsets_fit(p.T, p.q_st) && offsets_fit(p.T, p.k_st) && offsets_fit(p.T, p.v_st) && offsets_fit(p.T, p.do_st);
+}
+
 // The one-launch backward (sa_bwd_fused.h), 16-bit elements.
-template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 32 || D == 64); }
+template <typename T> constexpr bool fused_backward_exists(int D) { return sizeof(T) == 2 && (D == 16 || D == 32 || D == 64); }
 // Used while the query rows that a workgroup of 128 rows goes through for dK and dV are few: beyond its own 128 it reads and
 // multiplies rows that belong to its neighbours.  Forward and backward against the two launches, rows: gain -- D=64, B=8, H=16,
 // T=4096 128: 1.12 to 1.24; 192: 1.06 to 1.17; 256: 1.01 to 1.05; 320: 0.95 to 0.99; B=64, H=12, T=1354 1.17 to 1.31; 1.11 to 1.27; 1.04
 // to 1.06; 1.00 to 1.02; the backward alone, when it came, 384: 0.94; 448: 0.91.  D=32, B=225, H=4, T=993 and B=16, H=16, T=4096 128:
-// 1.06 to 1.22; 192: 1.06 to 1.19; 256: 1.02 to 1.04; the backward alone, when it came, 320: 0.98; 384: 0.91.
+// 1.06 to 1.22; 192: 1.06 to 1.19; 256: 1.02 to 1.04; the backward alone, when it came, 320: 0.98; 384: 0.91.  D=16, the same problems,
+// forward and backward: 192 80.0 against 88.3 us, 256 95.9 against 99.5 and 88 against 90.
 constexpr int BWD_FUSED_MAX_ROWS = 320;
 inline bool fused_backward(int D, int chunk, int back) {
   if (!fused_backward_exists<__bf16>(D)) return false;
@@ -185,7 +197,11 @@ inline bool fused_backward(int D, int chunk, int back) {
 // 10, 9 back 157.5 -> 151.7; on the other side 32, 3 back 130.1 -> 128.1 (64 x 8 x 1024: 104.9 -> 111.0), 64, 1 back 124.7 -> 122.2 (98.8 ->
 // 102.4), 128, none back 116.5 -> 122.4.  D=64, B=64, H=12, T=1354: 8, 3 back 339 -> 324; 16, 2 back 335 -> 323; 64, none back 306 -> 293; on the
 // other side 10, 9 back 463 -> 465, 32, 2 back 348 -> 347 (64 x 8 x 1024: 182 -> 189), 32, 3 back 390 -> 396, 128, none back 344 -> 365.
+// D=16 reads little and takes the small workgroups for all chunks below 128: B=225, H=4, T<=993; 64 x 8 x 1024, backward alone: 16, 2 back
+// 64.4 -> 53.5; 52.4 -> 46.3; 32, 3 back 66.8 -> 59.0; 56.2 -> 53.0; 64, 1 back 64.0 -> 55.4; 52.5 -> 49.0; 64, 2 back 71.2 -> 63.2; 61.0 ->
+// 61.1; on the other side 128, none back 60.4 -> 59.0; 44.3 -> 48.2.
 inline bool fused_backward_in_two_waves(int D, int chunk, int back) {
+  if (D == 16) return chunk < 128;
   return (D == 32 && !aligned_chunks(chunk)) || two_waves_read_no_more(chunk, back);
 }
 
@@ -205,7 +221,7 @@ template <typename T> struct Cfg {
 #ifdef SA_FWD2_DISABLE
   static constexpr bool fwd2(int) { return false; }
 #else
-  static constexpr bool fwd2(int D) { return sizeof(T) == 2 && (D == 32 || D == 64 || D == 128 || D == 256); }
+  static constexpr bool fwd2(int D) { return sizeof(T) == 2 && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256); }
 #endif
   // float32 on the 16-bit matrix pipe; at 256 the parts of the resident rows exceed the registers
   static constexpr bool split(int D) { return sizeof(T) == 4 && D <= 128; }
