@@ -806,6 +806,56 @@ SA_BOTH void key_tile_coords(int bid, int n_blocks, const TileMap& m, int ROWS, 
   }
 }
 
+// Inclusive sum over the lanes before a lane and itself.
+SA_DEV int lanes_scan(int x) {
+#define SA_SCAN_STEP(ctrl, rows) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false)
+  SA_SCAN_STEP(0x111, 0xf);   // from one, two, four and eight lanes back in a row of sixteen
+  SA_SCAN_STEP(0x112, 0xf);
+  SA_SCAN_STEP(0x114, 0xf);
+  SA_SCAN_STEP(0x118, 0xf);
+  SA_SCAN_STEP(0x142, 0xa);   // the first row's sum to the second, the third's to the fourth
+  SA_SCAN_STEP(0x143, 0xc);   // the first half's to the second
+#undef SA_SCAN_STEP
+  return x;
+}
+// tile_coords for windows that reach over the whole sequence, where a workgroup goes through all keys of its sequence: the longest
+// sequences first, tiles without a row below their sequence's length last.  So the last workgroups to start, which run while part
+// of the chip is idle, are the short ones.  An XCD has every eighth pair of (batch entry, head) in the order of the lengths, there
+// and back, so that none has the longer sequence of every two.  Every wave works that out by itself: the lengths, one to a lane, are
+// ranked (n batch entries, the earlier one first where they are equal), lane k takes the XCD's k-th pair, and the sums
+// of the tiles of the pairs before it say where its workgroups begin.
+template <int ROWS>
+SA_DEV void tile_coords_by_length(int bid, const TileMap& m, int n, const int32_t* lens, int64_t lens_stride, int T, int H, int lane,
+                                  int& bh, int& tile, int& L) {
+  const int x = bid & 7, nb = m.nbh >> 3;
+  int idx = bid >> 3, mine = -1;
+  if (lane < n) {
+    mine = lens[(int64_t)lane * lens_stride];
+    mine = mine < 0 ? 0 : (mine > T ? T : mine);
+  }
+  int rank = lane < n ? 0 : lane;
+  for (int j = 0; j < n; ++j) {
+    const int other = __builtin_amdgcn_readlane(mine, j);
+    rank += other > mine || (other == mine && j < lane && lane < n) ? (lane < n ? 1 : 0) : 0;
+  }
+  const int sorted = __builtin_amdgcn_ds_permute(rank * 4, mine);
+  const int pair = lane * 8 + (lane & 1 ? 7 - x : x), place = div_by(pair, m.by_heads);   // of lane's pair, in the order of the lengths
+  const int len = __builtin_amdgcn_ds_bpermute((lane < nb ? place : 0) * 4, sorted);
+  const int live = lane < nb ? (len + ROWS - 1) / ROWS : 0, dead = lane < nb ? m.n_tiles - live : 0;
+  const int live_sum = lanes_scan(live), dead_sum = (lane < nb ? (lane + 1) * m.n_tiles : nb * m.n_tiles) - live_sum;
+  const int all_live = __builtin_amdgcn_readlane(live_sum, 63);
+  const bool is_dead = idx >= all_live;
+  idx -= is_dead ? all_live : 0;
+  const int k = __builtin_popcountll(__builtin_amdgcn_ballot_w64((is_dead ? dead_sum : live_sum) <= idx));   // pairs that end before idx
+  const int before = is_dead ? __builtin_amdgcn_readlane(dead_sum, k) - __builtin_amdgcn_readlane(dead, k)
+                             : __builtin_amdgcn_readlane(live_sum, k) - __builtin_amdgcn_readlane(live, k);
+  const int its_live = __builtin_amdgcn_readlane(live, k), its_place = __builtin_amdgcn_readlane(place, k);
+  tile = is_dead ? its_live + (idx - before) : its_live - 1 - (idx - before);
+  const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n && rank == its_place));
+  bh = __builtin_amdgcn_readlane(pair, k) + (b - its_place) * H;
+  L = __builtin_amdgcn_readlane(len, k);
+}
+
 // Write four consecutive fp32 values as four elements of T.
 template <typename T> SA_DEV void store4(T* dst, float a, float b, float c, float d) {
   typename Elem<T>::Quad q;
@@ -913,6 +963,7 @@ struct FwdParams {
   ChunkDiv cdiv;      // division by C
   int period;         // TileOrder; 0: ascending
   ChunkDiv pdiv;      // division by period
+  int by_length;      // batch entries to put in the order of their lengths (tile_coords_by_length), or 0
 };
 
 struct BwdParams {

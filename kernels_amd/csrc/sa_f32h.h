@@ -294,12 +294,12 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && NW == 4 ? 1 : 2)) void fwd_ha
   const int lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bh, qt;
-  tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
-  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
+  int bh, qt, L = p.T;
+  if (p.by_length) tile_coords_by_length<TQ>(blockIdx.x, p.tiles, p.by_length, p.lens, p.lens_stride, p.T, p.H, lane, bh, qt, L);
+  else tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
   const int T_ = p.T;
-  int L = T_;
-  if (p.lens) {
+  const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
+  if (p.lens && !p.by_length) {
     L = p.lens[(int64_t)b * p.lens_stride];
     L = L < 0 ? 0 : (L > T_ ? T_ : L);
   }

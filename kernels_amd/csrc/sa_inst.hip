@@ -134,6 +134,7 @@ template <int D, int NW, int TK, bool SHORT> static int fwd2_launch(FwdParams p,
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, TQ, SHORT ? SHORT_LAST : PLAIN);
+  if (TK != 32) set_length_order(p, 768);
   set_tile_order(p, TQ, TK);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -169,6 +170,7 @@ template <int D, int NW> static int fwd_split_launch(FwdParams p, hipStream_t st
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
+  set_length_order(p, D == 128 ? 768 : 384);
   tile_order_f32<D>(p, 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -181,6 +183,7 @@ template <int D, int NW> static int fwd_halves_launch(FwdParams p, hipStream_t s
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
+  set_length_order(p, D == 128 ? 768 : 384);
   tile_order_f32<D>(p, D == 128 ? 256 : 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);

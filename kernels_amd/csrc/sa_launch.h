@@ -136,6 +136,20 @@ template <typename P> int64_t set_tiles(P& p, int rows, Tail tail) {
   m.by_heads = chunk_div(p.H);
   return nbh * m.n_tiles;
 }
+// tile_coords_by_length where it can (one length and one pair of an XCD to a lane, pairs that divide over the XCDs), on more workgroups
+// than CUs, and from the length on at which they live long enough to pay for it (about a microsecond each).  Forward in us, lengths in
+// [T/2, T] unless said otherwise, without -> with.  Float16, D=64: 8 x 12 x 1500 54.6 -> 48.3, any lengths 28.1 -> 25.2; 4 x 8 x 2048 36.8 ->
+// 34.8; 8 x 12 x 900, any lengths 24.3 -> 20.5; 32 x 8 x 1024, any lengths 45.7 -> 41.2; D=128, 3 x 8 x 2000 48.0 -> 41.5; D=32, 16 x 12 x
+// 1500 64.4 -> 58.5; D=16, 16 x 12 x 900 30.1 -> 28.1; D=256, 8 x 8 x 1500 119.6 -> 115.2.  On the other side, D=64: 16 x 12 x 700 28.8 ->
+// 29.3, 500 17.7 -> 17.0, 300 10.1 -> 10.9; 32 x 12 x 300, any lengths 11.9 -> 14.2; 192 workgroups, D=128, 2 x 12 x 1000 20.3 -> 20.7.
+// Float32: D=64, 8 x 8 x 1500 132.8 -> 120.1; D=32, 16 x 12 x 900 103.5 -> 88.0, 400 28.5 -> 26.2; D=128, 6 x 4 x 1800 119.5 -> 118.9; on the other
+// side D=64, 16 x 8 x 300 20.4 -> 20.9 (8 x 12 x 300 21.9 -> 19.8), D=128, 8 x 8 x 700 56.0 -> 56.5.  Longest sequences first with the empty tiles left among the others: 8 x 12 x 1500 51.1, any lengths
+// 31.0.
+inline void set_length_order(FwdParams& p, int shortest) {
+  const bool whole = (int64_t)p.C * ((int64_t)p.R + 1) >= p.T && p.T >= shortest;
+  const bool fits = p.B <= 32 && p.tiles.nbh % 8 == 0 && p.tiles.nbh <= 512;
+  p.by_length = p.lens && whole && fits && p.B > 1 && (int64_t)p.tiles.nbh * p.tiles.n_tiles > 256 ? p.B : 0;
+}
 template <typename P> void set_tile_order(P& p, int rows, int tile) {
   p.period = tiles_of_window(p.T, p.C, p.R, rows, tile);
   p.pdiv = chunk_div(p.period > 0 ? p.period : 1);
