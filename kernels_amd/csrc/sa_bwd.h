@@ -470,6 +470,46 @@ template <typename T, int D> SA_DEV typename Elem<T>::Frag dkdv2_keys(typename E
   }
   return k;
 }
+// The same for a tile of 64 keys that every query of the wave sees, at head dimension 256, where a SIMD has one wave: the vector work of a
+// block stands behind products, P behind those of its dP, dS behind the scores of the second block and the dQ products of the first.
+// Between them it stood in nothing's shadow: dQ alone in us, bf16 B=4, H=16, T=4096, chunks of 128, 4 back 375 -> 354 (P behind dP alone:
+// 2.5 % of it); float16 B=1, H=16, T=2048, chunks of 256, 6 back 88.7 -> 82.6; B=4, H=8, T<=3000, 32, 2 back 58.6 -> 56.7; at head dimensions
+// up to 128, with two and three waves on a SIMD, P behind dP changed nothing.  The sums are formed in the same order.
+template <typename T, int D, int NF, int DB>
+SA_DEV void dq2_tile_inside(f32x16 (&acc)[DB], const T* Kt, const T* Vt, const typename Elem<T>::Frag (&qf)[NF],
+                            const typename Elem<T>::Frag (&gf)[NF], float sl2e, float lse_q, const f32x16& dinit, int lane) {
+  static_assert(NF == 16 && DB == 8, "sixteen steps per product");
+  f32x16 s[2], dp[2];
+  float x[2][16];   // P, then -dS (not in the accumulators' registers, which would take them back and forth)
+  typename Elem<T>::Frag b[2][1][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[j][i] = 0.0f;
+    dp[j] = dinit;
+  }
+  auto form_p = [&](int j, int g) {   // one element behind every step but the first, two behind the second
+#pragma unroll
+    for (int i = g < 2 ? 0 : g; i <= g && g > 0; ++i) x[j][i] = fast_exp2(__builtin_fmaf(s[j][i], sl2e, -lse_q));
+  };
+  auto form_ds = [&](int j, int g) {   // rounded two at a time
+    x[j][g] *= dp[j][g];
+    if (g % 2 == 1)
+#pragma unroll
+      for (int i = g - 1; i <= g; ++i) b[j][0][i / 8][i % 8] = (T)x[j][i];
+  };
+  mma_rows_pair<T, D>(s[0], dp[0], Kt, Vt, 0, qf, gf, lane, [&](int it) {
+    if (it >= NF) form_p(0, it - NF);
+  });
+  mma_rows_pair<T, D>(s[1], dp[1], Kt, Vt, 32, qf, gf, lane, [&](int it) {
+    if (it < NF) form_ds(0, it);
+    else form_p(1, it - NF);
+  });
+  auto& acc_n = reinterpret_cast<f32x16 (&)[1][DB]>(acc);
+  mma_tr_n<T, D>(acc_n, Kt, 0, b[0], lane, [&](int it) { form_ds(1, it); });
+  mma_tr_n<T, D>(acc_n, Kt, 1, b[1], lane);
+}
+
 // dV^T += dO^T P and -dK^T += Q^T (-dS) for the TQ queries from qs on.  rows(r) gives the four lse and the four delta
 // values of the tile's rows r to r+3.  kf holds K * (-scale * log2 e), or K where the scores are scaled instead, vf holds -V.
 template <typename T, int D, int TQ, int PG, int NF, int DB, typename Rows>
@@ -646,17 +686,27 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
     for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
   wait_all_loads();
 
-  for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
+  int t = order.first, it = 0;
+  auto next_tile = [&] {   // waits for tile t, sends for the one after it
     wait_loads<0>();
     __syncthreads();
     if (order.next(t) != order.first) issue_tile(order.next(t), it + 1);
-
+  };
+  while (it < kt1 - kt0) {
+    if constexpr (D == 256) {   // a loop of their own: where two paths meet the compiler copies 128 accumulators
+      for (; it < kt1 - kt0 && t * TK >= win.lo_max && t * TK + TK <= win.hi_min; ++it, t = order.next(t)) {
+        next_tile();
+        const T* Kt = smem + (it & 1) * STAGE;
+        dq2_tile_inside<T, D>(acc, Kt, Kt + TILE, qf, gf, sl2e, lse_q, dinit, lane);
+      }
+      if (it == kt1 - kt0) break;
+    }
+    next_tile();
     const T* Kt = smem + (it & 1) * STAGE;
-    const T* Vt = Kt + TILE;
     const int k0 = t * TK;
-    if (k0 + TK <= win.lo_min || k0 >= win.hi_max) continue;   // outside this wave's windows
-
-    dq2_tile<T, D, TK>(acc, Kt, Vt, k0, win, qf, gf, sl2e, lse_q, dinit, lane);
+    if (k0 + TK > win.lo_min && k0 < win.hi_max)   // else outside this wave's windows
+      dq2_tile<T, D, TK>(acc, Kt, Kt + TILE, k0, win, qf, gf, sl2e, lse_q, dinit, lane);
+    ++it, t = order.next(t);
   }
 
   if (qrow >= L) {

@@ -194,6 +194,10 @@ SA_DEV constexpr int crow(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3);
 // N items in groups of G, load(i) returns the fragment of item i, use(i, frag) consumes it.
 SA_DEV void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
 
+struct NoSide {
+  SA_DEV void operator()(int) const {}
+};
+
 template <int N, int G, typename LoadF, typename UseF>
 SA_DEV void pipeline(LoadF&& load, UseF&& use) {
   static_assert(N % G == 0, "items must fill whole groups");
@@ -338,11 +342,12 @@ template <typename T> SA_DEV void pack_c(typename Elem<T>::Frag (&b)[2], const f
 
 // Two products that share the pipeline: acc0 += A0 * B0 and acc1 += A1 * B1, where A0 and A1
 // are the same 32 rows of two row-major LDS tiles (scores from Q and K, dP from dO and V).
-// One fragment stream means one exposed LDS latency instead of two.
-template <typename T, int D, int NF, int GRP = 4>
+// One fragment stream means one exposed LDS latency instead of two.  side(it) is vector work placed behind step it of
+// the 2 * NF.
+template <typename T, int D, int NF, int GRP = 4, typename Side = NoSide>
 SA_DEV void mma_rows_pair(f32x16& acc0, f32x16& acc1, const T* tile0, const T* tile1, int row0,
                           const typename Elem<T>::Frag (&b0)[NF], const typename Elem<T>::Frag (&b1)[NF],
-                          int lane) {
+                          int lane, Side&& side = Side()) {
   using G_ = TileGeom<T, D>;
   using Frag = typename Elem<T>::Frag;
   static_assert(NF == G_::NF, "one register fragment per 2*VEC slice of the head dimension");
@@ -359,6 +364,7 @@ SA_DEV void mma_rows_pair(f32x16& acc0, f32x16& acc1, const T* tile0, const T* t
       [&](int it, const Frag& a) {
         if (it < NF) mma(acc0, a, b0[it]);
         else mma(acc1, a, b1[it - NF]);
+        side(it);
       });
 }
 
@@ -396,10 +402,11 @@ SA_DEV void mma_tr_pair(f32x16 (&acc0)[NM], f32x16 (&acc1)[NM], const T* X0, con
       });
 }
 
-// 16-bit only: acc[q][m] += X^T * B[q] for 32-row block rb of tile X, B[q] packed by pack_c.
-template <typename T, int D, int NQ, int NM, int GRP = (D == 256 ? 2 : 4)>
+// 16-bit only: acc[q][m] += X^T * B[q] for 32-row block rb of tile X, B[q] packed by pack_c.  side(it) is vector work placed behind step it
+// of the 2 * NM.
+template <typename T, int D, int NQ, int NM, int GRP = (D == 256 ? 2 : 4), typename Side = NoSide>
 SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename Elem<T>::Frag (&b)[NQ][2],
-                     int lane) {
+                     int lane, Side&& side = Side()) {
   using E = Elem<T>;
   using G_ = TileGeom<T, D>;
   using Frag = typename E::Frag;
@@ -427,6 +434,7 @@ SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename E
         [&](int it, const Frag& a) {
 #pragma unroll
           for (int q = 0; q < NQ; ++q) mma(acc[q][it % NM], a, b[q][it / NM]);
+          side(it);
         });
     return;
   }
@@ -442,6 +450,7 @@ SA_DEV void mma_tr_n(f32x16 (&acc)[NQ][NM], const T* X, int rb, const typename E
       [&](int it, const Frag& a) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) mma(acc[q][it % NM], a, b[q][it / NM]);
+        side(it);
       });
 }
 

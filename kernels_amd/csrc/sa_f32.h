@@ -255,9 +255,6 @@ template <int D> struct HalfRow {
 
 // acc[row r][col c] += sum_k tile[r][k] * B[k][c] for the 32 rows of a split tile.  side(g) is vector work placed
 // behind the matrix instructions of step g: a wave that has a SIMD to itself has nothing else to fill them with.
-struct NoSide {
-  SA_DEV void operator()(int) const {}
-};
 template <int D, int ROWS, typename Side = NoSide>
 SA_DEV void mma_rows_split(f32x16& acc, const __bf16* tile, const Split8 (&b)[D / 16], int lane, Side&& side = Side()) {
   using G = TileGeom<__bf16, D, D == 16>;
