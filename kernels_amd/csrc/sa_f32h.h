@@ -163,7 +163,7 @@ SA_DEV void row_factors(float (&f)[16], const float* factors, int h) {
 // Keeps fragments that every step multiplies in accumulation registers, where the matrix instruction reads them.  Left alone the
 // compiler copies those that it has put there back for every use: 127 copies among the 960 instructions of a dQ step at D=128, 430 of
 // 1500 in dK/dV.  Counted over the 4k case below, with the masks by bits alone and the factors by v_max3: vector instructions of dQ
-// 108 -> 86 million, of dK/dV 182 -> 124, cycles 269 -> 254 and 393 -> 334; the clock follows the power, so the times less (two kernels
+// 108 -> 86 million, of dK/dV 182 -> 133, cycles 269 -> 257 and 393 -> 339; the clock follows the power, so the times less (two kernels
 // 1220 -> 1125 us).  Not where two waves share the registers of a SIMD (forward in eight waves: 80 registers spilled instead of 29).
 template <int N> SA_DEV void keep_in_agprs(Half8 (&f)[N]) {
 #pragma unroll
@@ -468,8 +468,8 @@ SA_DEV bool too_large(float factor) { return factor >= 0x1p45f; }
 // dQ, one wave per 32 queries, tiles of 32 keys, two stages, delta as in dq_split_kernel.  The next tile's parts are formed behind the
 // products of S and the exponentials behind those of dP.  Same problem as above, dQ and dK/dV together, us: D=128 1562 -> 1125 (traced
 // alone 713 -> 563; one wave per SIMD, whose vector work is what is left between products), D=64 812 -> 590, D=32 430 -> 350.
-// Tried at D=128: dS formed behind the products of the next tile and dQ added a step later, from three stages: 269 -> 277 million cycles;
-// the loads of the next tile right behind its predecessor's parts instead of at the end of a step: 254 -> 269.
+// Tried at D=128: dS formed behind the products of the next tile and dQ added a step later, from three stages: 257 -> 277 million cycles;
+// the loads of the next tile right behind its predecessor's parts instead of at the end of a step: 257 -> 269.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_halves_kernel(const BwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<_Float16, D>::DB;
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_halves_kernel(c
 
 // dK and dV, one wave per 32 keys, tiles of 32 queries, two stages, the vector work behind the products as in dkdv_split_f32_kernel
 // (times above; D=128 traced alone 881 -> 775).  Every tile is masked: a mask that is all ones costs two instructions per element, one that is
-// left out of inner tiles by a branch three, as the compiler makes a select of it (D=128 1210 -> 1087 vector instructions, no spills at 32);
+// left out of inner tiles by a branch three, as the compiler makes a select of it (a tenth of the vector instructions at D=128, no spills at 32);
 // two bodies, with and without, cost 240 copies of registers each.  The next tile's elements held in LDS on their way, to free 32
 // registers: no difference.  Held to 256 registers for a second wave per SIMD D=64 spills and
 // is slower.
