@@ -395,7 +395,7 @@ VARIANT_NAMES = {"fwd": ["narrow", "pipelined"], "dq": ["narrow", "pipelined"], 
 def step_kernels(lib, dtype, D, C, R):
     """{kernel: variant} of the launches of one step (`bwd`: one launch for the whole backward pass)."""
     if dtype == "float32":
-        kind = "float32 instruction" if D == 256 else "16-bit parts"
+        kind = "float32 instruction" if D == 256 else "bfloat16 parts"
         return dict.fromkeys(("fwd", "dq", "dkdv") if D <= 128 else ("fwd", "delta", "dq", "dkdv"), kind)
     if D == 256:
         return {"fwd": "narrow", "dq": "narrow", "dkdv": "split"}

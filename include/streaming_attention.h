@@ -33,12 +33,9 @@
  *     src/streaming_attention/kernel.py:1065-1066), whatever `prescale_qk` the caller of the Python
  *     operator passed: their probabilities differ from the forward's by about |score| * 2^-9 (bf16) /
  *     2^-12 (fp16) relative, inside the 16-bit accuracy bar.  Forward and dQ scale in float32.
- *   - float32 at D <= 128: every product is formed from 16-bit parts of its operands and summed in float32.  Three
- *     bfloat16 parts hold all 24 significand bits (D = 16; windows of less than 512 keys at D = 32, 192 at D = 64).  Two
- *     float16 parts of rows scaled by powers of two (the others) hold an element to 2^-24 of itself, or to 2^-39 of
- *     the largest of its row; the sums have fewer roundings and the results smaller errors.  What leaves the range of
- *     that (infinities, elements or sums beyond about 2^80; with two parts dO and V rows from 2^59 on) is computed with
- *     the float32 instruction, so it gives what float32 arithmetic gives.
+ *   - float32 at D <= 128: every product is formed from three bfloat16 parts per operand, which hold all 24
+ *     significand bits, and summed in float32.  What leaves the range of that (infinities, elements or sums beyond
+ *     about 2^80) is computed with the float32 instruction, so it gives what float32 arithmetic gives.
  */
 #ifndef STREAMING_ATTENTION_H
 #define STREAMING_ATTENTION_H

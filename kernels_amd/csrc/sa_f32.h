@@ -1,5 +1,4 @@
-// float32 kernels on the 16-bit matrix pipe with three bfloat16 parts per number: head dimension 16, and the short windows of 32 and 64
-// (the others have two float16 parts, sa_f32h.h; the copies, stores and windows here serve both).
+// float32 kernels on the 16-bit matrix pipe, head dimensions 16 to 128.
 //
 // v_mfma_f32_32x32x2_f32 does 64 flop per cycle and SIMD, v_mfma_f32_32x32x16_bf16 1024.  A float32
 // number is the sum of three bfloat16 numbers (24 = 8 + 8 + 8 significand bits; each part is the rounded
@@ -361,12 +360,13 @@ struct QueryWindow {
   }
 };
 
-// Forward.  One wave per 32 queries, tiles of 32 keys in two stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
-// bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back, us with the float32 instruction -> here: D=64 392 -> 220,
-// D=32 200 -> 125, D=16 167 -> 107 (with OwnRows32, whole-row stores and TileOrder 223 -> 218, 129 -> 128 at 64 and 32).
-// The register limits (four waves per SIMD up to 32, three at 64) make D=64 spill 19 registers per lane around the products.
-template <int D, int NW>
-__global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
+// Forward.  One wave per 32 queries, tiles of 32 keys in NST stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
+// bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back, us with the float32 instruction -> here: D=128 720 -> 455,
+// D=64 392 -> 220, D=32 200 -> 125, D=16 167 -> 107 (with OwnRows32, whole-row stores and TileOrder 456 -> 432, 223 -> 218, 129 -> 128).
+// The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 31
+// registers per lane, 82 in the four-wave form of 128, around the products.
+template <int D, int NW, int NST>
+__global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
   constexpr float kRescaleGap = 8.0f;
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_
   __syncthreads();
 
   for (int t = order.first, it = 0; it < kt1 - kt0; ++it, t = order.next(t)) {
-    const __bf16* Kt = smem + (it & 1) * 2 * TILE;
+    const __bf16* Kt = smem + (it % NST) * 2 * TILE;
     const __bf16* Vt = Kt + TILE;
     const bool more = order.next(t) != order.first;
     if (more) {
@@ -495,7 +495,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_
       mma_tr_split<D, TK>(oacc, Vt, pb, lane);   // O^T[d][q] += V^T P^T
     }
     if (more) {
-      __bf16* nxt = smem + (~it & 1) * 2 * TILE;
+      if (NST == 1) __syncthreads();   // the only stage has no reader left
+      __bf16* nxt = smem + ((it + 1) % NST) * 2 * TILE;
       sk.store(nxt, tid);
       sv.store(nxt + TILE, tid);
     }
@@ -523,10 +524,11 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : NW == 4 ? 3 : 2)) void fwd_
 
 // dQ, one wave per 32 queries, tiles of 32 keys, two stages.  delta = rowsum(O * dO) is formed in the prologue (the
 // O row is read beside the dO row) and written for the dK/dV kernel that runs after this one, or read when the caller
-// has computed it (p.delta_out == null).  Same problem as above: D=64 557 -> 309 us, D=32 274 -> 181, D=16 197 -> 117; forming
-// delta here saves a pass over O and dO (40 us at D=128).
+// has computed it (p.delta_out == null).  Same problem as above: D=128 1027 -> 679 us (one wave per SIMD: the parts of Q
+// and dO are 192 registers), D=64 557 -> 309, D=32 274 -> 181, D=16 197 -> 117; forming delta here saves a pass of 40 us over
+// O and dO at D=128.
 template <int D, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void dq_split_kernel(const BwdParams p) {
+__global__ __launch_bounds__(NW * 64, (D <= 64 ? 2 : 1)) void dq_split_kernel(const BwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, NF = D / 16, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
 
@@ -679,9 +681,10 @@ __global__ __launch_bounds__(NW * 64, 2) void dq_split_kernel(const BwdParams p)
 }
 
 // dK and dV, one wave per 32 keys, tiles of 32 queries, two stages.  Four products per tile; the vector work sits behind
-// their matrix instructions (the exponentials and the parts of P behind dP, dS and its parts behind dV): at head
-// dimension 64 a wave has its SIMD to itself.  Held to 256 registers for a second wave, D=64 spilled and measured
-// the same or slower.  Same problem as above: D=64 665 -> 476 us, D=32 351 -> 245, D=16 261 -> 194.
+// their matrix instructions (the exponentials and the parts of P behind dP, dS and its parts behind dV): from head
+// dimension 64 on a wave has its SIMD to itself.  Held to 256 registers for a second wave, D=64 spilled and measured
+// the same or slower.  Same problem as above: D=128 1470 -> 883 us (42 registers spilled), D=64 665 -> 476, D=32 351 -> 245,
+// D=16 261 -> 194.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 2 : 1)) void dkdv_split_f32_kernel(const BwdParams p) {
   constexpr int TKB = NW * 32, NT = NW * 64, TQ = 32, NF = D / 16, DB = TileGeom<__bf16, D, D == 16>::DB;

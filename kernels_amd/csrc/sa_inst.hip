@@ -6,7 +6,6 @@
 #include <mutex>
 #include "sa_launch.h"
 #include "sa_f32.h"
-#include "sa_f32h.h"
 #if SA_KIND == 0
 #include "sa_fwd.h"
 #ifndef SA_NO_ASM_KERNELS
@@ -83,19 +82,6 @@ template <typename P> static bool half_workgroups(const P& p) {
   return 10 * (back + ceil_div(64, p.C) * p.C) <= 9 * (back + ceil_div(128, p.C) * p.C);
 }
 
-// float32, head dimensions 32 and 64: whether the products are formed from two float16 parts (sa_f32h.h) or from three of bfloat16
-// (sa_f32.h).  Two parts take half the matrix time, but a wave sets its units in its first tiles and tests them in each, and rows are
-// scaled on their way into LDS: short windows have not the products that hide that.  By the keys of a window (never by the grid: the
-// two add in different orders, and a sequence has the same bits in any batch).  Three -> two parts, forward and backward in us:
-//   D=64, B=8, H=16, T=2000: 48 keys 49.6, 197 -> 54.8, 206; 100 68, 257 -> 72, 255; 160 80.6, 295 -> 79, 284; 192 70, 254 -> 67, 244;
-//     300 (one chunk) 125, 442 -> 114, 395; B*H=8, T=700: 80 keys 15.8, 39.8 -> 16.4, 40.7; 192 15.0, 39.5 -> 14.8, 38.4
-//   D=32: 192 keys 43.4, 144 -> 45.2, 151; 300 69, 218 -> 68, 220; 640 93.5, 310 -> 87.6, 288; 1500 230, 759 -> 217, 679; B*H=8, T=700, 384 keys
-//     18.0, 45.9 -> 18.8, 46.6
-// Head dimension 128 always takes two: 48 keys 71, 226 -> 69, 222.
-template <int D, typename P> static bool in_halves(const P& p) {
-  return ((int64_t)p.R + 1) * p.C >= (D == 64 ? 192 : 512);
-}
-
 // TileOrder of the float32 kernels, with the period of the largest workgroup that a kernel has at this head dimension, whatever
 // the grid picks: no window holds two multiples of it, so the windows of a smaller workgroup start at the same tile or have none of
 // them, and every row goes through its tiles in the same order.  At head dimension 16 the order gained nothing.
@@ -164,26 +150,13 @@ template <int D> static int fwd3_launch(FwdParams p, hipStream_t st) {
   }
 #endif
 }
-template <int D, int NW> static int fwd_split_launch(FwdParams p, hipStream_t st) {
-  constexpr size_t lds = split_lds<D, NW>((size_t)2 * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>, 1);
-  auto kern = fwd_split_kernel<D, NW>;
+template <int D, int NW, int NST> static int fwd_split_launch(FwdParams p, hipStream_t st) {
+  constexpr size_t lds = split_lds<D, NW>((size_t)NST * 2 * SplitTile<D, 32>::ELEMS * sizeof(__bf16), float_tiles<D>, 1);
+  auto kern = fwd_split_kernel<D, NW, NST>;
   static PrepareState once;
   if (int rc = prepare(kern, lds, once)) return rc;
   const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
-  set_length_order(p, D == 128 ? 768 : 384);
-  tile_order_f32<D>(p, 128);
-  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
-  return (int)hipGetLastError();
-}
-template <int D, int NW> static int fwd_halves_launch(FwdParams p, hipStream_t st) {
-  constexpr size_t tiles = (size_t)2 * 2 * (HalfTile<D>::ELEMS * sizeof(_Float16) + 32 * sizeof(float));
-  constexpr size_t lds = split_lds<D, NW>(tiles, float_tiles<D>, 1);
-  auto kern = fwd_halves_kernel<D, NW>;
-  static PrepareState once;
-  if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
-  set_length_order(p, D == 128 ? 768 : 384);
+  if (D != 128 || NW == 8) set_length_order(p, D == 128 ? 768 : 384);
   tile_order_f32<D>(p, D == 128 ? 256 : 128);
   if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
@@ -219,23 +192,15 @@ template <int D> static int fwd_d(FwdParams p, hipStream_t st) {
     }
     return fwd2_launch<D, C::NARROW_NW, C::FWD_TK, false>(p, st);
   } else if constexpr (C::split(D)) {
-    // Head dimension 128: eight waves with two on a SIMD, or four with a SIMD and 512 registers each while those make no second
-    // workgroup on a CU (which takes as long again).  us, eight -> four waves: chunks of 8, 5 back, T=402, 60 workgroups of four
-    // waves 27.2 -> 22.3; chunks of 64, 2 back, T=500, 128 of them 33.5 -> 24.9, T=1000, 256 34.6 -> 27.1; chunks of 256, 3 back,
-    // T=4000, 256 82.3 -> 76.4; past the line chunks of 32, 3 back, T=1000, 384 of them 35.8 -> 49.0, chunks of 128, 2 back, T=1000,
-    // 512 52.4 -> 52.8.
+    // Head dimension 128: eight waves share one workgroup's two 48 KiB stages, two waves per SIMD, once that makes a
+    // workgroup per CU; smaller grids run twice as many four-wave workgroups with one stage (B*H=24, T=1024: 34
+    // against 44 us; B*H=64, T=2048, 512 of the large ones: 91 against 82 us).
     if constexpr (D == 128) {
-      if ((int64_t)p.B * p.H * ceil_div(p.T, 128) <= 256) return fwd_halves_launch<D, 4>(p, st);
-      return fwd_halves_launch<D, 8>(p, st);
+      if ((int64_t)p.B * p.H * ceil_div(p.T, 256) < 256) return fwd_split_launch<D, 4, 1>(p, st);
+      return fwd_split_launch<D, 8, 2>(p, st);
     } else {
-      if constexpr (C::halves(D)) {
-        if (in_halves<D>(p)) {
-          if (half_workgroups(p)) return fwd_halves_launch<D, 2>(p, st);
-          return fwd_halves_launch<D, 4>(p, st);
-        }
-      }
-      if (half_workgroups(p)) return fwd_split_launch<D, 2>(p, st);
-      return fwd_split_launch<D, 4>(p, st);
+      if (half_workgroups(p)) return fwd_split_launch<D, 2, 2>(p, st);
+      return fwd_split_launch<D, 4, 2>(p, st);
     }
   } else {
     return fwd_first_launch<D>(p, st);
@@ -312,17 +277,6 @@ template <int D, int NW> static int dq_split_launch(BwdParams p, hipStream_t st)
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
-template <int D, int NW> static int dq_halves_launch(BwdParams p, hipStream_t st) {
-  constexpr size_t lds = split_lds<D, NW>((size_t)2 * 2 * (HalfTile<D>::ELEMS * sizeof(_Float16) + 32 * sizeof(float)), float_tiles<D>, 2);
-  auto kern = dq_halves_kernel<D, NW>;
-  static PrepareState once;
-  if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
-  tile_order_f32<D>(p, 128);
-  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
-  return (int)hipGetLastError();
-}
 template <int D> static int dq_first_launch(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   if (p.delta_out) return SA_ERR_ARG;
@@ -347,18 +301,10 @@ template <int D> static int dq_d(BwdParams p, hipStream_t st) {
     }
     return dq2_launch<D, C::NARROW_NW>(p, st);
   } else if constexpr (C::split(D)) {
-    if constexpr (D == 128) {
-      return dq_halves_launch<D, 4>(p, st);
-    } else {
-      if constexpr (C::halves(D)) {
-        if (in_halves<D>(p)) {
-          if (half_workgroups(p)) return dq_halves_launch<D, 2>(p, st);
-          return dq_halves_launch<D, 4>(p, st);
-        }
-      }
+    if constexpr (D <= 64) {
       if (half_workgroups(p)) return dq_split_launch<D, 2>(p, st);
-      return dq_split_launch<D, 4>(p, st);
     }
+    return dq_split_launch<D, 4>(p, st);
   } else {
     return dq_first_launch<D>(p, st);
   }
@@ -441,18 +387,6 @@ template <int D, int NW> static int dkdv_split_f32_launch(BwdParams p, hipStream
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
   return (int)hipGetLastError();
 }
-template <int D, int NW> static int dkdv_halves_launch(BwdParams p, hipStream_t st) {
-  constexpr size_t rows = (size_t)2 * 4 * 32 * sizeof(float);   // lse, delta and the factors
-  constexpr size_t lds = split_lds<D, NW>((size_t)2 * 2 * HalfTile<D>::ELEMS * sizeof(_Float16) + rows, float_tiles<D> + rows, 2);
-  auto kern = dkdv_halves_kernel<D, NW>;
-  static PrepareState once;
-  if (int rc = prepare(kern, lds, once)) return rc;
-  const int64_t blocks = set_tiles(p, NW * 32, SHORT_LAST);
-  tile_order_f32<D>(p, 128);
-  if (blocks > 0x7fffffffLL) return SA_ERR_TOO_LARGE;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), lds, st, p);
-  return (int)hipGetLastError();
-}
 template <int D> static int dkdv_first_launch(BwdParams p, hipStream_t st) {
   using C = Cfg<ElemT>;
   constexpr int TKB = C::NW * 32;
@@ -511,18 +445,10 @@ template <int D> static int dkdv_d(BwdParams p, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::DKDV2_NW * 64), lds, st, p);
     return (int)hipGetLastError();
   } else if constexpr (C::split(D)) {
-    if constexpr (D == 128) {
-      return dkdv_halves_launch<D, 4>(p, st);
-    } else {
-      if constexpr (C::halves(D)) {
-        if (in_halves<D>(p)) {
-          if (half_workgroups(p)) return dkdv_halves_launch<D, 2>(p, st);
-          return dkdv_halves_launch<D, 4>(p, st);
-        }
-      }
+    if constexpr (D <= 64) {
       if (half_workgroups(p)) return dkdv_split_f32_launch<D, 2>(p, st);
-      return dkdv_split_f32_launch<D, 4>(p, st);
     }
+    return dkdv_split_f32_launch<D, 4>(p, st);
   } else {
     return dkdv_first_launch<D>(p, st);
   }

@@ -142,9 +142,10 @@ template <typename P> int64_t set_tiles(P& p, int rows, Tail tail) {
 // 34.8; 8 x 12 x 900, any lengths 24.3 -> 20.5; 32 x 8 x 1024, any lengths 45.7 -> 41.2; D=128, 3 x 8 x 2000 48.0 -> 41.5; D=32, 16 x 12 x
 // 1500 64.4 -> 58.5; D=16, 16 x 12 x 900 30.1 -> 28.1; D=256, 8 x 8 x 1500 119.6 -> 115.2.  On the other side, D=64: 16 x 12 x 700 28.8 ->
 // 29.3, 500 17.7 -> 17.0, 300 10.1 -> 10.9; 32 x 12 x 300, any lengths 11.9 -> 14.2; 192 workgroups, D=128, 2 x 12 x 1000 20.3 -> 20.7.
-// Float32: D=64, 8 x 8 x 1500 132.8 -> 120.1; D=32, 16 x 12 x 900 103.5 -> 88.0, 400 28.5 -> 26.2; D=128, 6 x 4 x 1800 119.5 -> 118.9; on the other
-// side D=64, 16 x 8 x 300 20.4 -> 20.9 (8 x 12 x 300 21.9 -> 19.8), D=128, 8 x 8 x 700 56.0 -> 56.5.  Longest sequences first with the empty tiles left among the others: 8 x 12 x 1500 51.1, any lengths
-// 31.0.
+// Float32: D=64, 8 x 8 x 1500 157 -> 152, 16 x 8 x 600 at D=16 36 -> 32; D=32, 16 x 12 x 900 100 -> 84, 400 27.6 -> 25.2; D=16, 16 x 12 x 900 82 -> 69; below the
+// line either way, 16 x 8 x 300 at D=64 25.9 -> 24.2, 32 x 16 x 260 at 64, 32, 16 46.8 -> 48.2, 31.3 -> 32.9, 26.1 -> 28.0.  D=128 in eight waves, 8 x 8 x 1500 322
+// -> 306, 16 x 8 x 800 186 -> 160; below the line either way, 16 x 16 x 600 215 -> 217, 8 x 16 x 700 131 -> 134, 16 x 16 x 400 99.6 -> 94.5; in four waves 6 x 4 x
+// 1800 208 -> 214.  Longest sequences first with the empty tiles left among the others: float16, D=64, 8 x 12 x 1500 51.1, any lengths 31.0.
 inline void set_length_order(FwdParams& p, int shortest) {
   const bool whole = (int64_t)p.C * ((int64_t)p.R + 1) >= p.T && p.T >= shortest;
   const bool fits = p.B <= 32 && p.tiles.nbh % 8 == 0 && p.tiles.nbh <= 512;
@@ -237,10 +238,8 @@ template <typename T> struct Cfg {
 #else
   static constexpr bool fwd2(int D) { return sizeof(T) == 2 && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256); }
 #endif
-  // float32 on the 16-bit matrix pipe; at 256 the parts of the resident rows exceed the registers
+  // float32 on the 16-bit matrix pipe (sa_f32.h); at 256 the parts of the resident rows exceed the registers
   static constexpr bool split(int D) { return sizeof(T) == 4 && D <= 128; }
-  // which has kernels with two float16 parts per number (sa_f32h.h), and up to 64 with three bfloat16 parts (sa_f32.h)
-  static constexpr bool halves(int D) { return split(D) && D >= 32; }
 #ifdef SA_FWD_TK16
   static constexpr int FWD_TK = sizeof(T) == 4 ? 32 : SA_FWD_TK16;
 #else
