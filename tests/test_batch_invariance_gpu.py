@@ -44,3 +44,26 @@ def test_float32(D, C, R):
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_float32_long_windows(D):
     bits_alone_and_in_batches(torch.float32, 8, 1500, D, 96, 4, (2, 4, 6))   # 192 workgroups of 128 rows, 288 of 256
+
+
+@pytest.mark.parametrize("C,R", [(1000, 0), (96, 30), (64, 2)])   # one chunk over everything, chunks whose windows do, and those that do not
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_float32_padded_to_another_length(D, C, R):
+    """The padded length T of a batch, to which longer windows are cut, changes no bit either."""
+    from streaming_attention import streaming_attention
+
+    dev = torch.device("cuda:0")
+    B, H, L = 2, 8, 180
+    g = torch.Generator(device=dev).manual_seed(32)
+    q, k, v, d_o = (torch.randn(B, H, 1600, D, generator=g, device=dev) for _ in range(4))
+    lens = torch.tensor([L, L - 37], dtype=torch.int32, device=dev)
+
+    def step(T):
+        x = [t[:, :, :T].clone().requires_grad_() for t in (q, k, v)]
+        o, lse = streaming_attention(*x, lens, C, R, return_lse=True)
+        return [t[:, :, :L] for t in (o.detach(), lse.detach(), *torch.autograd.grad(o, x, d_o[:, :, :T]))]
+
+    short = step(L)
+    for T in (191, 192, 511, 512, 1600):
+        for name, a, b in zip(("O", "LSE", "dQ", "dK", "dV"), short, step(T)):
+            assert torch.equal(a, b), (name, T)
