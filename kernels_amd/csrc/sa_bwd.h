@@ -420,13 +420,6 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 // asynchronous global->LDS copies into a ring of two stages, one barrier per tile.
 // ---------------------------------------------------------------------------------------
 
-// The window of one lane's row (a query's keys, or a key's queries), of all rows of its wave and of any of them.
-struct WaveWindow {
-  int lo, hi;
-  int lo_max, hi_min;   // seen by every row of the wave
-  int lo_min, hi_max;   // seen by some row of the wave (empty for a wave of padding)
-};
-
 // -dQ^T += K^T (-dS^T) for the TK keys from k0 on: S, dP and dS of one 32-key block at a time, blocks outside the wave's
 // windows left out.  gf holds -dO and dinit delta, so that the dP accumulator ends at delta - dP.
 template <typename T, int D, int TK, int NF, int DB>
@@ -437,8 +430,8 @@ SA_DEV void dq2_tile(f32x16 (&acc)[DB], const T* Kt, const T* Vt, int k0, const 
 #pragma unroll
   for (int kb = 0; kb < TK / 32; ++kb) {
     const int kb0 = k0 + kb * 32;
-    if (kb0 + 32 <= win.lo_min || kb0 >= win.hi_max) continue;
-    const bool interior = (kb0 >= win.lo_max) && (kb0 + 32 <= win.hi_min);
+    if (!win.seen(kb0, 32)) continue;
+    const bool interior = win.inside(kb0, 32);
     f32x16 s[1], dp[1];
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[0][i] = 0.0f;
@@ -458,19 +451,7 @@ SA_DEV void dq2_tile(f32x16 (&acc)[DB], const T* Kt, const T* Vt, int k0, const 
   }
 }
 
-// A fragment of K as dkdv2_tile wants it: multiplied by -scale*log2(e) and rounded to the element type, so that the score accumulator
-// starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability.  At head dimension 16 the scores are
-// scaled in float32, which costs a multiplication per score of a kernel that is bound by memory and latency.
-constexpr bool scaled_scores(int D) { return D < 32; }
-template <typename T, int D> SA_DEV typename Elem<T>::Frag dkdv2_keys(typename Elem<T>::Frag k, float scale_log2e) {
-  if constexpr (!scaled_scores(D)) {
-    const float kmul = -scale_log2e;
-#pragma unroll
-    for (int e = 0; e < Elem<T>::VEC; ++e) k[e] = (T)((float)k[e] * kmul);
-  }
-  return k;
-}
-// The same for a tile of 64 keys that every query of the wave sees, at head dimension 256, where a SIMD has one wave: the vector work of a
+// dq2_tile for a tile of 64 keys that every query of the wave sees, at head dimension 256, where a SIMD has one wave: the vector work of a
 // block stands behind products, P behind those of its dP, dS behind the scores of the second block and the dQ products of the first.
 // Between them it stood in nothing's shadow: dQ alone in us, bf16 B=4, H=16, T=4096, chunks of 128, 4 back 375 -> 354 (P behind dP alone:
 // 2.5 % of it); float16 B=1, H=16, T=2048, chunks of 256, 6 back 88.7 -> 82.6; B=4, H=8, T<=3000, 32, 2 back 58.6 -> 56.7; at head dimensions
@@ -510,6 +491,19 @@ SA_DEV void dq2_tile_inside(f32x16 (&acc)[DB], const T* Kt, const T* Vt, const t
   mma_tr_n<T, D>(acc_n, Kt, 1, b[1], lane);
 }
 
+// A fragment of K as dkdv2_tile wants it: multiplied by -scale*log2(e) and rounded to the element type, so that the score accumulator
+// starts at lse and ends at lse - score*scale*log2(e), whose negated exp2 is the probability.  At head dimension 16 the scores are
+// scaled in float32, which costs a multiplication per score of a kernel that is bound by memory and latency.
+constexpr bool scaled_scores(int D) { return D < 32; }
+template <typename T, int D> SA_DEV typename Elem<T>::Frag dkdv2_keys(typename Elem<T>::Frag k, float scale_log2e) {
+  if constexpr (!scaled_scores(D)) {
+    const float kmul = -scale_log2e;
+#pragma unroll
+    for (int e = 0; e < Elem<T>::VEC; ++e) k[e] = (T)((float)k[e] * kmul);
+  }
+  return k;
+}
+
 // dV^T += dO^T P and -dK^T += Q^T (-dS) for the TQ queries from qs on.  rows(r) gives the four lse and the four delta
 // values of the tile's rows r to r+3.  kf holds K * (-scale * log2 e), or K where the scores are scaled instead, vf holds -V.
 template <typename T, int D, int TQ, int PG, int NF, int DB, typename Rows>
@@ -520,8 +514,8 @@ SA_DEV void dkdv2_tile(f32x16 (&dk)[DB], f32x16 (&dv)[DB], const T* Qt, const T*
 #pragma unroll
   for (int qb = 0; qb < TQ / 32; ++qb) {
     const int qb0 = qs + qb * 32;
-    if (qb0 + 32 <= win.lo_min || qb0 >= win.hi_max) continue;
-    const bool interior = (qb0 >= win.lo_max) && (qb0 + 32 <= win.hi_min);
+    if (!win.seen(qb0, 32)) continue;
+    const bool interior = win.inside(qb0, 32);
     f32x16 s[1], dp[1], lse;   // lse: scaled scores
     // lse / delta of the 16 rows this lane holds, fetched ahead of the products and read
     // straight into the score and dP accumulators
@@ -604,18 +598,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
 
   const int qrow = q0 + wave * 32 + c;
   const int qe = qrow < L ? qrow : L - 1;
-  const int qchunk = cdiv(qe);
-  const int lo = (qchunk > R ? qchunk - R : 0) * C;
-  const int hi = (qchunk + 1) * C < L ? (qchunk + 1) * C : L;
-  const int wq_first = q0 + wave * 32 < L ? q0 + wave * 32 : L - 1;
-  const int wq_last = q0 + wave * 32 + 31 < L ? q0 + wave * 32 + 31 : L - 1;
-  const int hi_min = (cdiv(wq_first) + 1) * C < L ? (cdiv(wq_first) + 1) * C : L;
-  const int lo_max = (cdiv(wq_last) > R ? cdiv(wq_last) - R : 0) * C;
-  // keys any query of this wave can see; a wave whose queries are all padding sees none
-  const bool wave_live = q0 + wave * 32 < L;
-  const int lo_min = (cdiv(wq_first) > R ? cdiv(wq_first) - R : 0) * C;
-  const int hi_max = !wave_live ? 0 : ((cdiv(wq_last) + 1) * C < L ? (cdiv(wq_last) + 1) * C : L);
-  const WaveWindow win{lo, hi, lo_max, hi_min, lo_min, hi_max};
+  const WaveWindow win = query_window(q0 + wave * 32, qrow, L, C, R, p.cdiv);
   const int gq_last = q0 + TQ - 1 < L ? q0 + TQ - 1 : L - 1;
   const int lo_wg = (cdiv(q0) > R ? cdiv(q0) - R : 0) * C;
   const int hi_wg = (cdiv(gq_last) + 1) * C < L ? (cdiv(gq_last) + 1) * C : L;
@@ -694,7 +677,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
   };
   while (it < kt1 - kt0) {
     if constexpr (D == 256) {   // a loop of their own: where two paths meet the compiler copies 128 accumulators
-      for (; it < kt1 - kt0 && t * TK >= win.lo_max && t * TK + TK <= win.hi_min; ++it, t = order.next(t)) {
+      for (; it < kt1 - kt0 && win.inside(t * TK, TK); ++it, t = order.next(t)) {
         next_tile();
         const T* Kt = smem + (it & 1) * STAGE;
         dq2_tile_inside<T, D>(acc, Kt, Kt + TILE, qf, gf, sl2e, lse_q, dinit, lane);
@@ -704,7 +687,7 @@ __global__ __launch_bounds__(NW * 64) void dq2_kernel(const BwdParams p) {
     next_tile();
     const T* Kt = smem + (it & 1) * STAGE;
     const int k0 = t * TK;
-    if (k0 + TK > win.lo_min && k0 < win.hi_max)   // else outside this wave's windows
+    if (win.seen(k0, TK))
       dq2_tile<T, D, TK>(acc, Kt, Kt + TILE, k0, win, qf, gf, sl2e, lse_q, dinit, lane);
     ++it, t = order.next(t);
   }
@@ -840,7 +823,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void dkdv2_kernel(const
     const T* Gt = Qt + TILE;
     const float* ld_t = reinterpret_cast<const float*>(stage + 2 * TILE * sizeof(T));
     const int qs = t * TQ;
-    if (qs + TQ <= win.lo_min || qs >= win.hi_max) continue;   // outside this wave's windows
+    if (!win.seen(qs, TQ)) continue;
 
     dkdv2_tile<T, D, TQ, PG>(dk, dv, Qt, Gt, qs, win, kf, vf, p.scale_log2e, [&](int r, f32x4& l4, f32x4& d4) {
       const float* chunk = ld_t + (r / RPW) * 2 * RPW + (r % RPW);

@@ -172,7 +172,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
       __syncthreads();   // tile t is in LDS and tile t - 1 has no reader left
       if (t + 2 < kt1) issue_tile(st == 0 ? 2 : st - 1);
       const T* Kt = smem + st * STAGE;
-      if (t * TT + TT <= wq.lo_min || t * TT >= wq.hi_max) continue;   // outside this wave's windows
+      if (!wq.seen(t * TT, TT)) continue;
       dq2_tile<T, D, TT>(acc, Kt, Kt + TILE, t * TT, wq, qf, gf, sl2e, lse_q, dinit, lane);
     }
     // the last three key tiles are still in LDS: as a rule the workgroup's own rows are among them
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(NW * 64, (D == 64 ? 3 : 1)) void bwd_fused_kernel(c
     __syncthreads();
     if (t + 2 < qt1) issue_tile(st == 0 ? 2 : st - 1);
     const T* Qt = smem + st * STAGE;
-    if (t * TT + TT <= wk.lo_min || t * TT >= wk.hi_max) continue;
+    if (!wk.seen(t * TT, TT)) continue;
     const float* l = lse_s + (t - qt0) * TT;
     const float* d = delta_s + (t - qt0) * TT;
     dkdv2_tile<T, D, TT, PG>(dk, dv, Qt, Qt + TILE, t * TT, wk, kf, vf, p.scale_log2e, [&](int r, f32x4& l4, f32x4& d4) {

@@ -959,6 +959,25 @@ struct TileOrder {
   SA_BOTH int next(int t) const { return t + 1 == t1 ? t0 : t + 1; }   // `first` again after the last one
 };
 
+// The window of one lane's row (a query's keys, or a key's queries), of all rows of its wave and of any of them.
+struct WaveWindow {
+  int lo, hi;
+  int lo_max, hi_min;   // seen by every row of the wave
+  int lo_min, hi_max;   // seen by some row of the wave; a wave of padding sees nothing: hi_max is 0
+  SA_BOTH bool seen(int first, int n) const { return first + n > lo_min && first < hi_max; }
+  SA_BOTH bool inside(int first, int n) const { return first >= lo_max && first + n <= hi_min; }   // every row sees all of them
+};
+// Of query `row` in the wave that has the 32 from first_row on, of a sequence of L.  Rows past L have the last valid row's window, but where
+// all of a wave's are, no key is inside it: its products would be thrown away.
+SA_BOTH WaveWindow query_window(int first_row, int row, int L, int C, int R, ChunkDiv cdiv) {
+  auto chunk = [&](int r) { return div_by(r < L ? r : L - 1, cdiv); };
+  auto begin = [&](int c) { return (c > R ? c - R : 0) * C; };
+  auto end = [&](int c) { return (c + 1) * C < L ? (c + 1) * C : L; };
+  const int own = chunk(row), first = chunk(first_row), last = chunk(first_row + 31);
+  const bool live = first_row < L;
+  return {begin(own), end(own), begin(last), live ? end(first) : 0, begin(first), live ? end(last) : 0};
+}
+
 struct FwdParams {
   const void *q, *k, *v;
   void* o;          // contiguous [B,H,T,D]

@@ -139,8 +139,43 @@ int main() {
 }
 """
 
+# What a dQ wave goes through: a tile is seen where one of its queries sees a key of it, inside where all of them see all of it, and a wave of
+# padding sees nothing and has nothing inside.
+QUERY_WINDOWS = HEAD + r"""
+int main() {
+  int waves = 0;
+  for (int C : {CHUNKS})
+    for (int R : {0, 1, 2, 5})
+      for (int L : {1, 31, 32, 33, 127, 128, 129, 300, 700})
+        for (int first = 0; first < 896; first += 32) {
+          WaveWindow w{};
+          bool live = false;
+          for (int row = first; row < first + 32; ++row) {
+            const WaveWindow mine = query_window(first, row, L, C, R, chunk_div(C));
+            if (row == first) w = mine;
+            CHECK(mine.lo_max == w.lo_max && mine.hi_min == w.hi_min && mine.lo_min == w.lo_min && mine.hi_max == w.hi_max, "row %d", row);
+            live |= row < L;
+          }
+          for (int tile : {32, 64})
+            for (int t = 0; t < L; t += tile) {
+              bool seen = false, inside = live;
+              for (int row = first; row < std::min(first + 32, L); ++row) {
+                const int lo = std::max(row / C - R, 0) * C, hi = std::min((row / C + 1) * C, L);
+                CHECK(query_window(first, row, L, C, R, chunk_div(C)).lo == lo && query_window(first, row, L, C, R, chunk_div(C)).hi == hi, "row %d", row);
+                seen |= t < hi && t + tile > lo;
+                inside &= t >= lo && t + tile <= hi;
+              }
+              CHECK(w.seen(t, tile) == seen, "C %d R %d L %d first %d t %d", C, R, L, first, t);
+              CHECK(w.inside(t, tile) == inside, "C %d R %d L %d first %d t %d", C, R, L, first, t);
+            }
+          ++waves;
+        }
+  printf("ok %d\n", waves);
+}
+""".replace("CHUNKS", CHUNKS)
 
-PROGRAMS = {"tile_order": (TILE_ORDER, 5000), "rows_in_reach": (ROWS_IN_REACH, 3000), "dispatch": (DISPATCH, 10000)}
+
+PROGRAMS = {"tile_order": (TILE_ORDER, 5000), "rows_in_reach": (ROWS_IN_REACH, 3000), "dispatch": (DISPATCH, 10000), "query_windows": (QUERY_WINDOWS, 10000)}
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="no compiler")
