@@ -111,8 +111,8 @@ int sa_bwd_dkdv(const void* q, const void* k, const void* v,
  * reference's `_streaming_attn_bwd_precompute` launch, kernel.py:433-514 -- is not launched; the
  * sums are added in another order than sa_bwd_delta adds them, so the gradients agree with those
  * of the separate calls to rounding, not bit for bit.  Replaces the body of
- * `attention_backward_adapter` (src/streaming_attention/kernel.py:1363-1442).  16-bit types at head dimensions 32 and 64
- * with windows of about a hundred keys run one kernel that forms all three gradients and `delta`. */
+ * `attention_backward_adapter` (src/streaming_attention/kernel.py:1363-1442).  16-bit types at head dimensions 16, 32 and
+ * 64 with windows of about a hundred keys run one kernel that forms all three gradients and `delta`. */
 int sa_backward(const void* q, const void* k, const void* v,
                 const int32_t* lens, int64_t lens_stride,
                 const void* o, const void* d_o, const float* lse, float* delta,

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(NW * 64) void dkdv_kernel(const BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Variants for 16-bit elements with swizzled tiles (D = 32, 64, 128; dQ also 256): tiles arrive by
+// Variants for 16-bit elements with swizzled tiles (D = 16 to 128; dQ also 256): tiles arrive by
 // asynchronous global->LDS copies into a ring of two stages, one barrier per tile.
 // ---------------------------------------------------------------------------------------
 

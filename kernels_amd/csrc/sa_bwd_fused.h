@@ -16,7 +16,7 @@
 // chunk of 128: 160 -> 127 us.
 // B=16, H=8, T=2048 ragged, D=64, chunks of 64, 1 back: 46 -> 39.  B=225, H=4, T=993 ragged, D=32, chunks of 16, 2 back: 94 -> 92.
 // Two waves and 32-row tiles instead of four and 64 where that reads no more rows per row of its own (and at D = 32 on
-// windows that lie across the 32-row blocks): fused_backward_in_two_waves in sa_launch.h has the rule and both sides' times.
+// windows that lie across the 32-row blocks, at D = 16 on all chunks below 128): fused_backward_in_two_waves in sa_launch.h has the rule and both sides' times.
 // A form that slides along a sequence and reads every row once (scores formed once, dS handed over in LDS) took 967 us
 // on the first problem and up to twice as long on windows of more than four 32-row blocks: one workgroup per CU, steps
 // in lockstep.

@@ -553,8 +553,8 @@ template <typename T, int D, int ROWS, int NW, bool ASM_COPIES = false> struct A
 // The copies of two tiles that a step reads together (K and V, or Q and dO), one behind the other in a stage.  Head dimension 16:
 // one instruction moves 32 rows, so a stage of 32 rows per pair of waves is one instruction per wave, half of the waves to a tile.
 // That, tiles without padding and the kernels of the wider heads instead of tiles staged through registers, float16, forward and with
-// backward in us: B=225, H=4, T<=993, chunks of 16, 2 back 67.4, 164.5 -> 21.1, 73.3; 64 x 8 x 1024, 40, 3 back 97.7, 225.9 -> 31.4, 112.9;
-// 64, 5 back 68.9, 218.4 -> 41.7, 145.5; one chunk, 8 x 8 x 1500 39.9, 143.7 -> 34.5, 121.1.  Bound by latency and the masks' vector work
+// backward in us: B=225, H=4, T<=993, chunks of 16, 2 back 65, 158 -> 20, 73; 64 x 8 x 1024, 40, 3 back 91, 204 -> 28, 99;
+// 64, 5 back 62, 188 -> 35, 125; one chunk, 8 x 8 x 1500 34, 121 -> 30, 102.  Bound by latency and the masks' vector work
 // (the first at 2.7 TB/s of its eight tensors).
 template <typename T, int D, int ROWS, int NW, bool ASM_COPIES> struct TilePair {
   static constexpr bool ONE_EACH = D < 32;

@@ -363,8 +363,8 @@ struct QueryWindow {
 // Forward.  One wave per 32 queries, tiles of 32 keys in NST stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
 // bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back, us with the float32 instruction -> here: D=128 720 -> 455,
 // D=64 392 -> 220, D=32 200 -> 125, D=16 167 -> 107 (with OwnRows32, whole-row stores and TileOrder 456 -> 432, 223 -> 218, 129 -> 128).
-// The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 31
-// registers per lane, 82 in the four-wave form of 128, around the products.
+// The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 29
+// registers per lane, 80 in the four-wave form of 128, around the products.
 template <int D, int NW, int NST>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D, D == 16>::DB;

@@ -235,7 +235,7 @@ struct Fwd2Slots {
   }
 };
 
-// Forward kernel for 16-bit elements with swizzled tiles (D = 32, 64, 128 or 256).
+// Forward kernel for 16-bit elements with swizzled tiles (D = 16, 32, 64, 128 or 256).
 //
 // Head dimension 256 goes through a tile of 64 keys half a tile at a time: one score block and 80 KiB of LDS (Fwd2Slots)
 // leave room for two waves per SIMD, one of which multiplies while the other one is at its exponentials; on whole tiles a

@@ -155,7 +155,7 @@ template <typename P> void set_tile_order(P& p, int rows, int tile) {
   p.period = tiles_of_window(p.T, p.C, p.R, rows, tile);
   p.pdiv = chunk_div(p.period > 0 ? p.period : 1);
 }
-// Short windows, head dimensions 32 and 64: workgroups of two waves (64 rows, tiles of 32) instead of four (128 rows,
+// Short windows, head dimensions 16 to 64: workgroups of two waves (64 rows, tiles of 32) instead of four (128 rows,
 // tiles of 64).  In the large workgroup every wave waits at the barriers of about twice as many tiles as it sees itself,
 // and half as many waves are resident; the small one goes through more rows per row of its own unless the windows begin and
 // end where its rows do.  So it is taken where that costs nothing (chunks divide 32 or are divided by it, and the
