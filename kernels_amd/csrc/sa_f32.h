@@ -363,9 +363,9 @@ struct QueryWindow {
 // Forward.  One wave per 32 queries, tiles of 32 keys in NST stages.  Bound by the matrix pipe: 1.1 PFLOP/s of
 // bfloat16 products.  B=4, H=16, T=4096, chunks of 128, 4 back, us with the float32 instruction -> here: D=128 720 -> 455,
 // D=64 392 -> 220, D=32 200 -> 125, D=16 167 -> 107 (with OwnRows32, whole-row stores and TileOrder 456 -> 432, 223 -> 218, 129 -> 128).
-// The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 29
-// registers per lane, 80 in the four-wave form of 128, around the products.
-template <int D, int NW, int NST>
+// The register limits (four waves per SIMD up to 32, three at 64, two at 128) make D=64 and 128 spill 19 and 31
+// registers per lane, 82 in the four-wave form of 128, around the products.
+template <int D, int NW, int NST, bool BY_LENGTH>
 __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)) void fwd_split_kernel(const FwdParams p) {
   constexpr int TQ = NW * 32, NT = NW * 64, TK = 32, DB = TileGeom<__bf16, D, D == 16>::DB;
   constexpr int TILE = SplitTile<D, TK>::ELEMS;
@@ -380,11 +380,11 @@ __global__ __launch_bounds__(NW * 64, (D <= 32 ? 4 : D == 64 && NW == 4 ? 3 : 2)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int bh, qt, L = p.T;
-  if (p.by_length) tile_coords_by_length<TQ>(blockIdx.x, p.tiles, p.by_length, p.lens, p.lens_stride, p.T, p.H, lane, bh, qt, L);
+  if (BY_LENGTH) tile_coords_by_length<TQ>(blockIdx.x, p.tiles, p.by_length, p.lens, p.lens_stride, p.T, p.H, lane, bh, qt, L);
   else tile_coords(blockIdx.x, gridDim.x, p.tiles, bh, qt);
   const int T_ = p.T;
   const int b = div_by(bh, p.tiles.by_heads), hd = bh - b * p.H;
-  if (p.lens && !p.by_length) {
+  if (p.lens && !BY_LENGTH) {
     L = p.lens[(int64_t)b * p.lens_stride];
     L = L < 0 ? 0 : (L > T_ ? T_ : L);
   }
